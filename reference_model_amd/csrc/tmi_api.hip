@@ -50,6 +50,7 @@ struct tmi_ctx
     uint32_t* flags_dev   = nullptr;    // latched REQUIRE conditions
     uint8_t* pages_dev    = nullptr;    // 256 pages of 64 bytes, page v filled with byte v: what padding reads
     uint32_t* flags_host  = nullptr;    // pinned staging word
+    tmi::DpPartial* dp_partials = nullptr;    // pinned: the DOT_PRODUCT check's partial results, written by the device
     void* workspace       = nullptr;    // scratch for operand re-layout (MATMUL's transposed B)
     size_t workspace_size = 0;
     std::vector<void*> retired;         // outgrown scratch blocks: captured graphs may still name them
@@ -647,13 +648,14 @@ int tmi_ctx_create(tmi_ctx_t** out_ctx, int device)
         return TMI_ERROR;
     }
     if (hipMalloc((void**)&ctx->flags_dev, 256) != hipSuccess ||
-        hipHostMalloc((void**)&ctx->flags_host, 256, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&ctx->flags_host, 256 + kDpCheckBlocks * sizeof(DpPartial), hipHostMallocDefault) != hipSuccess ||
         hipMemset(ctx->flags_dev, 0, 256) != hipSuccess)
     {
         tmi_ctx_destroy(ctx);
         return TMI_ERROR;
     }
     *ctx->flags_host = 0;
+    ctx->dp_partials = reinterpret_cast<DpPartial*>(reinterpret_cast<uint8_t*>(ctx->flags_host) + 256);
     {
         std::string pages(256 * 64, '\0');
         for (int v = 0; v < 256; v++)
@@ -1446,22 +1448,19 @@ int tmi_dot_product_check(tmi_ctx_t* ctx, int32_t out_dtype, int64_t n, const vo
     if (out_dtype != TMI_FP16 && out_dtype != TMI_BF16 && out_dtype != TMI_FP32)
         return fail(ctx, "dot product check: result type must be FP16, BF16 or FP32");
     TMI_HIP(ctx, hipSetDevice(ctx->device));
-    // accumulators: 3 doubles + 1 word in the upper half of the context's 256-byte flag block
-    uint8_t* acc = reinterpret_cast<uint8_t*>(ctx->flags_dev) + 128;
-    TMI_HIP(ctx, hipMemsetAsync(acc, 0, 32, ctx->stream));
     const int32_t abs_bound = 2 * ksb;
-    if (!launch_dp_check(ctx->stream, out_dtype, n, imp_dev, ref_dev, bnd_dev, abs_bound,
-                         reinterpret_cast<double*>(acc), reinterpret_cast<unsigned long long*>(acc + 24)))
+    if (!launch_dp_check(ctx->stream, out_dtype, n, imp_dev, ref_dev, bnd_dev, abs_bound, ctx->dp_partials))
         return fail(ctx, "dot product check: launch failed");
     ctx->last_kernel = "dot_product_check";
-    struct
-    {
-        double v[3];
-        unsigned long long bad;
-    } host;
-    TMI_HIP(ctx, hipMemcpyAsync(&host, acc, 32, hipMemcpyDeviceToHost, ctx->stream));
+    TMI_HIP(ctx, hipGetLastError());
     TMI_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    result->err_sum = host.v[0], result->err_sumsq = host.v[1], result->max_abs_err = host.v[2];
+    DpPartial host{ 0.0, 0.0, 0.0, 0 };
+    for (int i = 0; i < dp_check_blocks(n); i++)
+    {
+        const DpPartial& t = ctx->dp_partials[i];
+        host.sum += t.sum, host.sumsq += t.sumsq, host.worst = t.worst > host.worst ? t.worst : host.worst, host.bad += t.bad;
+    }
+    result->err_sum = host.sum, result->err_sumsq = host.sumsq, result->max_abs_err = host.worst;
     result->failed_elements = (int64_t)host.bad, result->elements = n;
     result->abs_bound = abs_bound, result->variance_bound = 4.0 * 0.4 * ksb;
     // validateDataDP: every element within its bound; for sets 3..5 |sum| <= sqrt(10 * var * T); sumsq <= var * T

@@ -123,16 +123,23 @@ const char* launch_depthwise_direct(hipStream_t st, int32_t in_dtype, int32_t ou
                                     const void* in, const void* w, const void* bias, int32_t in_zp, int32_t w_zp,
                                     const RescaleParams& rp, void* out, uint32_t* flag_word);
 // precise.hip: fp64 precise-mode / bounds-mode passes (abs_mode != 0: sums over absolute values) of CONV2D,
-// DEPTHWISE_CONV2D and MATMUL on fp16 / bf16 / fp32 operands, and the DOT_PRODUCT check as a reduction
-// (results: 3 doubles, counts: 1 word, both zero before the launch).  nullptr for another operand type.
+// DEPTHWISE_CONV2D and MATMUL on fp16 / bf16 / fp32 operands, and the DOT_PRODUCT check as a reduction that leaves one
+// partial result per workgroup (at most kDpCheckBlocks of them) in `partials`.  nullptr for another operand type.
 // abs_max_slot: device scratch of one double; when given together with abs_mode, every input element is replaced by
 // the input tensor's largest magnitude (the bounds pass of an operator whose local_bound attribute is false).
 const char* launch_conv_precise(hipStream_t st, int32_t in_dtype, bool depthwise, const ConvGeom& g, const void* in,
                                 const void* w, const void* bias, int32_t abs_mode, double* abs_max_slot, double* out);
 const char* launch_matmul_precise(hipStream_t st, int32_t in_dtype, int32_t N, int32_t H, int32_t C, int32_t W,
                                   const void* a, const void* b, int32_t abs_mode, double* out);
+struct DpPartial
+{
+    double sum, sumsq, worst;    // of the errors in units of the bound
+    uint64_t bad;                // elements that fail on their own
+};
+constexpr int kDpCheckBlocks = 512;
+int dp_check_blocks(int64_t n);
 const char* launch_dp_check(hipStream_t st, int32_t out_dtype, int64_t n, const void* imp, const double* ref,
-                            const double* bnd, int32_t abs_bound, double* results, unsigned long long* counts);
+                            const double* bnd, int32_t abs_bound, DpPartial* partials);
 
 // pool.hip: AVG_POOL2D (avg) / MAX_POOL2D; nullptr for a dtype without a kernel or 2^32 work items or more.
 const char* launch_pool(hipStream_t st, bool avg, int32_t dtype, int32_t N, int32_t IH, int32_t IW, int32_t C,
