@@ -9,8 +9,9 @@
 //    as a reduction: per element the error in units of the bound, then sum, sum of squares, largest
 //    magnitude and the number of elements that fail on their own.
 //
-// These are checkers for the fast kernels at shapes where a scalar CPU pass takes seconds to minutes; one
-// output element per lane, nothing tiled.
+// These are checkers for the fast kernels at shapes where a scalar CPU pass takes seconds to minutes.  CONV2D and MATMUL run
+// on the ordered tiles of ordered_gemm.hip; the kernels here, one output element per lane, take DEPTHWISE_CONV2D and the
+// shapes those decline (offsets or divisions beyond 32 bits).
 #include "tmi_kernels.h"
 
 namespace tmi
@@ -230,6 +231,8 @@ const char* launch_conv_precise(hipStream_t st, int32_t in_dtype, bool depthwise
         }
         a.input_abs_max = abs_max_slot;
     }
+    if (!depthwise && launch_ordered_conv(st, in_dtype, true, g, in, w, bias, abs_mode != 0, a.input_abs_max, out))
+        return abs_mode ? "conv_bounds_f64" : "conv_precise_f64";
     switch (in_dtype)
     {
         case TMI_FP16: hipLaunchKernelGGL(precise_conv_kernel<_Float16>, dim3(grid_for(a.total)), dim3(256), 0, st, a); break;
@@ -243,6 +246,8 @@ const char* launch_conv_precise(hipStream_t st, int32_t in_dtype, bool depthwise
 const char* launch_matmul_precise(hipStream_t st, int32_t in_dtype, int32_t N, int32_t H, int32_t C, int32_t W,
                                   const void* a, const void* b, int32_t abs_mode, double* out)
 {
+    if (launch_ordered_matmul(st, in_dtype, true, N, H, C, W, a, b, abs_mode != 0, out))
+        return abs_mode ? "matmul_bounds_f64" : "matmul_precise_f64";
     const int64_t total = (int64_t)N * H * W;
     const dim3 grid(grid_for(total)), block(256);
     const int eb      = in_dtype == TMI_FP32 ? 4 : 2;

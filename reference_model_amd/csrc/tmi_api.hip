@@ -608,6 +608,11 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
     }
     if (!name && ctx->kernel_choice >= 2)
         return fail(ctx, "%s: no MFMA / vector kernel is eligible for this shape", op);
+    // FP32 sums keep the reference's order: the tiles of ordered_gemm.hip, under the label of the one-result-per-lane kernel,
+    // whose results they are bit for bit
+    if (!name && !depthwise && ctx->kernel_choice == 0 && d->in_dtype == TMI_FP32 &&
+        launch_ordered_conv(ctx->stream, TMI_FP32, false, g, in, w, bias, false, nullptr, out))
+        name = "conv2d_direct_f32";
     if (!name && depthwise)
         name = launch_depthwise_direct(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                        ctx->flags_dev);
@@ -1364,6 +1369,9 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
     }
     if (!name && ctx->kernel_choice >= 2)
         return fail(ctx, "OpMatMul: no MFMA kernel is eligible for this shape");
+    if (!name && ctx->kernel_choice == 0 && in_dtype == TMI_FP32 &&
+        launch_ordered_matmul(ctx->stream, TMI_FP32, false, N, H, C, W, a_dev, b_dev, false, out_dev))
+        name = "matmul_direct_f32";
     if (!name)
         name = launch_matmul_direct(ctx->stream, in_dtype, N, H, C, W, a_dev, b_dev, a_zp, b_zp, out_dev);
     return after_launch(ctx, name);
