@@ -210,6 +210,7 @@ __global__ __launch_bounds__(256) void conv_i16_direct_kernel(ConvGeom g, const 
 {
     const int64_t total  = (int64_t)g.N * g.OH * g.OW * g.OC;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const bool vec       = g.IC % 8 == 0 && (((uintptr_t)in | (uintptr_t)w) & 15) == 0;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride)
     {
         const int oc = (int)(idx % g.OC);
@@ -238,7 +239,19 @@ __global__ __launch_bounds__(256) void conv_i16_direct_kernel(ConvGeom g, const 
                 else
                 {
                     const int64_t wb = (((int64_t)oc * g.KH + ky) * g.KW + kx) * g.IC;
-                    for (int ic = 0; ic < g.IC; ic++)
+                    int ic           = 0;
+                    if (vec)    // eight channels a step: 16 bytes of the input, 8 of the weights
+                        for (; ic < g.IC; ic += 8)
+                        {
+                            alignas(16) int16_t xv[8];
+                            alignas(8) int8_t wv[8];
+                            *reinterpret_cast<int4*>(xv) = *reinterpret_cast<const int4*>(in + ib + ic);
+                            *reinterpret_cast<int2*>(wv) = *reinterpret_cast<const int2*>(w + wb + ic);
+#pragma unroll
+                            for (int e = 0; e < 8; e++)
+                                acc += (int64_t)((int32_t)xv[e] * ((int32_t)wv[e] - w_zp));
+                        }
+                    for (; ic < g.IC; ic++)
                         acc += (int64_t)in[ib + ic] * (int64_t)((int32_t)w[wb + ic] - w_zp);
                 }
             }

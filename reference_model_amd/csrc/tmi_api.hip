@@ -426,11 +426,28 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         ctx->last_kernel = "empty";
         return TMI_VALID;
     }
+    auto in_scratch = [&](const void* p) {
+        return ctx->workspace && (const uint8_t*)p >= (const uint8_t*)ctx->workspace &&
+               (const uint8_t*)p < (const uint8_t*)ctx->workspace + ctx->workspace_size;
+    };
     if (d->in_dtype == TMI_INT16)
     {
         if (rp.enabled)
             return fail(ctx, "%s: the fused rescale needs an INT8 convolution", op);
-        return after_launch(ctx, launch_conv_i16_direct(ctx->stream, depthwise, g, in, w, bias, w_zp, out));
+        // Below 2^17 multiply-adds one result per lane (us direct / matrix cores: [1,8,8,16]->8 3x3 6.0 / 4.5, [3,5,5,33]->17 1x1 4.8 /
+        // 6.1, whose channels must be padded by a launch of its own, [1,28,28,8]->8 1x1 3.0 / 6.5; the other way [1,14,14,16]->16 3x3,
+        // 0.45 M, 6.2 / 4.6).
+        const bool tiny   = total * g.KH * g.KW * g.IC < (1 << 17);
+        const size_t need = depthwise || tiny || ctx->kernel_choice == 1 ? 0 : conv_i16_mfma_scratch_bytes(g, w_zp);
+        if (need && (need == 1 || (own_scratch && !in_scratch(in) && !in_scratch(w) && !in_scratch(out) && !in_scratch(bias))))
+        {
+            if (need > 1 && (rc = ensure_workspace(ctx, need)) != TMI_VALID)
+                return rc;
+            name = launch_conv_i16_mfma(ctx->stream, g, in, w, bias, out, ctx->workspace);
+        }
+        if (!name)
+            name = launch_conv_i16_direct(ctx->stream, depthwise, g, in, w, bias, w_zp, out);
+        return after_launch(ctx, name);
     }
     // Small depthwise layers: the vector kernel (a lane per four channels of a pixel, no LDS, no barrier) costs 3.15 us plus
     // 4.4 us per million results, the matrix-core kernel 3.3 us plus 3.7 ns per channel (its per-channel tables) and next
@@ -580,10 +597,6 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         if (!name && own_scratch && (ctx->kernel_choice == 5 || ctx->kernel_choice == 0))
         {
             const size_t need = conv2d_stem_scratch_bytes(d->in_dtype, out_dtype, g, w_zp, rp);
-            auto in_scratch   = [&](const void* p) {
-                return ctx->workspace && (const uint8_t*)p >= (const uint8_t*)ctx->workspace &&
-                       (const uint8_t*)p < (const uint8_t*)ctx->workspace + ctx->workspace_size;
-            };
             if (need && !in_scratch(in) && !in_scratch(w) && !in_scratch(out) && !in_scratch(bias))
             {
                 rc = ensure_workspace(ctx, need);

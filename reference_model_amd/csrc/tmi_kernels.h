@@ -233,6 +233,10 @@ const char* launch_conv3d_operands(hipStream_t st, int32_t row_bytes, int32_t OC
 const char* launch_depthwise_vec(hipStream_t st, int32_t in_dtype, int32_t out_dtype, const ConvGeom& g,
                                  const void* in, const void* w, const void* bias, int32_t in_zp, int32_t w_zp,
                                  const RescaleParams& rp, void* out, uint32_t* flag_word);
+// conv_i16.hip: INT16 x INT8 -> INT48 CONV2D on the int8 matrix cores.  conv_i16_mfma_scratch_bytes: 0 for a layer the form
+// does not take, 1 for one it reads in place, else the scratch its channel-padded operands need.
+size_t conv_i16_mfma_scratch_bytes(const ConvGeom& g, int32_t w_zp);
+const char* launch_conv_i16_mfma(hipStream_t st, const ConvGeom& g, const void* in, const void* w, const void* bias, void* out, void* scratch);
 // INT16 x INT8 -> INT48 CONV2D / DEPTHWISE_CONV2D and INT16 x INT16 -> INT48 MATMUL (int64 bias and results)
 const char* launch_conv_i16_direct(hipStream_t st, bool depthwise, const ConvGeom& g, const void* in, const void* w,
                                    const void* bias, int32_t w_zp, void* out);
