@@ -219,7 +219,7 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
             const int k    = unit / (RB / 16);
             const int pc   = (unit % (RB / 16)) ^ km_swizzle(k);
             int col        = oc0 * EB + pc * 16;
-            col            = col < a.N * EB - 16 ? col : a.N * EB - 16;    // pieces past the row end: never used
+            col            = col < a.ldw - 16 ? col : a.ldw - 16;    // pieces past the row end: never used
             voff[j]        = (uint32_t)k * (uint32_t)a.ldw + (uint32_t)col;
             gstep[j]       = (uint32_t)(64 / EB) * (uint32_t)a.ldw;
         }
@@ -1443,7 +1443,7 @@ const char* launch_gemm_mfma(hipStream_t st, int32_t in_dtype, int32_t out_dtype
     if (M < 128 || g.OC < 64 || M * kb >= (int64_t(1) << 32) || (int64_t)g.OC * kb >= (int64_t(1) << 32))
         return nullptr;
     // K-major weights: whole 16-byte pieces per K row
-    if (w_kmajor_stride && ((w_kmajor_stride & 15) || w_kmajor_stride != (int64_t)g.OC * eb))
+    if (w_kmajor_stride && ((w_kmajor_stride & 15) || w_kmajor_stride < (int64_t)g.OC * eb))
         return nullptr;
     // rows are multiples of 64 bytes, so 16-byte aligned bases keep every operand chunk aligned; the 16-byte
     // stores are only used when OC is a multiple of 16, which keeps every output row and batch aligned too

@@ -1,0 +1,371 @@
+// MATMUL int8 -> int32 and fp16 / bf16 -> fp32 of any size and alignment, for products the GEMM kernel does not read in place
+// or that offer it too few tiles: rows that are no multiple of 64 bytes, columns that are no whole 16-byte pieces, few rows.
+//
+// A tile is 32 rows x 64 columns and SPLIT waves share its K, a block of 64 bytes of K (two matrix instructions deep) at a
+// time, dealt round-robin.  Nothing is shared between waves before the end: a wave takes its part of the first operand
+// straight into the registers the matrix instruction reads (lane = row lane % 32, 16 bytes of K of half lane / 32), and moves
+// its part of the second operand, [K][W] as it lies, through a piece of LDS of its own, from which the transposing reads
+// (ds_read_b64_tr_b16 / _b8) return K-contiguous fragments; the next block's loads are in flight meanwhile.  Loads are 16 bytes
+// from any address (gfx950 takes global addresses of any alignment); only the end of a row of the first operand and the end of
+// the tensor go element by element.  The partial tiles meet in LDS.  Rows of the tile are rows of the result, so that 32
+// lanes store 128 neighbouring bytes.
+//
+// What bounds it: the first operand's fragments, a line per lane and load, for products of many tiles (fp16 at 130 TFLOP/s), the
+// chain of a wave's blocks otherwise.  us transposed copy + patch or GEMM kernel -> here: fp16 96 x [197,64]x[64,197] 33.6 -> 9.7
+// (34 MB with the next: 2.4 TB/s), 96 x [197,197]x[197,64] 45.3 -> 9.1, [1,4096]x[4096,4096] 49.7 -> 11.6, [1,3731]x[3731,144] 507 -> 8.8,
+// int8 3 x [1000,999]x[999,1001] 191 -> 30, [64,512]x[512,512] 11.5 -> 4.8.
+#include <type_traits>
+
+#include "tmi_mfma.h"
+
+namespace tmi
+{
+
+struct RaggedArgs
+{
+    const uint8_t* a;
+    const uint8_t* b;
+    uint8_t* out;    // 4-byte results
+    int64_t a_total, b_total;    // bytes of the whole operands
+    int32_t H, C, W;
+    int32_t za, zb;
+    int32_t tiles;    // of all batches
+    FastDiv per_batch, tiles_w;
+};
+
+struct __attribute__((packed)) Bytes16
+{
+    v4i v;
+};
+__device__ __forceinline__ v4i load16(const uint8_t* p)
+{
+    return reinterpret_cast<const Bytes16*>(p)->v;
+}
+
+// the first n bytes at p (n may be 0 or negative), then zeros
+template <int EB>
+__device__ __forceinline__ v4i load_front(const uint8_t* p, int n)
+{
+    uint32_t d[4] = { 0, 0, 0, 0 };
+#pragma unroll
+    for (int i = 0; i < 16; i += EB)
+        if (i < n)
+        {
+            const uint32_t e = EB == 1 ? *(p + i) : *reinterpret_cast<const uint16_t*>(p + i);
+            d[i >> 2] |= e << (8 * (i & 3));
+        }
+    return v4i{ (int)d[0], (int)d[1], (int)d[2], (int)d[3] };
+}
+
+template <typename T, int SPLIT>
+__global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_kernel(RaggedArgs p)
+{
+    using M             = Mma<T>;
+    using acc_t         = typename M::acc_t;
+    using word          = std::conditional_t<M::is_int, int32_t, float>;
+    constexpr int EB    = (int)sizeof(T);
+    constexpr int KB    = 64 / EB;              // k of a block
+    constexpr int RB    = 64 * EB;              // bytes of a k row of the tile
+    constexpr int LD    = RB + (EB == 2 ? 64 : 32);    // the 4 (8) k rows x 64 (32) bytes of a transposing read touch every bank once
+    constexpr int CPR   = RB / 16;              // 16-byte pieces of a k row
+    constexpr int NL    = KB * CPR / 64;        // loads of the second operand per lane and block
+    constexpr int kWaves = SPLIT > 4 ? SPLIT : 4;
+    constexpr int kWaveLds = KB * LD > 8192 && SPLIT > 1 ? KB * LD : (SPLIT > 1 ? 8192 : KB * LD);
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r32 = lane & 31, half = lane >> 5;
+    const uint32_t tile = (blockIdx.x * kWaves + wave) / SPLIT;
+    if (SPLIT < kWaves && SPLIT == 1 && tile >= (uint32_t)p.tiles)
+        return;
+    const bool live      = tile < (uint32_t)p.tiles;
+    const uint32_t t     = live ? tile : 0;
+    const uint32_t batch = fdiv(t, p.per_batch), in_batch = t - batch * p.per_batch.d, th = fdiv(in_batch, p.tiles_w);
+    const int h0 = (int)th * 32, w0 = (int)(in_batch - th * p.tiles_w.d) * 64;
+    uint8_t* mine = lds + wave * kWaveLds;
+
+    const int row_bytes  = p.C * EB;
+    const int h          = h0 + r32 < p.H ? h0 + r32 : p.H - 1;
+    const uint8_t* arow  = p.a + ((int64_t)batch * p.H + h) * row_bytes + 16 * half;
+    // (16 bytes from a row that is not the tensor's last may run into the next row)
+    const int64_t pitch  = (int64_t)p.W * EB;
+    const int64_t b_off  = (int64_t)batch * p.C * pitch + (int64_t)w0 * EB + (lane & (CPR - 1)) * 16;
+    const int krow       = lane / CPR;                       // k row of the lane's first load
+    const int blocks     = (p.C + KB - 1) / KB;
+    const bool col_ok    = w0 + (lane & (CPR - 1)) * (16 / EB) < p.W;
+
+    v4i av[2], bv[NL];
+    auto request = [&](int blk) {
+        const int k0 = blk * KB;
+        // the first operand: two pieces of 32 bytes of K, this lane's 16 of each
+        if (k0 + KB <= p.C)
+        {
+            av[0] = load16(arow + k0 * EB), av[1] = load16(arow + k0 * EB + 32);
+        }
+        else
+        {
+            const int left = row_bytes - k0 * EB - 16 * half;
+            av[0] = load_front<EB>(arow + k0 * EB, left), av[1] = load_front<EB>(arow + k0 * EB + 32, left - 32);
+        }
+        const uint8_t* src = p.b + b_off + (k0 + krow) * pitch;
+        if (k0 + KB <= p.C && b_off - (lane & (CPR - 1)) * 16 + (k0 + KB - 1) * pitch + RB <= p.b_total)
+        {
+#pragma unroll
+            for (int j = 0; j < NL; j++)
+                bv[j] = load16(src + j * (64 / CPR) * pitch);
+        }
+        else
+        {
+#pragma unroll
+            for (int j = 0; j < NL; j++)
+            {
+                const int k = k0 + krow + j * (64 / CPR);
+                const int64_t at = b_off + k * pitch;
+                bv[j] = v4i{ 0, 0, 0, 0 };
+                if (k < p.C && col_ok)
+                    bv[j] = at + 16 <= p.b_total ? load16(p.b + at) : load_front<EB>(p.b + at, (int)(p.b_total - at));
+            }
+        }
+    };
+
+    acc_t acc[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            acc[c][i] = 0;
+    int sum_a = 0, sum_b[2] = { 0, 0 };    // of the lane's row and columns (int8)
+    const bool sums = M::is_int && (p.za | p.zb) != 0;
+
+    const int first = wave % SPLIT;
+    // source of a transposing read: k row sl / 4 of four (sl / 2 of eight), 8 bytes of columns; see the GEMM kernel
+    const int sl = lane & 15, cblk = (lane >> 4) & 1;
+    const int tr = EB == 2 ? (8 * half + (sl >> 2)) * LD + (16 * cblk + 4 * (sl & 3)) * 2 : (16 * half + (sl >> 1)) * LD + 16 * cblk + 8 * (sl & 1);
+    if (live && first < blocks)
+        request(first);
+    for (int blk = first; live && blk < blocks; blk += SPLIT)
+    {
+#pragma unroll
+        for (int j = 0; j < NL; j++)
+            *reinterpret_cast<v4i*>(mine + (krow + j * (64 / CPR)) * LD + (lane & (CPR - 1)) * 16) = bv[j];
+        const v4i a0 = av[0], a1 = av[1];
+        __builtin_amdgcn_wave_barrier();
+        if (blk + SPLIT < blocks)
+            request(blk + SPLIT);
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+        {
+            const v4i a = s ? a1 : a0;
+            if (sums)
+                sum_a += dot4_ones(a);
+#pragma unroll
+            for (int c = 0; c < 2; c++)
+            {
+                v4i b;
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+                {
+                    const uint8_t* src = mine + tr + (KB / 2 * s + KB / 8 * r) * LD + 32 * c * EB;
+                    v2i part;
+                    if constexpr (EB == 2)
+                        part = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)src));
+                    else
+                        part = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)src);
+                    b[2 * r] = part.x, b[2 * r + 1] = part.y;
+                }
+                if (sums)
+                    sum_b[c] += dot4_ones(b);
+                acc[c] = M::mma(a, b, acc[c]);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (sums)
+    {
+        // each share brings its own part of the correction
+        sum_a += __shfl_xor(sum_a, 32);
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+        {
+            const int col = p.za * (sum_b[c] + __shfl_xor(sum_b[c], 32)) - (first == 0 ? p.C * p.za * p.zb : 0);
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                acc[c][i] -= (word)(col + p.zb * __shfl(sum_a, 8 * (i >> 2) + 4 * half + (i & 3)));
+        }
+    }
+    word* out   = reinterpret_cast<word*>(p.out) + (int64_t)batch * p.H * p.W;
+    auto store  = [&](int c, int i, word v) {
+        const int r = h0 + 8 * (i >> 2) + 4 * half + (i & 3), col = w0 + 32 * c + r32;
+        if (r < p.H && col < p.W)
+            out[(int64_t)r * p.W + col] = v;
+    };
+    if constexpr (SPLIT == 1)
+    {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                store(c, i, acc[c][i]);
+    }
+    else
+    {
+        // a wave's partial tile in its own 8 KB (its reads of the second operand are done), then 1 / SPLIT of the sums each
+        word* part = reinterpret_cast<word*>(mine);
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                part[(16 * c + i) * 64 + lane] = acc[c][i];
+        __syncthreads();
+        if (!live)
+            return;
+        const uint8_t* base = lds + wave / SPLIT * SPLIT * kWaveLds;
+        constexpr int kEach = 32 / SPLIT;
+#pragma unroll
+        for (int e = 0; e < kEach; e++)
+        {
+            const int j = first * kEach + e;
+            word v      = reinterpret_cast<const word*>(base)[j * 64 + lane];
+#pragma unroll
+            for (int s = 1; s < SPLIT; s++)
+                v += reinterpret_cast<const word*>(base + s * kWaveLds)[j * 64 + lane];
+            store(j >> 4, j & 15, v);
+        }
+    }
+}
+
+// Aligned copies of both operands for the GEMM kernel, in one launch: rows of the first become CP elements (a multiple of 64 bytes), the second
+// [N][C][W] becomes [N][CP][ldw bytes]; what is added holds the zero point, so that it contributes nothing.
+struct PadArgs
+{
+    const uint8_t* a;
+    const uint8_t* b;
+    uint8_t* ap;
+    uint8_t* bp;
+    int64_t units_a, units_b;    // 16-byte units of the copies (units_a 0: the first operand is read in place)
+    int32_t row_a, row_b;        // bytes of a row of each operand
+    int32_t C;
+    uint32_t fill_a, fill_b;     // zero points, replicated
+    FastDiv ua, ub, cp;          // units per padded row, padded k rows per batch
+};
+
+template <int EB>
+__global__ __launch_bounds__(256) void pad_operands_kernel(PadArgs p)
+{
+    for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < p.units_a + p.units_b; u += (int64_t)gridDim.x * 256)
+    {
+        const bool is_b   = u >= p.units_a;
+        const int64_t v   = is_b ? u - p.units_a : u;
+        const uint32_t d  = is_b ? p.ub.d : p.ua.d;
+        const int64_t row = v / d;
+        const int at      = (int)(v - row * d) * 16, bytes = is_b ? p.row_b : p.row_a;
+        const uint32_t fill = is_b ? p.fill_b : p.fill_a;
+        int64_t src_row   = row;
+        int left          = bytes - at;
+        if (is_b)
+        {
+            const int64_t n = row / p.cp.d;
+            const int k     = (int)(row - n * p.cp.d);
+            src_row         = n * p.C + k;
+            left            = k < p.C ? left : 0;
+        }
+        v4i q = { (int)fill, (int)fill, (int)fill, (int)fill };
+        if (left >= 16)
+            q = load16((is_b ? p.b : p.a) + src_row * bytes + at);
+        else if (left > 0)
+        {
+            q = load_front<EB>((is_b ? p.b : p.a) + src_row * bytes + at, left);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+            {
+                const int keep      = left - 4 * i;    // bytes of the word that are the operand's
+                const uint32_t mask = keep >= 4 ? ~0u : (keep <= 0 ? 0u : (1u << (8 * keep)) - 1u);
+                q[i]                = (int)(((uint32_t)q[i] & mask) | (fill & ~mask));
+            }
+        }
+        *reinterpret_cast<v4i*>((is_b ? p.bp : p.ap) + v * 16) = q;
+    }
+}
+
+// geometry of those copies; pad_a false: the first operand stays where it is
+void matmul_padded_sizes(int32_t eb, int32_t N, int32_t H, int32_t C, int32_t W, MatmulPad& m)
+{
+    m.pad_a   = (int64_t)C * eb % 64 != 0;
+    m.CP      = (int32_t)(((int64_t)C * eb + 63) / 64 * 64 / eb);
+    m.ldw     = ((int64_t)W * eb + 15) / 16 * 16;
+    m.a_bytes = m.pad_a ? (size_t)N * H * m.CP * eb : 0;
+    m.b_bytes = (size_t)N * m.CP * m.ldw;
+}
+
+bool launch_matmul_pad(hipStream_t st, int32_t eb, int32_t N, int32_t H, int32_t C, int32_t W, const MatmulPad& m, const void* a, const void* b,
+                       int32_t a_zp, int32_t b_zp, void* scratch)
+{
+    PadArgs p{};
+    p.a = (const uint8_t*)a, p.b = (const uint8_t*)b, p.ap = (uint8_t*)scratch, p.bp = (uint8_t*)scratch + m.a_bytes;
+    p.units_a = (int64_t)(m.a_bytes / 16), p.units_b = (int64_t)(m.b_bytes / 16);
+    p.row_a = C * eb, p.row_b = W * eb, p.C = C;
+    p.fill_a = (uint32_t)(a_zp & 255) * 0x01010101u, p.fill_b = (uint32_t)(b_zp & 255) * 0x01010101u;
+    p.ua = make_fastdiv((uint32_t)(m.CP * eb / 16)), p.ub = make_fastdiv((uint32_t)(m.ldw / 16)), p.cp = make_fastdiv((uint32_t)m.CP);
+    const int64_t blocks = (p.units_a + p.units_b + 255) / 256;
+    const dim3 grid((unsigned)(blocks > 8192 ? 8192 : blocks));
+    if (eb == 1)
+        hipLaunchKernelGGL(pad_operands_kernel<1>, grid, dim3(256), 0, st, p);
+    else
+        hipLaunchKernelGGL(pad_operands_kernel<2>, grid, dim3(256), 0, st, p);
+    return true;
+}
+
+template <typename T, int SPLIT>
+static bool launch_split(hipStream_t st, const RaggedArgs& p)
+{
+    constexpr int EB = (int)sizeof(T), kWaves = SPLIT > 4 ? SPLIT : 4, kBlock = 64 / EB * (64 * EB + (EB == 2 ? 64 : 32));
+    constexpr size_t lds_bytes = (size_t)kWaves * (SPLIT > 1 ? (kBlock > 8192 ? kBlock : 8192) : kBlock);
+    auto kern                  = matmul_ragged_kernel<T, SPLIT>;
+    static LdsLimit granted{};
+    if (lds_bytes > 65536 && !ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, granted))
+        return false;
+    const int64_t waves = (int64_t)p.tiles * SPLIT;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((waves + kWaves - 1) / kWaves)), dim3(64 * kWaves), lds_bytes, st, p);
+    return true;
+}
+
+template <typename T>
+static bool launch_ragged(hipStream_t st, const RaggedArgs& p)
+{
+    const int blocks = (p.C * (int)sizeof(T) + 63) / 64;
+    // K over as many waves as give the chip about two thousand, each with a block of its own at least
+    int split = 1;
+    while (split < 16 && (int64_t)p.tiles * split < 2048 && split * 2 <= blocks)
+        split *= 2;
+    switch (split)
+    {
+        case 1: return launch_split<T, 1>(st, p);
+        case 2: return launch_split<T, 2>(st, p);
+        case 4: return launch_split<T, 4>(st, p);
+        case 8: return launch_split<T, 8>(st, p);
+        default: return launch_split<T, 16>(st, p);
+    }
+}
+
+const char* launch_matmul_ragged(hipStream_t st, int32_t in_dtype, int32_t N, int32_t H, int32_t C, int32_t W, const void* a, const void* b,
+                                 int32_t a_zp, int32_t b_zp, void* out)
+{
+    const int eb        = in_dtype == TMI_INT8 ? 1 : 2;
+    const int64_t tw = ((int64_t)W + 63) / 64, per = ((int64_t)H + 31) / 32 * tw, tiles = per * N;
+    if (C < 1 || tiles > INT32_MAX / 16 || (int64_t)C * eb > INT32_MAX / 2 || !fastdiv_exact_up_to((uint64_t)tiles, (uint32_t)per) ||
+        !fastdiv_exact_up_to((uint64_t)per, (uint32_t)tw) || (eb == 2 && (((uintptr_t)a | (uintptr_t)b) & 1)))
+        return nullptr;
+    RaggedArgs p{};
+    p.a = (const uint8_t*)a, p.b = (const uint8_t*)b, p.out = (uint8_t*)out;
+    p.a_total = (int64_t)N * H * C * eb, p.b_total = (int64_t)N * C * W * eb;
+    p.H = H, p.C = C, p.W = W, p.za = a_zp, p.zb = b_zp, p.tiles = (int32_t)tiles;
+    p.per_batch = make_fastdiv((uint32_t)per), p.tiles_w = make_fastdiv((uint32_t)tw);
+    switch (in_dtype)
+    {
+        case TMI_INT8: return launch_ragged<int8_t>(st, p) ? "matmul_ragged_i8" : nullptr;
+        case TMI_FP16: return launch_ragged<_Float16>(st, p) ? "matmul_ragged_f16" : nullptr;
+        case TMI_BF16: return launch_ragged<bf16_t>(st, p) ? "matmul_ragged_bf16" : nullptr;
+        default: return nullptr;
+    }
+}
+
+}    // namespace tmi

@@ -1338,11 +1338,9 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
     if (ctx->kernel_choice != 1 && C > 0 && in_dtype != TMI_FP32)
     {
         // MFMA paths: one "image" per batch, pixels = rows of A, output channels = columns of B, 1x1 taps,
-        // per-image weights.  The bias operand is the permanently zero word kept after the flags.  The GEMM
-        // kernel takes B as it lies in memory ([C][W], transposed on its way out of LDS); what it does not
-        // take that way (rows of B that are not whole 16-byte pieces) is first made K-contiguous ([N,C,W] ->
-        // [N,W,C]) in the context's scratch buffer and offered to the GEMM kernel again, then to the
-        // implicit-GEMM kernel.
+        // per-image weights.  The bias operand is the permanently zero word kept after the flags.  The GEMM and the
+        // split kernel take B as it lies in memory ([C][W], transposed on its way out of LDS).  The patch kernel, and the
+        // GEMM kernel where a test asks for it, want B K-contiguous ([N,C,W] -> [N,W,C] in the context's scratch buffer).
         const int eb = in_dtype == TMI_INT8 ? 1 : 2;
         ConvGeom g{};
         g.N = N, g.IH = H, g.IW = 1, g.IC = C, g.OC = W, g.KH = 1, g.KW = 1, g.OH = H, g.OW = 1;
@@ -1350,11 +1348,50 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
         g.bias_len = 1, g.M = 1;
         RescaleParams none{};
         const int32_t out_dtype = in_dtype == TMI_INT8 ? TMI_INT32 : TMI_FP32;
+        const char* const label[3] = { in_dtype == TMI_INT8 ? "matmul_gemm_i8" : (in_dtype == TMI_FP16 ? "matmul_gemm_f16" : "matmul_gemm_bf16"),
+                                       in_dtype == TMI_INT8 ? "matmul_tgemm_i8" : (in_dtype == TMI_FP16 ? "matmul_tgemm_f16" : "matmul_tgemm_bf16"),
+                                       in_dtype == TMI_INT8 ? "matmul_mfma_i8" : (in_dtype == TMI_FP16 ? "matmul_mfma_f16" : "matmul_mfma_bf16") };
+        // What the GEMM kernel takes in place: rows of whole 64-byte pieces against rows of whole 16-byte pieces, from four tiles
+        // of 128 x 128 on.  Its tiles walk K one after the other, so where there are few of them and K is deep the kernel that
+        // splits K over waves leads: us GEMM / split, int8 [1,256,2048]x[..,1024] (16 tiles) 13.6 / 8.4, fp16 15.1 / 9.6,
+        // 2 x [256,4096]x[4096,256] (8) 25.0 / 14.5; the other way 64 x [128,128]x[128,128] 5.5 / 5.8, 4 x [128,64]x[64,128] 4.7 / 5.5.
+        const int64_t tiles128 = (((int64_t)H + 127) / 128) * (((int64_t)W + 127) / 128) * N;
+        const bool rows_whole  = (int64_t)C * eb % 64 == 0 && H >= 128 && W >= 64 && tiles128 >= 4;
+        const bool in_place    = rows_whole && (int64_t)W * eb % 16 == 0;
+        const bool few_deep    = tiles128 <= 32 && (int64_t)C * eb >= 1024;
+        // Products it cannot read in place: the split kernel, which reads anything, up to 4 G operations; beyond, aligned copies
+        // of the operands and the GEMM kernel.  us split / copies: int8 4 x [700,701]x[701,703] (2.8 G) 20.8 / 21.6, fp16 27.6 / 29.9,
+        // 4 x [1000,1001]x[1001,1003] (8 G) 37.6 / 32.9, fp16 56.9 / 42.9, [1000,..] (2 G) 14.7 / 19.7, 19.3 / 26.9, [2000,2001]x[2001,2003] (16 G)
+        // 65.4 / 38.8, 121 / 52.9.
+        const bool large = H >= 128 && W >= 64 && 2 * total * C > 4000000000ll;
+        if (ctx->kernel_choice == 0 && (in_place ? few_deep : !large))
+        {
+            name = launch_matmul_ragged(ctx->stream, in_dtype, N, H, C, W, a_dev, b_dev, a_zp, b_zp, out_dev);
+            // (products whose second operand alone has ragged rows keep the label they are known by)
+            if (name)
+                return after_launch(ctx, rows_whole && !in_place ? label[1] : name);
+        }
         if (ctx->kernel_choice != 2)
             name = launch_gemm_mfma(ctx->stream, in_dtype, out_dtype, g, a_dev, b_dev, ctx->flags_dev + 16, a_zp, b_zp,
                                     none, out_dev, (int64_t)W * C * eb, (int64_t)W * eb);
-        const bool direct = name != nullptr;    // B read as it lies, no transposed copy
-        if (!name)
+        if (name)
+            return after_launch(ctx, label[0]);
+        if (ctx->kernel_choice == 0 && large)
+        {
+            MatmulPad m;
+            matmul_padded_sizes(eb, N, H, C, W, m);
+            int rc = ensure_workspace(ctx, m.a_bytes + m.b_bytes);
+            if (rc != TMI_VALID)
+                return rc;
+            if (!launch_matmul_pad(ctx->stream, eb, N, H, C, W, m, a_dev, b_dev, a_zp, b_zp, ctx->workspace))
+                return fail(ctx, "OpMatMul: operand copy launch failed");
+            ConvGeom q = g;
+            q.IC       = m.CP;
+            name       = launch_gemm_mfma(ctx->stream, in_dtype, out_dtype, q, m.pad_a ? ctx->workspace : a_dev, (uint8_t*)ctx->workspace + m.a_bytes,
+                                          ctx->flags_dev + 16, a_zp, b_zp, none, out_dev, (int64_t)m.CP * m.ldw, m.ldw);
+            if (name)
+                return after_launch(ctx, label[1]);
+        }
         {
             const size_t bytes = (size_t)N * C * W * eb;
             int rc             = ensure_workspace(ctx, bytes);
@@ -1366,18 +1403,14 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
                 name = launch_gemm_mfma(ctx->stream, in_dtype, out_dtype, g, a_dev, ctx->workspace, ctx->flags_dev + 16,
                                         a_zp, b_zp, none, out_dev, (int64_t)W * C * eb);
         }
-        if (name && direct)
-            name = in_dtype == TMI_INT8 ? "matmul_gemm_i8" : (in_dtype == TMI_FP16 ? "matmul_gemm_f16" : "matmul_gemm_bf16");
-        else if (name)
-            name = in_dtype == TMI_INT8 ? "matmul_tgemm_i8"
-                                        : (in_dtype == TMI_FP16 ? "matmul_tgemm_f16" : "matmul_tgemm_bf16");
+        if (name)
+            name = label[1];
         else if (ctx->kernel_choice != 3)
         {
             name = launch_conv2d_mfma(ctx->stream, in_dtype, out_dtype, g, a_dev, ctx->workspace, ctx->flags_dev + 16,
                                       a_zp, b_zp, none, out_dev, ctx->flags_dev, (int64_t)W * C * eb);
             if (name)
-                name = in_dtype == TMI_INT8 ? "matmul_mfma_i8"
-                                            : (in_dtype == TMI_FP16 ? "matmul_mfma_f16" : "matmul_mfma_bf16");
+                name = label[2];
         }
     }
     if (!name && ctx->kernel_choice >= 2)

@@ -233,6 +233,22 @@ const char* launch_conv3d_operands(hipStream_t st, int32_t row_bytes, int32_t OC
 const char* launch_depthwise_vec(hipStream_t st, int32_t in_dtype, int32_t out_dtype, const ConvGeom& g,
                                  const void* in, const void* w, const void* bias, int32_t in_zp, int32_t w_zp,
                                  const RescaleParams& rp, void* out, uint32_t* flag_word);
+// matmul_ragged.hip: MATMUL int8 -> int32, fp16 / bf16 -> fp32 of any size and alignment, tiles of 32 x 64 results with K
+// split over waves; both operands read where they lie
+const char* launch_matmul_ragged(hipStream_t st, int32_t in_dtype, int32_t N, int32_t H, int32_t C, int32_t W, const void* a, const void* b,
+                                 int32_t a_zp, int32_t b_zp, void* out);
+// aligned copies of MATMUL's operands for the GEMM kernel ([N][H][CP] unless the first operand is read in place, then
+// [N][CP][ldw bytes], one behind the other in `scratch`)
+struct MatmulPad
+{
+    bool pad_a;
+    int32_t CP;
+    int64_t ldw;
+    size_t a_bytes, b_bytes;
+};
+void matmul_padded_sizes(int32_t eb, int32_t N, int32_t H, int32_t C, int32_t W, MatmulPad& m);
+bool launch_matmul_pad(hipStream_t st, int32_t eb, int32_t N, int32_t H, int32_t C, int32_t W, const MatmulPad& m, const void* a, const void* b,
+                       int32_t a_zp, int32_t b_zp, void* scratch);
 // conv_i16.hip: INT16 x INT8 -> INT48 CONV2D on the int8 matrix cores.  conv_i16_mfma_scratch_bytes: 0 for a layer the form
 // does not take, 1 for one it reads in place, else the scratch its channel-padded operands need.
 size_t conv_i16_mfma_scratch_bytes(const ConvGeom& g, int32_t w_zp);
