@@ -312,7 +312,9 @@ __global__ __launch_bounds__(512) void conv2d_patch_kernel(PatchArgs a)
     // past OC read row 0 of the block (valid memory) and are zeroed when written.
     const bool w_contig = !MULTI && VEC && a.rounds == 1 && row_bytes == blk_bytes;
     const int w_full    = n_pairs / LPR;    // slots in which every lane has a chunk
-    const uint8_t* w_lane_src = w_n + (w_oc_ok ? w_src_row : (uint32_t)oc0 * (uint32_t)(taps * row_bytes)) + w_part * 16;
+    // (a row of fewer chunks than lanes: the lanes past its end read its first chunk)
+    const uint8_t* w_lane_src = w_n + (w_oc_ok ? w_src_row : (uint32_t)oc0 * (uint32_t)(taps * row_bytes)) +
+                                (w_part < n_pairs ? w_part : 0) * 16;
     const int w_lane_dst      = w_row * a.wstride + w_part * 16;
     auto issue_weights_contig = [&]() {
 #pragma unroll
