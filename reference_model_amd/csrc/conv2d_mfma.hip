@@ -71,7 +71,7 @@ struct PatchArgs
     int32_t n_tiles;             // N * tiles_y * tiles_x
     int32_t n_ocb;               // blocks of output channels
     int32_t out_dtype;
-    int32_t xcd_remap;
+    int32_t xcd_remap;    // 0, or an eighth of the grid
     int32_t rounds;              // staging rounds per channel block
     int32_t pipelined;           // two LDS buffers, loads of the next block in flight during the MFMA loop
     int32_t buf_bytes;           // size of one LDS operand buffer (weight rows + patch)
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(512) void conv2d_patch_kernel(PatchArgs a)
     {
         // consecutive workgroups are dealt to the 8 XCDs in turn; give each XCD a contiguous run of tiles
         // so that neighbouring tiles (which share halo rows) share an L2
-        const uint32_t per = gridDim.x >> 3;
+        const uint32_t per = (uint32_t)a.xcd_remap;
         bid                = (bid & 7) * per + (bid >> 3);
     }
     // Grouped order: a run of kGroup pixel tiles times all channel blocks, the pixel tile running fastest.
@@ -1290,7 +1290,7 @@ static const char* launch_conv2d_mfma_t(hipStream_t st, const ConvGeom& g, int32
     if (blocks > 0x3fffffff || (int64_t)a.PH * a.PW * a.CH > (1 << 20))
         return nullptr;
     a.n_tiles     = (int)n_tiles;
-    a.xcd_remap   = (blocks % 8) == 0 && blocks >= 16;
+    a.xcd_remap   = (blocks % 8) == 0 && blocks >= 16 ? (int32_t)(blocks / 8) : 0;
     a.div_tw      = make_fastdiv(TW);
     a.div_pw      = make_fastdiv(a.PW);
     a.div_tiles_x = make_fastdiv(a.tiles_x);

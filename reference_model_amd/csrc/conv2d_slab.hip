@@ -32,6 +32,8 @@
 namespace tmi
 {
 
+// Kernel arguments are kept to 256 bytes where that is possible: writing them is part of every launch, and past that size a
+// launch takes the host about 0.8 us longer (2.5 us with 64 bytes, 3.2 with 256, 4.0 with 264).
 struct SlabArgs
 {
     const uint8_t* in;
@@ -41,16 +43,19 @@ struct SlabArgs
     void* out;
     uint32_t* flag_word;
     RescaleParams rp;
-    int32_t N, IH, IW, OC, OH, OW;
+    int32_t IH, IW, OC, OH, OW;
     int32_t sy, sx, dy, dx, pad_top, pad_left;
-    int32_t TH, TW, PH, PW, tiles_x, tiles_y;
+    int32_t TH, PH, PW;
     int32_t bias_len, za;
     int32_t n_ocb;
     int32_t out_kind;    // 0: int32 accumulators, 1: int8 through the RESCALE, 2: int16 through the RESCALE
     int32_t xcd_remap;    // 0, or grid / 8: workgroup b takes tile (b % 8) * (grid / 8) + b / 8
     int32_t pitch;               // 16-byte chunks per patch row in LDS: 5 per pixel plus the padding that spreads the banks
     int32_t step_row, step_chunk;    // 448 = step_row * pitch + step_chunk: how far 7 loads (448 slots) move
-    FastDiv div_tw, div_pitch, div_tiles_x, div_tiles_y, div_ocb;
+    FastDiv div_tw, div_pitch, div_tiles_x, div_tiles_y, div_ocb;    // (their divisors: tile width, patch pitch, tiles per row and column)
+};
+struct SlabArgsX : SlabArgs
+{
     // TRANSPOSE_CONV2D: IH x IW above are those of the input with up_y - 1 (up_x - 1) holes between its rows (columns),
     // which is never materialised; the tensor in memory is IHr x IWr
     int32_t up_y, up_x, IHr, IWr;
@@ -95,14 +100,14 @@ __device__ __forceinline__ void slab_barrier()
 // T: int8_t, or _Float16 / bf16_t: the same loads and LDS layout on channel vectors of CH * 8 values, fp32 accumulators that
 // start at the bias, results rounded to T (tensor_ops.cpp:828-882 with fp32 accumulation); no zero points, no RESCALE.
 template <int KH, int KW, int CH, bool ZA, bool FUSED, bool TC = false, int KD = 1, int NPT = 1, typename T = int8_t>
-__global__ __launch_bounds__(512) void conv2d_slab_kernel(SlabArgs a)
+__global__ __launch_bounds__(512) void conv2d_slab_kernel(std::conditional_t<(TC || KD > 1), SlabArgsX, SlabArgs> a)
 {
     static_assert(Mma<T>::is_int || (!ZA && !FUSED && !TC && KD == 1), "floating point: plain CONV2D only");
     // one field of every cache line of the arguments up front: a single scalar-cache round trip
     // every scalar argument the kernel reads, named once so that they are fetched together at the top (fields
     // first needed later are otherwise loaded one at a time, each with its own wait)
     asm volatile("" ::"s"(a.in), "s"(a.rp.shift), "s"(a.rp.out_zp), "s"(*reinterpret_cast<const uint32_t*>(&a.rp.scale32)),
-                 "s"(*reinterpret_cast<const uint32_t*>(&a.rp.in_bits)), "s"(a.rp.lo), "s"(a.N), "s"(a.TH), "s"(a.bias_len),
+                 "s"(*reinterpret_cast<const uint32_t*>(&a.rp.in_bits)), "s"(a.rp.lo), "s"(a.IH), "s"(a.TH), "s"(a.bias_len),
                  "s"(a.div_ocb.d));
     constexpr int TAPS   = KH * KW;
     constexpr int RW     = TAPS * CH + 1;    // chunks per weight row in LDS (odd)
@@ -145,10 +150,10 @@ __global__ __launch_bounds__(512) void conv2d_slab_kernel(SlabArgs a)
     const uint32_t tile = fdiv(bid, a.div_ocb);
     const int ocb       = bid - tile * a.n_ocb;
     const uint32_t trow = fdiv(tile, a.div_tiles_x);
-    const int txi       = tile - trow * a.tiles_x;
+    const int txi       = tile - trow * (int)a.div_tiles_x.d;
     const int n         = fdiv(trow, a.div_tiles_y);
-    const int tyi       = trow - n * a.tiles_y;
-    const int oy0 = tyi * a.TH, ox0 = txi * a.TW;
+    const int tyi       = trow - n * (int)a.div_tiles_y.d;
+    const int oy0 = tyi * a.TH, ox0 = txi * (int)a.div_tw.d;
     const int oc0 = ocb * 64;
     const int y0 = oy0 * a.sy - a.pad_top, x0 = ox0 * a.sx - a.pad_left;
 
@@ -184,11 +189,18 @@ __global__ __launch_bounds__(512) void conv2d_slab_kernel(SlabArgs a)
             }
         }
         {
-            const uint8_t* in_n = a.in + (size_t)n * (TC ? a.IHr * a.IWr : a.IH * a.IW) * KB;
+            int image_pixels = a.IH * a.IW;
+            if constexpr (TC)
+                image_pixels = a.IHr * a.IWr;
+            const uint8_t* in_n = a.in + (size_t)n * image_pixels * KB;
             constexpr int ICC   = CH / KD;    // chunks of a channel vector in memory
-            const int nb        = KD > 1 ? (int)fdiv(n, a.div_od) : 0;
-            const int slice0    = nb * a.ID;                              // first slice of the volume
-            const int z0        = (n - nb * a.OD) * a.sd - a.pd0;         // slice under depth tap 0
+            int slice0 = 0, z0 = 0;           // first slice of the volume, slice under depth tap 0
+            if constexpr (KD > 1)
+            {
+                const int nb = (int)fdiv(n, a.div_od);
+                slice0       = nb * a.ID;
+                z0           = (n - nb * a.OD) * a.sd - a.pd0;
+            }
             int lp              = wave + ((WLOADS - wave + LWAVES - 1) / LWAVES) * LWAVES - WLOADS;    // first patch load of this wave
             const int s0        = lp * 64 + lane;
             int py              = fdiv(s0, a.div_pitch);    // patch row and chunk inside the row
@@ -283,7 +295,7 @@ __global__ __launch_bounds__(512) void conv2d_slab_kernel(SlabArgs a)
     // A second accumulator tile (NPT = 2) holds 32 more pixels.
     constexpr int PXW  = 31;
     constexpr int WPIX = PXW + 32 * (NPT - 1);    // pixels of a wave
-    const int P        = a.TH * a.TW;
+    const int P        = a.TH * (int)a.div_tw.d;
     bool p_in_tile[NPT];
     int ty[NPT], tx[NPT];
 #pragma unroll
@@ -293,7 +305,7 @@ __global__ __launch_bounds__(512) void conv2d_slab_kernel(SlabArgs a)
         p_in_tile[k] = (k || li < PXW) && p < P;
         p            = p_in_tile[k] ? p : 0;
         ty[k]        = fdiv(p, a.div_tw);
-        tx[k]        = p - ty[k] * a.TW;
+        tx[k]        = p - ty[k] * (int)a.div_tw.d;
     }
     // The accumulators start at the bias of the lane's 16 channels (the zero-point column at zero).
     const int ocl = oct * 32 + 16 * lh;    // first of the lane's 16 channels inside the block
@@ -542,7 +554,7 @@ __global__ __launch_bounds__(512) void conv2d_slab_wreg_kernel(SlabArgs a)
     constexpr int KH = 3, KW = 3, CH = 4;    // 3x3 taps of 64 input channels: 18 weight fragments, 72 registers
     constexpr int NW = 8;
     asm volatile("" ::"s"(a.in), "s"(a.rp.shift), "s"(a.rp.out_zp), "s"(*reinterpret_cast<const uint32_t*>(&a.rp.scale32)),
-                 "s"(*reinterpret_cast<const uint32_t*>(&a.rp.in_bits)), "s"(a.rp.lo), "s"(a.N), "s"(a.TH), "s"(a.bias_len),
+                 "s"(*reinterpret_cast<const uint32_t*>(&a.rp.in_bits)), "s"(a.rp.lo), "s"(a.IH), "s"(a.TH), "s"(a.bias_len),
                  "s"(a.div_ocb.d));
     constexpr int TAPS   = KH * KW;
     constexpr int RW     = TAPS * CH + 1;    // chunks per weight row in LDS (odd)
@@ -583,10 +595,10 @@ __global__ __launch_bounds__(512) void conv2d_slab_wreg_kernel(SlabArgs a)
     const uint32_t tile = fdiv(bid, a.div_ocb);
     const int ocb       = bid - tile * a.n_ocb;
     const uint32_t trow = fdiv(tile, a.div_tiles_x);
-    const int txi       = tile - trow * a.tiles_x;
+    const int txi       = tile - trow * (int)a.div_tiles_x.d;
     const int n         = fdiv(trow, a.div_tiles_y);
-    const int tyi       = trow - n * a.tiles_y;
-    const int oy0 = tyi * a.TH, ox0 = txi * a.TW;
+    const int tyi       = trow - n * (int)a.div_tiles_y.d;
+    const int oy0 = tyi * a.TH, ox0 = txi * (int)a.div_tw.d;
     const int oc0 = ocb * 64;
     const int y0 = oy0 * a.sy - a.pad_top, x0 = ox0 * a.sx - a.pad_left;
 
@@ -735,7 +747,7 @@ __global__ __launch_bounds__(512) void conv2d_slab_wreg_kernel(SlabArgs a)
             start[4 * g] = b4[0], start[4 * g + 1] = b4[1], start[4 * g + 2] = b4[2], start[4 * g + 3] = b4[3];
         }
     }
-    const int P        = a.TH * a.TW;
+    const int P        = a.TH * (int)a.div_tw.d;
     const int NT       = (P + 31) >> 5;
     // the pixel fragments of step s + DEPTH are requested before the matrix instruction of step s, order pinned
     constexpr int AHEAD = 8;
@@ -778,7 +790,7 @@ __global__ __launch_bounds__(512) void conv2d_slab_wreg_kernel(SlabArgs a)
                     const bool in_tile = p < P;
                     p                  = in_tile ? p : 0;
                     const int ty       = fdiv(p, a.div_tw);
-                    const int tx       = p - ty * a.TW;
+                    const int tx       = p - ty * (int)a.div_tw.d;
                     const int oy = oy0 + ty, ox = ox0 + tx;
                     return Place{ (uint32_t)((ty * a.sy * a.pitch + tx * a.sx * RP) * 16 + lh * 16),
                                   (uint32_t)(((n * a.OH + oy) * a.OW + ox) * a.OC + oc0 + ocl),
@@ -896,7 +908,7 @@ __global__ __launch_bounds__(512) void conv2d_slab_wreg_kernel(SlabArgs a)
         const bool in_tile = p < P;
         p                  = in_tile ? p : 0;
         const int ty       = fdiv(p, a.div_tw);
-        const int tx       = p - ty * a.TW;
+        const int tx       = p - ty * (int)a.div_tw.d;
         const uint8_t* prow = pl + (ty * a.sy * a.pitch + tx * a.sx * RP) * 16 + lh * 16;
         v16i acc = start;
         v4i fb[STEPS];
@@ -998,31 +1010,31 @@ __global__ __launch_bounds__(512) void conv2d_slab_wreg_kernel(SlabArgs a)
 thread_local int32_t last_launch_shape[3] = { 0, 0, 0 };
 
 template <int KH, int KW, int CH, bool ZA, bool FUSED, bool TC = false, int KD = 1, int NPT = 1, typename T = int8_t>
-static bool launch_slab_kernel(hipStream_t st, const SlabArgs& a, int grid, int lds_bytes)
+static bool launch_slab_kernel(hipStream_t st, const SlabArgsX& a, int grid, int lds_bytes)
 {
     auto kern              = conv2d_slab_kernel<KH, KW, CH, ZA, FUSED, TC, KD, NPT, T>;
     static LdsLimit granted{};
     if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
         return false;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds_bytes, st, a);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds_bytes, st, static_cast<const std::conditional_t<(TC || KD > 1), SlabArgsX, SlabArgs>&>(a));
     last_launch_shape[0] = grid, last_launch_shape[1] = 512, last_launch_shape[2] = lds_bytes;
     return true;
 }
 
-static bool launch_slab_wreg(hipStream_t st, const SlabArgs& a, int grid, int lds_bytes)
+static bool launch_slab_wreg(hipStream_t st, const SlabArgsX& a, int grid, int lds_bytes)
 {
     auto launch = [&](auto kern) {
         static LdsLimit granted{};
         if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
             return false;
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds_bytes, st, a);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds_bytes, st, static_cast<const SlabArgs&>(a));
         last_launch_shape[0] = grid, last_launch_shape[1] = 512, last_launch_shape[2] = lds_bytes;
         return true;
     };
     // Weight loads through registers from five pixel tiles per workgroup on.  Measured on MI355X, us per launch with the
     // loads into LDS / through registers, [N,56,56,64]->64: N = 4 3.59 / 3.68, 8 4.04 / 4.09, 10 4.55 / 4.57, 12 4.70 / 4.60,
     // 16 5.25 / 5.10, 20 5.67 / 5.56, 32 6.96 / 6.64, 64 11.0 / 10.47.
-    const bool vl = (a.TH * a.TW + 31) / 32 >= 5;
+    const bool vl = (a.TH * (int)a.div_tw.d + 31) / 32 >= 5;
     if (vl)
         return a.za != 0 ? launch(conv2d_slab_wreg_kernel<true, true>) : launch(conv2d_slab_wreg_kernel<false, true>);
     return a.za != 0 ? launch(conv2d_slab_wreg_kernel<true, false>) : launch(conv2d_slab_wreg_kernel<false, false>);
@@ -1030,7 +1042,7 @@ static bool launch_slab_wreg(hipStream_t st, const SlabArgs& a, int grid, int ld
 
 // the floating-point instantiations: fp16 (kind 1) or bf16 (kind 2)
 template <int KH, int KW, int CH, bool WIDE_TOO = true>
-static bool launch_slab_taps_fp(hipStream_t st, const SlabArgs& a, int grid, int lds_bytes, int kind, bool wide)
+static bool launch_slab_taps_fp(hipStream_t st, const SlabArgsX& a, int grid, int lds_bytes, int kind, bool wide)
 {
     if constexpr (WIDE_TOO)
     {
@@ -1045,7 +1057,7 @@ static bool launch_slab_taps_fp(hipStream_t st, const SlabArgs& a, int grid, int
 }
 
 template <int KH, int KW, int CH, bool WIDE_TOO = true>
-static bool launch_slab_taps(hipStream_t st, const SlabArgs& a, int grid, int lds_bytes, bool fused, bool wide)
+static bool launch_slab_taps(hipStream_t st, const SlabArgsX& a, int grid, int lds_bytes, bool fused, bool wide)
 {
     if constexpr (!WIDE_TOO)
     {
@@ -1205,19 +1217,19 @@ const char* launch_conv2d_slab(hipStream_t st, int32_t in_dtype, int32_t out_dty
     if (!best_th)
         return nullptr;
 
-    SlabArgs a{};
+    SlabArgsX a{};
     a.in = (const uint8_t*)in, a.w = (const uint8_t*)w, a.bias = (const int32_t*)bias, a.out = out;
     a.pad_page = (const uint8_t*)pad_page, a.flag_word = flag_word, a.rp = rp;
-    a.N = g.N, a.IH = g.IH, a.IW = g.IW, a.OC = g.OC, a.OH = g.OH, a.OW = g.OW;
+    a.IH = g.IH, a.IW = g.IW, a.OC = g.OC, a.OH = g.OH, a.OW = g.OW;
     a.sy = g.stride_y, a.sx = g.stride_x, a.dy = g.dil_y, a.dx = g.dil_x, a.pad_top = g.pad_top, a.pad_left = g.pad_left;
-    a.TH = best_th, a.TW = best_tw;
+    a.TH = best_th;
     a.PH = (best_th - 1) * g.stride_y + (g.KH - 1) * g.dil_y + 1;
     a.PW = (best_tw - 1) * g.stride_x + (g.KW - 1) * g.dil_x + 1;
-    a.tiles_y = (g.OH + best_th - 1) / best_th, a.tiles_x = (g.OW + best_tw - 1) / best_tw;
+    const int tiles_y = (g.OH + best_th - 1) / best_th, tiles_x = (g.OW + best_tw - 1) / best_tw;
     a.bias_len = g.bias_len, a.za = in_zp, a.n_ocb = n_ocb;
     a.out_kind = !rp.enabled ? 0 : (out_dtype == TMI_INT8 ? 1 : 2);
-    const int64_t grid = (int64_t)g.N * a.tiles_y * a.tiles_x * n_ocb;
-    if (!tile_decode_is_exact(grid, (uint32_t)n_ocb, (uint32_t)a.tiles_x, (uint32_t)a.tiles_y))
+    const int64_t grid = (int64_t)g.N * tiles_y * tiles_x * n_ocb;
+    if (!tile_decode_is_exact(grid, (uint32_t)n_ocb, (uint32_t)tiles_x, (uint32_t)tiles_y))
         return nullptr;
     a.xcd_remap = (grid % 8 == 0 && n_ocb == 1) ? (int32_t)(grid / 8) : 0;
     // A patch pixel is R = CH + 1 chunks; the chunk of output pixel (ty, tx) under tap (0, 0) is ty * sy * pitch + R * sx * tx.
@@ -1229,12 +1241,12 @@ const char* launch_conv2d_slab(hipStream_t st, int32_t in_dtype, int32_t out_dty
     int pad = 0;
     if ((g.stride_x & 1) && (g.stride_y & 1))
         for (pad = 0; pad < 16; pad++)
-            if (((g.stride_y * (a.PW * rp_chunks + pad) - rp_chunks * g.stride_x * a.TW) & 15) == 0)
+            if (((g.stride_y * (a.PW * rp_chunks + pad) - rp_chunks * g.stride_x * best_tw) & 15) == 0)
                 break;
     a.pitch     = a.PW * rp_chunks + (pad & 15);
     a.step_row  = 448 / a.pitch, a.step_chunk = 448 % a.pitch;
-    a.div_tw = make_fastdiv((uint32_t)a.TW), a.div_pitch = make_fastdiv((uint32_t)a.pitch);
-    a.div_tiles_x = make_fastdiv((uint32_t)a.tiles_x), a.div_tiles_y = make_fastdiv((uint32_t)a.tiles_y);
+    a.div_tw = make_fastdiv((uint32_t)best_tw), a.div_pitch = make_fastdiv((uint32_t)a.pitch);
+    a.div_tiles_x = make_fastdiv((uint32_t)tiles_x), a.div_tiles_y = make_fastdiv((uint32_t)tiles_y);
     a.div_ocb = make_fastdiv((uint32_t)n_ocb);
     const int w_loads = taps * ch + 1, p_loads = (a.PH * a.pitch + 63) / 64;
     const int ones_bytes = (g.KH - 1) * g.dil_y * a.pitch * 16 + (g.KW - 1) * g.dil_x * rp_chunks * 16 + icb;

@@ -184,10 +184,10 @@ __global__ __launch_bounds__(256) void conv_i16_kernel(ConvI16Args a)
 // Copies of both operands with the channel vectors padded to ICP (a multiple of 16) channels of zeros, in one launch.
 __global__ __launch_bounds__(256) void pad_channels_i16_kernel(const int16_t* __restrict__ in, int64_t in_rows, const int8_t* __restrict__ w,
                                                                int64_t w_rows, int32_t IC, FastDiv icp, int16_t* __restrict__ in_out,
-                                                               int8_t* __restrict__ w_out)
+                                                               int8_t* __restrict__ w_out, int32_t blocks)
 {
     const int64_t n_in = in_rows * icp.d, total = n_in + w_rows * icp.d;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256)
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)blocks * 256)
     {
         const bool is_w   = i >= n_in;
         const int64_t j   = is_w ? i - n_in : i;
@@ -225,8 +225,9 @@ const char* launch_conv_i16_mfma(hipStream_t st, const ConvGeom& g, const void* 
         int16_t* in_pad = reinterpret_cast<int16_t*>(scratch);
         int8_t* w_pad   = reinterpret_cast<int8_t*>(scratch) + (in_rows * icp * 2 + 255) / 256 * 256;
         const int64_t blocks = (total + 255) / 256;
-        hipLaunchKernelGGL(pad_channels_i16_kernel, dim3((unsigned)(blocks > 8192 ? 8192 : blocks)), dim3(256), 0, st, (const int16_t*)in, in_rows,
-                           (const int8_t*)w, w_rows, g.IC, make_fastdiv((uint32_t)icp), in_pad, w_pad);
+        const unsigned grid = (unsigned)(blocks > 8192 ? 8192 : blocks);
+        hipLaunchKernelGGL(pad_channels_i16_kernel, dim3(grid), dim3(256), 0, st, (const int16_t*)in, in_rows, (const int8_t*)w, w_rows, g.IC,
+                           make_fastdiv((uint32_t)icp), in_pad, w_pad, (int32_t)grid);
         in = in_pad, w = w_pad;
     }
     else if ((((uintptr_t)in | (uintptr_t)w) & 15) != 0)

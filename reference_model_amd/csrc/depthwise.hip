@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void depthwise_dot4_kernel(DwArgs a)
 
     // consecutive workgroups are dealt to the 8 XCDs in turn: give each XCD a contiguous run of pixels, so
     // that the input rows shared by vertically adjacent outputs are found in its L2
-    const uint32_t per = gridDim.x >> 3;
+    const uint32_t per = ((uint32_t)a.blocks + 7) >> 3;    // an eighth of the grid
     const uint32_t bid = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (bid >= (uint32_t)a.blocks)
         return;

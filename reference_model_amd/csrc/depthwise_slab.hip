@@ -29,6 +29,7 @@
 namespace tmi
 {
 
+// (at most 256 bytes: see SlabArgs in conv2d_slab.hip)
 struct DwSlabArgs
 {
     const uint8_t* in;
@@ -38,19 +39,19 @@ struct DwSlabArgs
     void* out;
     uint32_t* flag_word;
     RescaleParams rp;
-    int32_t N, IH, IW, C, OH, OW;
+    int32_t IH, IW, C, OH, OW;
     int32_t sy, sx, dy, dx, pad_top, pad_left;
-    int32_t TH, TW, PH, PW, tiles_x, tiles_y;
+    int32_t TH, PH, PW;
     int32_t bias_len, za;
     int32_t out_kind;    // 0: int32 accumulators, 1: int8 through the RESCALE, 2: int16 through the RESCALE
     int32_t xcd_remap;    // 0, or grid / 8: workgroup b takes tile (b % 8) * (grid / 8) + b / 8
-    int32_t cpp;         // 16-byte chunks per pixel = C / 16
-    int32_t ppitch;      // chunks per patch pixel in LDS (odd)
-    int32_t pitch;       // chunks per patch row in LDS
-    int32_t step_row, step_px, step_ch;    // one round of loads (64 slots per wave) = step_row rows + step_px pixels + step_ch chunks
-    int32_t wrap_px, wrap_ch;    // a patch row in pixels and chunks: pitch = wrap_px * ppitch + wrap_ch (padding included)
-    int32_t n_cblk;      // channel blocks of 32
+    int32_t step_row;    // one round of loads (64 slots per wave) = step_row rows + step_px pixels + step_ch chunks
+    int16_t step_px, step_ch;
+    int16_t wrap_px, wrap_ch;    // a patch row in pixels and chunks: pitch = wrap_px * ppitch + wrap_ch (padding included)
+    int32_t nwaves;      // of a workgroup
     int32_t n_units;     // (pixel tiles of 32) x channel blocks
+    // (their divisors: tile width, 16-byte chunks per patch row and per patch pixel (odd) in LDS, tiles per row and column,
+    // channel blocks of 32)
     FastDiv div_tw, div_pitch, div_ppitch, div_tiles_x, div_tiles_y, div_cblk;
 };
 
@@ -62,18 +63,18 @@ __device__ __forceinline__ void dwslab_load(const void* src, uint32_t lds_addr)
 template <bool ZA, bool FUSED>
 __global__ __launch_bounds__(1024) void depthwise_slab_kernel(DwSlabArgs a)
 {
-    asm volatile("" ::"s"(a.in), "s"(a.rp.shift), "s"(a.rp.lo), "s"(a.N), "s"(a.TH), "s"(a.bias_len), "s"(a.n_units),
+    asm volatile("" ::"s"(a.in), "s"(a.rp.shift), "s"(a.rp.lo), "s"(a.IH), "s"(a.TH), "s"(a.bias_len), "s"(a.n_units),
                  "s"(a.div_cblk.d));
     constexpr int TAPS = 9;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid     = threadIdx.x;
     const int lane    = tid & 63;
     const int wave    = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nwaves  = blockDim.x >> 6;
+    const int nwaves  = a.nwaves;
     const int li      = lane & 31;
     const int lh      = lane >> 5;
     const int C       = a.C;
-    const int p_slots = a.PH * a.pitch;
+    const int p_slots = a.PH * (int)a.div_pitch.d;
     const int p_loads = (p_slots + 63) >> 6;
     // LDS: [patch][weights: 9 x C bytes][C x ChannelScale][C x HighWordScale][C multipliers][C x (bias - za * sum(w))][common shift per table wave]
     uint8_t* pl          = lds;
@@ -92,10 +93,10 @@ __global__ __launch_bounds__(1024) void depthwise_slab_kernel(DwSlabArgs a)
         bid                = (bid & 7) * per + (bid >> 3);
     }
     const uint32_t trow = fdiv(bid, a.div_tiles_x);
-    const int txi       = bid - trow * a.tiles_x;
+    const int txi       = bid - trow * (int)a.div_tiles_x.d;
     const int n         = fdiv(trow, a.div_tiles_y);
-    const int tyi       = trow - n * a.tiles_y;
-    const int oy0 = tyi * a.TH, ox0 = txi * a.TW;
+    const int tyi       = trow - n * (int)a.div_tiles_y.d;
+    const int oy0 = tyi * a.TH, ox0 = txi * (int)a.div_tw.d;
     const int y0 = oy0 * a.sy - a.pad_top, x0 = ox0 * a.sx - a.pad_left;
 
     // ---- per-channel operands: requested first, used after the patch loads have been issued ---------------------
@@ -124,28 +125,28 @@ __global__ __launch_bounds__(1024) void depthwise_slab_kernel(DwSlabArgs a)
         // slot s0 = (patch row py, pixel px, chunk ch); a round of loads later it is step_row rows, step_px pixels and
         // step_ch chunks further on, wrapped with additions only (a row ends with row_pad spare chunks)
         int py       = fdiv(s0, a.div_pitch);
-        const int r0 = s0 - py * a.pitch;
+        const int r0 = s0 - py * (int)a.div_pitch.d;
         int px       = fdiv(r0, a.div_ppitch);
-        int ch       = r0 - px * a.ppitch;
+        int ch       = r0 - px * (int)a.div_ppitch.d;
         uint32_t dst = lbase + wave * 1024;
         for (int l = wave; l < p_loads; l += nwaves)
         {
             const int iy = y0 + py, ix = x0 + px;
             const bool img = py < a.PH && px < a.PW && (unsigned)iy < (unsigned)a.IH && (unsigned)ix < (unsigned)a.IW;
-            const int cc   = ch < a.cpp ? ch : 0;    // the spare chunk of a pixel reads its first one
+            const int cc   = ch < (a.C >> 4) ? ch : 0;    // the spare chunk of a pixel reads its first one
             const uint8_t* src = img ? in_n + mad_u24(mad_u24((uint32_t)iy, (uint32_t)a.IW, (uint32_t)ix), (uint32_t)C, (uint32_t)(cc * 16))
                                      : a.pad_page + (cc & 3) * 16;
             dwslab_load(src, dst);
             dst += nwaves * 1024;
             py += a.step_row, px += a.step_px, ch += a.step_ch;
-            if (ch >= a.ppitch)
-                ch -= a.ppitch, px++;
+            if (ch >= (int)a.div_ppitch.d)
+                ch -= (int)a.div_ppitch.d, px++;
             // past the end of the row (pixels PW .. hold the row's spare chunks): on to the next row
-            if (__mul24(px, a.ppitch) + ch >= a.pitch)
+            if (__mul24(px, (int)a.div_ppitch.d) + ch >= (int)a.div_pitch.d)
             {
                 ch -= a.wrap_ch, px -= a.wrap_px, py++;
                 if (ch < 0)
-                    ch += a.ppitch, px--;
+                    ch += (int)a.div_ppitch.d, px--;
             }
         }
     }
@@ -201,9 +202,9 @@ __global__ __launch_bounds__(1024) void depthwise_slab_kernel(DwSlabArgs a)
     __syncthreads();
 
     // ---- units: (pixel tile of 32, channel block of 32) ---------------------------------------------------------
-    const int P        = a.TH * a.TW;
-    const int row_step = a.dy * a.pitch * 16;
-    const int col_step = a.dx * a.ppitch * 16;
+    const int P        = a.TH * (int)a.div_tw.d;
+    const int row_step = a.dy * (int)a.div_pitch.d * 16;
+    const int col_step = a.dx * (int)a.div_ppitch.d * 16;
     // operand row li of the diagonal matrix stands for channel wr of the block
     const int wr = 4 * (li & 4) + ((li >> 1) & 12) + (li & 3);
     // row li is non-zero at K index wr only, which lies in this lane's K half when wr / 16 == lh: byte wr % 4 of word
@@ -215,13 +216,13 @@ __global__ __launch_bounds__(1024) void depthwise_slab_kernel(DwSlabArgs a)
     for (int u = wave; u < a.n_units; u += nwaves)
     {
         const int pxt = fdiv(u, a.div_cblk);
-        const int cb  = u - pxt * a.n_cblk;
+        const int cb  = u - pxt * (int)a.div_cblk.d;
         const int c0  = cb * 32;
         int p         = pxt * 32 + li;
         const bool p_in_tile = p < P;
         p             = p_in_tile ? p : 0;
         const int ty  = fdiv(p, a.div_tw);
-        const int tx  = p - ty * a.TW;
+        const int tx  = p - ty * (int)a.div_tw.d;
         // Everything the nine MFMAs need is requested up front, in a pinned order: left alone, the compiler requests a
         // tap's pixel fragment right before its MFMA and a wave waits out the LDS latency nine times in a row.
         // The diagonal operands of this channel block are built from the replicated weight bytes (channels past C:
@@ -231,7 +232,7 @@ __global__ __launch_bounds__(1024) void depthwise_slab_kernel(DwSlabArgs a)
         // the nine tap addresses are this one plus scalars; kept opaque so that the products are not redistributed
         // over the taps (a 32-bit vector multiply runs at a quarter of the rate)
         uint32_t pbase = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)pl +
-                         (uint32_t)((ty * a.sy * a.pitch + tx * a.sx * a.ppitch) * 16 + c0 + lh * 16);
+                         (uint32_t)((ty * a.sy * (int)a.div_pitch.d + tx * a.sx * (int)a.div_ppitch.d) * 16 + c0 + lh * 16);
         asm volatile("" : "+v"(pbase));
         // (lane, register e) = channel c0 + 16 lh + e of pixel li; the accumulators start at the channel's bias term
         const int cl  = c0 + 16 * lh;
@@ -382,8 +383,9 @@ __global__ __launch_bounds__(1024) void depthwise_slab_kernel(DwSlabArgs a)
 }
 
 template <bool ZA, bool FUSED>
-static bool launch_dwslab_kernel(hipStream_t st, const DwSlabArgs& a, int grid, int threads, int lds_bytes)
+static bool launch_dwslab_kernel(hipStream_t st, DwSlabArgs a, int grid, int threads, int lds_bytes)
 {
+    a.nwaves     = threads / 64;
     auto kern = depthwise_slab_kernel<ZA, FUSED>;
     static LdsLimit granted{};
     if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
@@ -471,15 +473,14 @@ const char* launch_depthwise_slab(hipStream_t st, int32_t in_dtype, int32_t out_
     DwSlabArgs a{};
     a.in = (const uint8_t*)in, a.w = (const int8_t*)w, a.bias = (const int32_t*)bias, a.out = out;
     a.pad_page = (const uint8_t*)pad_page, a.flag_word = flag_word, a.rp = rp;
-    a.N = g.N, a.IH = g.IH, a.IW = g.IW, a.C = C, a.OH = g.OH, a.OW = g.OW;
+    a.IH = g.IH, a.IW = g.IW, a.C = C, a.OH = g.OH, a.OW = g.OW;
     a.sy = g.stride_y, a.sx = g.stride_x, a.dy = g.dil_y, a.dx = g.dil_x, a.pad_top = g.pad_top, a.pad_left = g.pad_left;
-    a.TH = best_th, a.TW = best_tw;
+    a.TH = best_th;
     a.PH = (best_th - 1) * g.stride_y + 2 * g.dil_y + 1;
     a.PW = (best_tw - 1) * g.stride_x + 2 * g.dil_x + 1;
-    a.tiles_y = (g.OH + best_th - 1) / best_th, a.tiles_x = (g.OW + best_tw - 1) / best_tw;
+    const int tiles_y = (g.OH + best_th - 1) / best_th, tiles_x = (g.OW + best_tw - 1) / best_tw;
     a.bias_len = g.bias_len, a.za = in_zp;
     a.out_kind = !rp.enabled ? 0 : (out_dtype == TMI_INT8 ? 1 : 2);
-    a.cpp = cpp, a.ppitch = ppitch, a.n_cblk = n_cblk;
     a.n_units = ((best_th * best_tw + 31) / 32) * n_cblk;
     // The chunk of tile pixel p = ty * TW + tx under tap (0, 0) is ty * sy * pitch + tx * sx * ppitch; the 16 lanes a
     // ds_read_b128 serves together differ modulo 16, so the reads are free of bank conflicts when that chunk is an odd
@@ -488,22 +489,22 @@ const char* launch_depthwise_slab(hipStream_t st, int32_t in_dtype, int32_t out_
     int pad = 0;
     if ((g.stride_x & 1) && (g.stride_y & 1))
         for (pad = 0; pad < 16; pad++)
-            if (((g.stride_y * (a.PW * ppitch + pad) - g.stride_x * ppitch * a.TW) & 15) == 0)
+            if (((g.stride_y * (a.PW * ppitch + pad) - g.stride_x * ppitch * best_tw) & 15) == 0)
                 break;
-    a.pitch = a.PW * ppitch + (pad & 15);
+    const int pitch = a.PW * ppitch + (pad & 15);
     const int per_round = best_nw * 64;
-    a.wrap_px = a.pitch / ppitch, a.wrap_ch = a.pitch % ppitch;
-    a.step_row = per_round / a.pitch;
-    a.step_px = (per_round % a.pitch) / ppitch, a.step_ch = (per_round % a.pitch) % ppitch;
-    const int64_t grid = (int64_t)g.N * a.tiles_y * a.tiles_x;
-    if (!tile_decode_is_exact(grid, 1u, (uint32_t)a.tiles_x, (uint32_t)a.tiles_y))
+    a.wrap_px = (int16_t)(pitch / ppitch), a.wrap_ch = (int16_t)(pitch % ppitch);    // (a patch row fits the LDS: below 2^15 chunks)
+    a.step_row = per_round / pitch;
+    a.step_px = (int16_t)((per_round % pitch) / ppitch), a.step_ch = (int16_t)((per_round % pitch) % ppitch);
+    const int64_t grid = (int64_t)g.N * tiles_y * tiles_x;
+    if (!tile_decode_is_exact(grid, 1u, (uint32_t)tiles_x, (uint32_t)tiles_y))
         return nullptr;
     a.xcd_remap = grid % 8 == 0 ? (int32_t)(grid / 8) : 0;
-    a.div_tw = make_fastdiv((uint32_t)a.TW), a.div_pitch = make_fastdiv((uint32_t)a.pitch);
+    a.div_tw = make_fastdiv((uint32_t)best_tw), a.div_pitch = make_fastdiv((uint32_t)pitch);
     a.div_ppitch = make_fastdiv((uint32_t)ppitch);
-    a.div_tiles_x = make_fastdiv((uint32_t)a.tiles_x), a.div_tiles_y = make_fastdiv((uint32_t)a.tiles_y);
+    a.div_tiles_x = make_fastdiv((uint32_t)tiles_x), a.div_tiles_y = make_fastdiv((uint32_t)tiles_y);
     a.div_cblk = make_fastdiv((uint32_t)n_cblk);
-    const int p_loads   = (a.PH * a.pitch + 63) / 64;
+    const int p_loads   = (a.PH * pitch + 63) / 64;
     const int lds_bytes = p_loads * 1024 + table_bytes;
     if (lds_bytes > lds_max)
         return nullptr;

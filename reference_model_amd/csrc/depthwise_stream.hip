@@ -36,6 +36,7 @@ struct DwStreamArgs
     int32_t n_tiles;        // pixel tiles of the layer
     int32_t tiles_per_part; // pixel tiles per part of the layer (part = workgroup index % 8)
     int32_t n_streams;      // waves per part and channel group
+    int32_t nw;             // waves of a workgroup
     FastDiv div_tiles_x, div_tiles_y, div_grp;
 };
 
@@ -47,7 +48,7 @@ __global__ __launch_bounds__(512) void depthwise_stream_kernel(DwStreamArgs a)
     const int tid  = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nw   = blockDim.x >> 6;
+    const int nw   = a.nw;
     const int li = lane & 31, lh = lane >> 5;
     const int C  = a.C;
     // LDS: [weights: 9 x C words, the byte in all four bytes][C x ChannelScale][C x HighWordScale][C x (bias - za * sum(w))]
@@ -360,8 +361,9 @@ __global__ __launch_bounds__(512) void depthwise_stream_kernel(DwStreamArgs a)
 }
 
 template <bool ZA, bool FUSED, int G>
-static bool launch_dwstream_kernel(hipStream_t st, const DwStreamArgs& a, int grid, int threads, int lds_bytes)
+static bool launch_dwstream_kernel(hipStream_t st, DwStreamArgs a, int grid, int threads, int lds_bytes)
 {
+    a.nw     = threads / 64;
     auto kern = depthwise_stream_kernel<ZA, FUSED, G>;
     static LdsLimit granted{};
     if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))

@@ -67,13 +67,13 @@ template <typename T, typename OutT>
 __global__ __launch_bounds__(256) void conv2d_direct_kernel(ConvGeom g, const T* __restrict__ in,
                                                             const T* __restrict__ w, const void* __restrict__ bias,
                                                             int32_t in_zp, int32_t w_zp, RescaleParams rp,
-                                                            OutT* __restrict__ out, uint32_t* flag_word)
+                                                            OutT* __restrict__ out, uint32_t* flag_word, int32_t blocks)
 {
     using acc_t          = typename Elem<T>::acc_t;
     const int64_t total  = (int64_t)g.N * g.OH * g.OW * g.OC;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t stride = (int64_t)blocks * 256;
     uint32_t flags       = 0;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride)
+    for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += stride)
     {
         const int oc = (int)(idx % g.OC);
         int64_t t    = idx / g.OC;
@@ -121,13 +121,13 @@ __global__ __launch_bounds__(256) void depthwise_direct_kernel(ConvGeom g, const
                                                                const T* __restrict__ w,
                                                                const void* __restrict__ bias, int32_t in_zp,
                                                                int32_t w_zp, RescaleParams rp, OutT* __restrict__ out,
-                                                               uint32_t* flag_word)
+                                                               uint32_t* flag_word, int32_t blocks)
 {
     using acc_t          = typename Elem<T>::acc_t;
     const int64_t total  = (int64_t)g.N * g.OH * g.OW * g.OC;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t stride = (int64_t)blocks * 256;
     uint32_t flags       = 0;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride)
+    for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += stride)
     {
         const int oc = (int)(idx % g.OC);
         int64_t t    = idx / g.OC;
@@ -173,12 +173,12 @@ __global__ __launch_bounds__(256) void depthwise_direct_kernel(ConvGeom g, const
 template <typename T, typename OutT>
 __global__ __launch_bounds__(256) void matmul_direct_kernel(int32_t N, int32_t H, int32_t C, int32_t W,
                                                             const T* __restrict__ a, const T* __restrict__ b,
-                                                            int32_t a_zp, int32_t b_zp, OutT* __restrict__ out)
+                                                            int32_t a_zp, int32_t b_zp, OutT* __restrict__ out, int32_t blocks)
 {
     using acc_t          = typename Elem<T>::acc_t;
     const int64_t total  = (int64_t)N * H * W;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride)
+    const int64_t stride = (int64_t)blocks * 256;
+    for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += stride)
     {
         const int x = (int)(idx % W);
         int64_t t   = idx / W;
@@ -206,12 +206,12 @@ template <bool DEPTHWISE>
 __global__ __launch_bounds__(256) void conv_i16_direct_kernel(ConvGeom g, const int16_t* __restrict__ in,
                                                               const int8_t* __restrict__ w,
                                                               const int64_t* __restrict__ bias, int32_t w_zp,
-                                                              int64_t* __restrict__ out)
+                                                              int64_t* __restrict__ out, int32_t blocks)
 {
     const int64_t total  = (int64_t)g.N * g.OH * g.OW * g.OC;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t stride = (int64_t)blocks * 256;
     const bool vec       = g.IC % 8 == 0 && (((uintptr_t)in | (uintptr_t)w) & 15) == 0;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride)
+    for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += stride)
     {
         const int oc = (int)(idx % g.OC);
         int64_t t    = idx / g.OC;
@@ -262,11 +262,11 @@ __global__ __launch_bounds__(256) void conv_i16_direct_kernel(ConvGeom g, const 
 
 __global__ __launch_bounds__(256) void matmul_i16_direct_kernel(int32_t N, int32_t H, int32_t C, int32_t W,
                                                                 const int16_t* __restrict__ a,
-                                                                const int16_t* __restrict__ b, int64_t* __restrict__ out)
+                                                                const int16_t* __restrict__ b, int64_t* __restrict__ out, int32_t blocks)
 {
     const int64_t total  = (int64_t)N * H * W;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += stride)
+    const int64_t stride = (int64_t)blocks * 256;
+    for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += stride)
     {
         const int x = (int)(idx % W);
         int64_t t   = idx / W;
@@ -291,7 +291,7 @@ static int grid_for(int64_t work_items)
 
 #define TMI_LAUNCH_CONV(KERNEL, T, OT)                                                                              \
     hipLaunchKernelGGL((KERNEL<T, OT>), dim3(grid_for(total)), dim3(256), 0, st, g, (const T*)in, (const T*)w, bias, \
-                       in_zp, w_zp, rp, (OT*)out, flag_word)
+                       in_zp, w_zp, rp, (OT*)out, flag_word, grid_for(total))
 
 #define TMI_DEFINE_CONV_LAUNCH(FUNC, KERNEL, LABEL)                                                                 \
     const char* FUNC(hipStream_t st, int32_t in_dtype, int32_t out_dtype, const ConvGeom& g, const void* in,        \
@@ -343,25 +343,25 @@ const char* launch_matmul_direct(hipStream_t st, int32_t in_dtype, int32_t N, in
     if (in_dtype == TMI_INT8)
     {
         hipLaunchKernelGGL((matmul_direct_kernel<int8_t, int32_t>), dim3(grid_for(total)), dim3(256), 0, st, N, H, C,
-                           W, (const int8_t*)a, (const int8_t*)b, a_zp, b_zp, (int32_t*)out);
+                           W, (const int8_t*)a, (const int8_t*)b, a_zp, b_zp, (int32_t*)out, grid_for(total));
         return "matmul_direct_i8";
     }
     if (in_dtype == TMI_FP16)
     {
         hipLaunchKernelGGL((matmul_direct_kernel<_Float16, float>), dim3(grid_for(total)), dim3(256), 0, st, N, H, C,
-                           W, (const _Float16*)a, (const _Float16*)b, 0, 0, (float*)out);
+                           W, (const _Float16*)a, (const _Float16*)b, 0, 0, (float*)out, grid_for(total));
         return "matmul_direct_f16";
     }
     if (in_dtype == TMI_BF16)
     {
         hipLaunchKernelGGL((matmul_direct_kernel<bf16_t, float>), dim3(grid_for(total)), dim3(256), 0, st, N, H, C,
-                           W, (const bf16_t*)a, (const bf16_t*)b, 0, 0, (float*)out);
+                           W, (const bf16_t*)a, (const bf16_t*)b, 0, 0, (float*)out, grid_for(total));
         return "matmul_direct_bf16";
     }
     if (in_dtype == TMI_FP32)
     {
         hipLaunchKernelGGL((matmul_direct_kernel<float, float>), dim3(grid_for(total)), dim3(256), 0, st, N, H, C, W,
-                           (const float*)a, (const float*)b, 0, 0, (float*)out);
+                           (const float*)a, (const float*)b, 0, 0, (float*)out, grid_for(total));
         return "matmul_direct_f32";
     }
     return nullptr;
@@ -375,10 +375,10 @@ const char* launch_conv_i16_direct(hipStream_t st, bool depthwise, const ConvGeo
         return "conv_direct_empty";
     if (depthwise)
         hipLaunchKernelGGL((conv_i16_direct_kernel<true>), dim3(grid_for(total)), dim3(256), 0, st, g, (const int16_t*)in,
-                           (const int8_t*)w, (const int64_t*)bias, w_zp, (int64_t*)out);
+                           (const int8_t*)w, (const int64_t*)bias, w_zp, (int64_t*)out, grid_for(total));
     else
         hipLaunchKernelGGL((conv_i16_direct_kernel<false>), dim3(grid_for(total)), dim3(256), 0, st, g, (const int16_t*)in,
-                           (const int8_t*)w, (const int64_t*)bias, w_zp, (int64_t*)out);
+                           (const int8_t*)w, (const int64_t*)bias, w_zp, (int64_t*)out, grid_for(total));
     return depthwise ? "depthwise_direct_i16_i48" : "conv2d_direct_i16_i48";
 }
 
@@ -389,7 +389,7 @@ const char* launch_matmul_i16_direct(hipStream_t st, int32_t N, int32_t H, int32
     if (total == 0)
         return "matmul_direct_empty";
     hipLaunchKernelGGL(matmul_i16_direct_kernel, dim3(grid_for(total)), dim3(256), 0, st, N, H, C, W, (const int16_t*)a,
-                       (const int16_t*)b, (int64_t*)out);
+                       (const int16_t*)b, (int64_t*)out, grid_for(total));
     return "matmul_direct_i16_i48";
 }
 

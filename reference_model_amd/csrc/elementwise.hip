@@ -19,12 +19,12 @@ struct alignas(sizeof(T) * N) Pack
 template <typename InT, typename OutT, int VEC, bool PRECISE>
 __global__ __launch_bounds__(256) void rescale_vec_kernel(RescaleParams p, const InT* __restrict__ in,
                                                           OutT* __restrict__ out, int64_t n_vec, int32_t C,
-                                                          uint32_t* flag_word)
+                                                          uint32_t* flag_word, int32_t blocks)
 {
     // C % VEC == 0, so a pack never straddles a row and its channels are c0 .. c0+VEC-1
     uint32_t flags       = 0;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_vec; i += stride)
+    const int64_t stride = (int64_t)blocks * 256;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_vec; i += stride)
     {
         const Pack<InT, VEC> a = reinterpret_cast<const Pack<InT, VEC>*>(in)[i];
         const int c0           = (int)((i * VEC) % C);
@@ -44,11 +44,11 @@ __global__ __launch_bounds__(256) void rescale_vec_kernel(RescaleParams p, const
 template <typename InT, typename OutT, bool PRECISE>
 __global__ __launch_bounds__(256) void rescale_scalar_kernel(RescaleParams p, const InT* __restrict__ in,
                                                              OutT* __restrict__ out, int64_t n, int32_t C,
-                                                             uint32_t* flag_word)
+                                                             uint32_t* flag_word, int32_t blocks)
 {
     uint32_t flags       = 0;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+    const int64_t stride = (int64_t)blocks * 256;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride)
     {
         const int c     = (int)(i % C);
         const int32_t m = load_multiplier(p, c);
@@ -115,10 +115,10 @@ __device__ __forceinline__ void rescale_store_row(const RescaleParams& p, const 
 template <typename OutT, bool HW, bool DR>
 __device__ __forceinline__ void rescale_walk(const RescaleParams& p, const RescaleLane& k, const int32_t* __restrict__ in,
                                              OutT* __restrict__ out, int64_t rows, int32_t C, int32_t rpi, int slot,
-                                             int c0, bool lane_on, uint32_t& flags)
+                                             int c0, bool lane_on, uint32_t& flags, int32_t blocks)
 {
     constexpr int U    = 4;
-    const int64_t step = (int64_t)gridDim.x * rpi;    // rows between two units of a workgroup
+    const int64_t step = (int64_t)blocks * rpi;    // rows between two units of a workgroup
     int64_t r          = (int64_t)blockIdx.x * rpi + slot;
     rs_v4i v[U];
 #pragma unroll
@@ -147,7 +147,7 @@ template <typename OutT>
 __global__ __launch_bounds__(256) void rescale_fast_kernel(RescaleParams p, const int32_t* __restrict__ in,
                                                            OutT* __restrict__ out, int64_t rows, int32_t C,
                                                            int32_t cgs, int32_t rpi, FastDiv div_cgs,
-                                                           uint32_t* flag_word)
+                                                           uint32_t* flag_word, int32_t blocks)
 {
     const int tid      = threadIdx.x;
     const int slot     = fdiv(tid, div_cgs);    // row slot of this lane inside a unit
@@ -183,12 +183,12 @@ __global__ __launch_bounds__(256) void rescale_fast_kernel(RescaleParams p, cons
         for (int c = 0; c < 4; c++)
             k.sh[c] -= 32;
         if (p.double_round)
-            rescale_walk<OutT, true, true>(p, k, in, out, rows, C, rpi, slot, c0, lane_on, flags);
+            rescale_walk<OutT, true, true>(p, k, in, out, rows, C, rpi, slot, c0, lane_on, flags, blocks);
         else
-            rescale_walk<OutT, true, false>(p, k, in, out, rows, C, rpi, slot, c0, lane_on, flags);
+            rescale_walk<OutT, true, false>(p, k, in, out, rows, C, rpi, slot, c0, lane_on, flags, blocks);
     }
     else
-        rescale_walk<OutT, false, false>(p, k, in, out, rows, C, rpi, slot, c0, lane_on, flags);
+        rescale_walk<OutT, false, false>(p, k, in, out, rows, C, rpi, slot, c0, lane_on, flags, blocks);
     raise_flags(flag_word, flags);
 }
 
@@ -209,7 +209,7 @@ static const char* launch_rescale_fast(hipStream_t st, const RescaleParams& p, c
     if (blocks < 1)
         blocks = 1;
     hipLaunchKernelGGL((rescale_fast_kernel<OutT>), dim3((int)blocks), dim3(256), 0, st, p, (const int32_t*)in,
-                       (OutT*)out, rows, C, cgs, rpi, make_fastdiv(cgs), flag_word);
+                       (OutT*)out, rows, C, cgs, rpi, make_fastdiv(cgs), flag_word, (int32_t)blocks);
     return "rescale_fast";
 }
 
@@ -240,18 +240,18 @@ static const char* launch_rescale_t(hipStream_t st, const RescaleParams& p, cons
         const int64_t n_vec = n / VEC;
         if (precise)
             hipLaunchKernelGGL((rescale_vec_kernel<InT, OutT, VEC, true>), dim3(grid_for(n_vec)), dim3(256), 0, st, p,
-                               (const InT*)in, (OutT*)out, n_vec, C, flag_word);
+                               (const InT*)in, (OutT*)out, n_vec, C, flag_word, grid_for(n_vec));
         else
             hipLaunchKernelGGL((rescale_vec_kernel<InT, OutT, VEC, false>), dim3(grid_for(n_vec)), dim3(256), 0, st, p,
-                               (const InT*)in, (OutT*)out, n_vec, C, flag_word);
+                               (const InT*)in, (OutT*)out, n_vec, C, flag_word, grid_for(n_vec));
         return precise ? "rescale_vec_precise" : "rescale_vec";
     }
     if (precise)
         hipLaunchKernelGGL((rescale_scalar_kernel<InT, OutT, true>), dim3(grid_for(n)), dim3(256), 0, st, p,
-                           (const InT*)in, (OutT*)out, n, C, flag_word);
+                           (const InT*)in, (OutT*)out, n, C, flag_word, grid_for(n));
     else
         hipLaunchKernelGGL((rescale_scalar_kernel<InT, OutT, false>), dim3(grid_for(n)), dim3(256), 0, st, p,
-                           (const InT*)in, (OutT*)out, n, C, flag_word);
+                           (const InT*)in, (OutT*)out, n, C, flag_word, grid_for(n));
     if (precise)
         return "rescale_scalar_precise";
     return "rescale_scalar";
@@ -294,12 +294,12 @@ const char* launch_rescale(hipStream_t st, const RescaleParams& p, int32_t in_dt
 // ------------------------------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void clamp_kernel(const T* __restrict__ in, T* __restrict__ out, int64_t n,
-                                                    int32_t lo, int32_t hi, int vectorised)
+                                                    int32_t lo, int32_t hi, int vectorised, int32_t blocks)
 {
     constexpr int VEC    = 16 / sizeof(T);
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t stride = (int64_t)blocks * 256;
     const int64_t n_vec  = vectorised ? n / VEC : 0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_vec; i += stride)
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_vec; i += stride)
     {
         Pack<T, VEC> a = reinterpret_cast<const Pack<T, VEC>*>(in)[i];
 #pragma unroll
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(256) void clamp_kernel(const T* __restrict__ in, T*
         }
         reinterpret_cast<Pack<T, VEC>*>(out)[i] = a;
     }
-    for (int64_t i = n_vec * VEC + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+    for (int64_t i = n_vec * VEC + (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride)
     {
         int32_t v = in[i];
         v         = v >= lo ? v : lo;
@@ -329,10 +329,10 @@ const char* launch_clamp(hipStream_t st, int32_t dtype, const void* in, void* ou
     const int vec = ((uintptr_t)in % 16 == 0) && ((uintptr_t)out % 16 == 0);
     if (dtype == TMI_INT8)
         hipLaunchKernelGGL(clamp_kernel<int8_t>, dim3(grid_for((n + 15) / 16)), dim3(256), 0, st, (const int8_t*)in,
-                           (int8_t*)out, n, lo, hi, vec);
+                           (int8_t*)out, n, lo, hi, vec, grid_for((n + 15) / 16));
     else if (dtype == TMI_INT16)
         hipLaunchKernelGGL(clamp_kernel<int16_t>, dim3(grid_for((n + 7) / 8)), dim3(256), 0, st,
-                           (const int16_t*)in, (int16_t*)out, n, lo, hi, vec);
+                           (const int16_t*)in, (int16_t*)out, n, lo, hi, vec, grid_for((n + 7) / 8));
     else
         return nullptr;
     return "clamp_vec";
@@ -375,10 +375,10 @@ __device__ __forceinline__ void clampf_store(bf16_t* p, int64_t i, float v)
 
 template <typename T>
 __global__ __launch_bounds__(256) void clamp_fp_kernel(const T* __restrict__ in, T* __restrict__ out, int64_t n, float lo,
-                                                       float hi, int nan_mode)
+                                                       float hi, int nan_mode, int32_t blocks)
 {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+    const int64_t stride = (int64_t)blocks * 256;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride)
     {
         float v = clampf_load<T>(in, i);
         if (v != v)
@@ -399,12 +399,12 @@ const char* launch_clamp_fp(hipStream_t st, int32_t dtype, const void* in, void*
         return "clamp_empty";
     const dim3 grid(grid_for(n)), block(256);
     if (dtype == TMI_FP32)
-        hipLaunchKernelGGL(clamp_fp_kernel<float>, grid, block, 0, st, (const float*)in, (float*)out, n, lo, hi, nan_mode);
+        hipLaunchKernelGGL(clamp_fp_kernel<float>, grid, block, 0, st, (const float*)in, (float*)out, n, lo, hi, nan_mode, (int32_t)grid.x);
     else if (dtype == TMI_FP16)
         hipLaunchKernelGGL(clamp_fp_kernel<_Float16>, grid, block, 0, st, (const _Float16*)in, (_Float16*)out, n, lo, hi,
-                           nan_mode);
+                           nan_mode, (int32_t)grid.x);
     else if (dtype == TMI_BF16)
-        hipLaunchKernelGGL(clamp_fp_kernel<bf16_t>, grid, block, 0, st, (const bf16_t*)in, (bf16_t*)out, n, lo, hi, nan_mode);
+        hipLaunchKernelGGL(clamp_fp_kernel<bf16_t>, grid, block, 0, st, (const bf16_t*)in, (bf16_t*)out, n, lo, hi, nan_mode, (int32_t)grid.x);
     else
         return nullptr;
     return "clamp_fp";

@@ -249,9 +249,9 @@ struct PadArgs
 };
 
 template <int EB>
-__global__ __launch_bounds__(256) void pad_operands_kernel(PadArgs p)
+__global__ __launch_bounds__(256) void pad_operands_kernel(PadArgs p, int32_t blocks)
 {
-    for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < p.units_a + p.units_b; u += (int64_t)gridDim.x * 256)
+    for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < p.units_a + p.units_b; u += (int64_t)blocks * 256)
     {
         const bool is_b   = u >= p.units_a;
         const int64_t v   = is_b ? u - p.units_a : u;
@@ -308,9 +308,9 @@ bool launch_matmul_pad(hipStream_t st, int32_t eb, int32_t N, int32_t H, int32_t
     const int64_t blocks = (p.units_a + p.units_b + 255) / 256;
     const dim3 grid((unsigned)(blocks > 8192 ? 8192 : blocks));
     if (eb == 1)
-        hipLaunchKernelGGL(pad_operands_kernel<1>, grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL(pad_operands_kernel<1>, grid, dim3(256), 0, st, p, (int32_t)grid.x);
     else
-        hipLaunchKernelGGL(pad_operands_kernel<2>, grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL(pad_operands_kernel<2>, grid, dim3(256), 0, st, p, (int32_t)grid.x);
     return true;
 }
 

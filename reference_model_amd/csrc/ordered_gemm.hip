@@ -112,6 +112,7 @@ __global__ __launch_bounds__(64 * WM * WN, 4) void ordered_gemm_kernel(OrderedAr
     constexpr int NA = BM / RPP, NB = BN / RPP;
     static_assert(NA * RPP == BM && NB * RPP == BN && NB * kThreads == KC * BN, "staging");
     __shared__ float sa[2][BM * LD], sb[2][BN * LD];
+    __shared__ int met_infinite;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // neighbouring tiles share operand rows: a contiguous run of tiles for each of the eight L2s
@@ -416,6 +417,8 @@ __global__ __launch_bounds__(64 * WM * WN, 4) void ordered_gemm_kernel(OrderedAr
     };
 
     const int stages = (p.K + BK - 1) / BK;
+    if (tid == 0)
+        met_infinite = 0;
     load_stage(0);
     store_stage(0);
     __syncthreads();
@@ -439,7 +442,14 @@ __global__ __launch_bounds__(64 * WM * WN, 4) void ordered_gemm_kernel(OrderedAr
     };
     // A tap outside the image adds nothing in the reference; here it adds 0 * weight, which is not nothing when the weight is
     // infinite or NaN.  A tile that met such a weight is summed again one result at a time.
-    if (!MATMUL && p.padded && __syncthreads_or(finite != 0.0f))
+    if (!MATMUL && p.padded)
+    {
+        // (not __syncthreads_or: it brings 256 bytes of hidden arguments into every launch)
+        if (finite != 0.0f)
+            met_infinite = 1;
+        __syncthreads();
+    }
+    if (!MATMUL && p.padded && met_infinite)
     {
         for (int t = tid; t < BM * BN; t += kThreads)
         {

@@ -31,7 +31,7 @@ struct PoolArgs
     int32_t nan_mode;    // MAX_POOL2D, floating point: 1 = PROPAGATE, 2 = IGNORE
     int32_t groups;      // channel groups of VEC elements per pixel
     int32_t full_mult, full_k;    // AVG_POOL2D: reciprocal_scale of a whole window (ky * kx taps), worked out on the host
-    int32_t xcd_remap;            // the grid is a multiple of 8 workgroups: give each XCD a contiguous range of pixels
+    int32_t xcd_blocks;           // workgroups of an XCD, an eighth of the grid: each takes a contiguous range of pixels
 };
 
 template <typename T>
@@ -108,10 +108,9 @@ __global__ __launch_bounds__(256) void pool_kernel(PoolArgs a)
     // share input rows with the next output row: XCD x takes workgroups [x * per, x * per + per) of the pixel order, so
     // that neighbouring output rows meet in one L2 instead of fetching the shared rows from HBM twice.
     uint32_t bid = blockIdx.x;
-    if (a.xcd_remap)
-        bid = (bid & 7) * (gridDim.x >> 3) + (bid >> 3);
+    bid = (bid & 7) * (uint32_t)a.xcd_blocks + (bid >> 3);
     {
-        const int64_t i = (int64_t)bid * blockDim.x + threadIdx.x;
+        const int64_t i = (int64_t)bid * 256 + threadIdx.x;
         if (i >= a.total)
             return;
         // (pixel, channel group); totals below 2^32 are checked on the host
@@ -323,7 +322,7 @@ static const char* launch_pool_t(hipStream_t st, PoolArgs& a, int32_t N, const c
             return vec_label;
         }
     const int64_t blocks = ((a.total + 255) / 256 + 7) & ~int64_t(7);    // whole groups of 8 for the XCD order
-    a.xcd_remap          = 1;
+    a.xcd_blocks         = (int32_t)(blocks / 8);
     if (vec)
         hipLaunchKernelGGL((pool_kernel<T, AVG, VEC>), dim3((int)blocks), dim3(256), 0, st, a);
     else

@@ -90,9 +90,9 @@ template <bool VEC>
 __device__ __forceinline__ void relayout_rows(const RelayoutArgs& a, int64_t block, int64_t n_blocks)
 {
     const int64_t total  = a.n_rows * a.pieces;
-    const int64_t stride = n_blocks * blockDim.x;
+    const int64_t stride = n_blocks * 256;
     const int fill_word  = (a.fill & 0xff) * 0x01010101;
-    for (int64_t i = block * blockDim.x + threadIdx.x; i < total; i += stride)
+    for (int64_t i = block * 256 + threadIdx.x; i < total; i += stride)
     {
         const int64_t r   = i / a.pieces;
         const int piece   = (int)(i - r * a.pieces);
@@ -110,16 +110,16 @@ __device__ __forceinline__ void relayout_rows(const RelayoutArgs& a, int64_t blo
 }
 
 template <bool VEC>
-__global__ __launch_bounds__(256) void relayout_kernel(RelayoutArgs a)
+__global__ __launch_bounds__(256) void relayout_kernel(RelayoutArgs a, int32_t blocks)
 {
-    relayout_rows<VEC>(a, blockIdx.x, gridDim.x);
+    relayout_rows<VEC>(a, blockIdx.x, blocks);
 }
 
 // Two re-layouts (an operator's weights and its input) in one launch: the first blocks_a workgroups take the first.
 struct RelayoutPair
 {
     RelayoutArgs a, b;
-    int32_t blocks_a;
+    int32_t blocks_a, blocks_b;
 };
 
 __global__ __launch_bounds__(256) void relayout_pair_kernel(RelayoutPair p)
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256) void relayout_pair_kernel(RelayoutPair p)
     if ((int)blockIdx.x < p.blocks_a)
         relayout_rows<true>(p.a, blockIdx.x, p.blocks_a);
     else
-        relayout_rows<true>(p.b, (int)blockIdx.x - p.blocks_a, (int)gridDim.x - p.blocks_a);
+        relayout_rows<true>(p.b, (int)blockIdx.x - p.blocks_a, p.blocks_b);
 }
 
 static bool relayout_vec(RelayoutArgs& a)
@@ -150,9 +150,9 @@ static const char* launch_relayout(hipStream_t st, RelayoutArgs& a)
     const bool vec       = relayout_vec(a);
     const int64_t blocks = relayout_blocks(a);
     if (vec)
-        hipLaunchKernelGGL(relayout_kernel<true>, dim3((int)blocks), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(relayout_kernel<true>, dim3((int)blocks), dim3(256), 0, st, a, (int32_t)blocks);
     else
-        hipLaunchKernelGGL(relayout_kernel<false>, dim3((int)blocks), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(relayout_kernel<false>, dim3((int)blocks), dim3(256), 0, st, a, (int32_t)blocks);
     return "relayout";
 }
 
@@ -161,8 +161,8 @@ static const char* launch_relayout_pair(hipStream_t st, RelayoutArgs& a, Relayou
 {
     if (a.n_rows > 0 && b.n_rows > 0 && a.row_bytes > 0 && b.row_bytes > 0 && relayout_vec(a) && relayout_vec(b))
     {
-        RelayoutPair p{ a, b, (int32_t)relayout_blocks(a) };
-        hipLaunchKernelGGL(relayout_pair_kernel, dim3(p.blocks_a + (int)relayout_blocks(b)), dim3(256), 0, st, p);
+        RelayoutPair p{ a, b, (int32_t)relayout_blocks(a), (int32_t)relayout_blocks(b) };
+        hipLaunchKernelGGL(relayout_pair_kernel, dim3(p.blocks_a + p.blocks_b), dim3(256), 0, st, p);
         return "relayout_pair";
     }
     launch_relayout(st, a);
