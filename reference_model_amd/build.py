@@ -3,7 +3,8 @@
     python -m reference_model_amd.build [--force]
 
 hipcc cross-compiles without a GPU.  Every translation unit is compiled to an object file under
-csrc/build/ (in parallel) and linked into reference_model_amd/libtosa_mi355.so.
+csrc/build/ (in parallel) and linked into reference_model_amd/libtosa_mi355.so; the C++ host side (the runner, its
+known-answer tests and the Python operator calls, _calls.so) is built on top of it with g++.
 """
 from __future__ import annotations
 
@@ -12,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -19,6 +21,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 BUILD = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libtosa_mi355.so")
 HOST_BIN = os.path.join(HERE, "tosa_mi355_run")
+CALLS = os.path.join(HERE, "_calls.so")
 
 ARCH = "gfx950"
 # -packed-fp32-ops off: hipcc must not form v_pk_*_f32 from float code on this hardware pool.
@@ -111,6 +114,18 @@ def build_host(force: bool = False) -> list:
             if r.stderr.strip():
                 sys.stderr.write(r.stderr)
         outs.append(exe)
+    # the operator calls of capi.Context as a CPython extension
+    src = os.path.join(host, "pycalls.cc")
+    if force or not os.path.exists(CALLS) or any(os.path.getmtime(d) > os.path.getmtime(CALLS) for d in (src, os.path.join(INCLUDE, "tosa_mi355.h"))):
+        cmd = ["g++", "-O2", "-std=c++17", "-Wall", "-Wextra", "-Wno-missing-field-initializers", "-fPIC", "-shared", f"-I{INCLUDE}",
+               "-I" + sysconfig.get_paths()["include"], src, "-o", CALLS, f"-L{HERE}", "-ltosa_mi355", "-Wl,-rpath,$ORIGIN",
+               "-Wl,-rpath-link,/opt/rocm/lib"]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"g++ failed on pycalls.cc:\n{r.stdout}\n{r.stderr}")
+        if r.stderr.strip():
+            sys.stderr.write(r.stderr)
+    outs.append(CALLS)
     return outs
 
 
