@@ -580,18 +580,23 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // Layers with taps that are small and deep (at most 2.4 G multiply-adds on at most 64 tiles of 128 x 128 results, or
         // on at most 100 from 160 input channels on) and not the slab kernel's: workgroups that own tiles of 32 x 32 results
         // with K split over their waves, before the patch and GEMM kernels, which would keep a fraction of the chip busy.
-        // us patch kernel / this kernel, 3x3, fused RESCALE: [8,14,14,256]->256 14.3 / 9.0, [8,28,28,256]->256 stride 2
-        // 16.2 / 9.1, [8,7,7,512]->512 21.1 / 10.8, [8,14,14,512]->512 stride 2 22.5 / 10.8, [8,14,14,160]->160 13.6 / 4.5,
-        // [1,14,14,256]->256 14.2 / 6.9, [16,14,14,256]->256 (50 tiles) 14.4 / 12.8, [20,14,14,256]->256 (62) 14.5 / 12.8,
-        // [8,14,14,384]->384 18.8 / 15.2, [8,14,14,256]->512 14.5 / 12.8, [8,14,14,512]->256 23.2 / 15.7, [16,7,7,512]->512
-        // 21.2 / 15.1, [8,14,14,320]->320 16.6 / 8.8, [8,28,28,160]->160 (98) 13.8 / 9.2, [8,28,28,192]->192 (98) 12.1 / 11.4,
-        // 5x5 [8,14,14,192]->192 31.1 / 11.1, [8,56,56,32]->32 stride 2 6.8 / 3.9; ties at [24,14,14,256]->256 (74 tiles, 2.8 G)
-        // 14.6 / 15.0 and [32,7,7,512]->512 21.2 / 21.8; the other way: [32,14,14,256]->256 (98, 3.7 G) 15.2 / 18.7,
-        // [16,14,14,512]->512 23.6 / 34.2, [8,56,56,32]->64 (196) 5.3 / 11.9, [8,112,112,32]->32 8.1 / 19.5.
-        const bool split_first = g.KH * g.KW > 1 && macs <= 2400000000ll && (tiles128 <= 64 || (g.IC >= 160 && tiles128 <= 100));
-        if (!name && g.KH * g.KW > 1 && (ctx->kernel_choice == 5 || (ctx->kernel_choice == 0 && split_first)))
+        // us patch kernel / this kernel, 3x3, fused RESCALE: [8,14,14,256]->256 14.3 / 6.8, [8,28,28,256]->256 stride 2
+        // 16.2 / 8.0, [8,7,7,512]->512 21.1 / 8.1, [8,14,14,512]->512 stride 2 22.5 / 8.8, [8,14,14,160]->160 13.6 / 4.5,
+        // [1,14,14,256]->256 14.2 / 5.5, [16,14,14,256]->256 (50 tiles) 14.4 / 9.1, [8,14,14,384]->384 18.8 / 10.7,
+        // [16,7,7,512]->512 21.2 / 9.9, [8,14,14,320]->320 16.6 / 8.8, [8,28,28,160]->160 (98) 13.8 / 9.2, [8,28,28,192]->192 (98) 12.1 / 11.4,
+        // 5x5 [8,14,14,192]->192 31.1 / 11.1, [8,56,56,32]->32 stride 2 6.8 / 3.9; the other way:
+        // [8,56,56,32]->64 (196) 5.3 / 11.9, [8,112,112,32]->32 8.1 / 19.5.
+        // On 256, 384 or 512 channels the K-split kernel has a form with both operands in LDS, whose workgroups walk several
+        // blocks with their weights in registers: it leads up to 100 tiles of 128 x 128 whatever the depth.  us best other
+        // kernel / this form: [32,14,14,256]->256 (98 tiles, 3.7 G) 15.1 / 12.8, [8,28,28,256]->256 15.2 / 13.3, [32,7,7,512]->512
+        // (52) 21.6 / 14.2, [64,7,7,512]->512 (100, 7.4 G) 33.4 / 23.6, [16,14,14,512]->512 (100) 24.0 / 21.0; the other way:
+        // [8,28,28,384]->384 (147) 24.6 / 28.1, [8,56,56,256]->64 (196) 15.1 / 16.7, [64,14,14,256]->256 (196) 19.3 / 22.1.
+        // (Layers with int32 results keep the first rule's bounds: the test of the automatic choice fixes their routes.)
+        const bool split_small = g.KH * g.KW > 1 && macs <= 2400000000ll && (tiles128 <= 64 || (g.IC >= 160 && tiles128 <= 100));
+        const bool split_patch = rp.enabled && g.KH == 3 && g.KW == 3 && (g.IC == 256 || g.IC == 384 || g.IC == 512) && tiles128 <= 100;
+        if (!name && g.KH * g.KW > 1 && (ctx->kernel_choice == 5 || (ctx->kernel_choice == 0 && (split_small || split_patch))))
             name = launch_conv2d_ksplit(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out, pad_page,
-                                        ctx->flags_dev);
+                                        ctx->flags_dev, ctx->kernel_choice == 5 || split_small);
         // First layers (at most 4 input channels, 3 x 3 ... 7 x 7 taps): a pre-pass into the scratch buffer and the pointwise
         // kernel with a K step per row of taps, unless an operand of this call lies in that buffer already.
         if (!name && own_scratch && (ctx->kernel_choice == 5 || ctx->kernel_choice == 0))

@@ -109,10 +109,11 @@ const char* launch_conv2d_stem(hipStream_t st, int32_t in_dtype, int32_t out_dty
                                void* scratch, uint32_t* flag_word);
 
 // conv_ksplit.hip: small int8 CONV2D layers with taps and a long reduction (IC a multiple of 32, weight_zp 0): a workgroup
-// per tile of 32 x 32 results, K split over its waves, operands straight from global memory into registers
+// per tile of 32 x 32 results, K split over its waves, operands straight from global memory into registers; 3 x 3 taps on 256,
+// 384 or 512 channels through LDS.  `small`: the first form may take the layer, not only the second.
 const char* launch_conv2d_ksplit(hipStream_t st, int32_t in_dtype, int32_t out_dtype, const ConvGeom& g, const void* in,
                                  const void* w, const void* bias, int32_t in_zp, int32_t w_zp, const RescaleParams& rp,
-                                 void* out, const void* pad_page, uint32_t* flag_word);
+                                 void* out, const void* pad_page, uint32_t* flag_word, bool small);
 
 // direct.hip: one output element per lane, any legal shape.  out_dtype is the stored output type
 // (INT32 without rescale; the rescale output type with it; FP16/BF16/FP32 for floating point).

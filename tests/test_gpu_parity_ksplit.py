@@ -37,6 +37,20 @@ SHAPES = [
 ]
 
 
+# The form with both operands in LDS (3 x 3 taps on 256, 384 or 512 channels)
+SHAPES += [
+    (3, 14, 14, 384, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),     # twelve waves, a ragged channel tile, blocks past the last row
+    (1, 5, 33, 256, 8, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),       # two blocks across, one of 32 output channels in use
+    (1, 3, 70, 512, 16, 3, 3, (0, 1, 2, 0), (1, 1), (1, 1)),      # three blocks across, uneven paddings
+    (1, 19, 1, 256, 24, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),      # blocks of one column
+    (2, 27, 23, 256, 32, 3, 3, (1, 1, 0, 0), (2, 2), (1, 1)),     # stride 2: more pieces of a patch than a lane holds at once
+    (1, 21, 20, 512, 8, 3, 3, (2, 2, 2, 2), (2, 1), (2, 3)),      # stride and dilation differ by direction
+    (12, 14, 14, 256, 264, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),   # two pixel tiles a block, several blocks a workgroup
+    (9, 4, 4, 256, 16, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),       # images of half a block: the form without a patch
+    (1, 12, 12, 512, 8, 3, 3, (40, 40, 40, 40), (1, 1), (40, 40)),    # a patch that does not fit: the form without one
+]
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_ksplit_int32_results(ctx, shape):
     n, ih, iw, ic, oc, kh, kw, pad, stride, dil = shape
@@ -51,7 +65,7 @@ def test_ksplit_int32_results(ctx, shape):
         assert st == capi.VALID and np.array_equal(got, want), int(np.count_nonzero(got != want))
 
 
-@pytest.mark.parametrize("shape", SHAPES[1:8])
+@pytest.mark.parametrize("shape", SHAPES[1:8] + [SHAPES[11], SHAPES[17]])
 @pytest.mark.parametrize("out_dtype,out_zp", [(np.int8, -4), (np.int16, 0)])
 @pytest.mark.parametrize("shifts", ["36 to 44", "mixed with small"])
 def test_ksplit_fused_rescale(ctx, shape, out_dtype, out_zp, shifts):
