@@ -16,9 +16,9 @@
 //
 // What bounds it: a k of 32 x 32 results costs a SIMD 33.6 ns in fp32 (the instruction's 13.6 ns and the additions' 15.7 do not
 // overlap: the two share the fp32 units) and four k 108 ns in fp64, where the matrix pipe is the limit.  us one result per
-// lane -> these tiles, [16,28,28,256]x[256,3,3,256] of fp32: the operator 27 100 -> 356 (41.5 TFLOP/s), precise pass 7 300 ->
-// 338, bounds pass 7 300 -> 328; a third of the distance to the 190 us of the fp64 pipe is the last round of tiles (3.06 to a
-// CU), the rest the conversions to fp64 and the stages' barriers.
+// lane -> these tiles, [16,28,28,256]x[256,3,3,256] of fp32: the operator 27 100 -> 299 (49 TFLOP/s), precise pass 7 300 ->
+// 257, bounds pass 7 300 -> 255 (58 TFLOP/s); the distance to the 190 us of the fp64 pipe is the conversions to fp64, the
+// stages' barriers and the tiles left over by whole rounds (see launch_ordered).
 #include "tmi_mfma.h"
 
 namespace tmi
@@ -39,6 +39,7 @@ struct OrderedArgs
     FastDiv ow, oh, ic, kw;         // divisors of the pixel decode (OW, OH) and of the k decode (IC, KW)
     FastDiv tiles_n;
     int32_t tiles;                  // per batch
+    int32_t n_big;                  // of these, tiles that are not cut into quarters
     int32_t bias_len;
     uint32_t abs_mask;              // 0x7fffffff in the bounds pass, else all ones
     int32_t vec_a, vec_b;           // operand rows are whole, aligned groups of four elements
@@ -101,27 +102,22 @@ enum OrderedMode
     kMatmul
 };
 
-template <typename T, bool F64, int MODE, int WM, int WN, int BK>
-__global__ __launch_bounds__(64 * WM * WN, 4) void ordered_gemm_kernel(OrderedArgs p)
+// One workgroup's tile of results from (m0, n0) on; a wave has WT x WT of them.
+template <typename T, bool F64, int MODE, int WM, int WN, int BK, int WT>
+__device__ __forceinline__ void ordered_tile(const OrderedArgs& p, int m0, int n0, float* lds)
 {
     using acc_t            = typename OrderedAcc<F64>::scalar;
     constexpr bool MATMUL  = MODE == kMatmul;
-    constexpr int kThreads = 64 * WM * WN, BM = 32 * WM, BN = 32 * WN, LD = BK + 4;
+    constexpr int kThreads = 64 * WM * WN, BM = WT * WM, BN = WT * WN, LD = BK + 4;
     constexpr int KC  = BK / 4;          // groups of four k in a stage
     constexpr int RPP = kThreads / KC;   // rows a pass of the workgroup stages
     constexpr int NA = BM / RPP, NB = BN / RPP;
     static_assert(NA * RPP == BM && NB * RPP == BN && NB * kThreads == KC * BN, "staging");
-    __shared__ float sa[2][BM * LD], sb[2][BN * LD];
-    __shared__ int met_infinite;
+    float (*sa)[BM * LD] = reinterpret_cast<float (*)[BM * LD]>(lds);
+    float (*sb)[BN * LD] = reinterpret_cast<float (*)[BN * LD]>(lds + 2 * BM * LD);
+    int& met_infinite    = *reinterpret_cast<int*>(lds + 2 * (BM + BN) * LD);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // neighbouring tiles share operand rows: a contiguous run of tiles for each of the eight L2s
-    const uint32_t per_xcd = ((uint32_t)p.tiles + 7) >> 3;
-    const uint32_t tile    = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (tile >= (uint32_t)p.tiles)
-        return;
-    const uint32_t tm = fdiv(tile, p.tiles_n), tn = tile - tm * p.tiles_n.d;
-    const int m0 = (int)tm * BM, n0 = (int)tn * BN;
     const int64_t batch = blockIdx.y;
     const T* __restrict__ a_base = reinterpret_cast<const T*>(p.a) + (MATMUL ? batch * p.M * p.K : 0);
     const T* __restrict__ b_base = reinterpret_cast<const T*>(p.b) + (MATMUL ? batch * p.K * p.OC : 0);
@@ -345,8 +341,11 @@ __global__ __launch_bounds__(64 * WM * WN, 4) void ordered_gemm_kernel(OrderedAr
 
     // 32 x 32 results of a wave.  fp32: one instruction of four blocks, block q = lane / 16 of the operands = (row half q / 2,
     // column half q % 2), results in registers 4 q + r.  fp64: four instructions.
-    const int wm = (wave / WN) * 32, wn = (wave % WN) * 32, l16 = lane & 15, q = lane >> 4;
+    // 16 x 16 results of a wave.  fp32: the four blocks are four k, whose products are added one after the other.  fp64: one
+    // instruction.
+    const int wm = (wave / WN) * WT, wn = (wave % WN) * WT, l16 = lane & 15, q = lane >> 4;
     v16f acc32;
+    v4f acc4 = { 0, 0, 0, 0 };
     v4d acc64[4];
     if constexpr (F64)
     {
@@ -361,7 +360,42 @@ __global__ __launch_bounds__(64 * WM * WN, 4) void ordered_gemm_kernel(OrderedAr
             acc32[t] = 0.0f;
     }
     auto compute = [&](int buf) {
-        if constexpr (F64)
+        if constexpr (WT == 16)
+        {
+            const float* pa = &sa[buf][(wm + l16) * LD + q];
+            const float* pb = &sb[buf][(wn + l16) * LD + q];
+            float fa[BK / 4], fb[BK / 4];
+#pragma unroll
+            for (int k = 0; k < BK / 4; k++)
+                fa[k] = pa[4 * k], fb[k] = pb[4 * k];
+            if constexpr (F64)
+            {
+#pragma unroll
+                for (int k = 0; k < BK / 4; k++)
+                    acc64[0] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)fa[k], (double)fb[k], acc64[0], 0, 0, 0);
+            }
+            else
+            {
+                const v16f zero = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+                v16f prod       = __builtin_amdgcn_mfma_f32_16x16x1f32(fa[0], fb[0], zero, 0, 0, 0);
+#pragma unroll
+                for (int k = 0; k < BK / 4; k++)
+                {
+                    v16f next = prod;
+                    if (k + 1 < BK / 4)
+                    {
+                        float x = fa[k + 1];
+                        asm volatile("" : "+v"(x), "+v"(acc4));    // (as below: one product ahead, no more)
+                        next = __builtin_amdgcn_mfma_f32_16x16x1f32(x, fb[k + 1], zero, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int t = 0; t < 16; t++)
+                        acc4[t & 3] = acc4[t & 3] + prod[t];
+                    prod = next;
+                }
+            }
+        }
+        else if constexpr (F64)
         {
             const float* pa = &sa[buf][(wm + l16) * LD + q];
             const float* pb = &sb[buf][(wn + l16) * LD + q];
@@ -483,7 +517,7 @@ __global__ __launch_bounds__(64 * WM * WN, 4) void ordered_gemm_kernel(OrderedAr
     {
         // row lane / 16 + 4 r, column lane % 16: 16 lanes store 128 bytes of one pixel
 #pragma unroll
-        for (int t = 0; t < 4; t++)
+        for (int t = 0; t < (WT == 16 ? 1 : 4); t++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
             {
@@ -495,13 +529,53 @@ __global__ __launch_bounds__(64 * WM * WN, 4) void ordered_gemm_kernel(OrderedAr
     else
     {
 #pragma unroll
-        for (int t = 0; t < 16; t++)
+        for (int t = 0; t < (WT == 16 ? 4 : 16); t++)
         {
             const int m = m0 + wm + 16 * (t >> 3) + 4 * q + (t & 3), oc = n0 + wn + 16 * ((t >> 2) & 1) + l16;
             if (m < p.M && oc < p.OC)
-                store_result(m, oc, acc32[t]);
+                store_result(m, oc, WT == 16 ? acc4[t & 3] : acc32[t]);
         }
     }
+}
+
+template <int BM, int BN, int BK>
+constexpr int ordered_lds_floats()
+{
+    return 2 * (BM + BN) * (BK + 4) + 1;
+}
+
+template <typename T, bool F64, int MODE, int WM, int WN, int BK>
+__global__ __launch_bounds__(64 * WM * WN, 4) void ordered_gemm_kernel(OrderedArgs p)
+{
+    constexpr int BM = 32 * WM, BN = 32 * WN;
+    __shared__ __attribute__((aligned(16))) float lds[ordered_lds_floats<BM, BN, BK>()];
+    // neighbouring tiles share operand rows: a contiguous run of tiles for each of the eight L2s
+    const uint32_t per_xcd = ((uint32_t)p.tiles + 7) >> 3;
+    const uint32_t tile    = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tile >= (uint32_t)p.tiles)
+        return;
+    const uint32_t tm = fdiv(tile, p.tiles_n), tn = tile - tm * p.tiles_n.d;
+    ordered_tile<T, F64, MODE, WM, WN, BK, 32>(p, (int)tm * BM, (int)tn * BN, lds);
+}
+
+// The first p.n_big tiles of 64 x 64 (a multiple of eight) as above, each of the others as four workgroups of 32 x 32 results.
+template <typename T, bool F64, int MODE>
+__global__ __launch_bounds__(256, 4) void ordered_gemm_tail_kernel(OrderedArgs p)
+{
+    __shared__ __attribute__((aligned(16))) float lds[ordered_lds_floats<64, 64, 32>()];
+    const uint32_t n_big = (uint32_t)p.n_big;
+    if (blockIdx.x < n_big)
+    {
+        const uint32_t tile = (blockIdx.x & 7) * (n_big >> 3) + (blockIdx.x >> 3);
+        const uint32_t tm = fdiv(tile, p.tiles_n), tn = tile - tm * p.tiles_n.d;
+        ordered_tile<T, F64, MODE, 2, 2, 32, 32>(p, (int)tm * 64, (int)tn * 64, lds);
+        return;
+    }
+    const uint32_t quarter = blockIdx.x - n_big, tile = n_big + (quarter >> 2);
+    const uint32_t tm = fdiv(tile, p.tiles_n), tn = tile - tm * p.tiles_n.d;
+    const int m0 = (int)tm * 64 + 32 * (int)((quarter >> 1) & 1), n0 = (int)tn * 64 + 32 * (int)(quarter & 1);
+    if (m0 < p.M && n0 < p.OC)
+        ordered_tile<T, F64, MODE, 2, 2, 32, 16>(p, m0, n0, lds);
 }
 
 template <typename T, bool F64, int MODE>
@@ -509,8 +583,8 @@ static bool launch_ordered(hipStream_t st, OrderedArgs p, int64_t batches)
 {
     // Workgroups of four waves and 64 x 64 results, in stages of 32 (of 16 where a reduction of at most 96 would leave half a
     // stage empty); of two waves and 64 x 32 or 32 x 64 where a ragged side would leave more than a quarter of those empty.  A
-    // wave has 32 x 32 results in every shape, so a smaller workgroup only shares fewer operand rows (us 64 x 64 / 32 x 64,
-    // fp64 [16,28,28,256]->256 332 / 389, [1,14,14,256]->256 106 / 120).
+    // wave has 32 x 32 results in every such shape, so a smaller workgroup only shares fewer operand rows (us 64 x 64 / 32 x 64,
+    // fp64 [16,28,28,256]->256 332 / 389).
     auto padded_area = [&](int bm, int bn) { return (int64_t)((p.M + bm - 1) / bm) * bm * ((p.OC + bn - 1) / bn) * bn; };
     const int64_t area = padded_area(64, 64);
     int bm = 64, bn = 64;
@@ -518,6 +592,25 @@ static bool launch_ordered(hipStream_t st, OrderedArgs p, int64_t batches)
         bn = 32;
     else if (4 * padded_area(32, 64) < 3 * area)
         bm = 32;
+    const bool short_stages = MODE != kTapStages && p.K <= 96 && (p.K & 31) != 0 && (p.K & 31) <= 16;
+    // Quarters: a round of tiles is one per CU, a wave on each SIMD, and takes as long for one tile as for 256.  Up to 192 tiles
+    // (together, or left over by whole rounds) are cut into four workgroups of 32 x 32 results, 16 x 16 a wave, which take a
+    // quarter of the time each and spread over four times the SIMDs; beyond, four quarters a CU are a round again.  us whole
+    // tiles / quarters, fp32 operator and fp64 pass: [16,28,28,256]->256 3x3 (784 tiles: 16 left over) 330 and 314 / 299 and 257,
+    // [1,14,14,256]->256 (16) 130 and 102 / 45 and 45, [4,28,28,128]->128 (98) 71 and 56 / 33 and 34, [3,28,28,256]->256 (148) 137
+    // and 104 / 85 and 85, [9,28,28,256]->256 (444: 188 left over) fp64 188 / 161, MATMUL 333 x 500 x 300 (30) 34 and 26 / 14 and 12.
+    const int64_t tiles64 = area / 4096, tn64 = (p.OC + 63) / 64;
+    const int64_t over       = tiles64 % 256;    // left over by whole rounds
+    const bool all_quarters  = tiles64 * batches <= 192;
+    const bool some_quarters = batches == 1 && bm == 64 && bn == 64 && !short_stages && over > 0 && over <= 192;
+    if ((all_quarters || some_quarters) && tiles64 <= INT32_MAX / 4 && fastdiv_exact_up_to((uint64_t)tiles64, (uint32_t)tn64))
+    {
+        p.n_big   = (int32_t)(all_quarters ? 0 : tiles64 - over);
+        p.tiles_n = make_fastdiv((uint32_t)tn64), p.tiles = (int32_t)tiles64;
+        const dim3 grid((unsigned)(p.n_big + 4 * (tiles64 - p.n_big)), (unsigned)batches);
+        hipLaunchKernelGGL((ordered_gemm_tail_kernel<T, F64, MODE>), grid, dim3(256), 0, st, p);
+        return true;
+    }
     const int64_t tiles = padded_area(bm, bn) / (bm * bn);
     const int64_t tn = (p.OC + bn - 1) / bn;
     if (!fastdiv_exact_up_to((uint64_t)tiles + 8, (uint32_t)tn) || tiles > INT32_MAX - 8 || batches > 65535)
@@ -528,7 +621,7 @@ static bool launch_ordered(hipStream_t st, OrderedArgs p, int64_t batches)
         hipLaunchKernelGGL((ordered_gemm_kernel<T, F64, MODE, 2, 1, 16>), grid, dim3(128), 0, st, p);
     else if (bm == 32)
         hipLaunchKernelGGL((ordered_gemm_kernel<T, F64, MODE, 1, 2, 16>), grid, dim3(128), 0, st, p);
-    else if (MODE != kTapStages && p.K <= 96 && (p.K & 31) != 0 && (p.K & 31) <= 16)
+    else if (short_stages)
         hipLaunchKernelGGL((ordered_gemm_kernel<T, F64, MODE, 2, 2, MODE == kTapStages ? 32 : 16>), grid, dim3(256), 0, st, p);
     else
         hipLaunchKernelGGL((ordered_gemm_kernel<T, F64, MODE, 2, 2, 32>), grid, dim3(256), 0, st, p);

@@ -25,6 +25,8 @@ CONVS = [  # n, ih, iw, ic, oc, k, pad, stride
     (1, 9, 9, 20, 70, 3, 1, 1),      # groups of four, stages across taps
     (2, 7, 9, 5, 66, 3, 1, 1),       # single elements
     (1, 9, 9, 16, 72, 1, 0, 1),      # a short reduction
+    (1, 63, 64, 32, 256, 2, 1, 1),   # 65 x 4 tiles: a whole round and four cut into quarters, the last row ragged
+    (1, 63, 64, 12, 200, 2, 1, 1),   # the same across taps, the last column ragged
 ]
 
 
@@ -56,7 +58,10 @@ def test_conv2d_in_the_references_order(ctx, case, infinite):
             assert np.array_equal(out.numpy(), want, equal_nan=True)
 
 
-@pytest.mark.parametrize("shape", [(1, 64, 32, 64), (2, 65, 33, 63), (3, 5, 17, 130), (1, 130, 100, 7), (2, 1, 3, 1), (1, 70, 96, 66)])
+@pytest.mark.parametrize("shape", [(1, 64, 32, 64), (2, 65, 33, 63), (3, 5, 17, 130), (1, 130, 100, 7), (2, 1, 3, 1), (1, 70, 96, 66),
+                                   # whole rounds of tiles, and with quarters behind; 64 x 32, 32 x 64, short stages; batches
+                                   (1, 1024, 50, 1000), (1, 4097, 35, 250), (1, 16600, 50, 20), (1, 20, 50, 16600), (1, 4097, 40, 250),
+                                   (70, 100, 33, 70), (48, 100, 33, 70)])
 def test_matmul_in_the_references_order(ctx, shape):
     n, h, c, w = shape
     rng = np.random.default_rng(h * c)
