@@ -173,6 +173,20 @@ int ensure_workspace(tmi_ctx* ctx, size_t bytes, bool exact = false)
     return TMI_VALID;
 }
 
+// The scratch buffer for a form that another kernel stands in for: false where the buffer would have to grow and cannot
+// (under capture, or out of memory), without an error.
+bool optional_workspace(tmi_ctx* ctx, size_t bytes)
+{
+    if (bytes <= ctx->workspace_size)
+        return true;
+    std::string before = ctx->last_error;
+    if (ensure_workspace(ctx, bytes) == TMI_VALID)
+        return true;
+    (void)hipGetLastError();
+    ctx->last_error = std::move(before);
+    return false;
+}
+
 int dtype_bits(int32_t dt)
 {
     switch (dt)
@@ -441,9 +455,8 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         const size_t need = depthwise || tiny || ctx->kernel_choice == 1 ? 0 : conv_i16_mfma_scratch_bytes(g, w_zp);
         if (need && (need == 1 || (own_scratch && !in_scratch(in) && !in_scratch(w) && !in_scratch(out) && !in_scratch(bias))))
         {
-            if (need > 1 && (rc = ensure_workspace(ctx, need)) != TMI_VALID)
-                return rc;
-            name = launch_conv_i16_mfma(ctx->stream, g, in, w, bias, out, ctx->workspace);
+            if (need == 1 || optional_workspace(ctx, need))
+                name = launch_conv_i16_mfma(ctx->stream, g, in, w, bias, out, ctx->workspace);
         }
         if (!name)
             name = launch_conv_i16_direct(ctx->stream, depthwise, g, in, w, bias, w_zp, out);
@@ -1381,13 +1394,11 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
                                     none, out_dev, (int64_t)W * C * eb, (int64_t)W * eb);
         if (name)
             return after_launch(ctx, label[0]);
+        MatmulPad m{};
         if (ctx->kernel_choice == 0 && large)
-        {
-            MatmulPad m;
             matmul_padded_sizes(eb, N, H, C, W, m);
-            int rc = ensure_workspace(ctx, m.a_bytes + m.b_bytes);
-            if (rc != TMI_VALID)
-                return rc;
+        if (ctx->kernel_choice == 0 && large && optional_workspace(ctx, m.a_bytes + m.b_bytes))
+        {
             if (!launch_matmul_pad(ctx->stream, eb, N, H, C, W, m, a_dev, b_dev, a_zp, b_zp, ctx->workspace))
                 return fail(ctx, "OpMatMul: operand copy launch failed");
             ConvGeom q = g;

@@ -161,3 +161,43 @@ def test_graph_of_transpose_conv_conv3d_and_avg_pool_matches_eager_on_every_repl
             assert len(torch.unique(t_out)) > 50 and len(torch.unique(c_out)) > 50 and len(torch.unique(p_out)) > 20
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("kind", ["int16", "int8"])
+def test_a_layer_with_ragged_channels_is_captured_without_scratch_memory(kind):
+    """Channel vectors of no whole pieces are copied into the scratch buffer where that buffer holds them or can grow.  A
+    context whose buffer is empty cannot grow it during capture: the layer then runs without the copies."""
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(3)
+    t = torch.int16 if kind == "int16" else torch.int8
+    n, hw, ic, oc = 2, 15, 137, 96
+    x = torch.from_numpy(rng.integers(-128, 128, (n, hw, hw, ic))).to(t).to(dev)
+    w = torch.from_numpy(rng.integers(-127, 128, (oc, 3, 3, ic)).astype(np.int8)).to(dev)
+    acc_t = torch.int64 if kind == "int16" else torch.int32
+    bias = torch.from_numpy(rng.integers(-9999, 9999, oc)).to(acc_t).to(dev)
+    results = []
+    for captured in (False, True):
+        ctx = Context(0)
+        try:
+            out = torch.zeros((n, hw, hw, oc), dtype=acc_t, device=dev)
+            d = ctx.conv_desc(capi.INT16 if kind == "int16" else capi.INT8, capi.INT48 if kind == "int16" else capi.INT32, tuple(x.shape),
+                              oc, 3, 3, (hw, hw), (1, 1, 1, 1), (1, 1), (1, 1), oc)
+            ctx.set_stream(torch.cuda.current_stream().cuda_stream)    # (leaves the context's own stream, outside the capture)
+            if captured:
+                graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+                side.wait_stream(torch.cuda.current_stream())
+                with torch.cuda.graph(graph, stream=side):
+                    ctx.set_stream(side.cuda_stream)
+                    ctx.conv2d(d, x, w, bias, 0, 0, out)
+                for _ in range(2):
+                    out.zero_()
+                    graph.replay()
+                    torch.cuda.synchronize()
+            else:
+                ctx.conv2d(d, x, w, bias, 0, 0, out)
+                assert ctx.sync() == capi.VALID
+            torch.cuda.synchronize()
+            results.append(out)
+        finally:
+            ctx.close()
+    assert torch.equal(*results) and len(torch.unique(results[0])) > 1000
