@@ -259,4 +259,71 @@ const char* launch_conv3d_operands(hipStream_t st, int32_t row_bytes, int32_t OC
     return launch_relayout_pair(st, a, b);
 }
 
+// Copies of CONV2D's operands with the channel vectors padded to whole steps of the matrix instruction (zeros; the weights'
+// zeros make whatever the input's are count for nothing), in one launch: a lane writes one 16-byte piece.  A piece that
+// crosses the end of its row is the row's last 16 bytes shifted down, so no lane reads past the tensor.
+struct PadRowsArgs
+{
+    const uint8_t *in, *w;
+    uint8_t *in_out, *w_out;
+    int64_t in_pieces, pieces;    // of the input's copy, of both
+    int32_t row_bytes, padded;    // bytes of a channel vector, before and after (at least 16; a multiple of 16)
+    FastDiv per_row;              // pieces of a padded row
+    int32_t grid;
+};
+
+typedef int rl_v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+
+__global__ __launch_bounds__(256) void pad_rows_kernel(PadRowsArgs a)
+{
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < a.pieces; i += (int64_t)a.grid * 256)
+    {
+        const bool is_w   = i >= a.in_pieces;
+        const uint32_t j  = (uint32_t)(is_w ? i - a.in_pieces : i);
+        const uint32_t row = fdiv(j, a.per_row);
+        const int at       = (int)(j - row * a.per_row.d) * 16;    // byte of the row
+        const uint8_t* src = (is_w ? a.w : a.in) + (int64_t)row * a.row_bytes;
+        const int left     = a.row_bytes - at;                     // bytes of the row from here on
+        rl_v4i v           = { 0, 0, 0, 0 };
+        if (left > 0)
+        {
+            const int from = left >= 16 ? at : a.row_bytes - 16;
+            v              = *reinterpret_cast<const rl_v4i_any*>(src + from);
+            if (left < 16)
+            {
+                const int s  = (16 - left) * 8;    // 8 ... 120 bits down
+                uint64_t lo  = (uint32_t)v.x | (uint64_t)(uint32_t)v.y << 32, hi = (uint32_t)v.z | (uint64_t)(uint32_t)v.w << 32;
+                lo           = s >= 64 ? hi >> (s - 64) : (lo >> s | hi << (64 - s));
+                hi           = s >= 64 ? 0 : hi >> s;
+                v            = rl_v4i{ (int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32) };
+            }
+        }
+        reinterpret_cast<rl_v4i*>(is_w ? a.w_out : a.in_out)[j] = v;
+    }
+}
+
+// 0 where the copies would be too large for 32-bit indices, else the bytes of both; `padded` is the padded row.
+size_t pad_channels_bytes(int64_t in_rows, int64_t w_rows, int32_t row_bytes, int32_t padded)
+{
+    if (row_bytes < 16 || in_rows * padded >= (int64_t(1) << 31) || w_rows * padded >= (int64_t(1) << 31) ||
+        !fastdiv_exact_up_to((uint64_t)(in_rows > w_rows ? in_rows : w_rows) * (padded / 16), (uint32_t)(padded / 16)))
+        return 0;
+    return (size_t)((in_rows * padded + 255) / 256 * 256 + w_rows * padded);
+}
+
+void launch_pad_channels(hipStream_t st, int64_t in_rows, int64_t w_rows, int32_t row_bytes, int32_t padded, const void* in, const void* w,
+                         void* scratch, const void** in_padded, const void** w_padded)
+{
+    PadRowsArgs a{};
+    a.in = (const uint8_t*)in, a.w = (const uint8_t*)w, a.in_out = (uint8_t*)scratch;
+    a.w_out     = a.in_out + (in_rows * padded + 255) / 256 * 256;
+    a.per_row   = make_fastdiv((uint32_t)padded / 16);
+    a.in_pieces = in_rows * (padded / 16), a.pieces = a.in_pieces + w_rows * (padded / 16);
+    a.row_bytes = row_bytes, a.padded = padded;
+    const int64_t blocks = (a.pieces + 255) / 256;
+    a.grid               = (int32_t)(blocks > 8192 ? 8192 : blocks);
+    hipLaunchKernelGGL(pad_rows_kernel, dim3(a.grid), dim3(256), 0, st, a);
+    *in_padded = a.in_out, *w_padded = a.w_out;
+}
+
 }    // namespace tmi

@@ -416,6 +416,40 @@ int validate_fused_rescale(tmi_ctx* ctx, const char* op, const tmi_conv_desc_t* 
     return TMI_VALID;
 }
 
+// CONV2D: the bytes a channel vector is padded to by a launch of its own (2.5 us and the copy), 0 to read the operands as they lie.
+// us as they lie / padded, graph replays, int8 with the fused RESCALE unless noted, 3x3 unless noted:
+int32_t padded_channel_bytes(int32_t in_dtype, const ConvGeom& g, int64_t total)
+{
+    const bool i8 = in_dtype == TMI_INT8;
+    if (!i8 && in_dtype != TMI_FP16 && in_dtype != TMI_BF16)
+        return 0;
+    const int32_t row = g.IC * (i8 ? 1 : 2);
+    if (row <= 16 || row > (1 << 20) || row % 32 == 0)
+        return 0;
+    const int32_t padded = (row + 31) / 32 * 32, taps = g.KH * g.KW;
+    // No whole words: the patch kernel stages them byte by byte.  [9,49,49,131]->112 82 / 25, [1,10,10,207]->400 56 / 8.1,
+    // [8,56,56,73]->72 54 / 21, [8,56,56,17]->64 10.7 / 8.0, [1,7,7,37]->24 10.3 / 6.0, 1x1 [8,56,56,65]->256 42 / 9.9, [8,112,112,37]->24
+    // 12.7 / 10.7, 5x5 [1,36,36,455]->16 176 / 52; fp16 [9,49,49,131]->112 138 / 31, [8,56,56,17]->64 13.8 / 6.9, 1x1 [8,56,56,65]->256 61 /
+    // 13.6; even: [8,112,112,18]->24 14.7 / 14.5, 1x1 [2,28,28,27]->32 4.9 / 4.9.
+    if (row % 4 != 0)
+        return padded;
+    // Whole words: where the slab kernel or the K-split kernel takes the padded layer and the patch kernel would have it else.
+    // [8,28,28,80]->80 9.7 / 7.0, [32,56,56,80]->80 48 / 32, [8,28,28,36]->64 7.4 / 6.1, [8,28,28,40]->64 6.8 / 6.1; [1,16,16,456]->160 35 /
+    // 11.6, [8,14,14,72]->72 13.0 / 6.7, [8,28,28,200]->128 19.8 / 14.0, [1,100,100,328]->16 25.8 / 14.2, stride 2 [2,28,28,464]->64 27 / 11.9;
+    // the other way: [8,28,28,40]->120 (49 tiles of 128 x 128) 9.6 / 11.4, [8,28,28,56]->56 8.0 / 8.1, [4,40,40,304]->100 20.2 / 23.1,
+    // 1x1 [8,28,28,200]->128 5.7 / 8.8.  fp16 [8,28,28,36]->64 10.4 / 5.9, [8,28,28,40]->64 7.1 / 6.0, [32,28,28,100]->100 40 / 30, 1x1
+    // [16,14,14,500]->300 30 / 17.5; the other way: [8,28,28,56]->56 7.6 / 10.0, [8,28,28,200]->128 19.2 / 23.3, [8,112,112,18]->24 11.4 / 17.0.
+    const int64_t pixels   = total / g.OC;
+    const int64_t tiles128 = ((pixels + 127) / 128) * ((g.OC + 127) / 128);
+    const bool slab        = taps == 9 && g.KH == 3 && g.OC % 16 == 0 && row > 32 && row <= 128;
+    if (!i8)
+        return (slab && !(g.stride_y * g.stride_x > 1)) || (row % 16 != 0 && g.IC >= 96) ? padded : 0;
+    const int64_t macs = total * padded * taps;
+    const bool split   = taps > 1 && row > 32 && g.OC % 8 == 0 && macs <= 2400000000ll && taps * (padded / 32) <= 160 &&
+                       tiles128 <= (padded >= 160 ? 100 : 32);
+    return slab || split ? padded : 0;
+}
+
 // check_level: false for the CONV2D that TRANSPOSE_CONV2D / CONV3D are evaluated as (their own limits were checked).
 // own_scratch: false when the caller holds operands of its own in a scratch buffer (the context's or the static one of
 // the entry point that allocates nothing): then no kernel that would grow or write the context's buffer is chosen.
@@ -492,6 +526,23 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
     if (depthwise && !name && ctx->kernel_choice != 1 && ctx->kernel_choice != 4 && ctx->kernel_choice != 6)
         name = launch_depthwise_vec(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                     ctx->flags_dev);
+    // Channel vectors of no whole steps, where kernels that need whole ones lead by more than the copies cost
+    if (!depthwise && ctx->kernel_choice == 0 && own_scratch && w_zp == 0)
+    {
+        const int32_t padded = padded_channel_bytes(d->in_dtype, g, total);
+        const int64_t in_rows = (int64_t)g.N * g.IH * g.IW, w_rows = (int64_t)g.OC * g.KH * g.KW;
+        const int32_t eb      = d->in_dtype == TMI_INT8 ? 1 : 2;
+        const size_t need     = padded ? pad_channels_bytes(in_rows, w_rows, g.IC * eb, padded) : 0;
+        if (need && !in_scratch(in) && !in_scratch(w) && !in_scratch(out) && !in_scratch(bias) && !in_scratch(rp.multiplier) &&
+            !in_scratch(rp.shift) && optional_workspace(ctx, need))
+        {
+            const void *in_padded, *w_padded;
+            launch_pad_channels(ctx->stream, in_rows, w_rows, g.IC * eb, padded, in, w, ctx->workspace, &in_padded, &w_padded);
+            tmi_conv_desc_t q = *d;
+            q.IC              = padded / eb;
+            return run_conv(ctx, op, false, &q, in_padded, w_padded, bias, in_zp, w_zp, rp, out_dtype, out, false, false);
+        }
+    }
     if (!depthwise && ctx->kernel_choice != 1)
     {
         // kernel choice 2 / 3 name one kernel; left open, the likely faster one is tried first

@@ -230,6 +230,10 @@ const char* launch_tconv_operands(hipStream_t st, int32_t row_bytes, int32_t OC,
 const char* launch_conv3d_operands(hipStream_t st, int32_t row_bytes, int32_t OC, int32_t KD, int32_t KHW, const void* w_src,
                                    void* w_dst, int32_t N, int32_t ID, int32_t OD, int32_t HW, int32_t stride_d,
                                    int32_t dilation_d, int32_t pad_d0, int32_t fill, const void* in_src, void* in_dst);
+// CONV2D's operands with the channel vectors padded from row_bytes to `padded` bytes of zeros, both in `scratch`
+size_t pad_channels_bytes(int64_t in_rows, int64_t w_rows, int32_t row_bytes, int32_t padded);
+void launch_pad_channels(hipStream_t st, int64_t in_rows, int64_t w_rows, int32_t row_bytes, int32_t padded, const void* in, const void* w,
+                         void* scratch, const void** in_padded, const void** w_padded);
 // depthwise.hip: 4 channels per lane, dot4 across taps, fused epilogue; nullptr when not eligible.
 const char* launch_depthwise_vec(hipStream_t st, int32_t in_dtype, int32_t out_dtype, const ConvGeom& g,
                                  const void* in, const void* w, const void* bias, int32_t in_zp, int32_t w_zp,
