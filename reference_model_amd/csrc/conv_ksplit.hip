@@ -542,6 +542,177 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void conv_ksplit_patch_kerne
     raise_flags(a.flag_word, flags);
 }
 
+// 1 x 1 layers with few tiles and a long reduction (the classifier of a network, the last projections): a workgroup of eight
+// waves per 32 channels x 32 pixels, an eighth of K to a wave.  Both operands come in whole lines, KS loads of each in flight,
+// and turn into fragments in the wave's own part of the LDS, which then takes its partial tile: one barrier in all.  What bounds
+// it is that chain: arguments, one trip to memory, LDS, the exchange.  The K-split pointwise form (a lane per row, as above) and
+// this one, us, graph replays, fused RESCALE: [8,7,7,2048]->512 8.0 / 4.8, [8,1,1,2048]->1000 6.8 / 4.4, [1,1,1,1280]->1000 5.8 /
+// 3.8, [64,1,1,2048]->4096 8.0 / 4.8, [8,14,14,2048]->256 (392 tiles) 11.3 / 7.6, [32,7,7,2048]->512 (784) 15.2 / 13.6, [8,7,7,512]->2048
+// (832) 7.0 / 6.0; more tiles than that were not measured and stay where weights are kept over several tiles.
+struct PointSplitArgs
+{
+    const uint8_t* in;
+    const int8_t* w;
+    const int32_t* bias;
+    void* out;
+    uint32_t* flag_word;
+    RescaleParams rp;
+    int32_t P, OC;    // pixels, output channels
+    int32_t za, bias_len;
+    int32_t out_kind;
+    FastDiv div_oct;
+};
+
+template <int KS, bool ZA>
+__global__ __launch_bounds__(512, 2) void point_split_kernel(PointSplitArgs a)
+{
+    constexpr int NW = 8, IC = NW * KS * 32, kPieces = 2 * KS, kRow = kPieces * 16 + 16;
+    constexpr int kOwn = 2 * 32 * kRow > 4096 ? 2 * 32 * kRow : 4096;    // a wave's weights and pixels, later its partial tile
+    // [32 x HighWordScale][32 x (m, s)][NW waves x 32 start values][form] and the waves' parts
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    asm volatile("" ::"s"(a.in), "s"(a.w), "s"(a.bias), "s"(a.out), "s"(a.flag_word), "s"(a.rp.multiplier), "s"(a.rp.shift), "s"(a.rp.out_zp),
+                 "s"(a.rp.lo), "s"(a.rp.hi), "s"(a.P), "s"(a.OC), "s"(a.za), "s"(a.bias_len), "s"(a.out_kind), "s"(a.div_oct.magic), "s"(a.div_oct.d));
+    const int tid  = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 31, lh = lane >> 5;
+    const uint32_t g = blockIdx.x;
+    const int pt = (int)fdiv(g, a.div_oct), oct = (int)g - pt * (int)a.div_oct.d;
+    HighWordScale* tab_hw = reinterpret_cast<HighWordScale*>(lds);
+    v2i* tab_ms           = reinterpret_cast<v2i*>(tab_hw + 32);
+    int32_t* wave_start   = reinterpret_cast<int32_t*>(tab_ms + 32) + wave * 32;
+    int32_t* form_word    = reinterpret_cast<int32_t*>(tab_ms + 32) + NW * 32;
+    uint8_t* parts        = reinterpret_cast<uint8_t*>(form_word + 4);
+    uint8_t* own          = parts + wave * kOwn;
+    const int wr = 4 * (li & 4) + ((li >> 1) & 12) + (li & 3);
+    const int ch = oct * 32 + wr;
+    int32_t b = 0, m_raw = 0, s_raw = 0;
+    if (wave == 0)
+    {
+        b = a.bias[a.bias_len == 1 ? 0 : (ch < a.OC ? ch : oct * 32)];
+        if (a.rp.enabled)
+        {
+            const int occ = oct * 32 + li < a.OC ? oct * 32 + li : oct * 32;
+            m_raw = load_multiplier(a.rp, occ), s_raw = load_shift(a.rp, occ);
+        }
+    }
+    v4i wb[KS], pb[KS];
+#pragma unroll
+    for (int i = 0; i < KS; i++)
+    {
+        const int r   = (i * 64 + lane) / kPieces, part = (i * 64 + lane) % kPieces;
+        const int row = oct * 32 + r, pix = pt * 32 + r;    // past the end: the last one again, zeroed or never stored
+        const uint32_t col = (uint32_t)(wave * KS * 32 + part * 16);
+        wb[i] = *reinterpret_cast<const v4i*>(a.w + ((uint32_t)(row < a.OC ? row : a.OC - 1) * (uint32_t)IC + col));
+        pb[i] = *reinterpret_cast<const v4i*>(a.in + ((uint32_t)(pix < a.P ? pix : a.P - 1) * (uint32_t)IC + col));
+    }
+#pragma unroll
+    for (int i = 0; i < KS; i++)
+    {
+        const int at = (i * 64 + lane + (i * 64 + lane) / kPieces) * 16;
+        *reinterpret_cast<v4i*>(own + at)             = wb[i];
+        *reinterpret_cast<v4i*>(own + 32 * kRow + at) = pb[i];
+    }
+    __builtin_amdgcn_wave_barrier();    // the wave's own LDS accesses complete in order
+    v4i fa[KS], fb[KS];
+#pragma unroll
+    for (int s = 0; s < KS; s++)
+    {
+        fa[s] = *reinterpret_cast<const v4i*>(own + wr * kRow + s * 32 + 16 * lh);
+        fb[s] = *reinterpret_cast<const v4i*>(own + 32 * kRow + li * kRow + s * 32 + 16 * lh);
+    }
+    uint32_t flags = 0;
+    if (wave == 0 && a.rp.enabled)
+        split_tables(a, oct, lane, m_raw, s_raw, tab_hw, tab_ms, form_word, flags);
+    if ((oct + 1) * 32 > a.OC)
+    {
+#pragma unroll
+        for (int s = 0; s < KS; s++)
+            fa[s] = ch < a.OC ? fa[s] : v4i{ 0, 0, 0, 0 };
+    }
+    if constexpr (ZA)
+    {
+        int sum = 0;
+#pragma unroll
+        for (int s = 0; s < KS; s++)
+            sum += dot4_ones(fa[s]);
+        sum += __builtin_amdgcn_ds_bpermute((lane ^ 32) * 4, sum);
+        b = (int32_t)((uint32_t)b - (uint32_t)a.za * (uint32_t)sum);
+    }
+    if (lh == 0)
+        wave_start[wr] = ch < a.OC ? b : 0;
+    __builtin_amdgcn_wave_barrier();
+    v16i acc;
+#pragma unroll
+    for (int gq = 0; gq < 4; gq++)
+    {
+        const v4i b4 = *reinterpret_cast<const v4i*>(wave_start + 16 * lh + 4 * gq);
+        acc[4 * gq] = b4[0], acc[4 * gq + 1] = b4[1], acc[4 * gq + 2] = b4[2], acc[4 * gq + 3] = b4[3];
+    }
+#pragma unroll
+    for (int s = 0; s < KS; s++)
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[s], fb[s], acc, 0, 0, 0);
+#pragma unroll
+    for (int gq = 0; gq < 4; gq++)
+        *reinterpret_cast<v4i*>(own + (gq * 64 + lane) * 16) = v4i{ acc[4 * gq], acc[4 * gq + 1], acc[4 * gq + 2], acc[4 * gq + 3] };
+    __syncthreads();    // the partial tiles and the tables are there
+    if (wave < 4)
+    {
+        const uint8_t* part = parts + wave * 1024 + lane * 16;
+        v4i sum = *reinterpret_cast<const v4i*>(part);
+#pragma unroll
+        for (int w2 = 1; w2 < NW; w2++)
+        {
+            const v4i o = *reinterpret_cast<const v4i*>(part + w2 * kOwn);
+            sum.x += o.x, sum.y += o.y, sum.z += o.z, sum.w += o.w;
+        }
+        const int p = pt * 32 + li, c0 = 16 * lh + 4 * wave, oc = oct * 32 + c0;
+        const bool store = p < a.P && oc < a.OC;    // OC is a multiple of 8: the four are in or out together
+        split_store(a, sum, c0, store ? (size_t)p * a.OC + oc : 0, store, a.rp.enabled ? *form_word : 0, tab_hw, tab_ms, flags);
+    }
+    raise_flags(a.flag_word, flags);
+}
+
+template <int KS>
+static bool launch_point_split_ks(hipStream_t st, const PointSplitArgs& a, int grid)
+{
+    constexpr int own = 2 * 32 * (KS * 32 + 16) > 4096 ? 2 * 32 * (KS * 32 + 16) : 4096;
+    constexpr int lds_bytes = 32 * 16 + 32 * 8 + 8 * 128 + 16 + 8 * own;
+    auto go = [&](auto kern, LdsLimit& granted) {
+        if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
+            return false;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds_bytes, st, a);
+        last_launch_shape[0] = grid, last_launch_shape[1] = 512, last_launch_shape[2] = lds_bytes;
+        return true;
+    };
+    static LdsLimit granted[2]{};
+    return a.za != 0 ? go(point_split_kernel<KS, true>, granted[1]) : go(point_split_kernel<KS, false>, granted[0]);
+}
+
+// False where the form does not apply.  (The caller has checked the layer: see launch_conv2d_pointwise.)
+bool launch_point_split(hipStream_t st, const ConvGeom& g, const void* in, const void* w, const void* bias, int32_t in_zp,
+                        const RescaleParams& rp, int32_t out_kind, void* out, uint32_t* flag_word)
+{
+    const int64_t P = (int64_t)g.N * g.OH * g.OW, n_oct = (g.OC + 31) / 32, tiles = (P + 31) / 32 * n_oct;
+    if (g.IC % 256 != 0 || tiles > 1024 || (int64_t)g.OC * g.IC >= (int64_t(1) << 31))
+        return false;
+    PointSplitArgs a{};
+    a.in = (const uint8_t*)in, a.w = (const int8_t*)w, a.bias = (const int32_t*)bias, a.out = out, a.flag_word = flag_word, a.rp = rp;
+    a.P = (int32_t)P, a.OC = g.OC, a.za = in_zp, a.bias_len = g.bias_len, a.out_kind = out_kind;
+    a.div_oct = make_fastdiv((uint32_t)n_oct);
+    switch (g.IC / 256)
+    {
+        case 2: return launch_point_split_ks<2>(st, a, (int)tiles);
+        case 3: return launch_point_split_ks<3>(st, a, (int)tiles);
+        case 4: return launch_point_split_ks<4>(st, a, (int)tiles);
+        case 5: return launch_point_split_ks<5>(st, a, (int)tiles);
+        case 6: return launch_point_split_ks<6>(st, a, (int)tiles);
+        case 7: return launch_point_split_ks<7>(st, a, (int)tiles);
+        case 8: return launch_point_split_ks<8>(st, a, (int)tiles);
+        default: return false;
+    }
+}
+
 template <int KS, int NW, bool ZA>
 static bool launch_conv_ksplit_za(hipStream_t st, const ConvSplitArgs& a, int grid)
 {

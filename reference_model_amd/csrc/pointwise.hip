@@ -568,6 +568,9 @@ const char* launch_conv2d_pointwise(hipStream_t st, int32_t in_dtype, int32_t ou
     a.n_oct    = (g.OC + 31) / 32;
     a.n_pt     = (int32_t)((P + 31) / 32);
     a.div_oct  = make_fastdiv((uint32_t)a.n_oct);
+    const char* split_label = rp.enabled ? "conv2d_pointwise_ksplit_i8_rescale" : "conv2d_pointwise_ksplit_i8";
+    if (launch_point_split(st, g, in, w, bias, in_zp, rp, a.out_kind, out, flag_word))
+        return split_label;
     if (g.IC > 160)
     {
         // K split over the four waves of a workgroup.  A workgroup walks several pixel tiles with its weight fragments in
@@ -592,7 +595,7 @@ const char* launch_conv2d_pointwise(hipStream_t st, int32_t in_dtype, int32_t ou
         else
             launch_pointwise_ksplit<16>(st, a, grid);
         last_launch_shape[0] = grid, last_launch_shape[1] = kSplitWaves * 64, last_launch_shape[2] = 34064;
-        return rp.enabled ? "conv2d_pointwise_ksplit_i8_rescale" : "conv2d_pointwise_ksplit_i8";
+        return split_label;
     }
     // as many groups as there are pixel tiles, up to the waves the 256 CUs hold at once (12 each up to 64 input channels,
     // 8 beyond: the fragments of two pixel tiles in flight take the registers)

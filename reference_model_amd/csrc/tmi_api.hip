@@ -597,6 +597,12 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // 20.1 / 22.7 / 12.9, [32,14,14,1024]->256 11.9 / 16.1 / 10.2.  int32 results: [32,56,56,256]->64 15.0 / 17.3 / 17.3,
         // [8,14,14,256]->1024 5.6 / 6.1 / 6.0, [8,14,14,1024]->256 4.4 / 6.3 / 8.3.
         const bool slab_deep = d->in_dtype == TMI_INT8 && g.KH * g.KW == 1 && g.IC > 128 && g.IC <= 1024 && (g.IC <= 256 || macs <= 900000000ll);
+        // One round of single tiles on 512, 768 or 1024 channels: the pointwise kernel's form with both operands in LDS.  us slab /
+        // this: [4,14,14,1024]->256 (200 tiles) 4.6 / 3.8, [4,7,7,1024]->512 4.6 / 3.8, [4,7,7,768]->768 4.2 / 3.7, [8,7,7,512]->512 4.0 / 3.6,
+        // [1,28,28,512]->256 3.9 / 3.6; the other way: [4,14,14,512]->512 (400) 4.0 / 4.2, [8,7,7,512]->2048 (832) 4.4 / 6.0.
+        if (!name && ctx->kernel_choice == 0 && slab_deep && g.IC >= 512 && g.IC % 256 == 0 && tiles32 <= 256)
+            name = launch_conv2d_pointwise(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
+                                           ctx->flags_dev);
         if (!name && ctx->kernel_choice == 0 && slab_deep)
             name = launch_conv2d_slab(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out, pad_page,
                                       ctx->flags_dev);

@@ -108,6 +108,10 @@ const char* launch_conv2d_stem(hipStream_t st, int32_t in_dtype, int32_t out_dty
                                const void* w, const void* bias, int32_t in_zp, int32_t w_zp, const RescaleParams& rp, void* out,
                                void* scratch, uint32_t* flag_word);
 
+// conv_ksplit.hip: the form of launch_conv2d_pointwise's layers with both operands through LDS (IC = 512 ... 2048 in multiples
+// of 256, at most 1024 tiles of 32 x 32 results); false where it does not apply
+bool launch_point_split(hipStream_t st, const ConvGeom& g, const void* in, const void* w, const void* bias, int32_t in_zp,
+                        const RescaleParams& rp, int32_t out_kind, void* out, uint32_t* flag_word);
 // conv_ksplit.hip: small int8 CONV2D layers with taps and a long reduction (IC a multiple of 32, weight_zp 0): a workgroup
 // per tile of 32 x 32 results, K split over its waves, operands straight from global memory into registers; 3 x 3 taps on 256,
 // 384 or 512 channels through LDS.  `small`: the first form may take the layer, not only the second.

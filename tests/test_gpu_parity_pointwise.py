@@ -146,7 +146,9 @@ def test_pointwise_split_k_int32_and_fused(ctx, ic, oc):
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 1, 256, 64), (1, 1, 33, 384, 24), (8, 14, 14, 1024, 256), (8, 7, 7, 2048, 512),
-                                   (8, 56, 56, 256, 64), (8, 14, 14, 384, 96)])
+                                   (8, 56, 56, 256, 64), (8, 14, 14, 384, 96),
+                                   # both operands in LDS: one pixel, ragged tiles either way; past its 1024 tiles
+                                   (1, 1, 1, 512, 40), (3, 5, 11, 768, 72), (1, 1, 33, 1792, 1000), (1, 1, 31, 1536, 8), (1, 33, 33, 512, 1000)])
 @pytest.mark.parametrize("shifts", ["33 to 40", "mixed with small"])
 def test_pointwise_split_k_layers_and_forms(ctx, shape, shifts):
     """projection layers of ResNet-50 and MobileNetV2 at batch 8 (several pixel tiles per workgroup on the largest), one
