@@ -14,6 +14,8 @@
 // a quarter of the tile each (4 consecutive channels per lane).
 //
 // weight_zp must be 0, IC a multiple of 32, OC a multiple of 8, and K at most 160 steps (16 waves of 10).
+//
+// Two more forms below take their operands through LDS: 3 x 3 taps on 256, 384 or 512 channels, and 1 x 1 on 512 ... 2048.
 #include "tmi_mfma.h"
 
 namespace tmi

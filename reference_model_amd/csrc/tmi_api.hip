@@ -572,10 +572,10 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // multiply-adds on at most 1600 such tiles, or up to 900 M where the GEMM kernel would have at most 64 tiles of
         // 128 x 128 for the chip.  us GEMM kernel / this form, fused RESCALE: [8,28,28,192]->32 9.2 / 3.3, [8,14,14,384]->64
         // 7.4 / 3.8, [8,7,7,960]->320 9.7 / 4.3, [8,7,7,320]->1280 7.4 / 4.2, [8,14,14,1024]->256 10.0 / 6.9, [8,7,7,2048]->512
-        // 14.2 / 7.5, [8,28,28,512]->128 8.1 / 6.5, [8,7,7,512]->2048 8.0 / 6.4, [8,14,14,256]->1024 7.2 / 6.7, [8,56,56,256]->64
+        // 14.2 / 4.8, [8,28,28,512]->128 8.1 / 6.5, [8,7,7,512]->2048 8.0 / 6.4, [8,14,14,256]->1024 7.2 / 6.7, [8,56,56,256]->64
         // 7.1 / 7.0, [8,28,28,256]->256 7.1 / 6.7, [32,14,14,384]->96 7.6 / 5.3, [8,28,28,256]->128 7.0 / 5.3, [32,7,7,960]->320
         // 9.7 / 5.7; 500 - 900 M: [8,14,14,1024]->512 (52 tiles) 10.0 / 8.6, [8,28,28,1024]->128 (49) 10.1 / 8.7, [8,14,14,2048]->256
-        // (26) 14.2 / 11.0; the other way: [8,28,28,192]->384 (2352 small tiles) 7.0 / 7.6, [8,28,28,512]->256 (98 tiles of
+        // (26) 14.2 / 7.6; the other way: [8,28,28,192]->384 (2352 small tiles) 7.0 / 7.6, [8,28,28,512]->256 (98 tiles of
         // 128 x 128) 8.2 / 8.8, [8,14,14,768]->768 (78) 9.1 / 10.1, [8,56,56,256]->128 7.4 / 10.5.
         const int64_t pixels   = (int64_t)g.N * g.OH * g.OW;
         const int64_t tiles128 = ((pixels + 127) / 128) * ((g.OC + 127) / 128);
