@@ -137,7 +137,9 @@ const char* tmi_last_kernel(const tmi_ctx_t* ctx);
  * call that needs more than the buffer holds allocates a larger block and keeps the old one until
  * tmi_ctx_destroy(), so launches already enqueued and HIP graphs captured earlier stay valid; while the context's
  * stream is being captured such a call returns TMI_ERROR instead of allocating -- size the buffer beforehand with
- * this function or with one eager call of the same operator.  Has no counterpart in the reference. */
+ * this function or with one eager call of the same operator.  CONV2D layers with ragged channel vectors and large ragged
+ * MATMULs use the buffer where it holds their copies or can grow, and run without copies otherwise.  Has no counterpart in
+ * the reference. */
 int tmi_ctx_reserve_workspace(tmi_ctx_t* ctx, size_t bytes);
 
 /* Size of the scratch buffer in use (`live`) and of the outgrown blocks still held (`retired`); either pointer may be

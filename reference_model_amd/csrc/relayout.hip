@@ -33,11 +33,33 @@ struct RelayoutArgs
     uint8_t* dst;
     int64_t n_rows;       // destination rows
     int32_t row_bytes;    // bytes of one channel vector
-    int32_t pieces;       // pieces per row (row_bytes / 16 or row_bytes)
+    int32_t out_bytes;    // 0, or the bytes a destination row is padded to with zeros (a multiple of 16, row_bytes >= 16)
+    int32_t pieces;       // pieces per row (of 16 bytes or of one)
     int32_t fill;         // byte stored where the source has no row (input_zp)
     int32_t mode;
     int32_t d[10];        // mode-specific dimensions, see source_row()
 };
+
+typedef int rl_v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+
+// Bytes at ... at + 15 of a row of row_bytes >= 16, zeros past its end.  A piece that crosses the end is the row's last 16 bytes
+// shifted down, so no lane reads past the tensor.
+__device__ __forceinline__ rl_v4i row_piece(const uint8_t* row, int row_bytes, int at)
+{
+    const int left = row_bytes - at;
+    if (left <= 0)
+        return rl_v4i{ 0, 0, 0, 0 };
+    rl_v4i v = *reinterpret_cast<const rl_v4i_any*>(row + (left >= 16 ? at : row_bytes - 16));
+    if (left < 16)
+    {
+        const int s = (16 - left) * 8;    // 8 ... 120 bits down
+        uint64_t lo = (uint32_t)v.x | (uint64_t)(uint32_t)v.y << 32, hi = (uint32_t)v.z | (uint64_t)(uint32_t)v.w << 32;
+        lo          = s >= 64 ? hi >> (s - 64) : (lo >> s | hi << (64 - s));
+        hi          = s >= 64 ? 0 : hi >> s;
+        v           = rl_v4i{ (int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32) };
+    }
+    return v;
+}
 
 // Source row of a destination row, or -1 when the destination is a fill row.
 __device__ __forceinline__ int64_t source_row(const RelayoutArgs& a, int64_t r)
@@ -101,8 +123,9 @@ __device__ __forceinline__ void relayout_rows(const RelayoutArgs& a, int64_t blo
         {
             rl_v4i v = rl_v4i{ fill_word, fill_word, fill_word, fill_word };
             if (src >= 0)
-                v = *reinterpret_cast<const rl_v4i*>(a.src + src * a.row_bytes + piece * 16);
-            *reinterpret_cast<rl_v4i*>(a.dst + r * a.row_bytes + piece * 16) = v;
+                v = a.out_bytes ? row_piece(a.src + src * a.row_bytes, a.row_bytes, piece * 16)
+                                : *reinterpret_cast<const rl_v4i*>(a.src + src * a.row_bytes + piece * 16);
+            *reinterpret_cast<rl_v4i*>(a.dst + r * (a.out_bytes ? a.out_bytes : a.row_bytes) + piece * 16) = v;
         }
         else
             a.dst[r * a.row_bytes + piece] = src >= 0 ? a.src[src * a.row_bytes + piece] : (uint8_t)a.fill;
@@ -132,6 +155,11 @@ __global__ __launch_bounds__(256) void relayout_pair_kernel(RelayoutPair p)
 
 static bool relayout_vec(RelayoutArgs& a)
 {
+    if (a.out_bytes)
+    {
+        a.pieces = a.out_bytes / 16;
+        return true;
+    }
     const bool vec = (a.row_bytes & 15) == 0 && (((uintptr_t)a.src | (uintptr_t)a.dst) & 15) == 0;
     a.pieces       = vec ? a.row_bytes / 16 : a.row_bytes;
     return vec;
@@ -239,13 +267,15 @@ const char* launch_permute_w3d(hipStream_t st, int32_t row_bytes, int32_t OC, in
     return launch_relayout(st, a);
 }
 
-// TRANSPOSE_CONV2D's two operands (flipped taps; input with holes) in one launch where possible.
-const char* launch_tconv_operands(hipStream_t st, int32_t row_bytes, int32_t OC, int32_t KH, int32_t KW, const void* w_src,
+// TRANSPOSE_CONV2D's two operands (flipped taps; input with holes) in one launch where possible; out_bytes: 0, or what the channel
+// vectors of both are padded to.
+const char* launch_tconv_operands(hipStream_t st, int32_t row_bytes, int32_t out_bytes, int32_t OC, int32_t KH, int32_t KW, const void* w_src,
                                   void* w_dst, int32_t N, int32_t IH, int32_t IW, int32_t sy, int32_t sx, int32_t fill,
                                   const void* in_src, void* in_dst)
 {
     RelayoutArgs a = flip_taps_args(row_bytes, OC, KH, KW, w_src, w_dst);
     RelayoutArgs b = upsample_args(row_bytes, N, IH, IW, sy, sx, fill, in_src, in_dst);
+    a.out_bytes = b.out_bytes = out_bytes;
     return launch_relayout_pair(st, a, b);
 }
 
@@ -260,8 +290,7 @@ const char* launch_conv3d_operands(hipStream_t st, int32_t row_bytes, int32_t OC
 }
 
 // Copies of CONV2D's operands with the channel vectors padded to whole steps of the matrix instruction (zeros; the weights'
-// zeros make whatever the input's are count for nothing), in one launch: a lane writes one 16-byte piece.  A piece that
-// crosses the end of its row is the row's last 16 bytes shifted down, so no lane reads past the tensor.
+// zeros make whatever the input's are count for nothing), in one launch: a lane writes one 16-byte piece.
 struct PadRowsArgs
 {
     const uint8_t *in, *w;
@@ -272,8 +301,6 @@ struct PadRowsArgs
     int32_t grid;
 };
 
-typedef int rl_v4i_any __attribute__((ext_vector_type(4), aligned(1)));
-
 __global__ __launch_bounds__(256) void pad_rows_kernel(PadRowsArgs a)
 {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < a.pieces; i += (int64_t)a.grid * 256)
@@ -283,22 +310,7 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(PadRowsArgs a)
         const uint32_t row = fdiv(j, a.per_row);
         const int at       = (int)(j - row * a.per_row.d) * 16;    // byte of the row
         const uint8_t* src = (is_w ? a.w : a.in) + (int64_t)row * a.row_bytes;
-        const int left     = a.row_bytes - at;                     // bytes of the row from here on
-        rl_v4i v           = { 0, 0, 0, 0 };
-        if (left > 0)
-        {
-            const int from = left >= 16 ? at : a.row_bytes - 16;
-            v              = *reinterpret_cast<const rl_v4i_any*>(src + from);
-            if (left < 16)
-            {
-                const int s  = (16 - left) * 8;    // 8 ... 120 bits down
-                uint64_t lo  = (uint32_t)v.x | (uint64_t)(uint32_t)v.y << 32, hi = (uint32_t)v.z | (uint64_t)(uint32_t)v.w << 32;
-                lo           = s >= 64 ? hi >> (s - 64) : (lo >> s | hi << (64 - s));
-                hi           = s >= 64 ? 0 : hi >> s;
-                v            = rl_v4i{ (int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32) };
-            }
-        }
-        reinterpret_cast<rl_v4i*>(is_w ? a.w_out : a.in_out)[j] = v;
+        reinterpret_cast<rl_v4i*>(is_w ? a.w_out : a.in_out)[j] = row_piece(src, a.row_bytes, at);
     }
 }
 

@@ -228,7 +228,7 @@ const char* launch_gather_depth(hipStream_t st, int32_t row_bytes, int32_t N, in
                                 const void* src, void* dst);
 const char* launch_permute_w3d(hipStream_t st, int32_t row_bytes, int32_t OC, int32_t KD, int32_t KHW,
                                const void* src, void* dst);
-const char* launch_tconv_operands(hipStream_t st, int32_t row_bytes, int32_t OC, int32_t KH, int32_t KW, const void* w_src,
+const char* launch_tconv_operands(hipStream_t st, int32_t row_bytes, int32_t out_bytes, int32_t OC, int32_t KH, int32_t KW, const void* w_src,
                                   void* w_dst, int32_t N, int32_t IH, int32_t IW, int32_t sy, int32_t sx, int32_t fill,
                                   const void* in_src, void* in_dst);
 const char* launch_conv3d_operands(hipStream_t st, int32_t row_bytes, int32_t OC, int32_t KD, int32_t KHW, const void* w_src,

@@ -59,6 +59,32 @@ def test_transpose_conv2d_i8_bit_exact(ctx, shape, zps):
         assert st == capi.VALID and np.array_equal(got, want), int(np.count_nonzero(got != want))
 
 
+RAGGED_TCONV = [  # channel vectors of no whole 16-byte pieces: padded while they are copied
+    (1, 5, 7, 17, 9, 3, 3, (0, 0, 0, 0), (2, 2)),
+    (2, 7, 11, 139, 40, 3, 3, (0, -1, 0, -1), (2, 2)),
+    (1, 6, 5, 58, 24, 4, 4, (-1, -1, -1, -1), (2, 2)),
+    (1, 9, 4, 31, 16, 2, 5, (1, 0, 0, 2), (1, 3)),
+]
+
+
+@pytest.mark.parametrize("shape", RAGGED_TCONV)
+@pytest.mark.parametrize("dtype", [capi.INT8, capi.FP16])
+def test_transpose_conv2d_with_ragged_channels(ctx, shape, dtype):
+    n, ih, iw, ic, oc, kh, kw, out_pad, stride = shape
+    rng = np.random.default_rng(ic)
+    if dtype == capi.INT8:
+        x, w = (rng.integers(-128, 128, s).astype(np.int8) for s in ((n, ih, iw, ic), (oc, kh, kw, ic)))
+        b = rng.integers(-9999, 9999, oc).astype(np.int32)
+        got, st = gpu_ops.transpose_conv2d(ctx, x, w, b, out_pad, stride, -5, 0)
+        assert st == capi.VALID and np.array_equal(got, oracle.transpose_conv2d("i8", x, w, b, out_pad, stride, -5, 0))
+        return
+    # whole quarters: the fp32 sums are exact, and one rounding of the result is all there is
+    x, w, b = (rng.integers(-8, 9, s).astype(np.float32) / 4 for s in ((n, ih, iw, ic), (oc, kh, kw, ic), (oc,)))
+    want = oracle.transpose_conv2d("f32", x, w, b, out_pad, stride)
+    got, st = gpu_ops.transpose_conv2d(ctx, *(v.astype(np.float16) for v in (x, w, b)), out_pad, stride, dtype=capi.FP16)
+    assert st == capi.VALID and np.all(np.abs(got.astype(np.float64) - want) <= 2.0 ** -11 * np.abs(want))
+
+
 SLAB_TCONV = [  # 3x3 taps, 64 / 96 / 128 input channels, zero weight_zp: both operands are read where they lie
     (2, 14, 14, 64, 48, (0, 0, 0, 0), (2, 2)),        # a decoder-style 2x upsampling layer
     (4, 28, 28, 128, 64, (0, -1, 0, -1), (2, 2)),     # cropped to exactly twice the input
