@@ -866,14 +866,16 @@ const char* launch_conv2d_ksplit(hipStream_t st, int32_t in_dtype, int32_t out_d
         !fastdiv_exact_up_to((uint64_t)P / g.OW + 1, (uint32_t)g.OH) || !fastdiv_exact_up_to((uint64_t)steps, (uint32_t)a.spt) ||
         !fastdiv_exact_up_to((uint64_t)taps, (uint32_t)g.KW))
         return nullptr;
-    bool ok = try_conv_ksplit_patch(st, g, a);
-    if (!ok && !small)
+    if (try_conv_ksplit_patch(st, g, a))
+        return rp.enabled ? "conv2d_ksplit_patch_i8_rescale" : "conv2d_ksplit_patch_i8";
+    if (!small)
         return nullptr;
-    if (!ok && nw == 4)
+    bool ok;
+    if (nw == 4)
         ok = ksw <= 4 ? launch_conv_ksplit<4, 4>(st, a, grid) : launch_conv_ksplit<10, 4>(st, a, grid);
-    else if (!ok && nw == 8)
+    else if (nw == 8)
         ok = launch_conv_ksplit<10, 8>(st, a, grid);
-    else if (!ok)
+    else
         ok = launch_conv_ksplit<10, 16>(st, a, grid);
     if (!ok)
         return nullptr;

@@ -579,7 +579,7 @@ __global__ __launch_bounds__(256, 4) void ordered_gemm_tail_kernel(OrderedArgs p
 }
 
 template <typename T, bool F64, int MODE>
-static bool launch_ordered(hipStream_t st, OrderedArgs p, int64_t batches)
+static OrderedForm launch_ordered(hipStream_t st, OrderedArgs p, int64_t batches)
 {
     // Workgroups of four waves and 64 x 64 results, in stages of 32 (of 16 where a reduction of at most 96 would leave half a
     // stage empty); of two waves and 64 x 32 or 32 x 64 where a ragged side would leave more than a quarter of those empty.  A
@@ -609,12 +609,12 @@ static bool launch_ordered(hipStream_t st, OrderedArgs p, int64_t batches)
         p.tiles_n = make_fastdiv((uint32_t)tn64), p.tiles = (int32_t)tiles64;
         const dim3 grid((unsigned)(p.n_big + 4 * (tiles64 - p.n_big)), (unsigned)batches);
         hipLaunchKernelGGL((ordered_gemm_tail_kernel<T, F64, MODE>), grid, dim3(256), 0, st, p);
-        return true;
+        return OrderedForm::quarters;
     }
     const int64_t tiles = padded_area(bm, bn) / (bm * bn);
     const int64_t tn = (p.OC + bn - 1) / bn;
     if (!fastdiv_exact_up_to((uint64_t)tiles + 8, (uint32_t)tn) || tiles > INT32_MAX - 8 || batches > 65535)
-        return false;
+        return OrderedForm::none;
     p.tiles_n = make_fastdiv((uint32_t)tn), p.tiles = (int32_t)tiles;
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)batches);
     if (bn == 32)
@@ -625,7 +625,7 @@ static bool launch_ordered(hipStream_t st, OrderedArgs p, int64_t batches)
         hipLaunchKernelGGL((ordered_gemm_kernel<T, F64, MODE, 2, 2, MODE == kTapStages ? 32 : 16>), grid, dim3(256), 0, st, p);
     else
         hipLaunchKernelGGL((ordered_gemm_kernel<T, F64, MODE, 2, 2, 32>), grid, dim3(256), 0, st, p);
-    return true;
+    return OrderedForm::tiles;
 }
 
 static bool aligned16(const void* p)
@@ -633,7 +633,7 @@ static bool aligned16(const void* p)
     return ((uintptr_t)p & 15) == 0;
 }
 
-bool launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w,
+OrderedForm launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w,
                          const void* bias, bool abs_mode, const double* input_abs_max, void* out)
 {
     const int64_t pixels = (int64_t)g.N * g.OH * g.OW, K = (int64_t)g.KH * g.KW * g.IC;
@@ -641,7 +641,7 @@ bool launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, const ConvG
     if (K < 1 || K > INT32_MAX - 64 || pixels > INT32_MAX - 64 || (int64_t)g.IH * g.IW * g.IC > INT32_MAX ||
         !fastdiv_exact_up_to((uint64_t)pixels, (uint32_t)g.OW) || !fastdiv_exact_up_to((uint64_t)pixels / g.OW, (uint32_t)g.OH) ||
         !fastdiv_exact_up_to((uint64_t)K, (uint32_t)g.IC) || !fastdiv_exact_up_to((uint64_t)g.KH * g.KW, (uint32_t)g.KW))
-        return false;
+        return OrderedForm::none;
     OrderedArgs p{};
     p.a = in, p.b = w, p.bias = bias, p.out = out, p.input_abs_max = input_abs_max;
     p.M = (int32_t)pixels, p.OC = g.OC, p.K = (int32_t)K, p.IH = g.IH, p.IW = g.IW, p.IC = g.IC, p.KW = g.KW;
@@ -654,34 +654,35 @@ bool launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, const ConvG
     const int64_t eb = in_dtype == TMI_FP32 ? 4 : 2;
     const bool taps  = p.vec_a && g.IC % 32 == 0 && (int64_t)g.N * g.IH * g.IW * g.IC * eb < INT32_MAX && (int64_t)g.OC * K * eb < INT32_MAX;
     if (!f64)
-        return in_dtype == TMI_FP32 && (taps ? launch_ordered<float, false, kTapStages>(st, p, 1) : launch_ordered<float, false, kAnyConv>(st, p, 1));
+        return in_dtype != TMI_FP32 ? OrderedForm::none
+                                    : (taps ? launch_ordered<float, false, kTapStages>(st, p, 1) : launch_ordered<float, false, kAnyConv>(st, p, 1));
     switch (in_dtype)
     {
         case TMI_FP16: return taps ? launch_ordered<_Float16, true, kTapStages>(st, p, 1) : launch_ordered<_Float16, true, kAnyConv>(st, p, 1);
         case TMI_BF16: return taps ? launch_ordered<bf16_t, true, kTapStages>(st, p, 1) : launch_ordered<bf16_t, true, kAnyConv>(st, p, 1);
         case TMI_FP32: return taps ? launch_ordered<float, true, kTapStages>(st, p, 1) : launch_ordered<float, true, kAnyConv>(st, p, 1);
-        default: return false;
+        default: return OrderedForm::none;
     }
 }
 
-bool launch_ordered_matmul(hipStream_t st, int32_t in_dtype, bool f64, int32_t N, int32_t H, int32_t C, int32_t W, const void* a,
+OrderedForm launch_ordered_matmul(hipStream_t st, int32_t in_dtype, bool f64, int32_t N, int32_t H, int32_t C, int32_t W, const void* a,
                            const void* b, bool abs_mode, void* out)
 {
     // 32-bit byte offsets inside a batch
     if (C < 1 || H > INT32_MAX - 64 || W > INT32_MAX - 64 || (int64_t)H * C > INT32_MAX / 4 || (int64_t)C * W > INT32_MAX / 4)
-        return false;
+        return OrderedForm::none;
     OrderedArgs p{};
     p.a = a, p.b = b, p.out = out, p.M = H, p.OC = W, p.K = C;
     p.bias_len = 1, p.abs_mask = abs_mode ? 0x7fffffffu : ~0u;
     p.vec_a = C % 4 == 0 && aligned16(a);
     if (!f64)
-        return in_dtype == TMI_FP32 && launch_ordered<float, false, kMatmul>(st, p, N);
+        return in_dtype != TMI_FP32 ? OrderedForm::none : launch_ordered<float, false, kMatmul>(st, p, N);
     switch (in_dtype)
     {
         case TMI_FP16: return launch_ordered<_Float16, true, kMatmul>(st, p, N);
         case TMI_BF16: return launch_ordered<bf16_t, true, kMatmul>(st, p, N);
         case TMI_FP32: return launch_ordered<float, true, kMatmul>(st, p, N);
-        default: return false;
+        default: return OrderedForm::none;
     }
 }
 

@@ -570,7 +570,7 @@ const char* launch_conv2d_pointwise(hipStream_t st, int32_t in_dtype, int32_t ou
     a.div_oct  = make_fastdiv((uint32_t)a.n_oct);
     const char* split_label = rp.enabled ? "conv2d_pointwise_ksplit_i8_rescale" : "conv2d_pointwise_ksplit_i8";
     if (launch_point_split(st, g, in, w, bias, in_zp, rp, a.out_kind, out, flag_word))
-        return split_label;
+        return rp.enabled ? "conv2d_pointwise_split_i8_rescale" : "conv2d_pointwise_split_i8";
     if (g.IC > 160)
     {
         // K split over the four waves of a workgroup.  A workgroup walks several pixel tiles with its weight fragments in

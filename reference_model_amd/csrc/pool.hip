@@ -306,7 +306,7 @@ __global__ __launch_bounds__(256) void pool_split_kernel(PoolArgs a)
 }
 
 template <typename T, bool AVG>
-static const char* launch_pool_t(hipStream_t st, PoolArgs& a, int32_t N, const char* vec_label, const char* label)
+static const char* launch_pool_t(hipStream_t st, PoolArgs& a, int32_t N, const char* vec_label, const char* label, const char* split_label = nullptr)
 {
     constexpr int VEC = 16 / (int)sizeof(T);
     const bool vec    = a.C % VEC == 0 && (((uintptr_t)a.in | (uintptr_t)a.out) & 15) == 0;
@@ -319,7 +319,7 @@ static const char* launch_pool_t(hipStream_t st, PoolArgs& a, int32_t N, const c
         if (vec && a.total <= 65536 && (int64_t)a.ky * a.kx >= 16 && (int64_t)a.ky * a.kx <= 65536)
         {
             hipLaunchKernelGGL((pool_split_kernel<T, AVG>), dim3((unsigned)((a.total + 15) / 16)), dim3(256), 0, st, a);
-            return vec_label;
+            return split_label;
         }
     const int64_t blocks = ((a.total + 255) / 256 + 7) & ~int64_t(7);    // whole groups of 8 for the XCD order
     a.xcd_blocks         = (int32_t)(blocks / 8);
@@ -354,12 +354,12 @@ const char* launch_pool(hipStream_t st, bool avg, int32_t dtype, int32_t N, int3
     {
         case TMI_INT8:
             a.qmin = -128, a.qmax = 127;
-            return avg ? launch_pool_t<int8_t, true>(st, a, N, "avg_pool2d_vec_i8", "avg_pool2d_i8")
-                       : launch_pool_t<int8_t, false>(st, a, N, "max_pool2d_vec_i8", "max_pool2d_i8");
+            return avg ? launch_pool_t<int8_t, true>(st, a, N, "avg_pool2d_vec_i8", "avg_pool2d_i8", "avg_pool2d_split_i8")
+                       : launch_pool_t<int8_t, false>(st, a, N, "max_pool2d_vec_i8", "max_pool2d_i8", "max_pool2d_split_i8");
         case TMI_INT16:
             a.qmin = -32768, a.qmax = 32767;
-            return avg ? launch_pool_t<int16_t, true>(st, a, N, "avg_pool2d_vec_i16", "avg_pool2d_i16")
-                       : launch_pool_t<int16_t, false>(st, a, N, "max_pool2d_vec_i16", "max_pool2d_i16");
+            return avg ? launch_pool_t<int16_t, true>(st, a, N, "avg_pool2d_vec_i16", "avg_pool2d_i16", "avg_pool2d_split_i16")
+                       : launch_pool_t<int16_t, false>(st, a, N, "max_pool2d_vec_i16", "max_pool2d_i16", "max_pool2d_split_i16");
         case TMI_FP16:
             return avg ? launch_pool_t<_Float16, true>(st, a, N, "avg_pool2d_vec_f16", "avg_pool2d_f16")
                        : launch_pool_t<_Float16, false>(st, a, N, "max_pool2d_vec_f16", "max_pool2d_f16");

@@ -231,8 +231,13 @@ const char* launch_conv_precise(hipStream_t st, int32_t in_dtype, bool depthwise
         }
         a.input_abs_max = abs_max_slot;
     }
-    if (!depthwise && launch_ordered_conv(st, in_dtype, true, g, in, w, bias, abs_mode != 0, a.input_abs_max, out))
-        return abs_mode ? "conv_bounds_f64" : "conv_precise_f64";
+    if (!depthwise)
+        switch (launch_ordered_conv(st, in_dtype, true, g, in, w, bias, abs_mode != 0, a.input_abs_max, out))
+        {
+            case OrderedForm::tiles: return abs_mode ? "conv_bounds_ordered_f64" : "conv_precise_ordered_f64";
+            case OrderedForm::quarters: return abs_mode ? "conv_bounds_ordered_tail_f64" : "conv_precise_ordered_tail_f64";
+            case OrderedForm::none: break;
+        }
     switch (in_dtype)
     {
         case TMI_FP16: hipLaunchKernelGGL(precise_conv_kernel<_Float16>, dim3(grid_for(a.total)), dim3(256), 0, st, a, grid_for(a.total)); break;
@@ -246,8 +251,12 @@ const char* launch_conv_precise(hipStream_t st, int32_t in_dtype, bool depthwise
 const char* launch_matmul_precise(hipStream_t st, int32_t in_dtype, int32_t N, int32_t H, int32_t C, int32_t W,
                                   const void* a, const void* b, int32_t abs_mode, double* out)
 {
-    if (launch_ordered_matmul(st, in_dtype, true, N, H, C, W, a, b, abs_mode != 0, out))
-        return abs_mode ? "matmul_bounds_f64" : "matmul_precise_f64";
+    switch (launch_ordered_matmul(st, in_dtype, true, N, H, C, W, a, b, abs_mode != 0, out))
+    {
+        case OrderedForm::tiles: return abs_mode ? "matmul_bounds_ordered_f64" : "matmul_precise_ordered_f64";
+        case OrderedForm::quarters: return abs_mode ? "matmul_bounds_ordered_tail_f64" : "matmul_precise_ordered_tail_f64";
+        case OrderedForm::none: break;
+    }
     const int64_t total = (int64_t)N * H * W;
     const dim3 grid(grid_for(total)), block(256);
     const int eb      = in_dtype == TMI_FP32 ? 4 : 2;

@@ -696,11 +696,15 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
     }
     if (!name && ctx->kernel_choice >= 2)
         return fail(ctx, "%s: no MFMA / vector kernel is eligible for this shape", op);
-    // FP32 sums keep the reference's order: the tiles of ordered_gemm.hip, under the label of the one-result-per-lane kernel,
-    // whose results they are bit for bit
-    if (!name && !depthwise && ctx->kernel_choice == 0 && d->in_dtype == TMI_FP32 &&
-        launch_ordered_conv(ctx->stream, TMI_FP32, false, g, in, w, bias, false, nullptr, out))
-        name = "conv2d_direct_f32";
+    // FP32 sums keep the reference's order: the tiles of ordered_gemm.hip, whose results are the one-result-per-lane kernel's bit
+    // for bit
+    if (!name && !depthwise && ctx->kernel_choice == 0 && d->in_dtype == TMI_FP32)
+        switch (launch_ordered_conv(ctx->stream, TMI_FP32, false, g, in, w, bias, false, nullptr, out))
+        {
+            case OrderedForm::tiles: name = "conv2d_ordered_f32"; break;
+            case OrderedForm::quarters: name = "conv2d_ordered_tail_f32"; break;
+            case OrderedForm::none: break;
+        }
     if (!name && depthwise)
         name = launch_depthwise_direct(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                        ctx->flags_dev);
@@ -1437,9 +1441,10 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
         g.bias_len = 1, g.M = 1;
         RescaleParams none{};
         const int32_t out_dtype = in_dtype == TMI_INT8 ? TMI_INT32 : TMI_FP32;
-        const char* const label[3] = { in_dtype == TMI_INT8 ? "matmul_gemm_i8" : (in_dtype == TMI_FP16 ? "matmul_gemm_f16" : "matmul_gemm_bf16"),
+        const char* const label[4] = { in_dtype == TMI_INT8 ? "matmul_gemm_i8" : (in_dtype == TMI_FP16 ? "matmul_gemm_f16" : "matmul_gemm_bf16"),
                                        in_dtype == TMI_INT8 ? "matmul_tgemm_i8" : (in_dtype == TMI_FP16 ? "matmul_tgemm_f16" : "matmul_tgemm_bf16"),
-                                       in_dtype == TMI_INT8 ? "matmul_mfma_i8" : (in_dtype == TMI_FP16 ? "matmul_mfma_f16" : "matmul_mfma_bf16") };
+                                       in_dtype == TMI_INT8 ? "matmul_mfma_i8" : (in_dtype == TMI_FP16 ? "matmul_mfma_f16" : "matmul_mfma_bf16"),
+                                       in_dtype == TMI_INT8 ? "matmul_pad_gemm_i8" : (in_dtype == TMI_FP16 ? "matmul_pad_gemm_f16" : "matmul_pad_gemm_bf16") };
         // What the GEMM kernel takes in place: rows of whole 64-byte pieces against rows of whole 16-byte pieces, from four tiles
         // of 128 x 128 on.  Its tiles walk K one after the other, so where there are few of them and K is deep the kernel that
         // splits K over waves leads: us GEMM / split, int8 [1,256,2048]x[..,1024] (16 tiles) 13.6 / 8.4, fp16 15.1 / 9.6,
@@ -1456,9 +1461,8 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
         if (ctx->kernel_choice == 0 && (in_place ? few_deep : !large))
         {
             name = launch_matmul_ragged(ctx->stream, in_dtype, N, H, C, W, a_dev, b_dev, a_zp, b_zp, out_dev);
-            // (products whose second operand alone has ragged rows keep the label they are known by)
             if (name)
-                return after_launch(ctx, rows_whole && !in_place ? label[1] : name);
+                return after_launch(ctx, name);
         }
         if (ctx->kernel_choice != 2)
             name = launch_gemm_mfma(ctx->stream, in_dtype, out_dtype, g, a_dev, b_dev, ctx->flags_dev + 16, a_zp, b_zp,
@@ -1477,7 +1481,7 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
             name       = launch_gemm_mfma(ctx->stream, in_dtype, out_dtype, q, m.pad_a ? ctx->workspace : a_dev, (uint8_t*)ctx->workspace + m.a_bytes,
                                           ctx->flags_dev + 16, a_zp, b_zp, none, out_dev, (int64_t)m.CP * m.ldw, m.ldw);
             if (name)
-                return after_launch(ctx, label[1]);
+                return after_launch(ctx, label[3]);
         }
         {
             const size_t bytes = (size_t)N * C * W * eb;
@@ -1502,9 +1506,13 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
     }
     if (!name && ctx->kernel_choice >= 2)
         return fail(ctx, "OpMatMul: no MFMA kernel is eligible for this shape");
-    if (!name && ctx->kernel_choice == 0 && in_dtype == TMI_FP32 &&
-        launch_ordered_matmul(ctx->stream, TMI_FP32, false, N, H, C, W, a_dev, b_dev, false, out_dev))
-        name = "matmul_direct_f32";
+    if (!name && ctx->kernel_choice == 0 && in_dtype == TMI_FP32)
+        switch (launch_ordered_matmul(ctx->stream, TMI_FP32, false, N, H, C, W, a_dev, b_dev, false, out_dev))
+        {
+            case OrderedForm::tiles: name = "matmul_ordered_f32"; break;
+            case OrderedForm::quarters: name = "matmul_ordered_tail_f32"; break;
+            case OrderedForm::none: break;
+        }
     if (!name)
         name = launch_matmul_direct(ctx->stream, in_dtype, N, H, C, W, a_dev, b_dev, a_zp, b_zp, out_dev);
     return after_launch(ctx, name);

@@ -129,10 +129,16 @@ const char* launch_depthwise_direct(hipStream_t st, int32_t in_dtype, int32_t ou
                                     const RescaleParams& rp, void* out, uint32_t* flag_word);
 // ordered_gemm.hip: CONV2D / MATMUL with the sums in the reference's order, tiled on the matrix cores: fp32 operands with fp32
 // sums (f64 false), or fp16 / bf16 / fp32 operands with fp64 sums and results (f64 true; abs_mode: over absolute values,
-// input_abs_max: device double that then replaces every input element, or nullptr).  false: not taken, nothing launched.
-bool launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w,
+// input_abs_max: device double that then replaces every input element, or nullptr).  none: not taken, nothing launched.
+enum class OrderedForm
+{
+    none,
+    tiles,       // ordered_gemm_kernel
+    quarters,    // ordered_gemm_tail_kernel: quarters of tiles, alone or behind whole rounds
+};
+OrderedForm launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w,
                          const void* bias, bool abs_mode, const double* input_abs_max, void* out);
-bool launch_ordered_matmul(hipStream_t st, int32_t in_dtype, bool f64, int32_t N, int32_t H, int32_t C, int32_t W, const void* a,
+OrderedForm launch_ordered_matmul(hipStream_t st, int32_t in_dtype, bool f64, int32_t N, int32_t H, int32_t C, int32_t W, const void* a,
                            const void* b, bool abs_mode, void* out);
 // precise.hip: fp64 precise-mode / bounds-mode passes (abs_mode != 0: sums over absolute values) of CONV2D,
 // DEPTHWISE_CONV2D and MATMUL on fp16 / bf16 / fp32 operands, and the DOT_PRODUCT check as a reduction that leaves one

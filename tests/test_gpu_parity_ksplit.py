@@ -40,15 +40,22 @@ SHAPES = [
 # The form with both operands in LDS (3 x 3 taps on 256, 384 or 512 channels)
 SHAPES += [
     (3, 14, 14, 384, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),     # twelve waves, a ragged channel tile, blocks past the last row
-    (1, 5, 33, 256, 8, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),       # two blocks across, one of 32 output channels in use
+    (1, 7, 49, 256, 8, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),       # two blocks across, one of 32 output channels in use
+    (1, 5, 33, 256, 8, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),       # two blocks across, too empty: the form without a patch
     (1, 3, 70, 512, 16, 3, 3, (0, 1, 2, 0), (1, 1), (1, 1)),      # three blocks across, uneven paddings
     (1, 19, 1, 256, 24, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),      # blocks of one column
     (2, 27, 23, 256, 32, 3, 3, (1, 1, 0, 0), (2, 2), (1, 1)),     # stride 2: more pieces of a patch than a lane holds at once
-    (1, 21, 20, 512, 8, 3, 3, (2, 2, 2, 2), (2, 1), (2, 3)),      # stride and dilation differ by direction
+    (1, 21, 28, 512, 8, 3, 3, (2, 2, 2, 2), (2, 1), (2, 3)),      # stride and dilation differ by direction
+    (1, 21, 20, 512, 8, 3, 3, (2, 2, 2, 2), (2, 1), (2, 3)),      # the same with blocks too empty: the form without a patch
     (12, 14, 14, 256, 264, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),   # two pixel tiles a block, several blocks a workgroup
     (9, 4, 4, 256, 16, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),       # images of half a block: the form without a patch
     (1, 12, 12, 512, 8, 3, 3, (40, 40, 40, 40), (1, 1), (40, 40)),    # a patch that does not fit: the form without one
 ]
+
+
+def kernel_of(shape, fused):
+    both_in_lds = shape[3] in (256, 384, 512) and shape[:4] not in ((1, 5, 33, 256), (1, 21, 20, 512), (9, 4, 4, 256), (1, 12, 12, 512))
+    return "conv2d_ksplit" + ("_patch" if both_in_lds else "") + "_i8" + ("_rescale" if fused else "")
 
 
 @pytest.mark.parametrize("shape", SHAPES)
@@ -61,11 +68,11 @@ def test_ksplit_int32_results(ctx, shape):
     for in_zp in (0, -128, 9):
         want = oracle.conv2d("i8", x, w, bias, pad, stride, dil, in_zp=in_zp, w_zp=0)
         got, st = gpu_ops.conv2d(ctx, x, w, bias, pad, stride, dil, in_zp=in_zp, w_zp=0)
-        assert ctx.last_kernel == "conv2d_ksplit_i8"
+        assert ctx.last_kernel == kernel_of(shape, False)
         assert st == capi.VALID and np.array_equal(got, want), int(np.count_nonzero(got != want))
 
 
-@pytest.mark.parametrize("shape", SHAPES[1:8] + [SHAPES[11], SHAPES[17]])
+@pytest.mark.parametrize("shape", SHAPES[1:8] + [SHAPES[11], SHAPES[19]])
 @pytest.mark.parametrize("out_dtype,out_zp", [(np.int8, -4), (np.int16, 0)])
 @pytest.mark.parametrize("shifts", ["36 to 44", "mixed with small"])
 def test_ksplit_fused_rescale(ctx, shape, out_dtype, out_zp, shifts):
@@ -84,7 +91,7 @@ def test_ksplit_fused_rescale(ctx, shape, out_dtype, out_zp, shifts):
         want = oracle.clamp(want, -90, 110)
         got, st = gpu_ops.conv2d(ctx, x, w, bias, pad, stride, dil, in_zp=-6, w_zp=0, clamp=(-90, 110),
                                  rescale=dict(mult=mult, shift=shift, out_zp=out_zp, out_dtype=out_dtype, rounding_mode=mode))
-        assert ctx.last_kernel == "conv2d_ksplit_i8_rescale"
+        assert ctx.last_kernel == kernel_of(shape, True)
         assert st == wst and np.array_equal(got, want), (st, wst, int(np.count_nonzero(got != want)))
     assert len(np.unique(got)) > 20
 
@@ -104,7 +111,7 @@ def test_ksplit_resnet_layers(ctx, shape):
     acc = cases.conv2d_exact_blas(x, w, bias, pad, (s, s), (1, 1), 4, 0)
     want, wst = oracle.rescale(acc, mult, shift, out_zp=1)
     got, st = gpu_ops.conv2d(ctx, x, w, bias, pad, (s, s), in_zp=4, w_zp=0, rescale=dict(mult=mult, shift=shift, out_zp=1))
-    assert ctx.last_kernel == "conv2d_ksplit_i8_rescale"
+    assert ctx.last_kernel == "conv2d_ksplit_patch_i8_rescale"
     assert st == wst == capi.VALID and np.array_equal(got, want), int(np.count_nonzero(got != want))
     assert len(np.unique(got)) > 100
 

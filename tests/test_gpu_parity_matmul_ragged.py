@@ -76,10 +76,10 @@ def test_large_products_on_aligned_copies(ctx, shape):
     rng = np.random.default_rng(h)
     a, b = rng.integers(-128, 128, (n, h, c)).astype(np.int8), rng.integers(-128, 128, (n, c, w)).astype(np.int8)
     got, st = gpu_ops.matmul(ctx, a, b, 7, -9)
-    assert st == capi.VALID and ctx.last_kernel == "matmul_tgemm_i8"
+    assert st == capi.VALID and ctx.last_kernel == "matmul_pad_gemm_i8"
     assert np.array_equal(got, np.matmul(a.astype(np.float64) - 7, b.astype(np.float64) + 9).astype(np.int64).astype(np.int32))
     x, y = (a / 64).astype(np.float16), (b / 64).astype(np.float16)
     got, st = gpu_ops.matmul(ctx, x, y, dtype=capi.FP16)
-    assert st == capi.VALID and ctx.last_kernel == "matmul_tgemm_f16"
+    assert st == capi.VALID and ctx.last_kernel == "matmul_pad_gemm_f16"
     x, y = x.astype(np.float64), y.astype(np.float64)
     assert dp.check(got, np.matmul(x, y), np.matmul(np.abs(x), np.abs(y)), "fp32", dp.kernel_size_bound(c, "fp32", has_bias=False))["ok"]

@@ -129,18 +129,19 @@ def test_pointwise_declines_what_it_does_not_take(ctx):
 def test_pointwise_split_k_int32_and_fused(ctx, ic, oc):
     """long channel vectors: the four waves of a workgroup take a quarter of K each (2, 4, 8 or 16 K steps a wave, the last
     wave's share ragged or empty) and meet in LDS"""
+    kernel = "conv2d_pointwise_split_i8" if ic % 256 == 0 and ic >= 512 else "conv2d_pointwise_ksplit_i8"    # the first: through LDS
     rng = np.random.default_rng(ic * 7 + oc)
     x, wt, bias = _operands(rng, 2, 5, 9, ic, oc)
     acc = oracle.conv2d("i8", x, wt, bias, in_zp=-9, w_zp=0)
     got, st = gpu_ops.conv2d(ctx, x, wt, bias, in_zp=-9, w_zp=0)
-    assert ctx.last_kernel == "conv2d_pointwise_ksplit_i8"
+    assert ctx.last_kernel == kernel
     assert st == capi.VALID and np.array_equal(got, acc), int(np.count_nonzero(got != acc))
     mult = rng.integers(1 << 30, 1 << 31, oc).astype(np.int32)
     shift = rng.integers(40, 46, oc).astype(np.int8)
     for out_dtype, out_zp in ((np.int8, 7), (np.int16, 0)):
         want, wst = oracle.rescale(acc, mult, shift, out_zp=out_zp, out_dtype=out_dtype)
         got, st = gpu_ops.conv2d(ctx, x, wt, bias, in_zp=-9, w_zp=0, rescale=dict(mult=mult, shift=shift, out_zp=out_zp, out_dtype=out_dtype))
-        assert ctx.last_kernel == "conv2d_pointwise_ksplit_i8_rescale"
+        assert ctx.last_kernel == kernel + "_rescale"
         assert st == wst == capi.VALID and np.array_equal(got, want), int(np.count_nonzero(got != want))
     assert len(np.unique(got)) > 50
 
@@ -154,6 +155,7 @@ def test_pointwise_split_k_layers_and_forms(ctx, shape, shifts):
     """projection layers of ResNet-50 and MobileNetV2 at batch 8 (several pixel tiles per workgroup on the largest), one
     pixel, a tile and one pixel; the high-word and the general form of the requantisation with zero input_zp and without"""
     n, h, w, ic, oc = shape
+    lds = ic % 256 == 0 and ic >= 512 and -(-n * h * w // 32) * -(-oc // 32) <= 1024
     rng = np.random.default_rng(n * h + ic + len(shifts))
     x, wt, bias = _operands(rng, n, h, w, ic, oc)
     small = shifts != "33 to 40"
@@ -167,5 +169,5 @@ def test_pointwise_split_k_layers_and_forms(ctx, shape, shifts):
         acc = cases.conv2d_exact_blas(x, wt, bias, (0, 0, 0, 0), (1, 1), (1, 1), in_zp, 0)
         want, wst = oracle.rescale(acc, mult, shift, out_zp=-1)
         got, st = gpu_ops.conv2d(ctx, x, wt, bias, in_zp=in_zp, w_zp=0, rescale=dict(mult=mult, shift=shift, out_zp=-1))
-        assert ctx.last_kernel == "conv2d_pointwise_ksplit_i8_rescale"
+        assert ctx.last_kernel == ("conv2d_pointwise_split_i8_rescale" if lds else "conv2d_pointwise_ksplit_i8_rescale")
         assert st == wst and np.array_equal(got, want), (st, wst, int(np.count_nonzero(got != want)))

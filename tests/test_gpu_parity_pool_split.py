@@ -28,6 +28,8 @@ def test_windows_over_sixteen_lanes(ctx, dtype, case):
     x = rng.integers(info.min, info.max + 1, (n, h, w, c)).astype(dtype)
     zps = (-7, 5) if dtype == np.int8 else (0, 0)
     got, st = gpu_ops.pool2d(ctx, x, k, s, p, True, *zps)
+    assert ctx.last_kernel == ("avg_pool2d_split_i8" if dtype == np.int8 else "avg_pool2d_split_i16")
     assert st == capi.VALID and np.array_equal(got, oracle.avg_pool2d(x, k, s, p, *zps))
     got, st = gpu_ops.pool2d(ctx, x, k, s, p, False)
+    assert ctx.last_kernel == ("max_pool2d_split_i8" if dtype == np.int8 else "max_pool2d_split_i16")
     assert st == capi.VALID and np.array_equal(got, oracle.max_pool2d(x, k, s, p))
