@@ -305,6 +305,25 @@ __global__ __launch_bounds__(256) void pool_split_kernel(PoolArgs a)
     raise_flags(a.flag_word, flags);
 }
 
+// Whether the split kernel leads, for `groups` results of `vec` channels under `taps` taps.  The other kernel's lane walks its
+// window in 0.165 us a tap whatever the number of groups, and in twice that where the image is larger than the eight L2s (32 MB);
+// this one's time is flat up to a wave per SIMD (4096 groups) and then grows with the groups, 0.52 us per 1000 on int8 and 0.13 -
+// 0.19 on int16, whose exchange is half as long.  us one lane a window / 16 lanes, AVG_POOL2D, graph replays: int8 4 x 4 taps, 64 groups 4.3 / 4.9, 16 384 5.0 / 9.9,
+// 65 536 5.1 / 31; 5 x 5, 1024 6.2 / 5.4, 6400 6.4 / 7.0, 65 536 6.6 / 32; 6 x 6, 8192 8.1 / 7.2, 12 288 8.1 / 8.9; 7 x 7, 1024 9.7 / 5.4,
+// 12 288 10.1 / 9.1, 16 384 10.1 / 11.1; 8 x 8, 16 384 12.4 / 11.1, overlapping windows 25 088 12.6 / 16.9; 10 x 10, 36 864 36 / 26, 65 536
+// 37 / 41; 12 x 12, 65 536 53 / 45; int16 4 x 4, 4096 4.4 / 3.5, 16 384 4.5 / 4.6; 5 x 5, 16 384 5.7 / 5.3, 36 864 5.7 / 8.5; 7 x 7, 36 864
+// 9.0 / 10.1; 8 x 8, 65 536 25 / 16; larger images: int8 8 x 8, 36 864 25 / 21.5, 65 536 26.5 / 36, 9 x 9, 36 864 30 / 25, 65 536 31 / 40, int16 7 x 7,
+// 65 536 18.5 / 15.  The kernel's divisions are exact up to 65 536 groups and taps.
+static bool pool_split_leads(int vec, int64_t groups, int64_t taps, int64_t image_bytes)
+{
+    if (groups > 65536 || taps > 65536)
+        return false;
+    const bool streams = image_bytes > (int64_t(32) << 20);
+    if (vec == 8)
+        return taps >= 16 && (taps >= 64 || taps * (streams ? 1500 : 750) >= groups);
+    return taps >= 24 && (taps >= 128 || (taps - 14) * 450 >= groups || (streams && taps * 650 >= groups));
+}
+
 template <typename T, bool AVG>
 static const char* launch_pool_t(hipStream_t st, PoolArgs& a, int32_t N, const char* vec_label, const char* label, const char* split_label = nullptr)
 {
@@ -314,9 +333,8 @@ static const char* launch_pool_t(hipStream_t st, PoolArgs& a, int32_t N, const c
     a.total           = (int64_t)N * a.OH * a.OW * a.groups;
     if (a.total >= (int64_t(1) << 32))
         return nullptr;
-    // few windows of many taps: below one wave per SIMD, from 16 taps on
     if constexpr (PoolType<T>::is_int)
-        if (vec && a.total <= 65536 && (int64_t)a.ky * a.kx >= 16 && (int64_t)a.ky * a.kx <= 65536)
+        if (vec && pool_split_leads(VEC, a.total, (int64_t)a.ky * a.kx, (int64_t)N * a.IH * a.IW * a.C * (int)sizeof(T)))
         {
             hipLaunchKernelGGL((pool_split_kernel<T, AVG>), dim3((unsigned)((a.total + 15) / 16)), dim3(256), 0, st, a);
             return split_label;
