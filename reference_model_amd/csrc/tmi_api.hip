@@ -416,9 +416,30 @@ int validate_fused_rescale(tmi_ctx* ctx, const char* op, const tmi_conv_desc_t* 
     return TMI_VALID;
 }
 
+// Tiny int8 layers: the patch kernel's set-up (4.4 us for a layer of a few workgroups, 1.8 more with the fused
+// RESCALE, 0.5 more when the channel vector is staged by 4- or 8-byte words and 1.8 when by bytes) exceeds what
+// the one-result-per-lane kernel takes, 2.6 us plus the longer of a lane's chain of K multiply-adds (90 ns each)
+// and the whole layer at 1000 multiply-adds per ns.  us patch kernel / direct kernel (graph replays, fused):
+// [1,32,32,8]->16 1x1 6.6 / 3.1, [1,64,64,8]->16 6.7 / 3.2, [8,32,32,8]->32 5.1 / 4.2, [1,32,32,16]->16 6.2 / 3.7,
+// [4,16,16,24]->48 6.5 / 4.2, 3x3 [1,32,32,3]->16 7.7 / 5.1, [1,112,112,3]->32 stride 2 6.9 / 5.8, int32 results
+// [2,32,32,8]->16 4.7 / 2.8, [1,32,32,16]->16 4.4 / 3.4; the other way: 3x3 [1,14,14,8]->16 6.7 / 8.5,
+// [1,28,28,12]->32 5.3 / 11.5, [1,224,224,3]->32 stride 2 7.7 / 11.9, 1x1 [8,56,56,8]->64 5.4 / 12.8,
+// [1,56,56,24]->144 6.3 / 9.9.
+double direct_us(const ConvGeom& g, int64_t total)
+{
+    const double k     = (double)g.KH * g.KW * g.IC;
+    const double chain = 0.09 * k, whole = (double)total * k * 1e-6;
+    return 2.6 + (chain > whole ? chain : whole);
+}
+bool direct_leads(const ConvGeom& g, int64_t total, bool fused)
+{
+    const double patch = 4.4 + ((g.IC & 15) == 0 ? 0.0 : ((g.IC & 3) == 0 ? 0.5 : 1.8)) + (fused ? 1.8 : 0.0);
+    return direct_us(g, total) + 0.3 < patch;
+}
+
 // CONV2D: the bytes a channel vector is padded to by a launch of its own (2.5 us and the copy), 0 to read the operands as they lie.
 // us as they lie / padded, graph replays, int8 with the fused RESCALE unless noted, 3x3 unless noted:
-int32_t padded_channel_bytes(int32_t in_dtype, const ConvGeom& g, int64_t total)
+int32_t padded_channel_bytes(int32_t in_dtype, const ConvGeom& g, int64_t total, bool fused)
 {
     const bool i8 = in_dtype == TMI_INT8;
     if (!i8 && in_dtype != TMI_FP16 && in_dtype != TMI_BF16)
@@ -427,6 +448,15 @@ int32_t padded_channel_bytes(int32_t in_dtype, const ConvGeom& g, int64_t total)
     if (row <= 16 || row > (1 << 20) || row % 32 == 0)
         return 0;
     const int32_t padded = (row + 31) / 32 * 32, taps = g.KH * g.KW;
+    // Tiny int8 layers that the one-result-per-lane kernel takes stay one launch: a second one costs an eager caller another 2.5 us on
+    // the host, and the copy 1.7 us on the device.  The padded layer is the better one where the pointwise kernel takes it and the
+    // chain of a lane is longer than that.  us as they lie / padded, eager calls and graph replays, fused 1x1: [1,8,8,17]->16 3.9 / 5.8
+    // and 3.8 / 4.3, [1,56,56,18]->24 4.6 / 6.2 and 4.6 / 5.1, [2,28,28,27]->32 4.8 / 6.3 and 4.8 / 5.1, [1,4,4,33]->8 4.9 / 5.7 and 5.1 / 4.3,
+    // [1,7,7,45]->64 6.1 / 6.3 and 6.2 / 4.8; not the pointwise kernel's: [1,28,28,21]->20 4.5 / 8.8 and 4.5 / 8.8, [1,14,14,33]->13 5.5 / 7.8
+    // and 5.4 / 7.9; int32 results: [1,56,56,17]->16 3.8 / 6.1 and 3.9 / 4.6, [1,14,14,33]->13 5.1 / 6.7 and 5.2 / 6.9.
+    const bool pointwise = taps == 1 && g.stride_y == 1 && g.stride_x == 1 && g.OH == g.IH && g.OW == g.IW && g.OC % 8 == 0;
+    if (i8 && direct_leads(g, total, fused) && (!pointwise || direct_us(g, total) < 5.6))
+        return 0;
     // No whole words: the patch kernel stages them byte by byte.  [9,49,49,131]->112 82 / 25, [1,10,10,207]->400 56 / 8.1,
     // [8,56,56,73]->72 54 / 21, [8,56,56,17]->64 10.7 / 8.0, [1,7,7,37]->24 10.3 / 6.0, 1x1 [8,56,56,65]->256 42 / 9.9, [8,112,112,37]->24
     // 12.7 / 10.7, 5x5 [1,36,36,455]->16 176 / 52; fp16 [9,49,49,131]->112 138 / 31, [8,56,56,17]->64 13.8 / 6.9, 1x1 [8,56,56,65]->256 61 /
@@ -529,7 +559,7 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
     // Channel vectors of no whole steps, where kernels that need whole ones lead by more than the copies cost
     if (!depthwise && ctx->kernel_choice == 0 && own_scratch && w_zp == 0)
     {
-        const int32_t padded = padded_channel_bytes(d->in_dtype, g, total);
+        const int32_t padded = padded_channel_bytes(d->in_dtype, g, total, rp.enabled);
         const int64_t in_rows = (int64_t)g.N * g.IH * g.IW, w_rows = (int64_t)g.OC * g.KH * g.KW;
         const int32_t eb      = d->in_dtype == TMI_INT8 ? 1 : 2;
         const size_t need     = padded ? pad_channels_bytes(in_rows, w_rows, g.IC * eb, padded) : 0;
@@ -624,25 +654,9 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         if (!name && ctx->kernel_choice == 0 && (g.IC <= 112 || deep_first))
             name = launch_conv2d_pointwise(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                            ctx->flags_dev);
-        // Tiny int8 layers: the patch kernel's set-up (4.4 us for a layer of a few workgroups, 1.8 more with the fused
-        // RESCALE, 0.5 more when the channel vector is staged by 4- or 8-byte words and 1.8 when by bytes) exceeds what
-        // the one-result-per-lane kernel takes, 2.6 us plus the longer of a lane's chain of K multiply-adds (90 ns each)
-        // and the whole layer at 1000 multiply-adds per ns.  us patch kernel / direct kernel (graph replays, fused):
-        // [1,32,32,8]->16 1x1 6.6 / 3.1, [1,64,64,8]->16 6.7 / 3.2, [8,32,32,8]->32 5.1 / 4.2, [1,32,32,16]->16 6.2 / 3.7,
-        // [4,16,16,24]->48 6.5 / 4.2, 3x3 [1,32,32,3]->16 7.7 / 5.1, [1,112,112,3]->32 stride 2 6.9 / 5.8, int32 results
-        // [2,32,32,8]->16 4.7 / 2.8, [1,32,32,16]->16 4.4 / 3.4; the other way: 3x3 [1,14,14,8]->16 6.7 / 8.5,
-        // [1,28,28,12]->32 5.3 / 11.5, [1,224,224,3]->32 stride 2 7.7 / 11.9, 1x1 [8,56,56,8]->64 5.4 / 12.8,
-        // [1,56,56,24]->144 6.3 / 9.9.
-        if (!name && ctx->kernel_choice == 0 && d->in_dtype == TMI_INT8)
-        {
-            const double k      = (double)g.KH * g.KW * g.IC;
-            const double chain  = 0.09 * k, whole = (double)total * k * 1e-6;
-            const double direct = 2.6 + (chain > whole ? chain : whole);
-            const double patch  = 4.4 + ((g.IC & 15) == 0 ? 0.0 : ((g.IC & 3) == 0 ? 0.5 : 1.8)) + (rp.enabled ? 1.8 : 0.0);
-            if (direct + 0.3 < patch)
-                name = launch_conv2d_direct(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
-                                            ctx->flags_dev);
-        }
+        if (!name && ctx->kernel_choice == 0 && d->in_dtype == TMI_INT8 && direct_leads(g, total, rp.enabled))
+            name = launch_conv2d_direct(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
+                                        ctx->flags_dev);
         // (left open, the slab kernel's layers with more than 128 input channels are the ones tried above)
         if (!name && (ctx->kernel_choice == 4 || (ctx->kernel_choice == 0 && g.IC <= 128 && d->in_dtype == TMI_INT8)))
             name = launch_conv2d_slab(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out, pad_page,

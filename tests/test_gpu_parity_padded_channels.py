@@ -17,16 +17,38 @@ def ctx():
     c.close()
 
 
-CASES = [  # n, h, w, ic, oc, k, pad, stride
-    (1, 7, 9, 17, 24, 3, 1, 1),       # one byte past a piece
-    (2, 9, 7, 31, 8, 3, 1, 1),        # one short of a step
-    (1, 8, 8, 33, 13, 1, 0, 1),
-    (3, 11, 5, 131, 40, 3, 1, 2),
-    (1, 6, 6, 207, 64, 2, 0, 1),
-    (2, 13, 13, 72, 72, 3, 1, 1),     # whole words, the K-split kernel
-    (2, 12, 12, 80, 80, 3, 1, 1),     # the slab kernel
-    (1, 10, 10, 245, 16, 3, 1, 1),    # padded to 256: both operands in LDS
-]
+CASES = {  # n, h, w, ic, oc, k, pad, stride: the kernel of the padded int8 layer (none of them takes it as it lies)
+    (1, 7, 9, 17, 24, 3, 1, 1): "conv2d_ksplit_i8",           # one byte past a piece
+    (2, 9, 7, 31, 8, 3, 1, 1): "conv2d_ksplit_i8",            # one short of a step
+    (1, 8, 8, 33, 13, 1, 0, 1): "conv2d_direct_i8",           # (tiny: stays as it lies)
+    (1, 8, 8, 65, 24, 1, 0, 1): "conv2d_pointwise_i8",
+    (3, 11, 5, 131, 40, 3, 1, 2): "conv2d_ksplit_i8",
+    (1, 6, 6, 207, 64, 2, 0, 1): "conv2d_ksplit_i8",
+    (2, 13, 13, 72, 72, 3, 1, 1): "conv2d_ksplit_i8",         # whole words
+    (2, 12, 12, 80, 80, 3, 1, 1): "conv2d_slab_i8",
+    (1, 10, 10, 245, 16, 3, 1, 1): "conv2d_ksplit_patch_i8",  # padded to 256: both operands in LDS
+}
+
+
+@pytest.mark.parametrize("ic, oc, fused, kernel", [
+    (17, 16, True, "conv2d_direct_i8_rescale"), (27, 32, True, "conv2d_direct_i8_rescale"), (45, 64, True, "conv2d_pointwise_i8_rescale"),
+    (21, 20, True, "conv2d_direct_i8_rescale"), (17, 16, False, "conv2d_direct_i8"), (37, 8, False, "conv2d_pointwise_i8")])
+def test_tiny_layers_stay_one_launch(ic, oc, fused, kernel):
+    """below the border the one-result-per-lane kernel reads the operands as they lie, without a copy in scratch memory"""
+    rng = np.random.default_rng(ic)
+    x, wt = rng.integers(-128, 128, (1, 9, 8, ic)).astype(np.int8), rng.integers(-128, 128, (oc, 1, 1, ic)).astype(np.int8)
+    bias = rng.integers(-999, 999, oc).astype(np.int32)
+    mult, shift = rng.integers(1 << 30, 1 << 31, oc).astype(np.int32), rng.integers(38, 43, oc).astype(np.int8)
+    want = oracle.conv2d("i8", x, wt, bias, (0, 0, 0, 0), (1, 1), (1, 1), in_zp=5, w_zp=0)
+    if fused:
+        want, _ = oracle.rescale(want, mult, shift, out_zp=3)
+    c = Context(0)
+    try:
+        got, st = gpu_ops.conv2d(c, x, wt, bias, in_zp=5, w_zp=0, rescale=dict(mult=mult, shift=shift, out_zp=3) if fused else None)
+        assert st == capi.VALID and np.array_equal(got, want)
+        assert c.last_kernel == kernel and (c.workspace_bytes() == (0, 0)) == ("direct" in kernel)
+    finally:
+        c.close()
 
 
 @pytest.mark.parametrize("case", CASES)
@@ -41,15 +63,15 @@ def test_int8(ctx, case, fused):
     want = oracle.conv2d("i8", x, wt, bias, pad, (s, s), (1, 1), in_zp=-11, w_zp=0)
     if not fused:
         got, st = gpu_ops.conv2d(ctx, x, wt, bias, pad, (s, s), in_zp=-11, w_zp=0)
-        assert st == capi.VALID and np.array_equal(got, want)
+        assert st == capi.VALID and np.array_equal(got, want) and ctx.last_kernel == CASES[case]
         return
     mult, shift = rng.integers(1 << 30, 1 << 31, oc).astype(np.int32), rng.integers(38, 43, oc).astype(np.int8)
     want, wst = oracle.rescale(want, mult, shift, out_zp=3)
     got, st = gpu_ops.conv2d(ctx, x, wt, bias, pad, (s, s), in_zp=-11, w_zp=0, rescale=dict(mult=mult, shift=shift, out_zp=3))
-    assert st == wst and np.array_equal(got, want) and len(np.unique(got)) > 20
+    assert st == wst and np.array_equal(got, want) and len(np.unique(got)) > 20 and ctx.last_kernel == CASES[case] + "_rescale"
 
 
-@pytest.mark.parametrize("case", CASES + [(1, 9, 9, 9, 16, 3, 1, 1), (1, 9, 9, 100, 40, 3, 1, 1), (2, 12, 12, 40, 64, 3, 1, 1)])
+@pytest.mark.parametrize("case", list(CASES) + [(1, 9, 9, 9, 16, 3, 1, 1), (1, 9, 9, 100, 40, 3, 1, 1), (2, 12, 12, 40, 64, 3, 1, 1)])
 @pytest.mark.parametrize("dtype", [capi.FP16, capi.BF16])
 def test_16_bit_floats(ctx, case, dtype):
     n, h, w, ic, oc, k, p, s = case
