@@ -1484,9 +1484,10 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
         if (name)
             return after_launch(ctx, label[0]);
         MatmulPad m{};
-        if (ctx->kernel_choice == 0 && large)
+        const bool copies = ctx->kernel_choice == 0 && !in_place && large && tiles128 >= 4;
+        if (copies)
             matmul_padded_sizes(eb, N, H, C, W, m);
-        if (ctx->kernel_choice == 0 && large && optional_workspace(ctx, m.a_bytes + m.b_bytes))
+        if (copies && optional_workspace(ctx, m.a_bytes + m.b_bytes))
         {
             if (!launch_matmul_pad(ctx->stream, eb, N, H, C, W, m, a_dev, b_dev, a_zp, b_zp, ctx->workspace))
                 return fail(ctx, "OpMatMul: operand copy launch failed");
@@ -1497,6 +1498,11 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
             if (name)
                 return after_launch(ctx, label[3]);
         }
+        // No room for the copies (the buffer cannot grow: under capture, or out of memory), or none that the GEMM kernel takes
+        if (ctx->kernel_choice == 0 && !in_place && large)
+            name = launch_matmul_ragged(ctx->stream, in_dtype, N, H, C, W, a_dev, b_dev, a_zp, b_zp, out_dev);
+        if (name)
+            return after_launch(ctx, name);
         {
             const size_t bytes = (size_t)N * C * W * eb;
             int rc             = ensure_workspace(ctx, bytes);

@@ -201,3 +201,38 @@ def test_a_layer_with_ragged_channels_is_captured_without_scratch_memory(kind):
         finally:
             ctx.close()
     assert torch.equal(*results) and len(torch.unique(results[0])) > 1000
+
+
+@pytest.mark.parametrize("kind, shape", [("int8", (1, 1300, 1301, 1303)), ("fp16", (2, 1100, 960, 1003)), ("int8", (1, 130, 250001, 66))])
+def test_a_large_ragged_product_is_captured_without_scratch_memory(kind, shape):
+    """Products whose operands would be copied into the scratch buffer, on a context whose buffer is empty and cannot grow: the
+    kernel that reads any operand where it lies, not an error.  (The last one has too few tiles for the copies in any case.)"""
+    dev = torch.device("cuda:0")
+    n, h, c, w = shape
+    rng = np.random.default_rng(h)
+    t, code, out_t = (torch.int8, capi.INT8, torch.int32) if kind == "int8" else (torch.float16, capi.FP16, torch.float32)
+    # whole numbers of at most 5: products and sums are exact in fp32
+    a, b = (torch.from_numpy(rng.integers(-5, 6, s)).to(t).to(dev) for s in ((n, h, c), (n, c, w)))
+    want = torch.from_numpy(np.matmul(a.cpu().numpy().astype(np.float64), b.cpu().numpy().astype(np.float64))).to(out_t).to(dev)
+    ctx = Context(0)
+    try:
+        out = torch.zeros((n, h, w), dtype=out_t, device=dev)
+        ctx.set_stream(torch.cuda.current_stream().cuda_stream)    # (leaves the context's own stream, outside the capture)
+        graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.graph(graph, stream=side):
+            ctx.set_stream(side.cuda_stream)
+            ctx.matmul(code, n, h, c, w, a, b, 0, 0, out)
+        assert ctx.last_kernel == ("matmul_ragged_i8" if kind == "int8" else "matmul_ragged_f16") and ctx.workspace_bytes() == (0, 0)
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+        ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+        out.zero_()
+        ctx.matmul(code, n, h, c, w, a, b, 0, 0, out)    # with room for them
+        assert ctx.sync() == capi.VALID and torch.equal(out, want)
+        assert ("pad_gemm" in ctx.last_kernel) == (h > 130)
+    finally:
+        ctx.close()
