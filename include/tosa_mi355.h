@@ -137,18 +137,24 @@ const char* tmi_last_kernel(const tmi_ctx_t* ctx);
  * call that needs more than the buffer holds allocates a larger block and keeps the old one until
  * tmi_ctx_destroy(), so launches already enqueued and HIP graphs captured earlier stay valid; while the context's
  * stream is being captured such a call returns TMI_ERROR instead of allocating -- size the buffer beforehand with
- * this function or with one eager call of the same operator.  CONV2D layers with ragged channel vectors and large ragged
- * MATMULs use the buffer where it holds their copies or can grow, and run without copies otherwise.  Has no counterpart in
- * the reference. */
+ * this function or with one eager call of the same operator.  Large ragged MATMULs use the buffer where it holds their
+ * copies or can grow, and run without copies otherwise.  Calls that use the buffer must not overlap in time: on one
+ * stream they are ordered, graphs captured from one context that hold such calls are not to run at once, nor beside
+ * eager calls of them on another stream.
+ * CONV2D layers with ragged channel vectors copy operands as well, into memory of their own: eager calls into one more
+ * buffer of the context, captured ones into a block that belongs to the capture and is kept with the outgrown ones (1 GiB
+ * in all; beyond, and where memory is short, they run without copies).  Graphs of such layers may run at once.
+ * Has no counterpart in the reference. */
 int tmi_ctx_reserve_workspace(tmi_ctx_t* ctx, size_t bytes);
 
-/* Size of the scratch buffer in use (`live`) and of the outgrown blocks still held (`retired`); either pointer may be
- * NULL.  An operator call that outgrows the buffer at least doubles it, so `retired` stays below `live` unless
- * tmi_ctx_reserve_workspace() was called with sizes of the caller's own choosing.  Has no counterpart in the reference. */
+/* Size of the scratch buffers in use (`live`) and of the blocks still held for launches and graphs (`retired`: outgrown
+ * ones and those of captured calls); either pointer may be NULL.  An operator call that outgrows a buffer at least doubles
+ * it, so the outgrown blocks sum to less than `live` unless tmi_ctx_reserve_workspace() was called with sizes of the
+ * caller's own choosing.  Has no counterpart in the reference. */
 int tmi_ctx_workspace_bytes(const tmi_ctx_t* ctx, size_t* live, size_t* retired);
 
-/* Frees the outgrown blocks after waiting for the context's stream.  Only for callers that hold no captured HIP graph
- * from before the last growth: such a graph may still name a block freed here.  Has no counterpart in the reference. */
+/* Frees the blocks counted in `retired` after waiting for the context's stream.  Only for callers that hold no captured
+ * HIP graph of this context: such a graph may still name a block freed here.  Has no counterpart in the reference. */
 int tmi_ctx_trim_workspace(tmi_ctx_t* ctx);
 
 /* ---- device memory (replaces Tensor::allocate / deallocate and the element-wise host copies of

@@ -53,7 +53,13 @@ struct tmi_ctx
     tmi::DpPartial* dp_partials = nullptr;    // pinned: the DOT_PRODUCT check's partial results, written by the device
     void* workspace       = nullptr;    // scratch for operand re-layout (MATMUL's transposed B)
     size_t workspace_size = 0;
-    std::vector<void*> retired;         // outgrown scratch blocks: captured graphs may still name them
+    void* copies          = nullptr;    // scratch for CONV2D's padded operands, eager calls only (see copy_scratch)
+    size_t copies_size    = 0;
+    void* captured        = nullptr;    // the same for the capture below: the last entry of `retired`
+    size_t captured_size  = 0;
+    unsigned long long capture_id = 0;
+    size_t captured_bytes = 0;          // of all such blocks in `retired`
+    std::vector<void*> retired;         // outgrown scratch blocks and those of captures: captured graphs may still name them
     size_t retired_bytes  = 0;          // their sizes, summed
     unsigned char* static_scratch = nullptr;    // this device's copy of the library's static scratch array
     uint32_t last_flags   = 0;
@@ -185,6 +191,62 @@ bool optional_workspace(tmi_ctx* ctx, size_t bytes)
     (void)hipGetLastError();
     ctx->last_error = std::move(before);
     return false;
+}
+
+// Scratch for the operand copies of a layer that another kernel would read where they lie: nullptr where there is none, without an
+// error.  Such layers share no buffer with anything that may run at the same time.  Eager calls use one of their own, ordered by
+// the context's stream; a call under capture gets a block that belongs to that capture (its launches are ordered too), kept like an
+// outgrown one until tmi_ctx_trim_workspace() or tmi_ctx_destroy(), at most 1 GiB of them in a context.
+void* copy_scratch(tmi_ctx* ctx, size_t bytes)
+{
+    constexpr size_t kMostCaptured = size_t(1) << 30;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    unsigned long long id     = 0;
+    if (hipStreamGetCaptureInfo(ctx->stream, &cs, &id) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    const bool capturing = cs == hipStreamCaptureStatusActive;
+    if (cs != hipStreamCaptureStatusNone && !capturing)
+        return nullptr;
+    if (capturing && ctx->captured && id == ctx->capture_id && bytes <= ctx->captured_size)
+        return ctx->captured;
+    if (!capturing && bytes <= ctx->copies_size)
+        return ctx->copies;
+    if (capturing && ctx->captured_bytes + bytes > kMostCaptured)
+        return nullptr;
+    const size_t want = !capturing && bytes < 2 * ctx->copies_size ? 2 * ctx->copies_size : bytes;
+    // an allocation is no part of a graph, but forbidden to a thread that captures in the default mode
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (capturing && hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    void* block        = nullptr;
+    const hipError_t e = hipMalloc(&block, want);
+    if (capturing)
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (capturing)
+    {
+        ctx->retired.push_back(block);
+        ctx->retired_bytes += want, ctx->captured_bytes += want;
+        ctx->captured = block, ctx->captured_size = want, ctx->capture_id = id;
+        return block;
+    }
+    if (ctx->copies)
+    {
+        ctx->retired.push_back(ctx->copies);
+        ctx->retired_bytes += ctx->copies_size;
+    }
+    ctx->copies = block, ctx->copies_size = want;
+    return block;
 }
 
 int dtype_bits(int32_t dt)
@@ -517,11 +579,9 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // 0.45 M, 6.2 / 4.6).
         const bool tiny   = total * g.KH * g.KW * g.IC < (1 << 17);
         const size_t need = depthwise || tiny || ctx->kernel_choice == 1 ? 0 : conv_i16_mfma_scratch_bytes(g, w_zp);
-        if (need && (need == 1 || (own_scratch && !in_scratch(in) && !in_scratch(w) && !in_scratch(out) && !in_scratch(bias))))
-        {
-            if (need == 1 || optional_workspace(ctx, need))
-                name = launch_conv_i16_mfma(ctx->stream, g, in, w, bias, out, ctx->workspace);
-        }
+        void* copies      = need > 1 && own_scratch ? copy_scratch(ctx, need) : nullptr;
+        if (need == 1 || copies)
+            name = launch_conv_i16_mfma(ctx->stream, g, in, w, bias, out, copies);
         if (!name)
             name = launch_conv_i16_direct(ctx->stream, depthwise, g, in, w, bias, w_zp, out);
         return after_launch(ctx, name);
@@ -563,11 +623,10 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         const int64_t in_rows = (int64_t)g.N * g.IH * g.IW, w_rows = (int64_t)g.OC * g.KH * g.KW;
         const int32_t eb      = d->in_dtype == TMI_INT8 ? 1 : 2;
         const size_t need     = padded ? pad_channels_bytes(in_rows, w_rows, g.IC * eb, padded) : 0;
-        if (need && !in_scratch(in) && !in_scratch(w) && !in_scratch(out) && !in_scratch(bias) && !in_scratch(rp.multiplier) &&
-            !in_scratch(rp.shift) && optional_workspace(ctx, need))
+        if (void* copies = need ? copy_scratch(ctx, need) : nullptr)
         {
             const void *in_padded, *w_padded;
-            launch_pad_channels(ctx->stream, in_rows, w_rows, g.IC * eb, padded, in, w, ctx->workspace, &in_padded, &w_padded);
+            launch_pad_channels(ctx->stream, in_rows, w_rows, g.IC * eb, padded, in, w, copies, &in_padded, &w_padded);
             tmi_conv_desc_t q = *d;
             q.IC              = padded / eb;
             return run_conv(ctx, op, false, &q, in_padded, w_padded, bias, in_zp, w_zp, rp, out_dtype, out, false, false);
@@ -791,6 +850,8 @@ int tmi_ctx_destroy(tmi_ctx_t* ctx)
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->workspace)
         (void)hipFree(ctx->workspace);
+    if (ctx->copies)
+        (void)hipFree(ctx->copies);
     for (void* block : ctx->retired)
         (void)hipFree(block);
     if (ctx->flags_dev)
@@ -934,7 +995,7 @@ int tmi_ctx_workspace_bytes(const tmi_ctx_t* ctx, size_t* live, size_t* retired)
     if (!ctx)
         return TMI_ERROR;
     if (live)
-        *live = ctx->workspace_size;
+        *live = ctx->workspace_size + ctx->copies_size;
     if (retired)
         *retired = ctx->retired_bytes;
     return TMI_VALID;
@@ -949,7 +1010,8 @@ int tmi_ctx_trim_workspace(tmi_ctx_t* ctx)
     for (void* b : ctx->retired)
         (void)hipFree(b);
     ctx->retired.clear();
-    ctx->retired_bytes = 0;
+    ctx->retired_bytes = ctx->captured_bytes = ctx->captured_size = 0;
+    ctx->captured      = nullptr;
     return TMI_VALID;
 }
 

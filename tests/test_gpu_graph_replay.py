@@ -164,9 +164,9 @@ def test_graph_of_transpose_conv_conv3d_and_avg_pool_matches_eager_on_every_repl
 
 
 @pytest.mark.parametrize("kind", ["int16", "int8"])
-def test_a_layer_with_ragged_channels_is_captured_without_scratch_memory(kind):
-    """Channel vectors of no whole pieces are copied into the scratch buffer where that buffer holds them or can grow.  A
-    context whose buffer is empty cannot grow it during capture: the layer then runs without the copies."""
+def test_a_layer_with_ragged_channels_is_captured(kind):
+    """Channel vectors of no whole pieces are copied: eagerly into a buffer of the context, under capture into memory that
+    belongs to the capture."""
     dev = torch.device("cuda:0")
     rng = np.random.default_rng(3)
     t = torch.int16 if kind == "int16" else torch.int8
@@ -234,5 +234,64 @@ def test_a_large_ragged_product_is_captured_without_scratch_memory(kind, shape):
         ctx.matmul(code, n, h, c, w, a, b, 0, 0, out)    # with room for them
         assert ctx.sync() == capi.VALID and torch.equal(out, want)
         assert ("pad_gemm" in ctx.last_kernel) == (h > 130)
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("kind", ["int8", "fp16", "int16"])
+def test_graphs_of_ragged_layers_replay_at_once(kind):
+    """Two graphs of one context and eager calls, each on a stream of its own and at the same time: CONV2D layers whose channel
+    vectors are padded on the way share no memory."""
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(5)
+    t, acc, code, out_code = {"int8": (torch.int8, torch.int32, capi.INT8, capi.INT32), "fp16": (torch.float16, torch.float16, capi.FP16, capi.FP16),
+                              "int16": (torch.int16, torch.int64, capi.INT16, capi.INT48)}[kind]
+    n, hw, ic, oc = 8, 56, 73, 72
+    wt = torch.int8 if kind == "int16" else t
+    layers = []
+    for _ in range(3):
+        x = torch.from_numpy(rng.integers(-9, 10, (n, hw, hw, ic))).to(t).to(dev)
+        w = torch.from_numpy(rng.integers(-1, 2, (oc, 3, 3, ic))).to(wt).to(dev)
+        bias = torch.from_numpy(rng.integers(-99, 100, oc)).to(acc).to(dev)
+        layers.append((x, w, bias, torch.zeros((n, hw, hw, oc), dtype=acc, device=dev)))
+    ctx = Context(0)
+    try:
+        d = ctx.conv_desc(code, out_code, (n, hw, hw, ic), oc, 3, 3, (hw, hw), (1, 1, 1, 1), (1, 1), (1, 1), oc)
+        main = torch.cuda.current_stream()
+        ctx.set_stream(main.cuda_stream)
+        want = []
+        for x, w, bias, out in layers:
+            ctx.conv2d(d, x, w, bias, 0, 0, out)
+            assert ctx.sync() == capi.VALID
+            want.append(out.clone())
+        kernel, (live, retired) = ctx.last_kernel, ctx.workspace_bytes()
+        assert live > 0 and retired == 0
+        graphs, streams = [], [torch.cuda.Stream(), torch.cuda.Stream()]
+        for layer, side in zip(layers, streams):
+            side.wait_stream(main)
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], stream=side):
+                ctx.set_stream(side.cuda_stream)
+                for _ in range(4):
+                    ctx.conv2d(d, *layer[:3], 0, 0, layer[3])
+            assert ctx.last_kernel == kernel
+            ctx.set_stream(main.cuda_stream)
+        # one block for each capture, of the size an eager call takes; the eager calls' buffer is untouched
+        assert ctx.workspace_bytes() == (live, 2 * live)
+        for _ in range(20):
+            for layer in layers:
+                layer[3].zero_()
+            torch.cuda.synchronize()
+            for graph, side in zip(graphs, streams):
+                with torch.cuda.stream(side):
+                    graph.replay()
+            for _ in range(4):
+                ctx.conv2d(d, *layers[2][:3], 0, 0, layers[2][3])
+            torch.cuda.synchronize()
+            assert all(torch.equal(layer[3], ref) for layer, ref in zip(layers, want))
+        assert ctx.sync() == capi.VALID
+        del graphs
+        ctx.trim_workspace()
+        assert ctx.workspace_bytes() == (live, 0)
     finally:
         ctx.close()
