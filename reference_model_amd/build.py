@@ -10,10 +10,12 @@ from __future__ import annotations
 
 import concurrent.futures
 import os
+import re
 import shutil
 import subprocess
 import sys
 import sysconfig
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -59,6 +61,50 @@ def kernels_with_scratch(remarks: str) -> list:
     return found
 
 
+_LISTED = re.compile(r"^<(?P<kernel>[^>\n]+)>:$"
+                     r"|^\s*(?P<shift>v_(?:lshlrev_b64|lshrrev_b64|ashrrev_i64))\S*\s+v\[\d+:\d+\],\s*v(?P<amount>\d+),", re.M)
+
+
+def shifts_by_the_last_register(remarks: str, listing: str) -> list:
+    """Kernels in which a 64-bit shift takes its amount from the last vector register of the wave's allocation (registers are
+    allocated in blocks of eight), from the compiler's kernel-resource-usage remarks and the objects' disassembly."""
+    kernel, registers = "", {}
+    for line in remarks.splitlines():
+        if "Function Name:" in line:
+            kernel = line.split("Function Name:")[1].split("[-Rpass")[0].strip()
+        else:
+            m = re.search(r"\b(VGPRs|AGPRs): (\d+)", line)
+            if m:
+                registers.setdefault(kernel, {})[m.group(1)] = int(m.group(2))
+    kernel, found = "", []
+    for m in _LISTED.finditer(listing):
+        if m.group("kernel"):
+            kernel = m.group("kernel")
+            continue
+        used = registers.get(kernel, {})
+        # (accumulation registers, where a kernel has any, come behind the others)
+        if not used.get("AGPRs") and used.get("VGPRs", 0) % 8 == 0 and int(m.group("amount")) == used.get("VGPRs", 0) - 1:
+            entry = f"{kernel}: {m.group('shift')} by v{m.group('amount')} of {used['VGPRs']} registers"
+            if entry not in found:
+                found.append(entry)
+    return found
+
+
+def _device_listing(obj: str) -> str:
+    """The disassembly of the gfx950 code in a freshly compiled object file."""
+    tools = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(_hipcc()))), "llvm", "bin")
+    with tempfile.TemporaryDirectory() as tmp:
+        fat, code = os.path.join(tmp, "fat"), os.path.join(tmp, "code")
+        for cmd in ([os.path.join(tools, "llvm-objcopy"), f"--dump-section=.hip_fatbin={fat}", obj, os.path.join(tmp, "rest.o")],
+                    [os.path.join(tools, "clang-offload-bundler"), "--unbundle", "--type=o", f"--targets=hipv4-amdgcn-amd-amdhsa--{ARCH}",
+                     f"--input={fat}", f"--output={code}"],
+                    [os.path.join(tools, "llvm-objdump"), "-d", "--no-leading-addr", code]):
+            r = subprocess.run(cmd, capture_output=True, text=True)
+            if r.returncode != 0:
+                raise RuntimeError(f"{cmd[0]} failed on {obj}:\n{r.stdout}\n{r.stderr}")
+        return r.stdout
+
+
 def _compile(src: str, force: bool) -> str:
     obj = os.path.join(BUILD, src[:-4] + ".o")
     deps = [os.path.join(CSRC, src)] + [os.path.join(CSRC, h) for h in os.listdir(CSRC) if h.endswith(".h")]
@@ -76,6 +122,13 @@ def _compile(src: str, force: bool) -> str:
     if with_scratch:
         os.remove(obj)
         raise RuntimeError(f"{src}: kernels with a scratch segment:\n  " + "\n  ".join(with_scratch))
+    # A kernel that shifts 64 bits by the last register of its allocation is refused: one such kernel (v87 of 88 registers) shifted
+    # by something else now and then, always in the element whose amount lay there, and never with the amount in another
+    # register.  Naming a register of the next block of eight in an empty asm moves the border.
+    by_last = shifts_by_the_last_register(r.stderr, _device_listing(obj))
+    if by_last:
+        os.remove(obj)
+        raise RuntimeError(f"{src}: 64-bit shifts by the last register of the allocation:\n  " + "\n  ".join(by_last))
     warn = "\n".join(l for l in r.stderr.splitlines()
                      if "packed-fp32-ops" not in l and "-Rpass-analysis" not in l and l.strip())
     if warn:

@@ -67,3 +67,29 @@ def test_build_refuses_kernels_with_a_scratch_segment():
     ])
     assert kernels_with_scratch(remarks) == ["_Z5spillPi: 184 bytes per lane"]
     assert kernels_with_scratch("") == []
+
+
+REMARKS = """a.hip:3:0: remark: Function Name: _Z4lastPi [-Rpass-analysis=kernel-resource-usage]
+a.hip:3:0: remark:     VGPRs: {vgprs} [-Rpass-analysis=kernel-resource-usage]
+a.hip:3:0: remark:     AGPRs: {agprs} [-Rpass-analysis=kernel-resource-usage]
+"""
+
+
+@pytest.mark.parametrize("vgprs, agprs, line, refused", [
+    (88, 0, "v_ashrrev_i64 v[2:3], v87, v[4:5]", True),
+    (88, 0, "v_lshlrev_b64 v[10:11], v87, 1", True),
+    (88, 0, "v_lshrrev_b64_e64 v[10:11], v87, s[4:5]", True),
+    (88, 0, "v_ashrrev_i64 v[2:3], v83, v[4:5]", False),
+    (88, 0, "v_ashrrev_i64 v[86:87], v4, v[86:87]", False),      # the value, not the amount
+    (88, 0, "v_ashrrev_i64 v[2:3], 31, v[86:87]", False),
+    (86, 0, "v_ashrrev_i64 v[2:3], v85, v[4:5]", False),         # two registers of the block unused behind it
+    (96, 0, "v_ashrrev_i64 v[2:3], v87, v[4:5]", False),
+    (88, 16, "v_ashrrev_i64 v[2:3], v87, v[4:5]", False),        # accumulation registers behind it
+    (88, 0, "v_ashrrev_i32 v2, v87, v4", False),
+])
+def test_build_refuses_64_bit_shifts_by_the_last_register(vgprs, agprs, line, refused):
+    from reference_model_amd.build import shifts_by_the_last_register
+    listing = "\n<_Z5otherPi>:\n\tv_ashrrev_i64 v[2:3], v87, v[4:5]   // 000000001800: D2910002\n" \
+              f"\n<_Z4lastPi>:\n\ts_nop 0\n\t{line}                   // 000000001900: D2910002\n"
+    found = shifts_by_the_last_register(REMARKS.format(vgprs=vgprs, agprs=agprs), listing)
+    assert len(found) == refused and all(f.startswith("_Z4lastPi") for f in found)
