@@ -4,7 +4,7 @@
 
 hipcc cross-compiles without a GPU.  Every translation unit is compiled to an object file under
 csrc/build/ (in parallel) and linked into reference_model_amd/libtosa_mi355.so; the C++ host side (the runner, its
-known-answer tests and the Python operator calls, _calls.so) is built on top of it with g++.
+known-answer tests and, where Python's headers are installed, its operator calls as an extension) is built on top of it with g++.
 """
 from __future__ import annotations
 
@@ -23,7 +23,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 BUILD = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libtosa_mi355.so")
 HOST_BIN = os.path.join(HERE, "tosa_mi355_run")
-CALLS = os.path.join(HERE, "_calls.so")
+CALLS = os.path.join(HERE, "_calls" + sysconfig.get_config_var("EXT_SUFFIX"))    # of this interpreter's ABI: no other loads it
 
 ARCH = "gfx950"
 # -packed-fp32-ops off: hipcc must not form v_pk_*_f32 from float code on this hardware pool.
@@ -167,19 +167,29 @@ def build_host(force: bool = False) -> list:
             if r.stderr.strip():
                 sys.stderr.write(r.stderr)
         outs.append(exe)
-    # the operator calls of capi.Context as a CPython extension
-    src = os.path.join(host, "pycalls.cc")
+    calls = build_calls(force)
+    return outs + [calls] if calls else outs
+
+
+def build_calls(force: bool = False) -> str | None:
+    """The operator calls of capi.Context as a CPython extension; None where Python's headers are not installed (the calls then
+    stay on ctypes)."""
+    src, headers = os.path.join(CSRC, "host", "pycalls.cc"), sysconfig.get_paths()["include"]
+    untagged = os.path.join(HERE, "_calls.so")    # what an interpreter of any version would load
+    if os.path.exists(untagged):
+        os.remove(untagged)
+    if not os.path.exists(os.path.join(headers, "Python.h")):
+        sys.stderr.write(f"no Python.h under {headers}: the operator calls stay on ctypes\n")
+        return None
     if force or not os.path.exists(CALLS) or any(os.path.getmtime(d) > os.path.getmtime(CALLS) for d in (src, os.path.join(INCLUDE, "tosa_mi355.h"))):
         cmd = ["g++", "-O2", "-std=c++17", "-Wall", "-Wextra", "-Wno-missing-field-initializers", "-fPIC", "-shared", f"-I{INCLUDE}",
-               "-I" + sysconfig.get_paths()["include"], src, "-o", CALLS, f"-L{HERE}", "-ltosa_mi355", "-Wl,-rpath,$ORIGIN",
-               "-Wl,-rpath-link,/opt/rocm/lib"]
+               f"-I{headers}", src, "-o", CALLS, f"-L{HERE}", "-ltosa_mi355", "-Wl,-rpath,$ORIGIN", "-Wl,-rpath-link,/opt/rocm/lib"]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"g++ failed on pycalls.cc:\n{r.stdout}\n{r.stderr}")
         if r.stderr.strip():
             sys.stderr.write(r.stderr)
-    outs.append(CALLS)
-    return outs
+    return CALLS
 
 
 if __name__ == "__main__":

@@ -182,11 +182,13 @@ def load_library() -> ctypes.CDLL:
         fn = getattr(lib, name)
         if fn.restype is ctypes.c_int:
             fn.restype = ctypes.c_int
+    # the operator calls as native methods, where they were built for this interpreter (2 us less host time a call)
     try:
         from . import _calls
-    except ImportError as e:
-        raise ImportError(f"the native operator calls do not load ({e}): run `python -m reference_model_amd.build`") from e
-    _calls.install(Context, DeviceTensor, TmiError, ctypes.ArgumentError, ConvDesc, TconvDesc, Conv3dDesc, PoolDesc, RescaleDesc)
+    except ModuleNotFoundError:
+        _calls = None
+    if _calls:
+        _calls.install(Context, DeviceTensor, TmiError, ctypes.ArgumentError, ConvDesc, TconvDesc, Conv3dDesc, PoolDesc, RescaleDesc)
     _lib = lib
     return lib
 
@@ -326,11 +328,47 @@ class Context:
         return r
 
     # -- operators (device pointers in, status out) ------------------------------------------
-    # conv2d, depthwise_conv2d, transpose_conv2d, conv3d (d, inp, w, bias, in_zp, w_zp, out), conv2d_rescale_clamp,
-    # depthwise_conv2d_rescale_clamp (d, inp, w, bias, in_zp, w_zp, r, mult, shift, out, clamp=None), matmul (in_dtype, n, h,
-    # c, w, a, b, a_zp, b_zp, out), rescale (r, rank, rows, c, inp, mult, shift, out), clamp (dtype, n, inp, lo, hi, out),
-    # avg_pool2d (d, inp, in_zp, out_zp, out) and max_pool2d (d, inp, out) are native methods (csrc/host/pycalls.cc), put
-    # here by load_library().  The calls below stay on ctypes.
+    # load_library() puts native methods (csrc/host/pycalls.cc) in the place of those named in PLAIN_OPERATORS, with the same
+    # arguments, results and errors.
+    def conv2d(self, d: ConvDesc, inp, w, bias, in_zp, w_zp, out) -> int:
+        return self._check(self.lib.tmi_conv2d(self.handle, ctypes.byref(d), _ptr(inp), _ptr(w), _ptr(bias), in_zp, w_zp, _ptr(out)))
+
+    def depthwise_conv2d(self, d: ConvDesc, inp, w, bias, in_zp, w_zp, out) -> int:
+        return self._check(self.lib.tmi_depthwise_conv2d(self.handle, ctypes.byref(d), _ptr(inp), _ptr(w), _ptr(bias), in_zp, w_zp, _ptr(out)))
+
+    def transpose_conv2d(self, d: TconvDesc, inp, w, bias, in_zp, w_zp, out) -> int:
+        return self._check(self.lib.tmi_transpose_conv2d(self.handle, ctypes.byref(d), _ptr(inp), _ptr(w), _ptr(bias), in_zp, w_zp, _ptr(out)))
+
+    def conv3d(self, d: Conv3dDesc, inp, w, bias, in_zp, w_zp, out) -> int:
+        return self._check(self.lib.tmi_conv3d(self.handle, ctypes.byref(d), _ptr(inp), _ptr(w), _ptr(bias), in_zp, w_zp, _ptr(out)))
+
+    def conv2d_rescale_clamp(self, d: ConvDesc, inp, w, bias, in_zp, w_zp, r: RescaleDesc, mult, shift, out, clamp=None) -> int:
+        lo, hi = clamp if clamp is not None else (0, 0)
+        return self._check(self.lib.tmi_conv2d_rescale_clamp(
+            self.handle, ctypes.byref(d), _ptr(inp), _ptr(w), _ptr(bias), in_zp, w_zp, ctypes.byref(r), _ptr(mult), _ptr(shift),
+            int(clamp is not None), lo, hi, _ptr(out)))
+
+    def depthwise_conv2d_rescale_clamp(self, d: ConvDesc, inp, w, bias, in_zp, w_zp, r: RescaleDesc, mult, shift, out, clamp=None) -> int:
+        lo, hi = clamp if clamp is not None else (0, 0)
+        return self._check(self.lib.tmi_depthwise_conv2d_rescale_clamp(
+            self.handle, ctypes.byref(d), _ptr(inp), _ptr(w), _ptr(bias), in_zp, w_zp, ctypes.byref(r), _ptr(mult), _ptr(shift),
+            int(clamp is not None), lo, hi, _ptr(out)))
+
+    def matmul(self, in_dtype, n, h, c, w, a, b, a_zp, b_zp, out) -> int:
+        return self._check(self.lib.tmi_matmul(self.handle, in_dtype, n, h, c, w, _ptr(a), _ptr(b), a_zp, b_zp, _ptr(out)))
+
+    def rescale(self, r: RescaleDesc, rank, rows, c, inp, mult, shift, out) -> int:
+        return self._check(self.lib.tmi_rescale(self.handle, ctypes.byref(r), rank, rows, c, _ptr(inp), _ptr(mult), _ptr(shift), _ptr(out)))
+
+    def clamp(self, dtype, n, inp, lo, hi, out) -> int:
+        return self._check(self.lib.tmi_clamp(self.handle, dtype, n, _ptr(inp), lo, hi, _ptr(out)))
+
+    def avg_pool2d(self, d: PoolDesc, inp, in_zp, out_zp, out) -> int:
+        return self._check(self.lib.tmi_avg_pool2d(self.handle, ctypes.byref(d), _ptr(inp), in_zp, out_zp, _ptr(out)))
+
+    def max_pool2d(self, d: PoolDesc, inp, out) -> int:
+        return self._check(self.lib.tmi_max_pool2d(self.handle, ctypes.byref(d), _ptr(inp), _ptr(out)))
+
     def transpose_conv2d_noalloc(self, d: TconvDesc, inp, w, bias, in_zp, w_zp, out) -> int:
         return self._check(self.lib.tmi_transpose_conv2d_noalloc(self.handle, ctypes.byref(d), _ptr(inp), _ptr(w),
                                                                  _ptr(bias), in_zp, w_zp, _ptr(out)))
@@ -384,6 +422,12 @@ class Context:
     def set_level(self, level=LEVEL_NONE):
         lv = Level(*level)
         self._check(self.lib.tmi_ctx_set_level(self.handle, ctypes.byref(lv)))
+
+
+# the operators on ctypes, whatever load_library() put in their place
+PLAIN_OPERATORS = {name: vars(Context)[name] for name in (
+    "conv2d", "depthwise_conv2d", "transpose_conv2d", "conv3d", "conv2d_rescale_clamp", "depthwise_conv2d_rescale_clamp", "matmul",
+    "rescale", "clamp", "avg_pool2d", "max_pool2d")}
 
 
 def _stored(zp: int, dtype: int) -> int:
