@@ -734,9 +734,11 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // kernel / this form: [32,14,14,256]->256 (98 tiles, 3.7 G) 15.1 / 12.8, [8,28,28,256]->256 15.2 / 13.3, [32,7,7,512]->512
         // (52) 21.6 / 14.2, [64,7,7,512]->512 (100, 7.4 G) 33.4 / 23.6, [16,14,14,512]->512 (100) 24.0 / 21.0; the other way:
         // [8,28,28,384]->384 (147) 24.6 / 28.1, [8,56,56,256]->64 (196) 15.1 / 16.7, [64,14,14,256]->256 (196) 19.3 / 22.1.
-        // (Layers with int32 results keep the first rule's bounds: the test of the automatic choice fixes their routes.)
+        // int32 results: [32,14,14,256]->256 (98) 16.3 / 11.5, [48,14,14,256]->128 (74) 15.5 / 9.8, [24,14,14,384]->256 (74) 19.9 / 14.3,
+        // [32,7,7,512]->512 (52) 21.1 / 12.7, [64,7,7,512]->512 (100) 32.9 / 20.3, [16,14,14,512]->512 (100) 24.7 / 18.4; even: stride 2
+        // [32,28,28,256]->256 (98) 18.3 / 18.4.
         const bool split_small = g.KH * g.KW > 1 && macs <= 2400000000ll && (tiles128 <= 64 || (g.IC >= 160 && tiles128 <= 100));
-        const bool split_patch = rp.enabled && g.KH == 3 && g.KW == 3 && (g.IC == 256 || g.IC == 384 || g.IC == 512) && tiles128 <= 100;
+        const bool split_patch = g.KH == 3 && g.KW == 3 && (g.IC == 256 || g.IC == 384 || g.IC == 512) && tiles128 <= 100;
         if (!name && g.KH * g.KW > 1 && (ctx->kernel_choice == 5 || (ctx->kernel_choice == 0 && (split_small || split_patch))))
             name = launch_conv2d_ksplit(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out, pad_page,
                                         ctx->flags_dev, ctx->kernel_choice == 5 || split_small);

@@ -420,14 +420,17 @@ def test_conv2d_fused_rescale_gemm_reports_require_conditions(ctx):
     (capi.INT8, (16, 28, 28, 1024, 256, 3, 1), "conv2d_mfma_i8"),      # 3x3 int8 whose patch (6 x 30 x 1 KB) does not fit
     (capi.INT8, (16, 14, 14, 1024, 1024, 1, 0), "gemm_mfma_i8"),       # pointwise: the GEMM kernel
     (capi.INT8, (64, 28, 28, 256, 256, 3, 1, 2), "gemm_mfma_i8"),      # 3x3 int8 with stride 2 and 200 tiles: the GEMM kernel
-    (capi.INT8, (32, 28, 28, 256, 256, 3, 1, 2), "conv2d_mfma_i8"),    # the same with 100 tiles: the patch kernel
+    (capi.INT8, (32, 28, 28, 256, 256, 3, 1, 2), "conv2d_ksplit_patch_i8"),    # the same with 98 tiles: K split over the waves, both operands in LDS
+    (capi.INT8, (32, 28, 28, 320, 256, 3, 1, 2), "conv2d_mfma_i8"),    # on 320 channels: the patch kernel
     (capi.INT8, (20, 28, 28, 1024, 256, 3, 1), "gemm_mfma_i8"),        # 3x3 int8 outside the patch form, 246 tiles: the GEMM kernel
-    (capi.INT8, (64, 7, 7, 512, 512, 3, 1), "gemm_mfma_i8"),           # images smaller than a tile, 100 tiles: the GEMM kernel
+    (capi.INT8, (64, 7, 7, 512, 512, 3, 1), "conv2d_ksplit_patch_i8"), # images smaller than a tile, 100 tiles: K split over the waves
+    (capi.INT8, (64, 7, 7, 640, 512, 3, 1), "gemm_mfma_i8"),           # on 640 channels: the GEMM kernel
     (capi.FP16, (16, 28, 28, 256, 256, 3, 1), "gemm_mfma_f16_patch"),  # 3x3 fp16, deep K, the patch fits the LDS
     (capi.FP16, (8, 28, 28, 512, 512, 3, 1), "gemm_mfma_f16"),         # the same with a patch that does not fit
     (capi.FP16, (4, 28, 28, 256, 256, 3, 1), "gemm_mfma_f16_patch"),   # 56 tiles of four output rows: enough for the patch form
     (capi.INT8, (16, 14, 14, 256, 256, 3, 1), "conv2d_ksplit_patch_i8"),    # 50 tiles, 1.8 G multiply-adds: K split over the waves of small workgroups
-    (capi.INT8, (32, 14, 14, 256, 256, 3, 1), "conv2d_mfma_i8"),       # 98 tiles, 3.7 G: too much for that, too few tiles for the GEMM kernel
+    (capi.INT8, (32, 14, 14, 256, 256, 3, 1), "conv2d_ksplit_patch_i8"),       # 98 tiles, 3.7 G
+    (capi.INT8, (32, 14, 14, 320, 256, 3, 1), "conv2d_mfma_i8"),       # 4.6 G on 320 channels: too much for that, too few tiles for the GEMM kernel
     (capi.INT8, (8, 14, 14, 1024, 512, 1, 0), "conv2d_slab_i8"),       # pointwise on 1024 channels, one round of workgroups: the slab kernel
     (capi.INT8, (8, 7, 7, 2048, 512, 1, 0), "conv2d_pointwise_split_i8"),    # 2048 channels, 411 M multiply-adds on 16 tiles: K split over waves
     (capi.INT8, (8, 28, 28, 512, 256, 1, 0), "conv2d_slab_i8"),        # pointwise on 512 channels, one round of workgroups: the slab kernel
