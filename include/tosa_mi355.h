@@ -252,10 +252,10 @@ typedef struct
 
 /* OpConv2d<In,W,Acc,Out>::eval, reference_model/src/ops/tensor_ops.cpp:723-882 (checks :120-226, :690-720).
  * INT8 x INT8 -> INT32 with int32 accumulation, or FP16 / BF16 / FP32 with fp32 accumulation and an output
- * of the input type (the instantiations at :2220-2229; FP32 runs on the one-element-per-lane kernels, in the
- * reference's summation order).  INT16 x INT8 -> INT48 (:2225; d->in_dtype TMI_INT16, weights INT8, bias and
- * output one int64 per element, the sum kept in 64 bits and REQUIREd to lie within 48 bits, :875-879) runs on a
- * one-element-per-lane kernel.  INT8 x INT4 -> INT32 (:2224) is the INT8 call with the weights handed over as one
+ * of the input type (the instantiations at :2220-2229; FP32 sums in the reference's order, on tiles that keep it or
+ * one element per lane).  INT16 x INT8 -> INT48 (:2225; d->in_dtype TMI_INT16, weights INT8, bias and
+ * output one int64 per element, the sum kept in 64 bits and REQUIREd to lie within 48 bits, :875-879) runs as two
+ * int8 products on the matrix cores, tiny layers and those with a weight zero point on a one-element-per-lane kernel.  INT8 x INT4 -> INT32 (:2224) is the INT8 call with the weights handed over as one
  * int8 value of -8 ... 7 per element and w_zp = 0, which the caller checks (the library cannot tell such weights from INT8
  * ones).  in_zp / w_zp are the values of operands 3 and 4: in_zp must be 0 unless the input is INT8, w_zp unless the
  * weights are (:804-811). */
@@ -312,7 +312,7 @@ int tmi_depthwise_conv2d_rescale_clamp(tmi_ctx_t* ctx, const tmi_conv_desc_t* d,
  * Evaluated as a stride-1 CONV2D with flipped taps over the input with stride-1 holes filled with input_zp.
  * INT8 with 3x3 taps, 64 / 96 / 128 input channels and w_zp 0 reads both operands in place (holes and flip are
  * part of the kernel's addressing); otherwise the re-laid-out operands live in the context's scratch buffer.
- * Element types as tmi_conv2d: INT8 -> INT32, FP16 / BF16 / FP32 (FP32 on the one-element-per-lane kernel, the sum in
+ * Element types as tmi_conv2d: INT8 -> INT32, FP16 / BF16 / FP32 (FP32: the sum in
  * the order of the equivalent CONV2D, not the reference's scatter order), INT16 x INT8 -> INT48 (:2291; clip :2190-2194). */
 int tmi_transpose_conv2d(tmi_ctx_t* ctx, const tmi_tconv_desc_t* d, const void* in_dev, const void* weight_dev,
                          const void* bias_dev, int32_t in_zp, int32_t w_zp, void* out_dev);
@@ -336,7 +336,7 @@ int tmi_transpose_conv2d_noalloc(tmi_ctx_t* ctx, const tmi_tconv_desc_t* d, cons
  * Evaluated as a CONV2D over N*OD images whose channels are the KD depth taps side by side.  INT8 with 3x3 taps in
  * the plane, KD*IC = 64 / 96 / 128 (IC 32 or 64) and w_zp 0 reads both operands in place; otherwise the gathered
  * input and the permuted weights live in the context's scratch buffer.  Element types as tmi_conv2d: INT8 -> INT32,
- * FP16 / BF16 / FP32 (FP32 on the one-element-per-lane kernel, the depth taps innermost in the sum), and INT16 x INT8 ->
+ * FP16 / BF16 / FP32 (FP32: the depth taps innermost in the sum), and INT16 x INT8 ->
  * INT48 (:2237; clip :1113-1117). */
 int tmi_conv3d(tmi_ctx_t* ctx, const tmi_conv3d_desc_t* d, const void* in_dev, const void* weight_dev,
                const void* bias_dev, int32_t in_zp, int32_t w_zp, void* out_dev);

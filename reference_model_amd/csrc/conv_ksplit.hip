@@ -324,7 +324,9 @@ __global__ __launch_bounds__(NW * 64, (NW + 3) / 4) void conv_ksplit_patch_kerne
 {
     constexpr int KS = 9, IC = NW * 32, NT = NW * 64;
     constexpr int kPieces = 2 * KS, kRow = kPieces * 16 + 16;    // 16-byte pieces of a wave's share of a weight row; its pitch in LDS
-    constexpr int CPP = IC / 16, kPitch = IC + 16;               // pieces of a pixel; its pitch: = 16 (mod 32), no bank conflicts
+    constexpr int CPP = IC / 16, kPitch = IC + 16;               // pieces of a pixel; its pitch: = 16 (mod 32), neighbours of a row in different banks
+    // (a block's next row of pixels starts PW - TW pixels further on and meets the banks of the last: 1.6 and 1.5 conflict cycles an LDS
+    // instruction measured on 14 x 14 x 256 and 7 x 7 x 512)
     constexpr int NC  = NW >= 14 ? 3 : 4;                        // pieces of the patch a lane has in flight
     // [32 x HighWordScale][32 x (m, s)][NW waves x 32 start values][form] and then the weights of all waves, later
     // [NPT x NW waves x 4 quarters x 64 lanes x 16 bytes][patch]

@@ -4,6 +4,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -216,6 +217,14 @@ void* copy_scratch(tmi_ctx* ctx, size_t bytes)
         return ctx->copies;
     if (capturing && ctx->captured_bytes + bytes > kMostCaptured)
         return nullptr;
+    try
+    {
+        ctx->retired.reserve(ctx->retired.size() + 1);    // (no exception may leave a C entry point)
+    }
+    catch (const std::exception&)
+    {
+        return nullptr;
+    }
     const size_t want = !capturing && bytes < 2 * ctx->copies_size ? 2 * ctx->copies_size : bytes;
     // an allocation is no part of a graph, but forbidden to a thread that captures in the default mode
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
