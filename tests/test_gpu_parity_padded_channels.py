@@ -71,6 +71,29 @@ def test_int8(ctx, case, fused):
     assert st == wst and np.array_equal(got, want) and len(np.unique(got)) > 20 and ctx.last_kernel == CASES[case] + "_rescale"
 
 
+def test_padded_layer_with_its_sums_in_the_scratch_buffer():
+    """a fused layer under precise-mode INEXACT_ROUND keeps its INT32 sums in the context's scratch buffer; the padded operands of
+    the same call lie elsewhere"""
+    n, h, w, ic, oc = 2, 12, 12, 131, 48
+    rng = np.random.default_rng(8)
+    x, wt = rng.integers(-128, 128, (n, h, w, ic)).astype(np.int8), rng.integers(-128, 128, (oc, 3, 3, ic)).astype(np.int8)
+    bias, pad = rng.integers(-9999, 9999, oc).astype(np.int32), (1, 1, 1, 1)
+    mult, shift = rng.integers(1 << 29, 1 << 30, oc).astype(np.int32), rng.integers(40, 44, oc).astype(np.int8)
+    acc = oracle.conv2d("i8", x, wt, bias, pad, (1, 1), (1, 1), in_zp=-11, w_zp=0)
+    want, wst = oracle.rescale(acc, mult, shift, out_zp=3, rounding_mode=capi.ROUND_INEXACT, inexact_mode=1)
+    c = Context(0)
+    try:
+        c.set_precise_mode(True)
+        for _ in range(2):
+            got, st = gpu_ops.conv2d(c, x, wt, bias, pad, in_zp=-11, w_zp=0,
+                                     rescale=dict(mult=mult, shift=shift, out_zp=3, rounding_mode=capi.ROUND_INEXACT))
+            assert st == wst and np.array_equal(got, want) and len(np.unique(got)) > 20
+        # the sums, and the padded operands of 160 channels
+        assert c.workspace_bytes()[0] >= 4 * n * h * w * oc + 160 * (n * h * w + 9 * oc)
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("case", list(CASES) + [(1, 9, 9, 9, 16, 3, 1, 1), (1, 9, 9, 100, 40, 3, 1, 1), (2, 12, 12, 40, 64, 3, 1, 1)])
 @pytest.mark.parametrize("dtype", [capi.FP16, capi.BF16])
 def test_16_bit_floats(ctx, case, dtype):
