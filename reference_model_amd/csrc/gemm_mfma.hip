@@ -157,6 +157,9 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     constexpr int LOADS    = ROWS / 128;    // direct loads per wave and block (16 rows each)
     constexpr int WLOADS   = WROWS / 128;   // of which carry weight rows
     constexpr int PLOADS   = LOADS - WLOADS;
+    // Single blocks: a block's loads are dealt to the second step of one block (EARLY) and the first step of the next
+    constexpr int EARLY    = (LOADS + 1) / 2;
+    constexpr int LATE     = LOADS - EARLY;
     static_assert(ROWS % 128 == 0, "a block must split evenly over the 8 waves");
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 
@@ -330,7 +333,7 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     }
     else if constexpr (APAIR)
     {
-        // in the order the loop continues: pixel pair 0, weights 0, weights 1, pixel pair 1, weights 2
+        // in the order the loop continues: pixel pair 0, weights 0, weights 1, half of pixel pair 1, weights 2
 #pragma unroll
         for (int q = 0; q < 2 * PLOADS; q++)
             issue_p(0, 0, q);
@@ -338,7 +341,7 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
         for (int j = 0; j < 2 * WLOADS; j++)
             issue_w(j / WLOADS, j % WLOADS);
 #pragma unroll
-        for (int q = 0; q < 2 * PLOADS; q++)
+        for (int q = 0; q < PLOADS; q++)
             issue_p(2, 1, q);
 #pragma unroll
         for (int j = 0; j < WLOADS; j++)
@@ -349,7 +352,7 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
 #pragma unroll
         for (int s = 0; s < kStages - 1; s++)
 #pragma unroll
-            for (int j = 0; j < LOADS; j++)
+            for (int j = 0; j < (s < kStages - 2 ? LOADS : EARLY); j++)
                 issue_one(s, s, j);
     }
 
@@ -487,17 +490,23 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     constexpr int NW = KM ? 2 * OCT : OCT;    // weight fragment reads per step
     constexpr int NR = NW + PXT;              // fragment reads per step
     v4i fa[2][OCT], fb[2][PXT];
-    // reads in the order the matrix instructions want them: pixel tile 0, the channel tiles, the other pixel tiles
+    // reads in the order the matrix instructions want them: pixel tile 0, channel tile 0, the other pixel tiles, the other
+    // channel tiles
     // wb: the stage's weight rows; pb: its pixel rows minus their offset in a whole stage (ap[] includes it)
     auto read_one = [&](const uint8_t* wb, const uint8_t* pb, int s, int j) {
         const uint8_t* sb = wb;
-        if (j == 0)
-            fb[s][0] = *reinterpret_cast<const v4i*>(pb + ap[s]);
-        else if (j <= NW)
+        constexpr int W1 = KM ? 2 : 1;    // weight reads per channel tile
+        if (j == 0 || (j > W1 && j < W1 + PXT))
         {
+            const int i = j == 0 ? 0 : j - W1;
+            fb[s][i]    = *reinterpret_cast<const v4i*>(pb + ap[s] + i * 2048);
+        }
+        else
+        {
+            const int w = j <= W1 ? j - 1 : j - PXT;    // which of the NW weight reads
             if constexpr (KM)
             {
-                const int t = (j - 1) >> 1, r = (j - 1) & 1;
+                const int t = w >> 1, r = w & 1;
                 const uint8_t* src = sb + akm[t] + (KSTEP * s + (KSTEP / 4) * r) * RB;
                 v2i half;
                 if constexpr (EB == 2)
@@ -509,24 +518,27 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                 fa[s][t][2 * r + 1] = half.y;
             }
             else
-                fa[s][j - 1] = *reinterpret_cast<const v4i*>(sb + aw[s] + (j - 1) * 2048);
+                fa[s][w] = *reinterpret_cast<const v4i*>(sb + aw[s] + w * 2048);
         }
-        else
-            fb[s][j - NW] = *reinterpret_cast<const v4i*>(pb + ap[s] + (j - NW) * 2048);
     };
-    auto sums = [&](int s) {
+    // The four waves that read the same weight rows take a fourth of the K-steps each for the rows' sums, the two that read the
+    // same pixel rows a half (every wave adding up every step: 16 vector instructions beside the 4 matrix instructions of a
+    // step of the 128 x 256 shape; int8 [8,1024,1024]x[8,1024,1024] 18.4 us, so 18.05); the parts meet in LDS after the loop.
+    auto sums = [&](int s, int odd) {
         if constexpr (ZP)
         {
+            if (wp == 2 * odd + s)
 #pragma unroll
-            for (int t = 0; t < OCT; t++)
-                wsum[t] += dot4_ones(fa[s][t]);
+                for (int t = 0; t < OCT; t++)
+                    wsum[t] += dot4_ones(fa[s][t]);
+            if (wo == s)
 #pragma unroll
-            for (int i = 0; i < PXT; i++)
-                psum[i] += dot4_ones(fb[s][i]);
+                for (int i = 0; i < PXT; i++)
+                    psum[i] += dot4_ones(fb[s][i]);
         }
     };
     auto mma_one = [&](int s, int k) {
-        const int i = k / OCT, t = k % OCT;
+        const int t = k / PXT, i = t & 1 ? PXT - 1 - k % PXT : k % PXT;    // (one operand changes at a time)
         acc[i][t]   = M::mma(fa[s][t], fb[s][i], acc[i][t]);
     };
     // A bare s_barrier: __syncthreads() would also drain this wave's LDS reads (the fragments of the step
@@ -544,51 +556,47 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     if constexpr (PAIR)
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PAIR ? (kStages / 2 - 2) * 2 * LOADS : 0) : "memory");
     else if constexpr (APAIR)
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PLOADS + 2 * WLOADS) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PLOADS + 2 * WLOADS) : "memory");
     else
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStages - 2) * LOADS) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStages - 3) * LOADS + EARLY) : "memory");
     __syncthreads();    // block 0 and the bias table are in LDS for every wave
 #pragma unroll
     for (int j = 0; j < NR; j++)
         read_one(lds, APAIR ? lds + PBASE - WB : lds, 0, j);
     __builtin_amdgcn_sched_barrier(0);
-    // first K-step of a block: its matrix instructions, and the requests for the fragments of the second step;
-    // two requests behind each of the first matrix instructions, so that the last ones of a step cover the
-    // latency of the fragments the next step starts with
-    auto first_step = [&](const uint8_t* cur, const uint8_t* curp) {
-        constexpr int PA = NR > 2 * NM ? (NR + NM - 1) / NM : 2;
-        sums(0);
+    // One K-step: the matrix instructions of step S, and behind them, spread evenly, NL direct loads and the requests for the
+    // fragments of the step that follows (step 1 - S, from the stage at wb / pb).  odd: the block's parity.  With the matrix instructions taken channel
+    // tile by channel tile a fragment is wanted as many instructions after its request as a step has, so a request waits for
+    // its turn at the LDS while the matrix cores work.  (All of a step's loads behind its first matrix instructions and the
+    // reads two by two: int8 [8,1024,1024]x[8,1024,1024] 18.8 us, so 18.4; bf16 [4,2048,4096]x[4,4096,2048] 112.5, so 111.5.
+    // What is left of the latter is the power the data takes: the same launch on zeros is 78 us, without any load or LDS
+    // read on random data 94.)
+    auto k_step = [&](auto S_tag, int odd, const uint8_t* wb, const uint8_t* pb, auto NL_tag, auto&& load) {
+        constexpr int S  = decltype(S_tag)::value;
+        constexpr int NL = decltype(NL_tag)::value;
+        sums(S, odd);
 #pragma unroll
         for (int k = 0; k < NM; k++)
         {
-            mma_one(0, k);
+            mma_one(S, k);
 #pragma unroll
-            for (int j = k * PA; j < (k + 1) * PA && j < NR; j++)
-                read_one(cur, curp, 1, j);
+            for (int q = 0; q < NL; q++)
+                if (q * NM / (NL ? NL : 1) == k)
+                    load(q);
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+                if (j * NM / NR == k)
+                    read_one(wb, pb, 1 - S, j);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // second K-step: its matrix instructions, NL direct loads (they have the longest way to go, so they come
-    // first) and the requests for the first fragments of the next block
-    auto second_step = [&](const uint8_t* next, const uint8_t* nextp, auto NL_tag, auto&& load) {
-        constexpr int NL = decltype(NL_tag)::value;
-        constexpr int NO = NL + NR;
-        constexpr int PB = NO > 2 * NM ? (NO + NM - 1) / NM : 2;
-        sums(1);
-#pragma unroll
-        for (int k = 0; k < NM; k++)
-        {
-            mma_one(1, k);
-#pragma unroll
-            for (int q = k * PB; q < (k + 1) * PB && q < NO; q++)
-            {
-                if (q < NL)
-                    load(q);
-                else
-                    read_one(next, nextp, 0, q - NL);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
+    constexpr std::integral_constant<int, 0> none{};
+    auto no_load = [](int) {};
+    auto first_step = [&](int odd, const uint8_t* cur, const uint8_t* curp, auto NL_tag, auto&& load) {
+        k_step(std::integral_constant<int, 0>{}, odd, cur, curp, NL_tag, load);
+    };
+    auto second_step = [&](int odd, const uint8_t* next, const uint8_t* nextp, auto NL_tag, auto&& load) {
+        k_step(std::integral_constant<int, 1>{}, odd, next, nextp, NL_tag, load);
     };
     if constexpr (PAIR)
     {
@@ -664,13 +672,13 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                     }
                 }
             };
-            first_step(cur0, PATCH ? lds : cur0);
+            first_step(0, cur0, PATCH ? lds : cur0, none, no_load);
             next_patch(sc + 1);
-            second_step(cur0 + STAGE, PATCH ? lds : cur0 + STAGE, std::integral_constant<int, 0>{}, [](int) {});
-            first_step(cur0 + STAGE, PATCH ? lds : cur0 + STAGE);
+            second_step(0, cur0 + STAGE, PATCH ? lds : cur0 + STAGE, none, no_load);
+            first_step(1, cur0 + STAGE, PATCH ? lds : cur0 + STAGE, none, no_load);
             publish_pair();    // the next pair is in LDS for every wave, and every wave is past the pair before
             next_patch(sc + 2);
-            second_step(lds + sn * STAGE, PATCH ? lds : lds + sn * STAGE, std::integral_constant<int, 2 * LOADS>{},
+            second_step(1, lds + sn * STAGE, PATCH ? lds : lds + sn * STAGE, std::integral_constant<int, 2 * LOADS>{},
                         [&](int q) {
                             if constexpr (fast)
                                 issue_fast(sc + (q & 1), q >> 1);
@@ -737,8 +745,8 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
         {
             // the last block of an odd count: the first half of a pair whose second half is a repeat
             const uint8_t* cur = lds + sc * STAGE;
-            first_step(cur, PATCH ? lds : cur);
-            second_step(cur + STAGE, PATCH ? lds : cur + STAGE, std::integral_constant<int, 0>{}, [](int) {});
+            first_step(0, cur, PATCH ? lds : cur, none, no_load);
+            second_step(0, cur + STAGE, PATCH ? lds : cur + STAGE, none, no_load);
         }
     }
     else if constexpr (APAIR)
@@ -757,17 +765,12 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
             const uint8_t* wb2  = lds + ((n + 2) & 3) * WB;
             const uint8_t* pb0  = lds + PBASE - WB + slot * 2 * PB;
             const uint8_t* pb2  = lds + PBASE - WB + slot_next * 2 * PB;
-            first_step(wb0, pb0);
+            first_step(0, wb0, pb0, std::integral_constant<int, PLOADS>{}, [&](int q) { issue_p(n + 2, slot_next, PLOADS + q); });
             asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * PLOADS + WLOADS) : "memory");
-            second_step(wb1, pb0 + PB, std::integral_constant<int, WLOADS>{}, [&](int q) { issue_w(n + 3, q); });
-            first_step(wb1, pb0 + PB);
-            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(WLOADS) : "memory");
-            second_step(wb2, pb2, std::integral_constant<int, 2 * PLOADS + WLOADS>{}, [&](int q) {
-                if (q < 2 * PLOADS)
-                    issue_p(n + 4, slot_free, q);
-                else
-                    issue_w(n + 4, q - 2 * PLOADS);
-            });
+            second_step(0, wb1, pb0 + PB, std::integral_constant<int, WLOADS>{}, [&](int q) { issue_w(n + 3, q); });
+            first_step(1, wb1, pb0 + PB, std::integral_constant<int, PLOADS>{}, [&](int q) { issue_p(n + 4, slot_free, q); });
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PLOADS + WLOADS) : "memory");
+            second_step(1, wb2, pb2, std::integral_constant<int, WLOADS>{}, [&](int q) { issue_w(n + 4, q); });
             slot = slot_next;
         }
         if (nb & 1)
@@ -775,8 +778,8 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
             // the last block of an odd count: published by the barrier before it, nothing left to request
             const uint8_t* wb = lds + ((nb - 1) & 3) * WB;
             const uint8_t* pb = lds + PBASE - WB + slot * 2 * PB;
-            first_step(wb, pb);
-            second_step(wb, pb, std::integral_constant<int, 0>{}, [](int) {});
+            first_step(0, wb, pb, none, no_load);
+            second_step(0, wb, pb, none, no_load);
         }
     }
     else
@@ -789,19 +792,19 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
         if constexpr (!TAPS && kStages == 4)
         {
             const uint8_t* fptr[LOADS];            // K-contiguous: source of block n + kStages
-            const uint8_t* kptr[LOADS][kStages];    // K-major: source of block n + kStages - 1 + r
+            const uint8_t* kptr[LOADS][kStages];    // K-major: source of block n + kStages - 1 + r (late loads: one less)
 #pragma unroll
             for (int j = 0; j < LOADS; j++)
             {
                 fptr[j] = gbase[j] + (size_t)kStages * gstep[j];
 #pragma unroll
                 for (int r = 0; r < kStages; r++)
-                    kptr[j][r] = gbase[j] + (size_t)(kStages - 1 + r) * gstep[j];
+                    kptr[j][r] = gbase[j] + (size_t)(kStages - 1 - (j < EARLY ? 0 : 1) + r) * gstep[j];
             }
-            auto issue_trip = [&](int r, int j) {
+            auto issue_trip = [&](int r, int j) {    // block n + kStages - 1 + r (late loads: one less)
                 if (KM && j < WLOADS)
                 {
-                    const uint32_t dst = ldst[j] + ((r + kStages - 1) % kStages) * STAGE;
+                    const uint32_t dst = ldst[j] + ((r + kStages - (j < EARLY ? 1 : 2)) % kStages) * STAGE;
                     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                                  :
                                  : "v"(voff[j]), "s"(kptr[j][r]), "s"(dst)
@@ -816,8 +819,9 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                        "n"(((R + kStages - 1) % kStages) * STAGE - (R - 1) * 64), "n"((R - 1) * 64)                    \
                      : "memory", "scc");                                                                               \
         break;
-                switch (r)
+                switch (j < EARLY ? r : r - 1)
                 {
+                    TMI_TRIP_LOAD(-1)
                     TMI_TRIP_LOAD(0)
                     TMI_TRIP_LOAD(1)
                     TMI_TRIP_LOAD(2)
@@ -833,9 +837,9 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                 {
                     const uint8_t* cur  = lds + r * STAGE;
                     const uint8_t* next = lds + ((r + 1) % kStages) * STAGE;
-                    first_step(cur, cur);
+                    first_step(r & 1, cur, cur, std::integral_constant<int, LATE>{}, [&](int q) { issue_trip(r, EARLY + q); });
                     publish();
-                    second_step(next, next, std::integral_constant<int, LOADS>{}, [&](int q) { issue_trip(r, q); });
+                    second_step(r & 1, next, next, std::integral_constant<int, EARLY>{}, [&](int q) { issue_trip(r, q); });
                 }
 #pragma unroll
                 for (int j = 0; j < LOADS; j++)
@@ -852,9 +856,11 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
         {
             const uint8_t* cur  = lds + (n % kStages) * STAGE;
             const uint8_t* next = lds + ((n + 1) % kStages) * STAGE;
-            first_step(cur, cur);
+            first_step(n & 1, cur, cur, std::integral_constant<int, LATE>{}, [&](int q) {
+                issue_one(n + kStages - 2, (n + kStages - 2) % kStages, EARLY + q);
+            });
             publish();    // block n+1 (after the last block: its repeat) is in LDS for every wave
-            second_step(next, next, std::integral_constant<int, LOADS>{}, [&](int q) {
+            second_step(n & 1, next, next, std::integral_constant<int, EARLY>{}, [&](int q) {
                 issue_one(n + kStages - 1, (n + kStages - 1) % kStages, q);
             });
         }
@@ -864,7 +870,9 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     // The loads issued past the last block are still on their way into LDS: let them land before a stage is
     // given another use.  The stage buffers are then free: the channel sums go through the first one.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    int* tab_wsum = reinterpret_cast<int*>(lds);    // WROWS words
+    int* tab_wsum = reinterpret_cast<int*>(lds);           // a row of WROWS words per wp
+    int* tab_psum = reinterpret_cast<int*>(lds + 5120);    // a row of PROWS words per wo
+    static_assert(WROWS * 16 <= 4096 && 5120 + PROWS * 8 <= 8192, "below the transposition buffers, beside the late bias table");
     if constexpr (ZP || APAIR)
     {
         __syncthreads();    // every wave has read its last fragments and seen its last loads land
@@ -876,14 +884,24 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
             for (int t = 0; t < OCT; t++)
             {
                 const int sum = wsum[t] + __shfl_xor(wsum[t], 32);
-                if (wp == 0 && h == 0)
-                    tab_wsum[wo * 32 * OCT + t * 32 + row_channel(rho)] = sum;
+                if (h == 0)
+                    tab_wsum[wp * WROWS + wo * 32 * OCT + t * 32 + row_channel(rho)] = sum;
             }
 #pragma unroll
             for (int i = 0; i < PXT; i++)
-                psum[i] += __shfl_xor(psum[i], 32);
+            {
+                const int sum = psum[i] + __shfl_xor(psum[i], 32);
+                if (h == 0)
+                    tab_psum[wo * PROWS + wp * 32 * PXT + i * 32 + rho] = sum;
+            }
         }
         __syncthreads();
+        if constexpr (ZP)
+        {
+#pragma unroll
+            for (int i = 0; i < PXT; i++)
+                psum[i] = tab_psum[wp * 32 * PXT + i * 32 + rho] + tab_psum[PROWS + wp * 32 * PXT + i * 32 + rho];
+        }
     }
     // Four-byte results (int32, fp32) whose rows are whole 128-byte lines per channel tile leave through LDS: a lane
     // holds 64 bytes of one pixel's row, so a store instruction straight from the accumulators is 64 separate
@@ -969,7 +987,11 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
 #pragma unroll
             for (int q = 0; q < 4; q++)
             {
-                const v4i sw = *reinterpret_cast<const v4i*>(tab_wsum + tl + group_channel(q));
+                const int* src = tab_wsum + tl + group_channel(q);
+                v4i sw         = *reinterpret_cast<const v4i*>(src);
+#pragma unroll
+                for (int r = 1; r < 4; r++)
+                    sw += *reinterpret_cast<const v4i*>(src + r * WROWS);
                 cb[4 * q] += kzz - a.za * sw.x, cb[4 * q + 1] += kzz - a.za * sw.y;
                 cb[4 * q + 2] += kzz - a.za * sw.z, cb[4 * q + 3] += kzz - a.za * sw.w;
             }
