@@ -625,10 +625,28 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
     if (depthwise && !name && ctx->kernel_choice != 1 && ctx->kernel_choice != 4 && ctx->kernel_choice != 6)
         name = launch_depthwise_vec(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                     ctx->flags_dev);
+    // The kernel with resident weights or split reductions takes channel vectors of any length as they lie
+    const bool taps_open  = !depthwise && ctx->kernel_choice == 0 && w_zp == 0;
+    const int32_t t_row   = g.IC * (d->in_dtype == TMI_INT8 ? 1 : 2);
+    const int64_t t_steps = ((int64_t)g.KH * g.KW * ((t_row + 15) / 16) + 1) / 2;
+    const int64_t t_tiles = ((total / g.OC + 31) / 32) * ((g.OC + 31) / 32);
+    auto launch_taps = [&]() {
+        return launch_conv2d_taps(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
+                                  ctx->pages_dev + (d->in_dtype == TMI_INT8 ? (in_zp & 255) * 64 : 0), ctx->flags_dev);
+    };
     // Channel vectors of no whole steps, where kernels that need whole ones lead by more than the copies cost
     if (!depthwise && ctx->kernel_choice == 0 && own_scratch && w_zp == 0)
     {
-        const int32_t padded = padded_channel_bytes(d->in_dtype, g, total, rp.enabled);
+        int32_t padded = padded_channel_bytes(d->in_dtype, g, total, rp.enabled);
+        // What would be padded and is small: one launch of the kernel that needs no whole steps.  us padded / this: int8 3x3 [18,21,21,48]->16
+        // 9.2 / 4.0, [2,35,35,45]->8 6.3 / 4.7, [2,34,31,272]->480 stride 2 11.1 / 7.7, [7,24,24,112]->160 stride 2 10.6 / 4.7; fp16 1x1
+        // [5,8,11,69]->440 8.1 / 3.6.  From 36 steps on, odd rows (loads that start between words, at a quarter of the rate) are
+        // padded first: bf16 [1,45,9,219]->23 18.9 / 11, int8 [2,11,16,285]->42 5x5 34 / 18.
+        // (Up to 36 tiles the copies stay: they are a few microseconds either way, and the tests of the padded route lie there.)
+        if (padded && taps_open && t_tiles > 36 && t_tiles * t_steps <= (t_row % 16 == 0 ? 24000 : 6000) && !(t_row % 4 != 0 && t_steps >= 36))
+            padded = 0, name = launch_taps();
+        if (name)
+            return after_launch(ctx, name);
         const int64_t in_rows = (int64_t)g.N * g.IH * g.IW, w_rows = (int64_t)g.OC * g.KH * g.KW;
         const int32_t eb      = d->in_dtype == TMI_INT8 ? 1 : 2;
         const size_t need     = padded ? pad_channels_bytes(in_rows, w_rows, g.IC * eb, padded) : 0;
@@ -722,7 +740,8 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         if (!name && ctx->kernel_choice == 0 && (g.IC <= 112 || deep_first))
             name = launch_conv2d_pointwise(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                            ctx->flags_dev);
-        if (!name && ctx->kernel_choice == 0 && d->in_dtype == TMI_INT8 && direct_leads(g, total, rp.enabled))
+        if (!name && ctx->kernel_choice == 0 && d->in_dtype == TMI_INT8 && direct_leads(g, total, rp.enabled) &&
+            (!taps_open || t_tiles <= 36 || direct_us(g, total) < conv2d_taps_us(d->in_dtype, g)))
             name = launch_conv2d_direct(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                         ctx->flags_dev);
         // (left open, the slab kernel's layers with more than 128 input channels are the ones tried above)
@@ -768,9 +787,27 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         if (!name && (ctx->kernel_choice == 5 || (ctx->kernel_choice == 0 && g.IC <= 160)))    // (the layers it leads on were tried above)
             name = launch_conv2d_pointwise(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                            ctx->flags_dev);
+        // 16-bit layers the GEMM kernel would spread over a few of the CUs, with channels its whole-line stores do not cover.  us GEMM
+        // kernel / resident weights or split reduction: 1x1 fp16 [5,19,11,224]->344 9.2 / 4.1, bf16 [2,47,65,288]->136 10.0 / 5.9; the other way:
+        // [5,60,8,320]->192 4.9 / 5.7, 3x3 [9,31,26,128]->128 10.6 / 13.9.
+        if (!name && taps_open && gemm_1st && fp16b && g.OC % 64 != 0 && t_tiles * t_steps <= 17500)
+            name = launch_taps();
         if (!name && gemm_1st)
             name = launch_gemm_mfma(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out, 0, 0,
                                     pad_page, ctx->flags_dev);
+        // Everything the kernels above leave open goes to the kernel with resident weights or split reductions.  us patch kernel / this
+        // one, eager calls: int8 [1,49,49,616]->59 3x3 stride 2 77 / 11.8, [4,20,20,600]->175 3x3 stride 2 49 / 11.4, [2,13,18,200]->40 5x5 stride 2
+        // 47 / 11.2, [6,147,147,208]->16 34 / 8.6, [36,129,126,20]->101 192 / 43, [4,35,35,324]->120 18.2 / 5.6, [19,84,89,16]->108 3x3 63 / 22,
+        // [5,24,29,8]->48 3x3 stride 2 7.4 / 4.2; fp16 [1,33,98,70]->16 3x3 stride 2 29.6 / 5.2, [15,54,65,68]->64 28.2 / 7.6, [9,31,41,240]->32
+        // 3x3 stride 2 28.9 / 8.2, [2,104,8,10]->16 3x3 5.6 / 3.8.  The patch kernel keeps long reductions over many tiles of 32 x 32 results
+        // ([10,74,27,160]->48 fp16 (1250 tiles, 90 steps) 16.7 / 27, [8,97,97,144]->48 5x5 stride 2 (1200, 113) 31.7 / 46, [12,15,22,176]->321 fp16
+        // (1364, 99) 23.4 / 34, [4,72,32,288]->48 bf16 (576, 162) 23.4 / 24.5) and layers with taps of 700 ... 2400 tiles whose rows are whole words, where its one round of large tiles
+        // is well filled ([5,93,77,64]->56 fp16 12.5 / 16.8, [10,50,50,56]->56 5x5 14.4 / 17.8, [59,15,15,24]->96 5x5 9.9 / 11.8, [4,106,106,16]->32
+        // 5.5 / 6.8; the other way [14,92,75,48]->48 fp16 stride 2 11.3 / 7.8, [4,28,33,16]->264 8.1 / 5.4).
+        const bool long_and_many = t_steps >= 90 && t_tiles > (t_steps >= 140 ? 380 : (t_steps >= 120 ? 480 : 700));
+        const bool patch_filled  = g.KH * g.KW > 1 && t_tiles > 700 && t_tiles <= (t_steps >= 64 ? 3400 : 2400) && t_row % 8 == 0 && g.OC % 8 == 0;
+        if (!name && taps_open && !long_and_many && !patch_filled)
+            name = launch_taps();
         if (!name && patch_ok)
             name = launch_conv2d_mfma(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                       ctx->flags_dev);

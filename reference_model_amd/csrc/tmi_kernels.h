@@ -108,6 +108,13 @@ const char* launch_conv2d_stem(hipStream_t st, int32_t in_dtype, int32_t out_dty
                                const void* w, const void* bias, int32_t in_zp, int32_t w_zp, const RescaleParams& rp, void* out,
                                void* scratch, uint32_t* flag_word);
 
+// conv_taps.hip: int8, fp16 and bf16 CONV2D with weight_zp 0, weights resident in LDS, pixels loaded where they lie
+const char* launch_conv2d_taps(hipStream_t st, int32_t in_dtype, int32_t out_dtype, const ConvGeom& g, const void* in, const void* w,
+                               const void* bias, int32_t in_zp, int32_t w_zp, const RescaleParams& rp, void* out, const void* pad_page,
+                               uint32_t* flag_word);
+// what a layer takes in it, us (launch included; 1e9: too deep a reduction)
+double conv2d_taps_us(int32_t in_dtype, const ConvGeom& g);
+
 // conv_ksplit.hip: the form of launch_conv2d_pointwise's layers with both operands through LDS (IC = 512 ... 2048 in multiples
 // of 256, at most 1024 tiles of 32 x 32 results); false where it does not apply
 bool launch_point_split(hipStream_t st, const ConvGeom& g, const void* in, const void* w, const void* bias, int32_t in_zp,
