@@ -209,7 +209,7 @@ static int grid_for(int64_t total)
 }
 
 const char* launch_conv_precise(hipStream_t st, int32_t in_dtype, bool depthwise, const ConvGeom& g, const void* in,
-                                const void* w, const void* bias, int32_t abs_mode, double* abs_max_slot, double* out)
+                                const void* w, const void* bias, int32_t abs_mode, double* abs_max_slot, double* out, void* copies)
 {
     PreciseConvArgs a{};
     a.g = g, a.in = in, a.w = w, a.bias = bias, a.out = out, a.abs_mode = abs_mode, a.depthwise = depthwise ? 1 : 0;
@@ -231,6 +231,8 @@ const char* launch_conv_precise(hipStream_t st, int32_t in_dtype, bool depthwise
         }
         a.input_abs_max = abs_max_slot;
     }
+    if (!depthwise && copies && launch_ordered_conv_copied(st, in_dtype, true, g, in, w, bias, abs_mode != 0, a.input_abs_max, out, copies))
+        return abs_mode ? "conv_bounds_copied_f64" : "conv_precise_copied_f64";
     if (!depthwise)
         switch (launch_ordered_conv(st, in_dtype, true, g, in, w, bias, abs_mode != 0, a.input_abs_max, out))
         {

@@ -508,6 +508,12 @@ bool direct_leads(const ConvGeom& g, int64_t total, bool fused)
     return direct_us(g, total) + 0.3 < patch;
 }
 
+// Scratch for the operand copies of ordered_copies.hip, or nullptr (bytes 0, or no memory for them).
+void* ordered_copies(tmi_ctx* ctx, size_t bytes)
+{
+    return bytes ? copy_scratch(ctx, bytes) : nullptr;
+}
+
 // CONV2D: the bytes a channel vector is padded to by a launch of its own (2.5 us and the copy), 0 to read the operands as they lie.
 // us as they lie / padded, graph replays, int8 with the fused RESCALE unless noted, 3x3 unless noted:
 int32_t padded_channel_bytes(int32_t in_dtype, const ConvGeom& g, int64_t total, bool fused)
@@ -819,6 +825,10 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         return fail(ctx, "%s: no MFMA / vector kernel is eligible for this shape", op);
     // FP32 sums keep the reference's order: the tiles of ordered_gemm.hip, whose results are the one-result-per-lane kernel's bit
     // for bit
+    if (!name && !depthwise && ctx->kernel_choice == 0 && d->in_dtype == TMI_FP32 && own_scratch)
+        if (void* copies = ordered_copies(ctx, ordered_conv_copies_bytes(false, g)))
+            if (launch_ordered_conv_copied(ctx->stream, TMI_FP32, false, g, in, w, bias, false, nullptr, out, copies))
+                name = "conv2d_copied_f32";
     if (!name && !depthwise && ctx->kernel_choice == 0 && d->in_dtype == TMI_FP32)
         switch (launch_ordered_conv(ctx->stream, TMI_FP32, false, g, in, w, bias, false, nullptr, out))
         {
@@ -1670,7 +1680,8 @@ static int run_conv_precise(tmi_ctx* ctx, const char* op, bool depthwise, const 
     // one double of the context's 256-byte block (bytes 160..167) holds the input's largest magnitude
     double* abs_max_slot = (bounds_mode && !local_bound) ? reinterpret_cast<double*>(reinterpret_cast<uint8_t*>(ctx->flags_dev) + 160)
                                                          : nullptr;
-    const char* name = launch_conv_precise(ctx->stream, d->in_dtype, depthwise, g, in, w, bias, bounds_mode, abs_max_slot, out);
+    const char* name = launch_conv_precise(ctx->stream, d->in_dtype, depthwise, g, in, w, bias, bounds_mode, abs_max_slot, out,
+                                           depthwise ? nullptr : ordered_copies(ctx, ordered_conv_copies_bytes(true, g)));
     if (!name)
         return fail(ctx, "%s: operand type without a precise-mode kernel", op);
     return after_launch(ctx, name);

@@ -147,13 +147,18 @@ OrderedForm launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, cons
                          const void* bias, bool abs_mode, const double* input_abs_max, void* out);
 OrderedForm launch_ordered_matmul(hipStream_t st, int32_t in_dtype, bool f64, int32_t N, int32_t H, int32_t C, int32_t W, const void* a,
                            const void* b, bool abs_mode, void* out);
+// ordered_copies.hip: the same on copies of the operands in `copies` (ordered_conv_copies_bytes() of 256-byte aligned memory; 0: not taken)
+size_t ordered_conv_copies_bytes(bool f64, const ConvGeom& g);
+bool launch_ordered_conv_copied(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w,
+                                const void* bias, bool abs_mode, const double* input_abs_max, void* out, void* copies);
 // precise.hip: fp64 precise-mode / bounds-mode passes (abs_mode != 0: sums over absolute values) of CONV2D,
 // DEPTHWISE_CONV2D and MATMUL on fp16 / bf16 / fp32 operands, and the DOT_PRODUCT check as a reduction that leaves one
 // partial result per workgroup (at most kDpCheckBlocks of them) in `partials`.  nullptr for another operand type.
 // abs_max_slot: device scratch of one double; when given together with abs_mode, every input element is replaced by
 // the input tensor's largest magnitude (the bounds pass of an operator whose local_bound attribute is false).
+// copies: scratch of ordered_copies.hip for layers that are to run there, or nullptr.
 const char* launch_conv_precise(hipStream_t st, int32_t in_dtype, bool depthwise, const ConvGeom& g, const void* in,
-                                const void* w, const void* bias, int32_t abs_mode, double* abs_max_slot, double* out);
+                                const void* w, const void* bias, int32_t abs_mode, double* abs_max_slot, double* out, void* copies);
 const char* launch_matmul_precise(hipStream_t st, int32_t in_dtype, int32_t N, int32_t H, int32_t C, int32_t W,
                                   const void* a, const void* b, int32_t abs_mode, double* out);
 struct DpPartial

@@ -1,0 +1,77 @@
+"""The ordered sums on copies of the operands (fp32 CONV2D and its fp64 passes): bit for bit the oracle's loop nest, at the edges of tiles,
+granules and stages, and where a weight is infinite under a tap outside the image."""
+import numpy as np
+import pytest
+
+import gpu_ops
+import oracle
+from reference_model_amd import Context, capi
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = Context(0)
+    yield c
+    c.close()
+
+
+CASES = [  # n, ih, iw, ic, oc, kh, kw, pads, strides, dilations, fp32 sums on copies too
+    (1, 5, 6, 50, 33, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), True),       # 450: single elements, odd granules, one column past a tile
+    (2, 4, 5, 45, 7, 3, 3, (1, 0, 1, 0), (1, 1), (1, 1), True),        # few channels
+    (1, 9, 9, 26, 66, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1), False),      # 234
+    (1, 7, 8, 65, 64, 2, 4, (2, 2, 1, 3), (1, 2), (2, 1), True),       # dilated, strided, uneven padding
+    (1, 6, 4, 116, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), True),      # 1044, whole groups of four
+    (1, 6, 5, 128, 65, 3, 3, (0, 0, 0, 0), (1, 1), (1, 1), False),     # 1152, whole stages, no padding
+    (1, 2, 3, 51, 5, 2, 2, (0, 0, 0, 0), (1, 1), (1, 1), False),       # two results in a row of 204
+    (1, 114, 113, 59, 65, 2, 2, (1, 0, 0, 1), (1, 1), (1, 1), False),  # a whole round of tiles and quarters
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("infinite", [False, True])
+def test_conv2d_on_copies(ctx, case, infinite):
+    n, ih, iw, ic, oc, kh, kw, pad, stride, dil, f32 = case
+    rng = np.random.default_rng(ic * oc)
+    x = rng.normal(0, 1, (n, ih, iw, ic)).astype(np.float32)
+    w = rng.normal(0, 0.3, (oc, kh, kw, ic)).astype(np.float32)
+    b = rng.normal(0, 1, oc if ic % 2 else 1).astype(np.float32)
+    if infinite:
+        w[oc // 2, 0, 0, 1] = np.inf
+    oh, ow = oracle.conv_out_hw(ih, iw, kh, kw, pad, stride, dil)
+    bias = np.broadcast_to(b, oc)
+    with np.errstate(invalid="ignore"):
+        if f32:
+            got, st = gpu_ops.conv2d(ctx, x, w, b, pad, stride, dil, dtype=capi.FP32)
+            assert st == capi.VALID and ctx.last_kernel == "conv2d_copied_f32"
+            assert np.array_equal(got, oracle.conv2d("f32", x, w, bias, pad, stride, dil), equal_nan=True)
+        d = ctx.conv_desc(capi.FP32, capi.FP32, x.shape, oc, kh, kw, (oh, ow), pad, stride, dil, len(b))
+        dev = [ctx.upload(v) for v in (x, w, b)]
+        for bounds in (False,) if infinite else (False, True):    # (the oracle's bounds pass multiplies the padding out: NaN)
+            for local in (True, False) if bounds else (True,):
+                out = ctx.empty((n, oh, ow, oc), capi.F64)
+                ctx.conv2d_precise(d, *dev, bounds, out, local_bound=local)
+                assert ctx.sync() == capi.VALID and ctx.last_kernel == ("conv_bounds" if bounds else "conv_precise") + "_copied_f64"
+                xs = x.astype(np.float64) if local else np.full(x.shape, np.abs(x).max(), np.float64)
+                want = oracle.conv2d("f64", xs, w.astype(np.float64), bias.astype(np.float64), pad, stride, dil, abs_mode=bounds)
+                assert np.array_equal(out.numpy(), want, equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+def test_precise_pass_of_sixteen_bit_operands(ctx, dtype):
+    """An image of infinities and NaN: only products of its own elements may see them."""
+    rng = np.random.default_rng(5)
+    ih, iw, ic, oc = 6, 7, 27, 35
+    x, w, b = (rng.integers(-8, 9, s).astype(np.float32) / 4 for s in ((1, ih, iw, ic), (oc, 3, 3, ic), (oc,)))
+    x[0, 2, 3, ic - 1], x[0, 5, 6, 0] = np.inf, np.nan
+    code = capi.FP16 if dtype == "fp16" else capi.BF16
+    narrow = (lambda v: v.astype(np.float16)) if dtype == "fp16" else (lambda v: (v.view(np.uint32) >> 16).astype(np.uint16))    # (exact)
+    d = ctx.conv_desc(code, code, x.shape, oc, 3, 3, (ih, iw), (1, 1, 1, 1), (1, 1), (1, 1), oc)
+    dev = [ctx.upload(narrow(v), code) for v in (x, w, b)]
+    out = ctx.empty((1, ih, iw, oc), capi.F64)
+    ctx.conv2d_precise(d, *dev, False, out)
+    assert ctx.sync() == capi.VALID and ctx.last_kernel == "conv_precise_copied_f64"
+    with np.errstate(invalid="ignore"):
+        want = oracle.conv2d("f64", *(v.astype(np.float64) for v in (x, w, b)), (1, 1, 1, 1), (1, 1), (1, 1))
+    assert np.array_equal(out.numpy(), want, equal_nan=True)
