@@ -6,14 +6,15 @@
 // straight into the registers the matrix instruction reads (lane = row lane % 32, 16 bytes of K of half lane / 32), and moves
 // its part of the second operand, [K][W] as it lies, through a piece of LDS of its own, from which the transposing reads
 // (ds_read_b64_tr_b16 / _b8) return K-contiguous fragments; the next block's loads are in flight meanwhile.  Loads are 16 bytes
-// from any address (gfx950 takes global addresses of any alignment); only the end of a row of the first operand and the end of
-// the tensor go element by element.  The partial tiles meet in LDS.  Rows of the tile are rows of the result, so that 32
-// lanes store 128 neighbouring bytes.
+// from any address (gfx950 takes global addresses of any alignment), the last of a tensor from its last 16 bytes.  The partial
+// tiles meet in LDS.  Rows of the tile are rows of the result, so that 32 lanes store 128 neighbouring bytes.  Workgroups of
+// neighbouring tiles share an L2 (us without / with: fp16 7 x [78,853]x[853,2096] 20.6 / 17.2, int8 [1,4096]x[4096,4096] 8.7 / 6.5; fp16
+// the same 10.0 / 10.7).
 //
 // What bounds it: the first operand's fragments, a line per lane and load, for products of many tiles (fp16 at 130 TFLOP/s), the
-// chain of a wave's blocks otherwise.  us transposed copy + patch or GEMM kernel -> here: fp16 96 x [197,64]x[64,197] 33.6 -> 9.7
-// (34 MB with the next: 2.4 TB/s), 96 x [197,197]x[197,64] 45.3 -> 9.1, [1,4096]x[4096,4096] 49.7 -> 11.6, [1,3731]x[3731,144] 507 -> 8.8,
-// int8 3 x [1000,999]x[999,1001] 191 -> 30, [64,512]x[512,512] 11.5 -> 4.8.
+// chain of a wave's blocks otherwise.  us transposed copy + patch or GEMM kernel -> here: fp16 96 x [197,64]x[64,197] 33.6 -> 8.8
+// (34 MB with the next: 2.2 TB/s), 96 x [197,197]x[197,64] 45.3 -> 7.3, [1,4096]x[4096,4096] 49.7 -> 9.4, int8 4 x [700,701]x[701,703]
+// 13.4 (20.8 before its ends were read in one piece), [64,512]x[512,512] 11.5 -> 4.8.
 #include <type_traits>
 
 #include "tmi_mfma.h"
@@ -30,6 +31,7 @@ struct RaggedArgs
     int32_t H, C, W;
     int32_t za, zb;
     int32_t tiles;    // of all batches
+    uint32_t per_xcd;    // workgroups / 8, rounded down
     FastDiv per_batch, tiles_w;
 };
 
@@ -57,7 +59,39 @@ __device__ __forceinline__ v4i load_front(const uint8_t* p, int n)
     return v4i{ (int)d[0], (int)d[1], (int)d[2], (int)d[3] };
 }
 
-template <typename T, int SPLIT>
+// v without its first n bytes, zeros behind (n < 16)
+__device__ __forceinline__ v4i drop_bytes(v4i v, int n)
+{
+    uint64_t lo = (uint32_t)v[0] | (uint64_t)(uint32_t)v[1] << 32, hi = (uint32_t)v[2] | (uint64_t)(uint32_t)v[3] << 32;
+    if (n & 8)
+        lo = hi, hi = 0;
+    const int bits = 8 * (n & 7);
+    if (bits)
+        lo = lo >> bits | hi << (64 - bits), hi >>= bits;
+    return v4i{ (int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32) };
+}
+// the first n bytes of v, zeros behind (n may be negative)
+__device__ __forceinline__ v4i keep_bytes(v4i v, int n)
+{
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+    {
+        const int m = n - 4 * k;
+        v[k]        = m >= 4 ? v[k] : (m <= 0 ? 0 : v[k] & (int)((1u << (8 * m)) - 1u));
+    }
+    return v;
+}
+
+// bytes of LDS of a wave: a block of the second operand, then its partial tile
+template <typename T, int SPLIT, int NC>
+constexpr int ragged_wave_lds()
+{
+    constexpr int EB = (int)sizeof(T), block = 64 / EB * (32 * NC * EB + (NC == 2 ? 32 * EB : 0));
+    return SPLIT > 1 && block < 4096 * NC ? 4096 * NC : block;
+}
+
+// NC: column blocks of 32 in a tile.  TINY: an operand of less than 16 bytes, read element by element
+template <typename T, int SPLIT, int NC, bool TINY>
 __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_kernel(RaggedArgs p)
 {
     using M             = Mma<T>;
@@ -65,92 +99,137 @@ __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_ke
     using word          = std::conditional_t<M::is_int, int32_t, float>;
     constexpr int EB    = (int)sizeof(T);
     constexpr int KB    = 64 / EB;              // k of a block
-    constexpr int RB    = 64 * EB;              // bytes of a k row of the tile
-    constexpr int LD    = RB + (EB == 2 ? 64 : 32);    // the 4 (8) k rows x 64 (32) bytes of a transposing read touch every bank once
+    constexpr int RB    = 32 * NC * EB;         // bytes of a k row of the tile
+    constexpr int LD    = RB + (NC == 2 ? 32 * EB : 0);    // the 4 (8) k rows x 64 (32) bytes of a transposing read touch every bank once
     constexpr int CPR   = RB / 16;              // 16-byte pieces of a k row
     constexpr int NL    = KB * CPR / 64;        // loads of the second operand per lane and block
     constexpr int kWaves = SPLIT > 4 ? SPLIT : 4;
-    constexpr int kWaveLds = KB * LD > 8192 && SPLIT > 1 ? KB * LD : (SPLIT > 1 ? 8192 : KB * LD);
+    constexpr int kWaveLds = ragged_wave_lds<T, SPLIT, NC>();
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r32 = lane & 31, half = lane >> 5;
-    const uint32_t tile = (blockIdx.x * kWaves + wave) / SPLIT;
+    // a contiguous run of tiles for each of the eight L2s (workgroups go to them in turn)
+    uint32_t bid = blockIdx.x;
+    if (bid < p.per_xcd * 8)
+        bid = (bid & 7) * p.per_xcd + (bid >> 3);
+    const uint32_t tile = (bid * kWaves + wave) / SPLIT;
     if (SPLIT < kWaves && SPLIT == 1 && tile >= (uint32_t)p.tiles)
         return;
     const bool live      = tile < (uint32_t)p.tiles;
     const uint32_t t     = live ? tile : 0;
     const uint32_t batch = fdiv(t, p.per_batch), in_batch = t - batch * p.per_batch.d, th = fdiv(in_batch, p.tiles_w);
-    const int h0 = (int)th * 32, w0 = (int)(in_batch - th * p.tiles_w.d) * 64;
+    const int h0 = (int)th * 32, w0 = (int)(in_batch - th * p.tiles_w.d) * 32 * NC;
     uint8_t* mine = lds + wave * kWaveLds;
 
-    const int row_bytes  = p.C * EB;
-    const int h          = h0 + r32 < p.H ? h0 + r32 : p.H - 1;
-    const uint8_t* arow  = p.a + ((int64_t)batch * p.H + h) * row_bytes + 16 * half;
-    // (16 bytes from a row that is not the tensor's last may run into the next row)
-    const int64_t pitch  = (int64_t)p.W * EB;
-    const int64_t b_off  = (int64_t)batch * p.C * pitch + (int64_t)w0 * EB + (lane & (CPR - 1)) * 16;
-    const int krow       = lane / CPR;                       // k row of the lane's first load
-    const int blocks     = (p.C + KB - 1) / KB;
-    const bool col_ok    = w0 + (lane & (CPR - 1)) * (16 / EB) < p.W;
+    const int row_bytes = p.C * EB, piece = (lane & (CPR - 1)) * 16, krow = lane / CPR;    // (krow: k row of the lane's first load)
+    const int rows      = p.H - h0 < 32 ? p.H - h0 : 32;
+    const int64_t pitch = (int64_t)p.W * EB;
+    const int64_t a_tile = ((int64_t)batch * p.H + h0) * row_bytes, b_tile = (int64_t)batch * p.C * pitch + (int64_t)w0 * EB;
+    const uint32_t a_lane = (uint32_t)(r32 < rows ? r32 : rows - 1) * (uint32_t)row_bytes + 16 * half, b_lane = (uint32_t)krow * (uint32_t)pitch + piece;
+    const int blocks = (p.C + KB - 1) / KB, first = wave % SPLIT;
+    const int shares = live && first < blocks ? (blocks - first + SPLIT - 1) / SPLIT : 0;    // blocks of this wave
 
+    // Loads are 16 bytes wherever they begin, at the last 16 bytes of the tensor at the latest; what they bring from behind a row of the
+    // first operand, from behind K or from before their place (the end of the tensor) goes in finish(), which loads nothing.  (Where the
+    // ends were read element by element, a wave waited for eight loads one after the other: us then / now, fp16 96 x [197,197]x[197,64]
+    // 8.0 / 7.2, 10 x [55,40]x[40,55] 6.3 / 4.0, int8 8 x [4,125]x[125,922] 6.7 / 4.5.  Two and three blocks of registers instead of one: the
+    // products of many tiles lose more to fewer waves than they gain, fp16 127 x [203,128]x[128,203] 15.5 / 19.1 with three.)
+    struct Place
+    {
+        const uint8_t* base;
+        uint32_t extra, most;    // what to add to an offset, and how large the sum may be
+    };
+    auto place = [&](const uint8_t* t, int64_t total, int64_t at) {
+        const int64_t to = at < total - 16 ? at : total - 16, room = total - 16 - to;
+        return Place{ t + to, (uint32_t)(at - to), room < INT32_MAX ? (uint32_t)room : (uint32_t)INT32_MAX };
+    };
     v4i av[2], bv[NL];
-    auto request = [&](int blk) {
-        const int k0 = blk * KB;
-        // the first operand: two pieces of 32 bytes of K, this lane's 16 of each
-        if (k0 + KB <= p.C)
-        {
-            av[0] = load16(arow + k0 * EB), av[1] = load16(arow + k0 * EB + 32);
-        }
-        else
-        {
-            const int left = row_bytes - k0 * EB - 16 * half;
-            av[0] = load_front<EB>(arow + k0 * EB, left), av[1] = load_front<EB>(arow + k0 * EB + 32, left - 32);
-        }
-        const uint8_t* src = p.b + b_off + (k0 + krow) * pitch;
-        if (k0 + KB <= p.C && b_off - (lane & (CPR - 1)) * 16 + (k0 + KB - 1) * pitch + RB <= p.b_total)
+    auto request = [&](int share) {
+        const int k0 = (first + share * SPLIT) * KB;
+        if constexpr (TINY)
         {
 #pragma unroll
-            for (int j = 0; j < NL; j++)
-                bv[j] = load16(src + j * (64 / CPR) * pitch);
-        }
-        else
-        {
+            for (int j = 0; j < 2; j++)
+                av[j] = load_front<EB>(p.a + a_tile + (int64_t)(r32 < rows ? r32 : rows - 1) * row_bytes + 16 * half + k0 * EB + 32 * j, row_bytes - k0 * EB - 16 * half - 32 * j);
 #pragma unroll
             for (int j = 0; j < NL; j++)
             {
-                const int k = k0 + krow + j * (64 / CPR);
-                const int64_t at = b_off + k * pitch;
-                bv[j] = v4i{ 0, 0, 0, 0 };
-                if (k < p.C && col_ok)
-                    bv[j] = at + 16 <= p.b_total ? load16(p.b + at) : load_front<EB>(p.b + at, (int)(p.b_total - at));
+                const int k      = k0 + krow + j * (64 / CPR);
+                const int64_t at = b_tile + k * pitch + piece, left = p.b_total - at;
+                bv[j]         = load_front<EB>(p.b + at, k < p.C ? (left < 16 ? (int)left : 16) : 0);
+            }
+            return;
+        }
+        const Place pa = place(p.a, p.a_total, a_tile + k0 * EB), pb = place(p.b, p.b_total, b_tile + k0 * pitch);
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+        {
+            const uint32_t off = a_lane + pa.extra + 32 * j;
+            av[j]           = load16(pa.base + (off < pa.most ? off : pa.most));
+        }
+#pragma unroll
+        for (int j = 0; j < NL; j++)
+        {
+            const uint32_t off = b_lane + pb.extra + j * (64 / CPR) * (uint32_t)pitch;
+            bv[j]           = load16(pb.base + (off < pb.most ? off : pb.most));
+        }
+    };
+    auto finish = [&](int share) {
+        int k0 = (first + share * SPLIT) * KB;
+        asm volatile("" : "+s"(k0));    // (worked out again rather than kept from request())
+        const bool k_tail = k0 + KB > p.C;
+        if (k_tail)
+        {
+            const Place pa = place(p.a, p.a_total, a_tile + k0 * EB);
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+            {
+                const uint32_t off = a_lane + pa.extra + 32 * j;
+                if (off > pa.most)
+                    av[j] = drop_bytes(av[j], (int)(off - pa.most) & 15);
+                av[j] = keep_bytes(av[j], row_bytes - k0 * EB - 16 * half - 32 * j);
+            }
+        }
+        if (k_tail || b_tile + (k0 + KB - 1) * pitch + RB > p.b_total)
+        {
+            const Place pb = place(p.b, p.b_total, b_tile + k0 * pitch);
+#pragma unroll
+            for (int j = 0; j < NL; j++)
+            {
+                const uint32_t off = b_lane + pb.extra + j * (64 / CPR) * (uint32_t)pitch;
+                if (off > pb.most)
+                    bv[j] = drop_bytes(bv[j], (int)(off - pb.most) & 15);
+                if (k0 + krow + j * (64 / CPR) >= p.C)
+                    bv[j] = v4i{ 0, 0, 0, 0 };
             }
         }
     };
 
-    acc_t acc[2];
+    acc_t acc[NC];
 #pragma unroll
-    for (int c = 0; c < 2; c++)
+    for (int c = 0; c < NC; c++)
 #pragma unroll
         for (int i = 0; i < 16; i++)
             acc[c][i] = 0;
-    int sum_a = 0, sum_b[2] = { 0, 0 };    // of the lane's row and columns (int8)
+    int sum_a = 0, sum_b[NC] = {};    // of the lane's row and columns (int8)
     const bool sums = M::is_int && (p.za | p.zb) != 0;
 
-    const int first = wave % SPLIT;
     // source of a transposing read: k row sl / 4 of four (sl / 2 of eight), 8 bytes of columns; see the GEMM kernel
     const int sl = lane & 15, cblk = (lane >> 4) & 1;
     const int tr = EB == 2 ? (8 * half + (sl >> 2)) * LD + (16 * cblk + 4 * (sl & 3)) * 2 : (16 * half + (sl >> 1)) * LD + 16 * cblk + 8 * (sl & 1);
-    if (live && first < blocks)
-        request(first);
-    for (int blk = first; live && blk < blocks; blk += SPLIT)
+    if (shares > 0)
+        request(0);
+    for (int i = 0; i < shares; i++)
     {
+        if constexpr (!TINY)
+            finish(i);
 #pragma unroll
         for (int j = 0; j < NL; j++)
             *reinterpret_cast<v4i*>(mine + (krow + j * (64 / CPR)) * LD + (lane & (CPR - 1)) * 16) = bv[j];
         const v4i a0 = av[0], a1 = av[1];
         __builtin_amdgcn_wave_barrier();
-        if (blk + SPLIT < blocks)
-            request(blk + SPLIT);
+        if (i + 1 < shares)
+            request(i + 1);
 #pragma unroll
         for (int s = 0; s < 2; s++)
         {
@@ -158,7 +237,7 @@ __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_ke
             if (sums)
                 sum_a += dot4_ones(a);
 #pragma unroll
-            for (int c = 0; c < 2; c++)
+            for (int c = 0; c < NC; c++)
             {
                 v4i b;
 #pragma unroll
@@ -184,7 +263,7 @@ __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_ke
         // each share brings its own part of the correction
         sum_a += __shfl_xor(sum_a, 32);
 #pragma unroll
-        for (int c = 0; c < 2; c++)
+        for (int c = 0; c < NC; c++)
         {
             const int col = p.za * (sum_b[c] + __shfl_xor(sum_b[c], 32)) - (first == 0 ? p.C * p.za * p.zb : 0);
 #pragma unroll
@@ -201,7 +280,7 @@ __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_ke
     if constexpr (SPLIT == 1)
     {
 #pragma unroll
-        for (int c = 0; c < 2; c++)
+        for (int c = 0; c < NC; c++)
 #pragma unroll
             for (int i = 0; i < 16; i++)
                 store(c, i, acc[c][i]);
@@ -211,7 +290,7 @@ __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_ke
         // a wave's partial tile in its own 8 KB (its reads of the second operand are done), then 1 / SPLIT of the sums each
         word* part = reinterpret_cast<word*>(mine);
 #pragma unroll
-        for (int c = 0; c < 2; c++)
+        for (int c = 0; c < NC; c++)
 #pragma unroll
             for (int i = 0; i < 16; i++)
                 part[(16 * c + i) * 64 + lane] = acc[c][i];
@@ -219,7 +298,7 @@ __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_ke
         if (!live)
             return;
         const uint8_t* base = lds + wave / SPLIT * SPLIT * kWaveLds;
-        constexpr int kEach = 32 / SPLIT;
+        constexpr int kEach = 16 * NC / SPLIT;
 #pragma unroll
         for (int e = 0; e < kEach; e++)
         {
@@ -314,30 +393,31 @@ bool launch_matmul_pad(hipStream_t st, int32_t eb, int32_t N, int32_t H, int32_t
     return true;
 }
 
-template <typename T, int SPLIT>
-static bool launch_split(hipStream_t st, const RaggedArgs& p)
+template <typename T, int SPLIT, int NC = 2>
+static bool launch_split(hipStream_t st, RaggedArgs& p)
 {
-    constexpr int EB = (int)sizeof(T), kWaves = SPLIT > 4 ? SPLIT : 4, kBlock = 64 / EB * (64 * EB + (EB == 2 ? 64 : 32));
-    constexpr size_t lds_bytes = (size_t)kWaves * (SPLIT > 1 ? (kBlock > 8192 ? kBlock : 8192) : kBlock);
-    auto kern                  = matmul_ragged_kernel<T, SPLIT>;
+    constexpr int EB = (int)sizeof(T), kWaves = SPLIT > 4 ? SPLIT : 4;
+    constexpr size_t lds_bytes = (size_t)kWaves * ragged_wave_lds<T, SPLIT, NC>();
+    // (and operands whose tile is beyond 32-bit offsets: element by element)
+    const bool tiny            = p.a_total < 16 || p.b_total < 16 || (int64_t)p.C * EB > INT32_MAX / 33 || (int64_t)p.W * EB > INT32_MAX / 65;
+    auto kern                  = tiny ? matmul_ragged_kernel<T, SPLIT, NC, true> : matmul_ragged_kernel<T, SPLIT, NC, false>;
     static LdsLimit granted{};
     if (lds_bytes > 65536 && !ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, granted))
         return false;
-    const int64_t waves = (int64_t)p.tiles * SPLIT;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((waves + kWaves - 1) / kWaves)), dim3(64 * kWaves), lds_bytes, st, p);
+    const int64_t grid = ((int64_t)p.tiles * SPLIT + kWaves - 1) / kWaves;
+    p.per_xcd          = (uint32_t)(grid / 8);
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * kWaves), lds_bytes, st, p);
     return true;
 }
 
 template <typename T>
-static bool launch_ragged(hipStream_t st, const RaggedArgs& p)
+static bool launch_ragged(hipStream_t st, RaggedArgs& p)
 {
     const int blocks = (p.C * (int)sizeof(T) + 63) / 64;
-    // K over as many waves as give the chip two thousand (two a SIMD), each with a block of its own at least.  us for 512 / 1024 / 2048 /
-    // 4096 waves: fp16 96 x [197,197]x[197,64] (672 tiles) 8.5 / 10.0 / 8.1 / 8.0, 96 x [197,64]x[64,197] (2688) 8.5 / 8.5 / 8.4 / 12.3,
-    // 64 x [8,512]x[512,512] (512) 10.5 / 7.5 / 6.5 / 6.9, 4 x [300,301]x[301,303] (200) 6.9 / 6.1 / 6.1 / 6.1, [600,601]x[601,603] (190)
-    // 8.9 / 8.1 / 8.0 / 8.0, [1,4096]x[4096,4096] (64) 10.4 / 9.6 / 9.6 / 9.6; int8 the same in this order 6.7 / 6.6 / 5.8 / 5.8, 7.3 / 7.3 / 7.3 /
-    // 7.4, 5.6 / 4.9 / 5.0 / 5.2, 7.9 / 7.9 / 7.9 / 7.9, 7.5 / 7.1 / 7.1 / 7.1, 7.0 / 7.4 / 7.3 / 7.4; the other way [500,2000]x[2000,500] (128)
-    // fp16 10.2 / 8.7 / 9.1 / 9.0, int8 8.0 / 7.0 / 7.6 / 7.6.
+    // K over as many waves as give the chip two thousand (two a SIMD), each with a block of its own at least.  us for 1024 / 2048 / 4096
+    // waves: fp16 96 x [197,197]x[197,64] (672 tiles) 8.6 / 7.3 / 7.1, 96 x [197,64]x[64,197] (2688) 8.8 / 8.8 / 9.9, 64 x [8,512]x[512,512]
+    // (512) 6.8 / 5.5 / 5.5, 7 x [78,853]x[853,2096] 22.5 / 17.2 / 16.8, 4 x [300,301]x[301,303] (200) 4.8 / 4.9 / 4.8; int8 in this order 6.7 / 5.9 /
+    // 5.7, 7.2 / 7.3 / 7.2, 4.8 / 4.4 / 4.2; the other way [500,2000]x[2000,500] (128) fp16 7.6 / 8.3 / 8.1, int8 5.9 / 6.2 / 6.2.
     int split = 1;
     while (split < 16 && (int64_t)p.tiles * split < 2048 && split * 2 <= blocks)
         split *= 2;
@@ -347,8 +427,20 @@ static bool launch_ragged(hipStream_t st, const RaggedArgs& p)
         case 2: return launch_split<T, 2>(st, p);
         case 4: return launch_split<T, 4>(st, p);
         case 8: return launch_split<T, 8>(st, p);
-        default: return launch_split<T, 16>(st, p);
+        default: break;
     }
+    // Sixteen waves a tile and still few tiles: a workgroup, and the lines its CU's L1 takes in, bound it; tiles of 32 columns then put
+    // twice as many CUs to work, while those fit beside each other.  us 64 / 32 columns: fp16 [1,4096]x[4096,4096] (64 tiles of 64) 11.0 / 9.4,
+    // [13,3215]x[3215,235] x 5 (20) 18.6 / 14.9, [64,4000]x[4000,64] (2) 11.2 / 8.9, [20,1500]x[1500,3000] x 2 (94) 7.7 / 6.0, int8 5.0 / 4.5;
+    // [500,2000]x[2000,500] (128) 8.2 / 8.1, int8 6.2 / 6.4; the other way [100,1100]x[1100,700] x 3 (132) 5.8 / 7.4, 4.9 / 5.8.
+    const int64_t wide = p.tiles_w.d, narrow = ((int64_t)p.W + 31) / 32, rows = p.tiles / wide;
+    if (p.tiles > 112 || !fastdiv_exact_up_to((uint64_t)(rows * narrow), (uint32_t)(p.per_batch.d / wide * narrow)) ||
+        !fastdiv_exact_up_to((uint64_t)(p.per_batch.d / wide * narrow), (uint32_t)narrow))
+        return launch_split<T, 16>(st, p);
+    p.per_batch = make_fastdiv((uint32_t)(p.per_batch.d / wide * narrow));
+    p.tiles     = (int32_t)(rows * narrow);
+    p.tiles_w   = make_fastdiv((uint32_t)narrow);
+    return launch_split<T, 16, 1>(st, p);
 }
 
 const char* launch_matmul_ragged(hipStream_t st, int32_t in_dtype, int32_t N, int32_t H, int32_t C, int32_t W, const void* a, const void* b,

@@ -1588,10 +1588,11 @@ int tmi_matmul(tmi_ctx_t* ctx, int32_t in_dtype, int32_t N, int32_t H, int32_t C
         const bool in_place    = rows_whole && (int64_t)W * eb % 16 == 0;
         const bool few_deep    = tiles128 <= 32 && (int64_t)C * eb >= 1024;
         // Products it cannot read in place: the split kernel, which reads anything, up to 4 G operations; beyond, aligned copies
-        // of the operands and the GEMM kernel.  us split / copies: int8 4 x [700,701]x[701,703] (2.8 G) 20.8 / 21.6, fp16 27.6 / 29.9,
-        // 4 x [1000,1001]x[1001,1003] (8 G) 37.6 / 32.9, fp16 56.9 / 42.9, [1000,..] (2 G) 14.7 / 19.7, 19.3 / 26.9, [2000,2001]x[2001,2003] (16 G)
-        // 65.4 / 38.8, 121 / 52.9.
-        const bool large = H >= 128 && W >= 64 && 2 * total * C > 4000000000ll;
+        // of the operands and the GEMM kernel, but for few tiles and deep K.  us split / copies: int8 4 x [700,701]x[701,703] (2.8 G) 13.6 /
+        // 14.8, fp16 20.7 / 18.7, 4 x [1000,1001]x[1001,1003] (8 G) 31.6 / 21.4, fp16 54.8 / 27.0, 17 x [1850,64]x[64,427] (1.7 G) 13.6 / 20.3,
+        // 17.5 / 19.6, 9 x [217,1403]x[1403,2092] (11.5 G) 53.3 / 31.7, 93.3 / 45.9; 2 x [150,5000]x[5000,1500] (4.5 G, 24 tiles) 16.7 / 37.1, 25.0 / 51.2.
+        // Over 240 drawn products of 0.5 ... 20 G the line is 2.6 % from the better one of each.
+        const bool large = H >= 128 && W >= 64 && 2 * total * C > 4000000000ll && !few_deep;
         if (ctx->kernel_choice == 0 && (in_place ? few_deep : !large))
         {
             name = launch_matmul_ragged(ctx->stream, in_dtype, N, H, C, W, a_dev, b_dev, a_zp, b_zp, out_dev);
