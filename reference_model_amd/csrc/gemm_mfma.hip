@@ -903,21 +903,24 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                 psum[i] = tab_psum[wp * 32 * PXT + i * 32 + rho] + tab_psum[PROWS + wp * 32 * PXT + i * 32 + rho];
         }
     }
-    // Four-byte results (int32, fp32) whose rows are whole 128-byte lines per channel tile leave through LDS: a lane
-    // holds 64 bytes of one pixel's row, so a store instruction straight from the accumulators is 64 separate
+    // Results leave through LDS: a lane holds 64 bytes of one pixel's row, so a store instruction straight from the accumulators is 64 separate
     // 16-byte requests to the L2 (4.2 M of them for the named bf16 MATMUL, which kept its 256 workgroups storing
     // for 22 us at the end); transposed through a per-wave 4.5 KB buffer, an instruction writes 8 whole lines.
+    // Rows of no whole 16 bytes leave word by word (16-bit results: element by element), neighbouring lanes side by side.
+    // us when only whole lines went this way / now: fp16 MATMUL 40 x [300,160]x[160,1304] 86 / 22, 3 x [1300,416]x[416,1304] 41 / 13,
+    // 8 x [1024,1024]x[1024,1000] 59 / 27, on aligned copies 25 x [224,544]x[544,1359] 74 / 43, int8 4 x [1000,1001]x[1001,1003] 30 / 21; fp16
+    // CONV2D [32,28,28,128]->200 1x1 25.8 / 6.9, [8,56,56,64]->136 1x1 20.9 / 5.7, [16,28,28,256]->264 3x3 48 / 36, ->260 48 / 39.
     // (The buffer lies in the stage memory: every wave must be done with its fragments first.)
     const bool wide_out = M::is_int ? !(!APAIR && a.rp.enabled) : a.out_is_wide != 0;
-    const bool lines    = wide_out && (a.N & 31) == 0;
+    constexpr bool ANY_ROWS = KM || !M::is_int;    // (int8 CONV2D: whole lines only, its registers are spoken for)
+    const bool lines        = wide_out && (ANY_ROWS || (a.N & 31) == 0);
     // Floating-point results of the input type (2 bytes): a pixel's OCT x 32 channels are 128 or 256 bytes, gathered
     // from all the wave's channel tiles before they leave.
     constexpr int HROW   = OCT * 64;    // bytes of a pixel's channels held by this wave
     constexpr int HPITCH = HROW + 16;
-    const bool half_lines = !M::is_int && !wide_out && (a.N & 63) == 0 && oc0 + (wo + 1) * 32 * OCT <= a.N;
-    const bool any_half_lines = !M::is_int && !wide_out && (a.N & 63) == 0;    // the same for every wave
+    const bool half_lines = !M::is_int && !wide_out;
     if constexpr (!(ZP || APAIR))
-        if (lines || any_half_lines)
+        if (lines || half_lines)
             __syncthreads();
     constexpr int TPITCH = 144;    // bytes per pixel row in the buffer: 128 + 16, so that rows spread over the banks
     uint8_t* tbuf        = lds + 8192 + wave * (32 * (HPITCH > TPITCH ? HPITCH : TPITCH));
@@ -956,15 +959,34 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                     reinterpret_cast<v4i*>(d)[0] = reinterpret_cast<const v4i*>(packed)[0];
                     reinterpret_cast<v4i*>(d)[1] = reinterpret_cast<const v4i*>(packed)[1];
                 }
-                constexpr int PIECES = HROW / 16;      // 16-byte pieces per pixel row: 8 or 16
-                constexpr int RPI    = 64 / PIECES;    // rows per store instruction
-#pragma unroll
-                for (int j = 0; j < 32 / RPI; j++)
+                const int left = a.N - oc0 - wo * 32 * OCT;    // channels from the wave's first on
+                uint8_t* to    = out_b + ((size_t)pt0 * a.N + oc0 + wo * 32 * OCT) * 2;
+                if ((a.N & 7) == 0)
                 {
-                    const int row = lane / PIECES + RPI * j, piece = lane % PIECES;
-                    const v4i d   = *reinterpret_cast<const v4i*>(tbuf + row * HPITCH + piece * 16);
-                    if (pt0 + row < m_end)
-                        *reinterpret_cast<v4i*>(out_b + ((size_t)(pt0 + row) * a.N + oc0 + wo * 32 * OCT) * 2 + piece * 16) = d;
+                    constexpr int PIECES = HROW / 16;      // 16-byte pieces per pixel row: 8 or 16
+                    constexpr int RPI    = 64 / PIECES;    // rows per store instruction
+#pragma unroll
+                    for (int j = 0; j < 32 / RPI; j++)
+                    {
+                        const int row = lane / PIECES + RPI * j, piece = lane % PIECES;
+                        const v4i d   = *reinterpret_cast<const v4i*>(tbuf + row * HPITCH + piece * 16);
+                        if (pt0 + row < m_end && piece * 8 < left)
+                            *reinterpret_cast<v4i*>(to + (size_t)row * a.N * 2 + piece * 16) = d;
+                    }
+                }
+                else
+                {
+                    // (rows of no whole 16 bytes: a row's elements side by side)
+                    const int rows = m_end - pt0 < 32 ? m_end - pt0 : 32;
+#pragma unroll 4
+                    for (int row = 0; row < rows; row++)
+                    {
+#pragma unroll
+                        for (int u = 0; u < OCT / 2; u++)
+                            if (64 * u + lane < left)
+                                *reinterpret_cast<uint16_t*>(to + 128 * u + 2 * lane) = *reinterpret_cast<const uint16_t*>(tbuf + row * HPITCH + 128 * u + 2 * lane);
+                        to += (size_t)a.N * 2;
+                    }
                 }
             }
             return;
@@ -1023,13 +1045,33 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                 for (int q = 0; q < 4; q++)
                     *reinterpret_cast<v4i*>(tbuf + rho * TPITCH + group_channel(q) * 4) =
                         v4i{ w4[4 * q], w4[4 * q + 1], w4[4 * q + 2], w4[4 * q + 3] };
-#pragma unroll
-                for (int j = 0; j < 4; j++)
+                const int left = a.N - oc0 - tl;    // channels from the tile's first on
+                if (!ANY_ROWS || (a.N & 3) == 0)
                 {
-                    const int row = (lane >> 3) + 8 * j, piece = lane & 7;
-                    const v4i d   = *reinterpret_cast<const v4i*>(tbuf + row * TPITCH + piece * 16);
-                    if (pt0 + row < m_end)
-                        *reinterpret_cast<v4i*>(out_b + ((size_t)(pt0 + row) * a.N + oc0 + tl) * 4 + piece * 16) = d;
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                    {
+                        const int row = (lane >> 3) + 8 * j, piece = lane & 7;
+                        const v4i d   = *reinterpret_cast<const v4i*>(tbuf + row * TPITCH + piece * 16);
+                        if (pt0 + row < m_end && (!ANY_ROWS || piece * 4 < left))
+                            *reinterpret_cast<v4i*>(out_b + ((size_t)(pt0 + row) * a.N + oc0 + tl) * 4 + piece * 16) = d;
+                    }
+                }
+                else
+                {
+                    const int c    = lane & 31, row0 = lane >> 5;
+                    uint8_t* dst   = out_b + ((size_t)(pt0 + row0) * a.N + oc0 + tl + c) * 4;
+                    const uint8_t* src = tbuf + row0 * TPITCH + c * 4;
+                    int rows       = c < left ? m_end - pt0 - row0 : 0;
+#pragma unroll 1
+                    for (int j = 0; j < 4; j++)
+                    {
+#pragma unroll
+                        for (int u = 0; u < 4; u++)
+                            if (2 * u < rows)
+                                *reinterpret_cast<int*>(dst + (size_t)(2 * u) * a.N * 4) = *reinterpret_cast<const int*>(src + 2 * u * TPITCH);
+                        dst += (size_t)8 * a.N * 4, src += 8 * TPITCH, rows -= 8;
+                    }
                 }
                 continue;
             }
@@ -1096,73 +1138,29 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                     }
                     continue;
                 }
-                int32_t* row    = reinterpret_cast<int32_t*>(out_b) + (size_t)p * a.N;
-#pragma unroll
-                for (int q = 0; q < 4; q++)
+                if constexpr (!ANY_ROWS)
                 {
-                    const int oc = oc0 + tl + group_channel(q);
-                    int v[4];
+                    int32_t* row = reinterpret_cast<int32_t*>(out_b) + (size_t)p * a.N;
 #pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        v[e] = acc[i][t][4 * q + e] + cb[4 * q + e] - pcorr;
-                    if (rows4)
+                    for (int q = 0; q < 4; q++)
                     {
-                        if (oc < a.N)
-                            *reinterpret_cast<v4i*>(row + oc) = v4i{ v[0], v[1], v[2], v[3] };
-                    }
-                    else
-                    {
+                        const int oc = oc0 + tl + group_channel(q);
+                        int v[4];
 #pragma unroll
                         for (int e = 0; e < 4; e++)
-                            if (oc + e < a.N)
-                                row[oc + e] = v[e];
-                    }
-                }
-            }
-            else
-            {
-                const int oc = oc0 + tl + 16 * h;    // floating point: always 16 consecutive channels
-                if (oc >= a.N)
-                    continue;
-                float v[16];
+                            v[e] = acc[i][t][4 * q + e] + cb[4 * q + e] - pcorr;
+                        if (rows4)
+                        {
+                            if (oc < a.N)
+                                *reinterpret_cast<v4i*>(row + oc) = v4i{ v[0], v[1], v[2], v[3] };
+                        }
+                        else
+                        {
 #pragma unroll
-                for (int e = 0; e < 16; e++)
-                    v[e] = acc[i][t][e] + __int_as_float(cb[e]);
-                if (a.out_is_wide)
-                {
-                    float* dst = reinterpret_cast<float*>(out_b) + (size_t)p * a.N + oc;
-                    if (rows16)
-                    {
-#pragma unroll
-                        for (int q = 0; q < 4; q++)
-                            reinterpret_cast<v4f*>(dst)[q] = v4f{ v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3] };
-                    }
-                    else
-                    {
-#pragma unroll
-                        for (int e = 0; e < 16; e++)
-                            if (oc + e < a.N)
-                                dst[e] = v[e];
-                    }
-                }
-                else
-                {
-                    T* dst = reinterpret_cast<T*>(out_b) + (size_t)p * a.N + oc;
-                    if (rows16)
-                    {
-                        alignas(16) T packed[16];
-#pragma unroll
-                        for (int e = 0; e < 16; e++)
-                            store_from_float(packed + e, v[e]);
-                        reinterpret_cast<v4i*>(dst)[0] = reinterpret_cast<const v4i*>(packed)[0];
-                        reinterpret_cast<v4i*>(dst)[1] = reinterpret_cast<const v4i*>(packed)[1];
-                    }
-                    else
-                    {
-#pragma unroll
-                        for (int e = 0; e < 16; e++)
-                            if (oc + e < a.N)
-                                store_from_float(dst + e, v[e]);
+                            for (int e = 0; e < 4; e++)
+                                if (oc + e < a.N)
+                                    row[oc + e] = v[e];
+                        }
                     }
                 }
             }
@@ -1468,7 +1466,7 @@ const char* launch_gemm_mfma(hipStream_t st, int32_t in_dtype, int32_t out_dtype
     if (w_kmajor_stride && ((w_kmajor_stride & 15) || w_kmajor_stride < (int64_t)g.OC * eb))
         return nullptr;
     // rows are multiples of 64 bytes, so 16-byte aligned bases keep every operand chunk aligned; the 16-byte
-    // stores are only used when OC is a multiple of 16, which keeps every output row and batch aligned too
+    // stores are only used where an output row is whole 16-byte pieces, which keeps every row and batch aligned too
     if ((((uintptr_t)in | (uintptr_t)w | (uintptr_t)out | (uintptr_t)pad_page) & 15) || (w_batch_stride & 15))
         return nullptr;
     // (enough work to fill the CUs: checked by the launcher of the form that takes the layer)

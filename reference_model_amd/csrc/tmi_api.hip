@@ -793,10 +793,11 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         if (!name && (ctx->kernel_choice == 5 || (ctx->kernel_choice == 0 && g.IC <= 160)))    // (the layers it leads on were tried above)
             name = launch_conv2d_pointwise(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                            ctx->flags_dev);
-        // 16-bit layers the GEMM kernel would spread over a few of the CUs, with channels its whole-line stores do not cover.  us GEMM
-        // kernel / resident weights or split reduction: 1x1 fp16 [5,19,11,224]->344 9.2 / 4.1, bf16 [2,47,65,288]->136 10.0 / 5.9; the other way:
-        // [5,60,8,320]->192 4.9 / 5.7, 3x3 [9,31,26,128]->128 10.6 / 13.9.
-        if (!name && taps_open && gemm_1st && fp16b && g.OC % 64 != 0 && t_tiles * t_steps <= 17500)
+        // 16-bit layers the GEMM kernel would spread over a few of the CUs, with channels its tiles do not divide.  us GEMM
+        // kernel / resident weights or split reduction, fp16 1x1 (pixels): [570,256]->116 5.6 / 4.0, [1512,288]->288 (432 tiles of 32 x 32, 18
+        // steps) 6.0 / 4.9, [2432,320]->112 (304, 20) 6.1 / 5.2, [1368,64]->392 (559, 4) 5.0 / 4.1; the other way: [1692,288]->330 (583, 18)
+        // 7.1 / 7.6, [2100,224]->312 (660, 14) 4.6 / 5.3, [4752,64]->216 (1043, 4) 4.1 / 5.6, 3x3 [3564,128]->393 (1456, 72) 17.4 / 24.3.
+        if (!name && taps_open && gemm_1st && fp16b && g.OC % 64 != 0 && t_tiles <= 650 && t_tiles * t_steps <= 8000)
             name = launch_taps();
         if (!name && gemm_1st)
             name = launch_gemm_mfma(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out, 0, 0,
