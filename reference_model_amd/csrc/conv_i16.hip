@@ -11,8 +11,8 @@
 // result, so that 32 lanes hold neighbouring channels of one pixel and a store instruction writes two runs of 256 bytes.
 //
 // What bounds it: the lines its loads touch, 32 to an instruction of which 32 bytes each are used before the L1 has let go
-// of them: time follows the number of load instructions.  [8,56,56,64]->64 3x3 on one result per lane 1750 us, here 12.6;
-// [16,56,56,64]->64 1x1 365 -> 8.8 (32 MB: 3.7 TB/s).
+// of them: time follows the number of load instructions.  [8,56,56,64]->64 3x3 on one result per lane 1750 us, here 12.2 (10.5 with the
+// weights in LDS: conv_i16_taps.hip, which leads on most layers; long reductions over few pixels, whose weights fill the LDS, are this one's).
 #include "tmi_mfma.h"
 
 namespace tmi

@@ -593,10 +593,15 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // 6.1, whose channels must be padded by a launch of its own, [1,28,28,8]->8 1x1 3.0 / 6.5; the other way [1,14,14,16]->16 3x3,
         // 0.45 M, 6.2 / 4.6).
         const bool tiny   = total * g.KH * g.KW * g.IC < (1 << 17);
-        const size_t need = depthwise || tiny || ctx->kernel_choice == 1 ? 0 : conv_i16_mfma_scratch_bytes(g, w_zp);
-        void* copies      = need > 1 && own_scratch ? copy_scratch(ctx, need) : nullptr;
-        if (need == 1 || copies)
+        const bool matrix = !depthwise && !tiny && ctx->kernel_choice != 1 && w_zp == 0;
+        const size_t need = matrix ? conv_i16_mfma_scratch_bytes(g, w_zp) : 0;
+        if (matrix)
+            name = launch_conv_i16_taps(ctx->stream, g, in, w, bias, out, ctx->pages_dev, need == 1 || (need > 1 && own_scratch));
+        void* copies = !name && need > 1 && own_scratch ? copy_scratch(ctx, need) : nullptr;
+        if (!name && (need == 1 || copies))
             name = launch_conv_i16_mfma(ctx->stream, g, in, w, bias, out, copies);
+        if (!name && matrix)    // (no memory for the copies)
+            name = launch_conv_i16_taps(ctx->stream, g, in, w, bias, out, ctx->pages_dev, false);
         if (!name)
             name = launch_conv_i16_direct(ctx->stream, depthwise, g, in, w, bias, w_zp, out);
         return after_launch(ctx, name);

@@ -280,6 +280,9 @@ bool launch_matmul_pad(hipStream_t st, int32_t eb, int32_t N, int32_t H, int32_t
 // does not take, 1 for one it reads in place, else the scratch its channel-padded operands need.
 size_t conv_i16_mfma_scratch_bytes(const ConvGeom& g, int32_t w_zp);
 const char* launch_conv_i16_mfma(hipStream_t st, const ConvGeom& g, const void* in, const void* w, const void* bias, void* out, void* scratch);
+// conv_i16_taps.hip: the same with the weights in LDS, any channel count; zeros: 64 bytes of them; or_gather: nullptr also where conv_i16.hip leads
+const char* launch_conv_i16_taps(hipStream_t st, const ConvGeom& g, const void* in, const void* w, const void* bias, void* out, const void* zeros,
+                                 bool or_gather);
 // INT16 x INT8 -> INT48 CONV2D / DEPTHWISE_CONV2D and INT16 x INT16 -> INT48 MATMUL (int64 bias and results)
 const char* launch_conv_i16_direct(hipStream_t st, bool depthwise, const ConvGeom& g, const void* in, const void* w,
                                    const void* bias, int32_t w_zp, void* out);
