@@ -1260,6 +1260,11 @@ static int run_transpose_conv2d(tmi_ctx* ctx, bool static_only, const tmi_tconv_
         const SlabHoles h{ d->stride[0], d->stride[1], d->IH, d->IW };
         const char* name = launch_conv2d_slab(ctx->stream, d->in_dtype, d->out_dtype, g, in_dev, weight_dev, bias_dev, in_zp,
                                               w_zp, none, out_dev, ctx->pages_dev + (in_zp & 255) * 64, ctx->flags_dev, &h);
+        // with a stride: class by class of output pixels, nothing copied (on the static scratch memory only what would fit there)
+        const bool fits = !static_only || align256((size_t)d->OC * d->KH * d->KW * row_bytes) + align256((size_t)d->N * UH * UW * row_bytes) <=
+                                              (size_t)TMI_NOALLOC_SCRATCH_BYTES;
+        if (!name && ctx->kernel_choice == 0 && holes && w_zp == 0 && d->out_dtype == TMI_INT32 && fits)
+            name = launch_tconv_taps(ctx->stream, *d, in_dev, weight_dev, bias_dev, in_zp, out_dev, ctx->pages_dev + (in_zp & 255) * 64);
         if (name)
             return after_launch(ctx, name);
     }

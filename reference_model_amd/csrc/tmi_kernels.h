@@ -236,6 +236,8 @@ const char* launch_conv2d_mfma(hipStream_t st, int32_t in_dtype, int32_t out_dty
 // elementwise.hip: [N, R, C] -> [N, C, R] for 1- or 2-byte elements (MATMUL's second operand becomes K-contiguous).
 const char* launch_transpose(hipStream_t st, int32_t elem_bytes, int32_t N, int32_t R, int32_t C, const void* in,
                              void* out);
+// tconv_taps.hip: TRANSPOSE_CONV2D int8 -> int32 with strides, weight_zp 0, class by class; page: 16 bytes of input_zp; nullptr: not taken
+const char* launch_tconv_taps(hipStream_t st, const tmi_tconv_desc_t& d, const void* in, const void* w, const void* bias, int32_t in_zp, void* out, const void* page);
 // relayout.hip: whole-channel-vector copies that turn TRANSPOSE_CONV2D / CONV3D operands into CONV2D operands.
 const char* launch_flip_taps(hipStream_t st, int32_t row_bytes, int32_t OC, int32_t KH, int32_t KW, const void* src,
                              void* dst);
