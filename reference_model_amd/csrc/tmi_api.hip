@@ -606,6 +606,10 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
             name = launch_conv_i16_direct(ctx->stream, depthwise, g, in, w, bias, w_zp, out);
         return after_launch(ctx, name);
     }
+    // 5x5 taps: the kernel that walks down the rows, which loads and permutes an input row once (us one pixel a lane / this one: [1,8,13,16]
+    // 7.0 / 3.4, [41,8,13,440] 28 / 8)
+    if (depthwise && ctx->kernel_choice == 0 && g.KH == 5)
+        name = launch_depthwise_rows(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out, ctx->flags_dev);
     // Small depthwise layers: the vector kernel (a lane per four channels of a pixel, no LDS, no barrier) costs 3.15 us plus
     // 4.4 us per million results, the matrix-core kernel 3.3 us plus 3.7 ns per channel (its per-channel tables) and next
     // to nothing per result.  us matrix-core / vector kernel, 3x3, fused RESCALE: [8,14,14,384] stride 2 4.3 / 3.3,
@@ -615,7 +619,7 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
     // fp16 / bf16 depthwise layers with channels in multiples of 8: the vector kernel (us one-result-per-lane kernel / this
     // one, fp16 3x3: [8,112,112,96] stride 2 25.6 / 8.1, [8,112,112,32] 31.0 / 8.6, [8,56,56,144] 31.6 / 10.7, [8,28,28,192]
     // 11.4 / 5.6, [8,14,14,576] 9.4 / 5.2, [64,112,112,96] stride 2 182 / 38.5)
-    if (depthwise && ctx->kernel_choice != 1 && !rp.enabled && (d->in_dtype == TMI_FP16 || d->in_dtype == TMI_BF16))
+    if (depthwise && !name && ctx->kernel_choice != 1 && !rp.enabled && (d->in_dtype == TMI_FP16 || d->in_dtype == TMI_BF16))
         name = launch_depthwise_fp_vec(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, out);
     if (depthwise && !name && ctx->kernel_choice == 0 && total < 34000 + 850 * (int64_t)g.IC)
         name = launch_depthwise_vec(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
@@ -633,6 +637,10 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
     if (depthwise && !name && (ctx->kernel_choice == 0 || ctx->kernel_choice == 4))
         name = launch_depthwise_slab(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                      ctx->pages_dev + (in_zp & 255) * 64, ctx->flags_dev);
+    // what the matrix-core kernels leave, with 3x3 taps: the same (us one pixel a lane / this one: [10,131,128,40] 16.5 / 11.4; channels that are no
+    // multiple of four, one result a lane: [34,13,18,445] 33 / 11, [5,22,22,65] 4.9 / 3.6)
+    if (depthwise && !name && ctx->kernel_choice == 0)
+        name = launch_depthwise_rows(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out, ctx->flags_dev);
     if (depthwise && !name && ctx->kernel_choice != 1 && ctx->kernel_choice != 4 && ctx->kernel_choice != 6)
         name = launch_depthwise_vec(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                     ctx->flags_dev);

@@ -258,6 +258,9 @@ const char* launch_conv3d_operands(hipStream_t st, int32_t row_bytes, int32_t OC
 size_t pad_channels_bytes(int64_t in_rows, int64_t w_rows, int32_t row_bytes, int32_t padded);
 void launch_pad_channels(hipStream_t st, int64_t in_rows, int64_t w_rows, int32_t row_bytes, int32_t padded, const void* in, const void* w,
                          void* scratch, const void** in_padded, const void** w_padded);
+// depthwise_rows.hip: 3x3 and 5x5 taps, strides 1 and 2, any channel count, weight_zp 0; nullptr: not taken
+const char* launch_depthwise_rows(hipStream_t st, int32_t in_dtype, int32_t out_dtype, const ConvGeom& g, const void* in, const void* w, const void* bias,
+                                  int32_t in_zp, int32_t w_zp, const RescaleParams& rp, void* out, uint32_t* flag_word);
 // depthwise.hip: 4 channels per lane, dot4 across taps, fused epilogue; nullptr when not eligible.
 const char* launch_depthwise_vec(hipStream_t st, int32_t in_dtype, int32_t out_dtype, const ConvGeom& g,
                                  const void* in, const void* w, const void* bias, int32_t in_zp, int32_t w_zp,
