@@ -919,8 +919,10 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     constexpr int HROW   = OCT * 64;    // bytes of a pixel's channels held by this wave
     constexpr int HPITCH = HROW + 16;
     const bool half_lines = !M::is_int && !wide_out;
+    const bool rows16     = (a.N & 15) == 0;    // every lane's 16 channels are inside the tensor or all outside
+    const bool gathered   = M::is_int && !KM && !wide_out && !rows16;    // RESCALE results of no whole pieces: a channel tile's at a time
     if constexpr (!(ZP || APAIR))
-        if (lines || half_lines)
+        if (lines || half_lines || gathered)
             __syncthreads();
     constexpr int TPITCH = 144;    // bytes per pixel row in the buffer: 128 + 16, so that rows spread over the banks
     uint8_t* tbuf        = lds + 8192 + wave * (32 * (HPITCH > TPITCH ? HPITCH : TPITCH));
@@ -928,9 +930,30 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     // A lane's 16 accumulator registers of a tile are four groups of 4 consecutive channels: group q starts at
     // channel 16h + 4q (all 16 consecutive), or 8q + 4h with the in-order row assignment.
     auto group_channel = [&](int q) { return IDENT ? 8 * q + 4 * h : 16 * h + 4 * q; };
-    const bool rows16 = (a.N & 15) == 0;    // every lane's 16 channels are inside the tensor or all outside
     const bool rows4  = (a.N & 3) == 0;     // the same for a group of 4
     uint8_t* out_b    = reinterpret_cast<uint8_t*>(a.out) + batch * a.o_batch;
+    constexpr int GPITCH = 80;    // bytes of a pixel's 32 channels (at most 64) in the buffer, and 16
+    auto store_gathered  = [&](int pt0, int tl) {
+        // words of a row side by side where its length allows, else elements
+        const int left = a.N - oc0 - tl, rows = m_end - pt0 < 32 ? m_end - pt0 : 32, bytes = (left < 32 ? left : 32) * a.out_bytes;
+        const uint32_t pitch = (uint32_t)a.N * (uint32_t)a.out_bytes;
+        const int unit = (pitch & 3) == 0 ? 4 : a.out_bytes, log_lanes = 5 + (a.out_bytes >> 1) - (unit >> 1);    // lanes of a row: its 32 elements' bytes / unit
+        const int at   = (lane & ((1 << log_lanes) - 1)) * unit;
+        uint8_t* to    = out_b + (size_t)pt0 * pitch + (size_t)(oc0 + tl) * a.out_bytes + at;
+#pragma unroll 1
+        for (int row = lane >> log_lanes; row < rows; row += 64 >> log_lanes)
+            if (at < bytes)
+            {
+                const uint8_t* from = tbuf + row * GPITCH + at;
+                uint8_t* dst        = to + (size_t)row * pitch;
+                if (unit == 4)
+                    *reinterpret_cast<int*>(dst) = *reinterpret_cast<const int*>(from);
+                else if (unit == 2)
+                    *reinterpret_cast<uint16_t*>(dst) = *reinterpret_cast<const uint16_t*>(from);
+                else
+                    *dst = *from;
+            }
+    };
     if constexpr (!M::is_int)
     {
         if (half_lines)
@@ -1075,48 +1098,38 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                 }
                 continue;
             }
-            if (p >= m_end || oc0 + tl >= a.N)
-                continue;
-            if constexpr (M::is_int)
-            {
-                const int pcorr = ZP ? a.zw * psum[i] : 0;
-                if (!APAIR && a.rp.enabled)
+            if constexpr (M::is_int && !APAIR && !KM)
+                if (a.rp.enabled)
                 {
-                    // fused RESCALE (+ CLAMP): the lane's 16 consecutive channels leave as 16 (32) bytes
-                    const int ocl = tl + 16 * h;
-                    const int oc  = oc0 + ocl;
-                    if (oc >= a.N)
+                    // fused RESCALE (+ CLAMP): the lane's 16 consecutive channels leave as 16 (32) bytes, by way of the buffer where rows
+                    // are no whole pieces (byte by byte from the lanes, us then / now: 1x1 [32,28,28,256]->520 51 / 27, [32,28,28,512]->264 32 / 20,
+                    // 3x3 [32,28,28,192]->200 42 / 31, [16,28,28,256]->250 25.0 / 20.6)
+                    const int ocl   = tl + 16 * h, oc = oc0 + ocl, pt0 = p0 + wp * 32 * PXT + i * 32;
+                    const int pcorr = ZP ? a.zw * psum[i] : 0;
+                    if (pt0 >= m_end || oc0 + tl >= a.N)
                         continue;
-                    int r[16];
+                    if (p < m_end && oc < a.N)
+                    {
+                        int r[16];
 #pragma unroll
-                    for (int e = 0; e < 16; e++)
-                    {
-                        const ChannelScale cs = tab_cs[ocl + e];
-                        r[e] = fast_rescale(acc[i][t][e] + cb[e] - pcorr, cs, a.rp.out_zp, a.rp.lo, a.rp.hi, flags);
-                    }
-                    uint8_t* dst = out_b + ((size_t)p * a.N + oc) * a.out_bytes;
-                    if (a.out_bytes == 1)
-                    {
-                        if (rows16)
+                        for (int e = 0; e < 16; e++)
+                        {
+                            const ChannelScale cs = tab_cs[ocl + e];
+                            r[e] = fast_rescale(acc[i][t][e] + cb[e] - pcorr, cs, a.rp.out_zp, a.rp.lo, a.rp.hi, flags);
+                        }
+                        if (a.out_bytes == 1)
                         {
                             v4i packed;
 #pragma unroll
                             for (int q = 0; q < 4; q++)
                                 packed[q] = (r[4 * q] & 0xff) | ((r[4 * q + 1] & 0xff) << 8) |
                                             ((r[4 * q + 2] & 0xff) << 16) | ((r[4 * q + 3] & 0xff) << 24);
-                            *reinterpret_cast<v4i*>(dst) = packed;
+                            if (gathered)
+                                *reinterpret_cast<v4i*>(tbuf + rho * GPITCH + 16 * h) = packed;
+                            else
+                                *reinterpret_cast<v4i*>(out_b + (size_t)p * a.N + oc) = packed;
                         }
                         else
-                        {
-#pragma unroll
-                            for (int e = 0; e < 16; e++)
-                                if (oc + e < a.N)
-                                    dst[e] = (uint8_t)r[e];
-                        }
-                    }
-                    else
-                    {
-                        if (rows16)
                         {
 #pragma unroll
                             for (int hq = 0; hq < 2; hq++)
@@ -1125,19 +1138,22 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
 #pragma unroll
                                 for (int q = 0; q < 4; q++)
                                     packed[q] = (r[8 * hq + 2 * q] & 0xffff) | ((r[8 * hq + 2 * q + 1] & 0xffff) << 16);
-                                reinterpret_cast<v4i*>(dst)[hq] = packed;
+                                if (gathered)
+                                    *reinterpret_cast<v4i*>(tbuf + rho * GPITCH + 32 * h + 16 * hq) = packed;
+                                else
+                                    reinterpret_cast<v4i*>(out_b + ((size_t)p * a.N + oc) * 2)[hq] = packed;
                             }
                         }
-                        else
-                        {
-#pragma unroll
-                            for (int e = 0; e < 16; e++)
-                                if (oc + e < a.N)
-                                    reinterpret_cast<int16_t*>(dst)[e] = (int16_t)r[e];
-                        }
                     }
+                    if (gathered)
+                        store_gathered(pt0, tl);
                     continue;
                 }
+            if (p >= m_end || oc0 + tl >= a.N)
+                continue;
+            if constexpr (M::is_int)
+            {
+                const int pcorr = ZP ? a.zw * psum[i] : 0;
                 if constexpr (!ANY_ROWS)
                 {
                     int32_t* row = reinterpret_cast<int32_t*>(out_b) + (size_t)p * a.N;
