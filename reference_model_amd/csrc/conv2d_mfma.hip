@@ -1121,9 +1121,8 @@ static constexpr int kCUs    = 256;
 template <typename T, int WOC, int OCT, int PXT, int EPI, bool VEC, bool MULTI>
 static bool launch_patch(hipStream_t st, PatchArgs& a, size_t lds_bytes, int blocks)
 {
-    auto kern                = conv2d_patch_kernel<T, WOC, OCT, PXT, EPI, VEC, MULTI>;
-    static LdsLimit granted{};
-    if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, granted))
+    constexpr auto kern      = conv2d_patch_kernel<T, WOC, OCT, PXT, EPI, VEC, MULTI>;
+    if (!ensure_dynamic_lds<kern>(lds_bytes))
         return false;
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(512), lds_bytes, st, a);
     return true;

@@ -1012,9 +1012,8 @@ thread_local int32_t last_launch_shape[3] = { 0, 0, 0 };
 template <int KH, int KW, int CH, bool ZA, bool FUSED, bool TC = false, int KD = 1, int NPT = 1, typename T = int8_t>
 static bool launch_slab_kernel(hipStream_t st, const SlabArgsX& a, int grid, int lds_bytes)
 {
-    auto kern              = conv2d_slab_kernel<KH, KW, CH, ZA, FUSED, TC, KD, NPT, T>;
-    static LdsLimit granted{};
-    if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
+    constexpr auto kern    = conv2d_slab_kernel<KH, KW, CH, ZA, FUSED, TC, KD, NPT, T>;
+    if (!ensure_dynamic_lds<kern>((size_t)lds_bytes))
         return false;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds_bytes, st, static_cast<const std::conditional_t<(TC || KD > 1), SlabArgsX, SlabArgs>&>(a));
     last_launch_shape[0] = grid, last_launch_shape[1] = 512, last_launch_shape[2] = lds_bytes;
@@ -1023,9 +1022,9 @@ static bool launch_slab_kernel(hipStream_t st, const SlabArgsX& a, int grid, int
 
 static bool launch_slab_wreg(hipStream_t st, const SlabArgsX& a, int grid, int lds_bytes)
 {
-    auto launch = [&](auto kern) {
-        static LdsLimit granted{};
-        if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
+    auto launch = [&](auto kernel) {
+        constexpr auto kern = decltype(kernel)::value;
+        if (!ensure_dynamic_lds<kern>((size_t)lds_bytes))
             return false;
         hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds_bytes, st, static_cast<const SlabArgs&>(a));
         last_launch_shape[0] = grid, last_launch_shape[1] = 512, last_launch_shape[2] = lds_bytes;
@@ -1036,8 +1035,8 @@ static bool launch_slab_wreg(hipStream_t st, const SlabArgsX& a, int grid, int l
     // 16 5.25 / 5.10, 20 5.67 / 5.56, 32 6.96 / 6.64, 64 11.0 / 10.47.
     const bool vl = (a.TH * (int)a.div_tw.d + 31) / 32 >= 5;
     if (vl)
-        return a.za != 0 ? launch(conv2d_slab_wreg_kernel<true, true>) : launch(conv2d_slab_wreg_kernel<false, true>);
-    return a.za != 0 ? launch(conv2d_slab_wreg_kernel<true, false>) : launch(conv2d_slab_wreg_kernel<false, false>);
+        return a.za != 0 ? launch(kernel_constant<conv2d_slab_wreg_kernel<true, true>>{}) : launch(kernel_constant<conv2d_slab_wreg_kernel<false, true>>{});
+    return a.za != 0 ? launch(kernel_constant<conv2d_slab_wreg_kernel<true, false>>{}) : launch(kernel_constant<conv2d_slab_wreg_kernel<false, false>>{});
 }
 
 // the floating-point instantiations: fp16 (kind 1) or bf16 (kind 2)

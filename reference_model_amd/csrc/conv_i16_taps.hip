@@ -373,9 +373,8 @@ template <int CT, bool SPLIT, bool RAGGED>
 static bool launch_i16_taps(hipStream_t st, I16TapsArgs& a)
 {
     const int64_t lds = i16_taps_lds<CT, SPLIT>(a.steps);
-    auto kern         = conv_i16_taps_kernel<CT, SPLIT, RAGGED>;
-    static LdsLimit granted{};
-    if (lds > 65536 && !ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds, granted))
+    constexpr auto kern = conv_i16_taps_kernel<CT, SPLIT, RAGGED>;
+    if (lds > 65536 && !ensure_dynamic_lds<kern>((size_t)lds))
         return false;
     // as many workgroups as the chip holds, for each channel block
     const int64_t blocks = (a.OC + 16 * CT - 1) / (16 * CT), rounds = SPLIT ? a.n_pt : (a.n_pt + 3) / 4;

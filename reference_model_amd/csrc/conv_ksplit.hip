@@ -682,15 +682,15 @@ static bool launch_point_split_ks(hipStream_t st, const PointSplitArgs& a, int g
 {
     constexpr int own = 2 * 32 * (KS * 32 + 16) > 4096 ? 2 * 32 * (KS * 32 + 16) : 4096;
     constexpr int lds_bytes = 32 * 16 + 32 * 8 + 8 * 128 + 16 + 8 * own;
-    auto go = [&](auto kern, LdsLimit& granted) {
-        if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
+    auto go = [&](auto kernel) {
+        constexpr auto kern = decltype(kernel)::value;
+        if (!ensure_dynamic_lds<kern>((size_t)lds_bytes))
             return false;
         hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds_bytes, st, a);
         last_launch_shape[0] = grid, last_launch_shape[1] = 512, last_launch_shape[2] = lds_bytes;
         return true;
     };
-    static LdsLimit granted[2]{};
-    return a.za != 0 ? go(point_split_kernel<KS, true>, granted[1]) : go(point_split_kernel<KS, false>, granted[0]);
+    return a.za != 0 ? go(kernel_constant<point_split_kernel<KS, true>>{}) : go(kernel_constant<point_split_kernel<KS, false>>{});
 }
 
 // False where the form does not apply.  (The caller has checked the layer: see launch_conv2d_pointwise.)
@@ -721,9 +721,8 @@ template <int KS, int NW, bool ZA>
 static bool launch_conv_ksplit_za(hipStream_t st, const ConvSplitArgs& a, int grid)
 {
     constexpr int lds_bytes = NW * 4096 + 32 * 16 + 32 * 8 + NW * 128 + 16;
-    static LdsLimit granted{};
-    auto kern = conv_ksplit_i8_kernel<KS, NW, ZA>;
-    if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
+    constexpr auto kern = conv_ksplit_i8_kernel<KS, NW, ZA>;
+    if (!ensure_dynamic_lds<kern>((size_t)lds_bytes))
         return false;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), lds_bytes, st, a);
     last_launch_shape[0] = grid, last_launch_shape[1] = NW * 64, last_launch_shape[2] = lds_bytes;
@@ -739,16 +738,16 @@ static bool launch_conv_ksplit(hipStream_t st, const ConvSplitArgs& a, int grid)
 template <int NW, int NPT>
 static bool launch_conv_ksplit_patch(hipStream_t st, const ConvPatchSplitArgs& a, int lds_bytes)
 {
-    auto go = [&](auto kern, LdsLimit& granted) {
-        if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
+    auto go = [&](auto kernel) {
+        constexpr auto kern = decltype(kernel)::value;
+        if (!ensure_dynamic_lds<kern>((size_t)lds_bytes))
             return false;
         const int grid = a.n_groups * (int)a.div_oct.d;
         hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), lds_bytes, st, a);
         last_launch_shape[0] = grid, last_launch_shape[1] = NW * 64, last_launch_shape[2] = lds_bytes;
         return true;
     };
-    static LdsLimit granted[2]{};
-    return a.za != 0 ? go(conv_ksplit_patch_kernel<NW, NPT, true>, granted[1]) : go(conv_ksplit_patch_kernel<NW, NPT, false>, granted[0]);
+    return a.za != 0 ? go(kernel_constant<conv_ksplit_patch_kernel<NW, NPT, true>>{}) : go(kernel_constant<conv_ksplit_patch_kernel<NW, NPT, false>>{});
 }
 
 // Cuts the layer into blocks of up to `slots` output pixels whose patch fits the LDS beside `other` bytes.  False if none does.

@@ -846,10 +846,9 @@ static bool launch_taps(hipStream_t st, TapsArgs& a)
     // results whose rows are no whole words and all of one workgroup
     a.rows_bytes           = (a.OC & 3) && a.OC <= 32 * OCT && a.out_kind != 0 ? 32 * a.OC * (a.out_kind == 1 ? 1 : 2) : 0;
     const size_t lds_bytes = (size_t)taps_lds_bytes<OCT>(a.steps) + kTapsWaves * a.rows_bytes;
-    auto kern              = conv_taps_kernel<T, OCT, RAGGED>;
-    static LdsLimit granted{};
+    constexpr auto kern    = conv_taps_kernel<T, OCT, RAGGED>;
     unsigned grid;
-    if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, granted) ||
+    if (!ensure_dynamic_lds<kern>(lds_bytes) ||
         !taps_grid(a, OCT, (a.n_pt + kTapsWaves - 1) / kTapsWaves, lds_bytes > 80 * 1024 ? 1 : (lds_bytes > 53 * 1024 ? 2 : 3), grid))
         return false;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kTapsWaves * 64), lds_bytes, st, a);

@@ -386,9 +386,8 @@ template <bool ZA, bool FUSED>
 static bool launch_dwslab_kernel(hipStream_t st, DwSlabArgs a, int grid, int threads, int lds_bytes)
 {
     a.nwaves     = threads / 64;
-    auto kern = depthwise_slab_kernel<ZA, FUSED>;
-    static LdsLimit granted{};
-    if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
+    constexpr auto kern = depthwise_slab_kernel<ZA, FUSED>;
+    if (!ensure_dynamic_lds<kern>((size_t)lds_bytes))
         return false;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds_bytes, st, a);
     return true;

@@ -365,9 +365,8 @@ template <bool ZA, bool FUSED, int G>
 static bool launch_dwstream_kernel(hipStream_t st, DwStreamArgs a, int grid, int threads, int lds_bytes)
 {
     a.nw     = threads / 64;
-    auto kern = depthwise_stream_kernel<ZA, FUSED, G>;
-    static LdsLimit granted{};
-    if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds_bytes, granted))
+    constexpr auto kern = depthwise_stream_kernel<ZA, FUSED, G>;
+    if (!ensure_dynamic_lds<kern>((size_t)lds_bytes))
         return false;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds_bytes, st, a);
     return true;

@@ -1198,9 +1198,8 @@ static bool launch_gemm_pipe(hipStream_t st, const GemmArgs& a, int blocks)
                                         ? (size_t)STAGES * 64 * OCT * 64 + (size_t)a.patch_bytes
                                         : (size_t)STAGES * (64 * OCT + 128 * PXT) * 64) +
                                        64 * OCT * 4 + 64 * OCT * 32;
-    auto kern                  = gemm_lds_kernel<T, OCT, PXT, ZP, MODE, STAGES, PIPE>;
-    static LdsLimit granted{};
-    if (!ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, granted))
+    constexpr auto kern        = gemm_lds_kernel<T, OCT, PXT, ZP, MODE, STAGES, PIPE>;
+    if (!ensure_dynamic_lds<kern>(lds_bytes))
         return false;
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(512), lds_bytes, st, a);
     return true;

@@ -393,21 +393,27 @@ bool launch_matmul_pad(hipStream_t st, int32_t eb, int32_t N, int32_t H, int32_t
     return true;
 }
 
-template <typename T, int SPLIT, int NC = 2>
-static bool launch_split(hipStream_t st, RaggedArgs& p)
+template <typename T, int SPLIT, int NC, bool TINY>
+static bool launch_split_form(hipStream_t st, RaggedArgs& p)
 {
-    constexpr int EB = (int)sizeof(T), kWaves = SPLIT > 4 ? SPLIT : 4;
+    constexpr int kWaves       = SPLIT > 4 ? SPLIT : 4;
     constexpr size_t lds_bytes = (size_t)kWaves * ragged_wave_lds<T, SPLIT, NC>();
-    // (and operands whose tile is beyond 32-bit offsets: element by element)
-    const bool tiny            = p.a_total < 16 || p.b_total < 16 || (int64_t)p.C * EB > INT32_MAX / 33 || (int64_t)p.W * EB > INT32_MAX / 65;
-    auto kern                  = tiny ? matmul_ragged_kernel<T, SPLIT, NC, true> : matmul_ragged_kernel<T, SPLIT, NC, false>;
-    static LdsLimit granted{};
-    if (lds_bytes > 65536 && !ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, granted))
+    constexpr auto kern        = matmul_ragged_kernel<T, SPLIT, NC, TINY>;
+    if (lds_bytes > 65536 && !ensure_dynamic_lds<kern>(lds_bytes))
         return false;
     const int64_t grid = ((int64_t)p.tiles * SPLIT + kWaves - 1) / kWaves;
     p.per_xcd          = (uint32_t)(grid / 8);
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * kWaves), lds_bytes, st, p);
     return true;
+}
+
+template <typename T, int SPLIT, int NC = 2>
+static bool launch_split(hipStream_t st, RaggedArgs& p)
+{
+    constexpr int EB = (int)sizeof(T);
+    // (and operands whose tile is beyond 32-bit offsets: element by element)
+    const bool tiny = p.a_total < 16 || p.b_total < 16 || (int64_t)p.C * EB > INT32_MAX / 33 || (int64_t)p.W * EB > INT32_MAX / 65;
+    return tiny ? launch_split_form<T, SPLIT, NC, true>(st, p) : launch_split_form<T, SPLIT, NC, false>(st, p);
 }
 
 template <typename T>

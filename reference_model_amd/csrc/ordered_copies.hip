@@ -565,11 +565,10 @@ static bool launch_copied(hipStream_t st, CopiedArgs& p)
     p.n_big   = tiles <= 192 || p.OC <= 32 ? 0 : (int32_t)(over <= 192 ? tiles - over : tiles / 8 * 8);
     const int64_t grid = p.n_big + 4 * (tiles - p.n_big);
     // few workgroups: a long ring, for the waves of one workgroup hide nothing of each other's loads
-    static LdsLimit granted_long{}, granted_short{};
-    const bool longer = grid <= 256 && ensure_dynamic_lds(reinterpret_cast<const void*>(ordered_copied_kernel<F64, 8>), 8 * 16384, granted_long);
+    const bool longer = grid <= 256 && ensure_dynamic_lds<ordered_copied_kernel<F64, 8>>(8 * 16384);
     if (longer)
         hipLaunchKernelGGL((ordered_copied_kernel<F64, 8>), dim3((unsigned)grid), dim3(256), 8 * 16384, st, p);
-    else if (ensure_dynamic_lds(reinterpret_cast<const void*>(ordered_copied_kernel<F64, 4>), 4 * 16384, granted_short))
+    else if (ensure_dynamic_lds<ordered_copied_kernel<F64, 4>>(4 * 16384))
         hipLaunchKernelGGL((ordered_copied_kernel<F64, 4>), dim3((unsigned)grid), dim3(256), 4 * 16384, st, p);
     else
         return false;

@@ -310,9 +310,8 @@ static bool launch_tconv(hipStream_t st, TconvArgs& a)
 {
     static_assert(sizeof(TconvArgs) <= 256, "see there");
     const int64_t lds = tconv_lds<CT>(a.steps);
-    auto kern         = tconv_taps_kernel<CT, RAGGED>;
-    static LdsLimit granted{};
-    if (lds > 65536 && !ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (size_t)lds, granted))
+    constexpr auto kern = tconv_taps_kernel<CT, RAGGED>;
+    if (lds > 65536 && !ensure_dynamic_lds<kern>((size_t)lds))
         return false;
     // as many workgroups as the chip holds, for each channel block and class
     const int64_t units = (int64_t)((a.OC + 16 * CT - 1) / (16 * CT)) * a.classes, rounds = (a.n_pt + 3) / 4;

@@ -12,27 +12,30 @@
 namespace tmi
 {
 
-// A kernel's dynamic LDS limit is a per-device attribute of the function.  `done` holds, per device, the largest
-// size already granted to one kernel instantiation; the attribute is set again only when a launch needs more.
-// Safe for contexts used from different host threads.
+// A kernel's dynamic LDS limit is a per-device attribute of the function.  `granted` holds, per device, the largest size already
+// granted to this kernel; the attribute is set again only when a launch needs more.  The kernel is a template argument, so that no
+// two kernels can share a grant (kernels of one signature have one type).  Safe for contexts used from different host threads.
 constexpr int kMaxDevices = 16;
-struct LdsLimit
+template <auto Kernel>
+struct kernel_constant    // a kernel as the argument of a generic lambda
 {
-    std::atomic<size_t> done[kMaxDevices];
+    static constexpr auto value = Kernel;
 };
-inline bool ensure_dynamic_lds(const void* kernel, size_t bytes, LdsLimit& lim)
+template <auto Kernel>
+inline bool ensure_dynamic_lds(size_t bytes)
 {
+    static std::atomic<size_t> granted[kMaxDevices];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
         return false;
-    if (bytes <= lim.done[dev].load(std::memory_order_acquire))
+    if (bytes <= granted[dev].load(std::memory_order_acquire))
         return true;
-    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
     {
         (void)hipGetLastError();    // the caller goes on to another kernel, whose launch must not inherit this error
         return false;
     }
-    lim.done[dev].store(bytes, std::memory_order_release);
+    granted[dev].store(bytes, std::memory_order_release);
     return true;
 }
 
