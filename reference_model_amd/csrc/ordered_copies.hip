@@ -59,7 +59,7 @@ struct CopiedArgs
     int32_t tiles, n_big;          // all; those not cut into quarters (a multiple of eight)
     int32_t IC, IH, IW, KH, pieces;
     int32_t pad_top, pad_left, stride_y, stride_x, dil_y, dil_x;
-    int32_t padded;
+    int32_t padded;                // a tap can fall outside the image, and adds nothing there
     FastDiv ow, oh, tiles_n;
 };
 
@@ -620,7 +620,8 @@ bool launch_ordered_conv_copied(hipStream_t st, int32_t in_dtype, bool f64, cons
     p.IC = g.IC, p.IH = g.IH, p.IW = g.IW, p.pad_top = g.pad_top, p.pad_left = g.pad_left;
     p.stride_y = g.stride_y, p.stride_x = g.stride_x, p.dil_y = g.dil_y, p.dil_x = g.dil_x;
     p.ow = make_fastdiv((uint32_t)g.OW), p.oh = make_fastdiv((uint32_t)g.OH);
-    p.padded = g.pad_top > 0 || g.pad_left > 0 || c.rows_y - g.pad_top > g.IH || c.rows_x - g.pad_left > g.IW;
+    // (the bounds pass multiplies the padding out, tensor_ops.cpp:845-852: an infinite weight there makes NaN, as the zeros in the copy do)
+    p.padded = !abs_mode && (g.pad_top > 0 || g.pad_left > 0 || c.rows_y - g.pad_top > g.IH || c.rows_x - g.pad_left > g.IW);
     if (!launch_copies(st, in_dtype, f64, k))
         return false;
     return f64 ? launch_copied<true>(st, p) : launch_copied<false>(st, p);

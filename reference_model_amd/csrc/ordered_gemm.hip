@@ -43,7 +43,7 @@ struct OrderedArgs
     int32_t bias_len;
     uint32_t abs_mask;              // 0x7fffffff in the bounds pass, else all ones
     int32_t vec_a, vec_b;           // operand rows are whole, aligned groups of four elements
-    int32_t padded;                 // a tap can fall outside the image
+    int32_t padded;                 // a tap can fall outside the image, and adds nothing there
 };
 
 template <typename T>
@@ -474,8 +474,8 @@ __device__ __forceinline__ void ordered_tile(const OrderedArgs& p, int m0, int n
         }
         reinterpret_cast<acc_t*>(p.out)[(batch * p.M + m) * p.OC + oc] = v;
     };
-    // A tap outside the image adds nothing in the reference; here it adds 0 * weight, which is not nothing when the weight is
-    // infinite or NaN.  A tile that met such a weight is summed again one result at a time.
+    // A tap outside the image adds nothing in the reference (but in its bounds pass); here it adds 0 * weight, which is not nothing
+    // when the weight is infinite or NaN.  A tile that met such a weight is summed again one result at a time.
     if (!MATMUL && p.padded)
     {
         // (not __syncthreads_or: it brings 256 bytes of hidden arguments into every launch)
@@ -649,8 +649,10 @@ OrderedForm launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, cons
     p.ow = make_fastdiv((uint32_t)g.OW), p.oh = make_fastdiv((uint32_t)g.OH), p.ic = make_fastdiv((uint32_t)g.IC), p.kw = make_fastdiv((uint32_t)g.KW);
     p.bias_len = g.bias_len, p.abs_mask = abs_mode ? 0x7fffffffu : ~0u;
     p.vec_a = p.vec_b = g.IC % 4 == 0 && aligned16(in) && aligned16(w);
-    p.padded = g.pad_top > 0 || g.pad_left > 0 || (int64_t)(g.OH - 1) * g.stride_y - g.pad_top + (int64_t)(g.KH - 1) * g.dil_y >= g.IH ||
-               (int64_t)(g.OW - 1) * g.stride_x - g.pad_left + (int64_t)(g.KW - 1) * g.dil_x >= g.IW;
+    // (the bounds pass multiplies the padding out, tensor_ops.cpp:845-852: an infinite weight there makes NaN, as zeros in the operand do)
+    p.padded = !abs_mode &&
+               (g.pad_top > 0 || g.pad_left > 0 || (int64_t)(g.OH - 1) * g.stride_y - g.pad_top + (int64_t)(g.KH - 1) * g.dil_y >= g.IH ||
+                (int64_t)(g.OW - 1) * g.stride_x - g.pad_left + (int64_t)(g.KW - 1) * g.dil_x >= g.IW);
     const int64_t eb = in_dtype == TMI_FP32 ? 4 : 2;
     const bool taps  = p.vec_a && g.IC % 32 == 0 && (int64_t)g.N * g.IH * g.IW * g.IC * eb < INT32_MAX && (int64_t)g.OC * K * eb < INT32_MAX;
     if (!f64)

@@ -86,6 +86,8 @@ __global__ __launch_bounds__(256) void precise_conv_kernel(PreciseConvArgs a, in
     const int64_t stride = (int64_t)blocks * 256;
     const bool flat      = a.input_abs_max != nullptr;    // the input is one constant
     const double gmax    = flat ? *a.input_abs_max : 0.0;
+    // (CONV2D's bounds pass multiplies the padding out, tensor_ops.cpp:845-852: an infinite weight there makes NaN)
+    const bool outside_adds_nothing = a.depthwise || !a.abs_mode;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < a.total; i += stride)
     {
         const int oc      = (int)(i % g.OC);
@@ -96,14 +98,20 @@ __global__ __launch_bounds__(256) void precise_conv_kernel(PreciseConvArgs a, in
         double acc        = 0.0;
         for (int ky = 0; ky < g.KH; ky++)
         {
-            const int y = oh * g.stride_y - g.pad_top + ky * g.dil_y;
-            if (y < 0 || y >= g.IH)
+            const int y     = oh * g.stride_y - g.pad_top + ky * g.dil_y;
+            const bool y_in = y >= 0 && y < g.IH;
+            if (!y_in && outside_adds_nothing)
                 continue;
             for (int kx = 0; kx < g.KW; kx++)
             {
                 const int x = ow * g.stride_x - g.pad_left + kx * g.dil_x;
-                if (x < 0 || x >= g.IW)
+                if (!y_in || x < 0 || x >= g.IW)
+                {
+                    if (!outside_adds_nothing)
+                        for (int ic = 0; ic < g.IC; ic++)
+                            acc = acc + 0.0 * fabs(widen<T>(a.w, (((size_t)oc * g.KH + ky) * g.KW + kx) * g.IC + ic));
                     continue;
+                }
                 const size_t in_base = (((size_t)n * g.IH + y) * g.IW + x) * g.IC;
                 if (a.depthwise)
                 {

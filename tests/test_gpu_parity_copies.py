@@ -48,7 +48,7 @@ def test_conv2d_on_copies(ctx, case, infinite):
             assert np.array_equal(got, oracle.conv2d("f32", x, w, bias, pad, stride, dil), equal_nan=True)
         d = ctx.conv_desc(capi.FP32, capi.FP32, x.shape, oc, kh, kw, (oh, ow), pad, stride, dil, len(b))
         dev = [ctx.upload(v) for v in (x, w, b)]
-        for bounds in (False,) if infinite else (False, True):    # (the oracle's bounds pass multiplies the padding out: NaN)
+        for bounds in (False, True):    # (the bounds pass multiplies the padding out: an infinite weight there makes NaN)
             for local in (True, False) if bounds else (True,):
                 out = ctx.empty((n, oh, ow, oc), capi.F64)
                 ctx.conv2d_precise(d, *dev, bounds, out, local_bound=local)
@@ -75,3 +75,27 @@ def test_precise_pass_of_sixteen_bit_operands(ctx, dtype):
     with np.errstate(invalid="ignore"):
         want = oracle.conv2d("f64", *(v.astype(np.float64) for v in (x, w, b)), (1, 1, 1, 1), (1, 1), (1, 1))
     assert np.array_equal(out.numpy(), want, equal_nan=True)
+
+
+@pytest.mark.parametrize("shape, kernel", [
+    ((2, 9, 8, 12, 20), "conv_bounds_ordered"),       # read as they lie
+    ((2, 9, 8, 64, 40), "conv_bounds_ordered"),       # channels of whole stages
+    ((1, 2, 65536, 1, 2), "conv_bounds_f64")])        # too wide for the tiles: one result a lane
+@pytest.mark.parametrize("local", [True, False])
+def test_bounds_pass_multiplies_the_padding_out(ctx, shape, kernel, local):
+    """an infinite weight under a tap outside the image: NaN in the bounds pass, nothing in the others"""
+    n, h, w, ic, oc = shape
+    rng = np.random.default_rng(ic)
+    x, wt, b = rng.normal(0, 1, (n, h, w, ic)).astype(np.float32), rng.normal(0, 0.3, (oc, 3, 3, ic)).astype(np.float32), rng.normal(0, 1, oc).astype(np.float32)
+    wt[oc // 2, 0, 0, 0], wt[0, 2, 1, ic - 1] = -np.inf, np.nan
+    d = ctx.conv_desc(capi.FP32, capi.FP32, x.shape, oc, 3, 3, (h, w), (1, 1, 1, 1), (1, 1), (1, 1), oc)
+    dev = [ctx.upload(v) for v in (x, wt, b)]
+    for bounds in (False, True):
+        out = ctx.empty((n, h, w, oc), capi.F64)
+        ctx.conv2d_precise(d, *dev, bounds, out, local_bound=local)
+        assert ctx.sync() == capi.VALID and ctx.last_kernel.startswith(kernel if bounds else kernel.replace("bounds", "precise"))
+        xs = np.full(x.shape, np.abs(x).max()) if bounds and not local else x
+        with np.errstate(invalid="ignore"):
+            want = oracle.conv2d("f64", *(v.astype(np.float64) for v in (xs, wt, b)), (1, 1, 1, 1), (1, 1), (1, 1), abs_mode=bounds)
+        assert np.array_equal(out.numpy(), want, equal_nan=True)
+        assert np.isnan(want).any() and np.isinf(want).any()
