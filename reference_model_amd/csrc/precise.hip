@@ -292,8 +292,6 @@ struct DpCheckArgs
     int32_t normal_frac;
     double normal_min;
     DpPartial* partials;
-    uint32_t* tags;    // per block: the call whose partial result is complete; nullptr: the host waits for the stream
-    uint32_t tag;
 };
 
 template <typename T>
@@ -382,11 +380,6 @@ __global__ __launch_bounds__(256) void dp_check_kernel(DpCheckArgs a, int32_t bl
         for (int w = 1; w < 4; w++)
             t.sum += red[w].sum, t.sumsq += red[w].sumsq, t.worst = fmax(t.worst, red[w].worst), t.bad += red[w].bad;
         a.partials[blockIdx.x] = t;
-        if (a.tags)
-        {
-            __threadfence_system();
-            __hip_atomic_store(&a.tags[blockIdx.x], a.tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
     }
 }
 
@@ -397,10 +390,10 @@ int dp_check_blocks(int64_t n)
 }
 
 const char* launch_dp_check(hipStream_t st, int32_t out_dtype, int64_t n, const void* imp, const double* ref,
-                            const double* bnd, int32_t abs_bound, DpPartial* partials, uint32_t* tags, uint32_t tag)
+                            const double* bnd, int32_t abs_bound, DpPartial* partials)
 {
     DpCheckArgs a{};
-    a.imp = imp, a.ref = ref, a.bnd = bnd, a.n = n, a.abs_bound = abs_bound, a.partials = partials, a.tags = tags, a.tag = tag;
+    a.imp = imp, a.ref = ref, a.bnd = bnd, a.n = n, a.abs_bound = abs_bound, a.partials = partials;
     const dim3 grid(dp_check_blocks(n)), block(256);
     switch (out_dtype)
     {

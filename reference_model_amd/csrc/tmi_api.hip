@@ -1,7 +1,6 @@
 // C ABI of the library: context, device memory, operand validation and kernel selection.
 // Validation follows the reference operator's checkTensorAttributes()/eval() checks so that the same
 // malformed node is rejected with the same status; arithmetic lives in the kernel files.
-#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -53,8 +52,6 @@ struct tmi_ctx
     uint8_t* pages_dev    = nullptr;    // 256 pages of 64 bytes, page v filled with byte v: what padding reads
     uint32_t* flags_host  = nullptr;    // pinned staging word
     tmi::DpPartial* dp_partials = nullptr;    // pinned: the DOT_PRODUCT check's partial results, written by the device
-    uint32_t* dp_tags = nullptr;              // behind them: the check each is of
-    uint32_t dp_calls = 0;
     void* workspace       = nullptr;    // scratch for operand re-layout (MATMUL's transposed B)
     size_t workspace_size = 0;
     void* copies          = nullptr;    // scratch for CONV2D's padded operands, eager calls only (see copy_scratch)
@@ -893,7 +890,7 @@ int tmi_ctx_create(tmi_ctx_t** out_ctx, int device)
         return TMI_ERROR;
     }
     if (hipMalloc((void**)&ctx->flags_dev, 256) != hipSuccess ||
-        hipHostMalloc((void**)&ctx->flags_host, 256 + kDpCheckBlocks * (sizeof(DpPartial) + sizeof(uint32_t)), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&ctx->flags_host, 256 + kDpCheckBlocks * sizeof(DpPartial), hipHostMallocDefault) != hipSuccess ||
         hipMemset(ctx->flags_dev, 0, 256) != hipSuccess)
     {
         tmi_ctx_destroy(ctx);
@@ -901,8 +898,6 @@ int tmi_ctx_create(tmi_ctx_t** out_ctx, int device)
     }
     *ctx->flags_host = 0;
     ctx->dp_partials = reinterpret_cast<DpPartial*>(reinterpret_cast<uint8_t*>(ctx->flags_host) + 256);
-    ctx->dp_tags     = reinterpret_cast<uint32_t*>(ctx->dp_partials + kDpCheckBlocks);
-    memset(ctx->dp_tags, 0, kDpCheckBlocks * sizeof(uint32_t));
     {
         std::string pages(256 * 64, '\0');
         for (int v = 0; v < 256; v++)
@@ -1764,35 +1759,13 @@ int tmi_dot_product_check(tmi_ctx_t* ctx, int32_t out_dtype, int64_t n, const vo
         return fail(ctx, "dot product check: result type must be FP16, BF16 or FP32");
     TMI_HIP(ctx, hipSetDevice(ctx->device));
     const int32_t abs_bound = 2 * ksb;
-    // The partial results of a few workgroups are awaited where they arrive: waiting for the stream costs the runtime's way to the end of the
-    // kernel on top.  Each workgroup then fences its result, which writes back an L2, so many wait for the stream.  Call to verdict, us, stream /
-    // polled: 512 elements (a workgroup) 14.3 / 9.7, 28 K (56) 15.4 / 13.6, 126 K (246) 18.2 / 31.
-    const int blocks   = dp_check_blocks(n);
-    const bool polled  = blocks <= 32;
-    const uint32_t tag = ++ctx->dp_calls ? ctx->dp_calls : ++ctx->dp_calls;
-    if (!launch_dp_check(ctx->stream, out_dtype, n, imp_dev, ref_dev, bnd_dev, abs_bound, ctx->dp_partials, polled ? ctx->dp_tags : nullptr, tag))
+    if (!launch_dp_check(ctx->stream, out_dtype, n, imp_dev, ref_dev, bnd_dev, abs_bound, ctx->dp_partials))
         return fail(ctx, "dot product check: launch failed");
     ctx->last_kernel = "dot_product_check";
     TMI_HIP(ctx, hipGetLastError());
-    int arrived = 0;
-    if (polled)
-    {
-        // at most a millisecond: after that - long work before the check, a capture, a failure - the stream it is
-        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
-        for (int spins = 0; arrived < blocks; spins++)
-        {
-            if (__atomic_load_n(&ctx->dp_tags[arrived], __ATOMIC_ACQUIRE) == tag)
-                arrived++;
-            else if ((spins & 255) == 255 && std::chrono::steady_clock::now() > until)
-                break;
-            else
-                __builtin_ia32_pause();
-        }
-    }
-    if (arrived < blocks)
-        TMI_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    TMI_HIP(ctx, hipStreamSynchronize(ctx->stream));
     DpPartial host{ 0.0, 0.0, 0.0, 0 };
-    for (int i = 0; i < blocks; i++)
+    for (int i = 0; i < dp_check_blocks(n); i++)
     {
         const DpPartial& t = ctx->dp_partials[i];
         host.sum += t.sum, host.sumsq += t.sumsq, host.worst = t.worst > host.worst ? t.worst : host.worst, host.bad += t.bad;

@@ -171,9 +171,8 @@ struct DpPartial
 };
 constexpr int kDpCheckBlocks = 512;
 int dp_check_blocks(int64_t n);
-// tags: nullptr, or where a workgroup says with `tag` that its partial result is complete (memory the host may poll)
 const char* launch_dp_check(hipStream_t st, int32_t out_dtype, int64_t n, const void* imp, const double* ref,
-                            const double* bnd, int32_t abs_bound, DpPartial* partials, uint32_t* tags, uint32_t tag);
+                            const double* bnd, int32_t abs_bound, DpPartial* partials);
 
 // pool.hip: AVG_POOL2D (avg) / MAX_POOL2D; nullptr for a dtype without a kernel or 2^32 work items or more.
 const char* launch_pool(hipStream_t st, bool avg, int32_t dtype, int32_t N, int32_t IH, int32_t IW, int32_t C,

@@ -1,5 +1,7 @@
-"""The DOT_PRODUCT check whose partial results are awaited where they arrive: one workgroup, the most that are polled and one more, fresh results
-call after call, and a check behind work that outlasts the polling."""
+"""The DOT_PRODUCT check on its own: sizes from one workgroup to many, fresh results call after call, a check behind work of several
+milliseconds, and a stream with nothing left to do when the call returns."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -51,3 +53,23 @@ def test_behind_work_of_several_milliseconds(ctx):
     r = ctx.dot_product_check(capi.FP32, 3000, *dev, 9)
     assert r.failed_elements == 0 and r.max_abs_err == pytest.approx(want["max_err"], rel=1e-12)
     assert r.err_sumsq == pytest.approx(want["err_sumsq"], rel=1e-9)
+
+
+@pytest.mark.parametrize("n", [1, 512, 512 * 32, 40_000])
+def test_the_stream_is_idle_on_return(n):
+    c = Context(0)
+    hip = c.lib    # (the runtime the library is linked with)
+    stream = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+    try:
+        c.set_stream(stream.value)
+        ref, bnd, imp = _data(np.random.default_rng(n), n)
+        dev = [c.upload(imp), c.upload(ref, capi.F64), c.upload(bnd, capi.F64)]
+        left = []
+        for _ in range(200):
+            c.dot_product_check(capi.FP32, n, *dev, 9)
+            left.append(hip.hipStreamQuery(stream))
+        assert not any(left)
+    finally:
+        c.close()
+        hip.hipStreamDestroy(stream)
