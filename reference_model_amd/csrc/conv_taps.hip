@@ -269,6 +269,66 @@ __device__ __forceinline__ void finish_taps(const TapsArgs& a, const TapsTables&
     }
 }
 
+// A tap outside the image adds nothing in the reference (tensor_ops.cpp:845-852); in the matrix instruction it adds zero times the
+// weight, which is NaN where the weight is infinite or NaN.  A wave that met a NaN in a layer with padding goes over its tiles once more
+// at the end, and sums results that are NaN and whose window leaves the image one at a time without those taps.  (Here, behind the
+// loop and from arguments read anew, it costs the loop a test of the results and no register: summed again in the loop, two channel
+// tiles a wave fall from four waves a SIMD to two.)
+__device__ __forceinline__ bool leaves_image(const TapsArgs& a, int y0, int x0)
+{
+    return y0 < 0 || x0 < 0 || y0 + (a.KH - 1) * a.dy >= a.IH || x0 + (a.KW - 1) * a.dx >= a.IW;
+}
+template <int N, typename R>
+__device__ __forceinline__ bool any_nan(const R& v)
+{
+    bool nan = false;
+#pragma unroll
+    for (int e = 0; e < N; e += 2)
+        nan |= __builtin_isunordered(v[e], v[e + 1]);
+    return __any(nan);
+}
+__device__ __forceinline__ TapsArgs args_read_anew()
+{
+    auto* args = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));    // (not the values the kernel began with, which would have to be kept)
+    TapsArgs a;
+    __builtin_memcpy(&a, (const void*)args, sizeof(a));
+    return a;
+}
+// the lane's pixel p, `tiles` tiles of 32 channels of which it holds `each` from channel oc on
+template <typename T>
+__device__ __forceinline__ void sum_again(const TapsArgs& a, int p, int oc, int tiles, int each)
+{
+    if (p >= a.P)
+        return;
+    const int r = (int)fdiv((uint32_t)p, a.div_ow), n = (int)fdiv((uint32_t)r, a.div_oh), IC = a.row_bytes / 2;
+    const int y0 = (r - n * a.OH) * a.sy - a.pad_top, x0 = (p - r * a.OW) * a.sx - a.pad_left;
+    if (!leaves_image(a, y0, x0))
+        return;
+    T* out = reinterpret_cast<T*>(a.out) + (size_t)p * a.OC;
+#pragma unroll 1
+    for (int k = 0; k < tiles * each; k++)
+    {
+        const int c = oc + k / each * 32 + k % each;
+        if (c >= a.OC || load_as_float<T>(out, c) == load_as_float<T>(out, c))
+            continue;
+        float sum = 0.0f;
+#pragma unroll 1
+        for (int tap = 0; tap < a.KH * a.KW; tap++)
+        {
+            const int ky = (int)fdiv((uint32_t)tap, a.div_kw), y = y0 + ky * a.dy, x = x0 + (tap - ky * a.KW) * a.dx;
+            if ((unsigned)y >= (unsigned)a.IH || (unsigned)x >= (unsigned)a.IW)
+                continue;
+            const uint8_t* u = a.in + (uint32_t)(((n * a.IH + y) * a.IW + x) * a.row_bytes);
+            const uint8_t* w = a.w + (uint32_t)((c * a.KH * a.KW + tap) * a.row_bytes);
+#pragma unroll 1
+            for (int i = 0; i < IC; i++)
+                sum += load_as_float<T>(u, i) * load_as_float<T>(w, i);
+        }
+        store_from_float(out + c, sum + load_as_float<T>(a.bias, a.bias_len == 1 ? 0 : c));
+    }
+}
+
 template <typename T, int OCT, bool RAGGED>
 __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs a)
 {
@@ -467,7 +527,9 @@ __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs 
 
     const uint8_t* wfrag = wl + lh * PITCH + li * 16;
     uint8_t* rows        = wl + 2 * a.steps * PITCH + wave * a.rows_bytes;
-    for (int pt = first_pt; pt < a.n_pt; pt += pt_step)
+    bool met_nan         = false;
+    int pt               = first_pt;
+    for (; pt < a.n_pt; pt += pt_step)
     {
         acc_t acc[OCT];
 #pragma unroll
@@ -546,6 +608,8 @@ __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs 
 #pragma unroll
         for (int t = 0; t < OCT; t++)
         {
+            if constexpr (!M::is_int)
+                met_nan |= any_nan<16>(acc[t]);
             finish_taps<T, 16>(a, TapsTables{ tab_hw + 32 * t, tab_ms + 32 * t, tab_start + 32 * t, tab_form + t }, acc[t],
                                oc0 + 32 * t + 16 * lh, 16 * lh, p, flags, a.rows_bytes ? rows : nullptr);
             __builtin_amdgcn_sched_barrier(0);    // (one channel tile's values at a time)
@@ -567,6 +631,13 @@ __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs 
     }
     if constexpr (M::is_int)
         raise_flags(a.flag_word, flags);
+    else if (met_nan)
+    {
+        __threadfence();    // (gathered rows were stored by other lanes)
+        const TapsArgs b = args_read_anew();
+        while ((pt -= pt_step) >= 0)
+            sum_again<T>(b, pt * 32 + li, oc0 + 16 * lh, OCT, 16);
+    }
 }
 
 // Few tiles and a long reduction: a workgroup of NW waves shares a tile of 32 channels x 32 pixels (or several of pixels, one
@@ -739,8 +810,9 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_ker
     }
 
     const bool keep = share <= KSW;
-    bool have_start = false;
-    for (int pt = grp; pt < a.n_pt; pt += a.groups)
+    bool have_start = false, met_nan = false;
+    int pt = grp;
+    for (; pt < a.n_pt; pt += a.groups)
     {
         enter_tile(pt);
         acc_t acc;
@@ -818,6 +890,8 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_ker
             const int cb = 16 * lh + 4 * wave;
             if constexpr (M::is_int)
                 total += *reinterpret_cast<const v4i*>(&tab_start[NW][cb]);
+            if constexpr (!M::is_int)
+                met_nan |= any_nan<4>(total);
             finish_taps<T, 4>(a, TapsTables{ tab_hw, tab_ms, tab_start[NW], &tab_form }, total, oc0 + cb, cb, pt * 32 + li, flags);
         }
         if (pt + a.groups < a.n_pt)
@@ -825,6 +899,12 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_ker
     }
     if constexpr (M::is_int)
         raise_flags(a.flag_word, flags);
+    else if (met_nan)
+    {
+        const TapsArgs b = args_read_anew();
+        while ((pt -= b.groups) >= 0)
+            sum_again<T>(b, pt * 32 + li, oc0 + 16 * lh + 4 * wave, 1, 4);
+    }
 }
 
 // Workgroups: as many as the CUs hold at once.  (Neighbours walk one tile more or less, and neighbours lie on different CUs; fewer

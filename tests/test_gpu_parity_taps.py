@@ -115,6 +115,36 @@ def test_infinities_stay_where_they_are(ctx, dtype, shape):
     assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want)) and not np.isnan(got).any()
 
 
+@pytest.mark.parametrize("dtype", [capi.FP16, capi.BF16])
+@pytest.mark.parametrize("shape, stride", [
+    ((2, 20, 21, 9, 40), 1),       # a split reduction, ragged
+    ((1, 9, 23, 8, 44), 1),        # whole pieces
+    ((9, 50, 50, 6, 33), 1),       # resident weights; rows gathered in LDS
+    ((9, 50, 50, 16, 70), 1),      # several channel tiles a wave
+    ((15, 54, 65, 68, 60), 2)])
+def test_infinite_weights_under_taps_outside_the_image(ctx, dtype, shape, stride):
+    """a tap outside the image adds nothing, whatever its weight; inside, an infinity or a NaN reaches its results"""
+    n, h, w, ic, oc = shape
+    n, h, w, ic, oc, k, pad, _, _ = _fitting((n, h, w, ic, oc, (3, 3), (1, 1, 1, 1), (stride, stride), (1, 1)))
+    rng = np.random.default_rng(6)
+    x, wt, bias = (rng.integers(-8, 9, sh).astype(np.float32) / 4 for sh in ((n, h, w, ic), (oc, 3, 3, ic), (oc,)))
+    wt[oc // 2, 0, 0, 1], wt[oc - 1, 2, 1, 0], wt[1, 1, 2, ic - 1] = np.inf, np.nan, -np.inf
+    x[0, 0, 1, 0] = np.nan
+    with np.errstate(invalid="ignore"):
+        want = oracle.conv2d("f64", *(v.astype(np.float64) for v in (x, wt, bias)), pad, (stride, stride), (1, 1))
+    if dtype == capi.FP16:
+        args = [v.astype(np.float16) for v in (x, wt, bias)]
+    else:
+        args = [(v.view(np.uint32) >> 16).astype(np.uint16) for v in (x, wt, bias)]
+    got, st = gpu_ops.conv2d(ctx, *args, pad, (stride, stride), dtype=dtype)
+    got = got.astype(np.float64) if dtype == capi.FP16 else (got.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    assert st == capi.VALID and "taps" in ctx.last_kernel
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isinf(want).any() and np.isnan(want).any()
+    finite = np.isfinite(want)
+    assert np.array_equal(got[~finite], want[~finite], equal_nan=True)
+    assert np.all(np.abs(got[finite] - want[finite]) <= (2.0 ** -11 if dtype == capi.FP16 else 2.0 ** -8) * np.abs(want[finite]))
+
+
 def test_values_out_of_range_are_latched(ctx):
     """apply_scale_32's value range, by stored results only"""
     for shape in ((1, 9, 23, 8, 44), (9, 64, 62, 7, 84)):
