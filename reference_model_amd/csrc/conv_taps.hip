@@ -995,8 +995,6 @@ static int64_t taps_steps(int64_t taps, int64_t row)
 double conv2d_taps_us(int32_t in_dtype, const ConvGeom& g)
 {
     const int64_t row = (int64_t)g.IC * (in_dtype == TMI_INT8 ? 1 : 2), steps = taps_steps((int64_t)g.KH * g.KW, row);
-    if (steps > 1024)
-        return 1e9;
     return taps_form(((int64_t)g.N * g.OH * g.OW + 31) / 32, g.OC, steps, row % 16 == 0 ? 0 : (row % 4 == 0 ? 1 : 2)).us;
 }
 
@@ -1022,33 +1020,43 @@ static bool launch_taps_t(hipStream_t st, TapsArgs& a, bool ragged)
     return false;
 }
 
+// the results by out_kind, -1: none of this kernel's
+static int taps_kind(int32_t in_dtype, int32_t out_dtype, const RescaleParams& rp)
+{
+    if (in_dtype == TMI_INT8)
+        return !rp.enabled ? (out_dtype == TMI_INT32 ? 0 : -1) : (!rp.fast ? -1 : (out_dtype == TMI_INT8 ? 1 : (out_dtype == TMI_INT16 ? 2 : -1)));
+    return (in_dtype == TMI_FP16 || in_dtype == TMI_BF16) && !rp.enabled && out_dtype == in_dtype ? 3 : -1;
+}
+static int64_t taps_window(const ConvGeom& g, int64_t row)    // the last chunk's offset from its window's first tap
+{
+    return ((int64_t)(g.KH - 1) * g.dil_y * g.IW + (int64_t)(g.KW - 1) * g.dil_x) * row + (row - 1) / 16 * 16;
+}
+bool conv2d_taps_takes(int32_t in_dtype, int32_t out_dtype, const ConvGeom& g, int32_t w_zp, const RescaleParams& rp, const void* out)
+{
+    if (w_zp != 0 || g.KH > 13 || g.KW > 13 || taps_kind(in_dtype, out_dtype, rp) < 0 || ((uintptr_t)out & 15))
+        return false;
+    const int64_t P        = (int64_t)g.N * g.OH * g.OW, row = (int64_t)g.IC * (in_dtype == TMI_INT8 ? 1 : 2), taps = (int64_t)g.KH * g.KW;
+    const int64_t in_bytes = (int64_t)g.N * g.IH * g.IW * row, w_bytes = (int64_t)g.OC * taps * row, chunks = taps * ((row + 15) / 16);
+    // 32-bit offsets (a window's first tap may lie before the tensor)
+    if (P < 1 || g.OC < 1 || P > (1 << 30) || in_bytes < 16 || w_bytes < 16 || in_bytes >= (int64_t(1) << 30) || w_bytes >= (int64_t(1) << 30) ||
+        (int64_t)(g.pad_top + 1) * g.IW * row >= (int64_t(1) << 30) || (int64_t)g.pad_left * row >= (int64_t(1) << 29) ||
+        taps_window(g, row) >= (int64_t(1) << 30) || taps_steps(taps, row) > 1024)
+        return false;
+    return fastdiv_exact_up_to((uint64_t)P, (uint32_t)g.OW) && fastdiv_exact_up_to((uint64_t)P / g.OW + 1, (uint32_t)g.OH) &&
+           fastdiv_exact_up_to((uint64_t)128 * chunks, (uint32_t)chunks);
+}
+
 const char* launch_conv2d_taps(hipStream_t st, int32_t in_dtype, int32_t out_dtype, const ConvGeom& g, const void* in, const void* w,
                                const void* bias, int32_t in_zp, int32_t w_zp, const RescaleParams& rp, void* out, const void* pad_page,
                                uint32_t* flag_word)
 {
-    if (w_zp != 0 || !flag_word || !pad_page || g.KH > 13 || g.KW > 13)
+    if (!flag_word || !pad_page || !conv2d_taps_takes(in_dtype, out_dtype, g, w_zp, rp, out))
         return nullptr;
-    const bool i8 = in_dtype == TMI_INT8;
-    int kind      = -1;
-    if (i8)
-        kind = !rp.enabled ? (out_dtype == TMI_INT32 ? 0 : -1) : (!rp.fast ? -1 : (out_dtype == TMI_INT8 ? 1 : (out_dtype == TMI_INT16 ? 2 : -1)));
-    else if ((in_dtype == TMI_FP16 || in_dtype == TMI_BF16) && !rp.enabled)
-        kind = out_dtype == in_dtype ? 3 : -1;
-    if (kind < 0 || ((uintptr_t)out & 15))
-        return nullptr;
-    const int eb           = i8 ? 1 : 2;
-    const int64_t P        = (int64_t)g.N * g.OH * g.OW, row = (int64_t)g.IC * eb, taps = (int64_t)g.KH * g.KW;
-    const int64_t in_bytes = (int64_t)g.N * g.IH * g.IW * row, w_bytes = (int64_t)g.OC * taps * row;
-    // 32-bit offsets (a window's first tap may lie before the tensor)
-    if (P < 1 || g.OC < 1 || P > (1 << 30) || in_bytes < 16 || w_bytes < 16 || in_bytes >= (int64_t(1) << 30) || w_bytes >= (int64_t(1) << 30) ||
-        (int64_t)(g.pad_top + 1) * g.IW * row >= (int64_t(1) << 30) || (int64_t)g.pad_left * row >= (int64_t(1) << 29))
-        return nullptr;
-    const int64_t window = ((int64_t)(g.KH - 1) * g.dil_y * g.IW + (int64_t)(g.KW - 1) * g.dil_x) * row + (row - 1) / 16 * 16;
-    if (window >= (int64_t(1) << 30))
-        return nullptr;
+    const bool i8          = in_dtype == TMI_INT8;
+    const int kind         = taps_kind(in_dtype, out_dtype, rp);
+    const int64_t P        = (int64_t)g.N * g.OH * g.OW, row = (int64_t)g.IC * (i8 ? 1 : 2), taps = (int64_t)g.KH * g.KW;
+    const int64_t in_bytes = (int64_t)g.N * g.IH * g.IW * row, w_bytes = (int64_t)g.OC * taps * row, window = taps_window(g, row);
     const int64_t pieces = (row + 15) / 16, chunks = taps * pieces;
-    if (taps_steps(taps, row) > 1024)
-        return nullptr;
     TapsArgs a{};
     a.steps = (int32_t)taps_steps(taps, row);
     a.in = (const uint8_t*)in, a.w = (const uint8_t*)w, a.bias = bias, a.out = out, a.pad_page = (const uint8_t*)pad_page;
@@ -1062,9 +1070,6 @@ const char* launch_conv2d_taps(hipStream_t st, int32_t in_dtype, int32_t out_dty
     a.div_ow = make_fastdiv((uint32_t)g.OW), a.div_oh = make_fastdiv((uint32_t)g.OH), a.div_chunks = make_fastdiv((uint32_t)chunks);
     a.row_skip = (int32_t)(kTapsWaves * 64 / chunks), a.chunk_skip = (int32_t)(kTapsWaves * 64 % chunks);
     a.div_pieces = make_fastdiv((uint32_t)pieces), a.div_kw = make_fastdiv((uint32_t)g.KW);
-    if (!fastdiv_exact_up_to((uint64_t)P, (uint32_t)g.OW) || !fastdiv_exact_up_to((uint64_t)P / g.OW + 1, (uint32_t)g.OH) ||
-        !fastdiv_exact_up_to((uint64_t)128 * chunks, (uint32_t)chunks))
-        return nullptr;
     const bool ragged = row % 16 != 0 || (((uintptr_t)in | (uintptr_t)w) & 15);
     const bool ok     = i8 ? launch_taps_t<int8_t>(st, a, ragged)
                            : (in_dtype == TMI_FP16 ? launch_taps_t<_Float16>(st, a, ragged) : launch_taps_t<bf16_t>(st, a, ragged));

@@ -645,7 +645,12 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         name = launch_depthwise_vec(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                     ctx->flags_dev);
     // The kernel with resident weights or split reductions takes channel vectors of any length as they lie
-    const bool taps_open  = !depthwise && ctx->kernel_choice == 0 && w_zp == 0;
+    int taps_taken        = -1;    // (asked for where a rule needs it)
+    auto taps_open        = [&]() {
+        if (taps_taken < 0)
+            taps_taken = !depthwise && ctx->kernel_choice == 0 && conv2d_taps_takes(d->in_dtype, out_dtype, g, w_zp, rp, out) ? 1 : 0;
+        return taps_taken == 1;
+    };
     const int32_t t_row   = g.IC * (d->in_dtype == TMI_INT8 ? 1 : 2);
     const int64_t t_steps = ((int64_t)g.KH * g.KW * ((t_row + 15) / 16) + 1) / 2;
     const int64_t t_tiles = ((total / g.OC + 31) / 32) * ((g.OC + 31) / 32);
@@ -657,12 +662,17 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
     if (!depthwise && ctx->kernel_choice == 0 && own_scratch && w_zp == 0)
     {
         int32_t padded = padded_channel_bytes(d->in_dtype, g, total, rp.enabled);
+        // Results off 16 bytes or 16-bit multipliers: the kernels that lead on whole steps decline, and the patch kernel has the layer either way;
+        // it gains from the copies only where it would stage the rows byte by byte (us padded / as they lie: [18,21,21,48]->16 3x3 10.6 /
+        // 8.1, with 16-bit multipliers 17.1 / 14.6; the other way [2,35,35,45]->8 3x3 9.9 / 13.0).
+        if (padded && t_row % 4 == 0 && ((((uintptr_t)out) & 15) || (rp.enabled && !rp.fast)))
+            padded = 0;
         // What would be padded and is small: one launch of the kernel that needs no whole steps.  us padded / this: int8 3x3 [18,21,21,48]->16
         // 9.2 / 4.0, [2,35,35,45]->8 6.3 / 4.7, [2,34,31,272]->480 stride 2 11.1 / 7.7, [7,24,24,112]->160 stride 2 10.6 / 4.7; fp16 1x1
         // [5,8,11,69]->440 8.1 / 3.6.  From 36 steps on, odd rows (loads that start between words, at a quarter of the rate) are
         // padded first: bf16 [1,45,9,219]->23 18.9 / 11, int8 [2,11,16,285]->42 5x5 34 / 18.
         // (Up to 36 tiles the copies stay: they are a few microseconds either way, and the tests of the padded route lie there.)
-        if (padded && taps_open && t_tiles > 36 && t_tiles * t_steps <= (t_row % 16 == 0 ? 24000 : 6000) && !(t_row % 4 != 0 && t_steps >= 36))
+        if (padded && t_tiles > 36 && t_tiles * t_steps <= (t_row % 16 == 0 ? 24000 : 6000) && !(t_row % 4 != 0 && t_steps >= 36) && taps_open())
             padded = 0, name = launch_taps();
         if (name)
             return after_launch(ctx, name);
@@ -760,7 +770,7 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
             name = launch_conv2d_pointwise(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                            ctx->flags_dev);
         if (!name && ctx->kernel_choice == 0 && d->in_dtype == TMI_INT8 && direct_leads(g, total, rp.enabled) &&
-            (!taps_open || t_tiles <= 36 || direct_us(g, total) < conv2d_taps_us(d->in_dtype, g)))
+            (t_tiles <= 36 || !taps_open() || direct_us(g, total) < conv2d_taps_us(d->in_dtype, g)))
             name = launch_conv2d_direct(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                         ctx->flags_dev);
         // (left open, the slab kernel's layers with more than 128 input channels are the ones tried above)
@@ -810,7 +820,7 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // kernel / resident weights or split reduction, fp16 1x1 (pixels): [570,256]->116 5.6 / 4.0, [1512,288]->288 (432 tiles of 32 x 32, 18
         // steps) 6.0 / 4.9, [2432,320]->112 (304, 20) 6.1 / 5.2, [1368,64]->392 (559, 4) 5.0 / 4.1; the other way: [1692,288]->330 (583, 18)
         // 7.1 / 7.6, [2100,224]->312 (660, 14) 4.6 / 5.3, [4752,64]->216 (1043, 4) 4.1 / 5.6, 3x3 [3564,128]->393 (1456, 72) 17.4 / 24.3.
-        if (!name && taps_open && gemm_1st && fp16b && g.OC % 64 != 0 && t_tiles <= 650 && t_tiles * t_steps <= 8000)
+        if (!name && gemm_1st && fp16b && g.OC % 64 != 0 && t_tiles <= 650 && t_tiles * t_steps <= 8000 && taps_open())
             name = launch_taps();
         if (!name && gemm_1st)
             name = launch_gemm_mfma(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out, 0, 0,
@@ -826,7 +836,7 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // 5.5 / 6.8; the other way [14,92,75,48]->48 fp16 stride 2 11.3 / 7.8, [4,28,33,16]->264 8.1 / 5.4).
         const bool long_and_many = t_steps >= 90 && t_tiles > (t_steps >= 140 ? 380 : (t_steps >= 120 ? 480 : 700));
         const bool patch_filled  = g.KH * g.KW > 1 && t_tiles > 700 && t_tiles <= (t_steps >= 64 ? 3400 : 2400) && t_row % 8 == 0 && g.OC % 8 == 0;
-        if (!name && taps_open && !long_and_many && !patch_filled)
+        if (!name && !long_and_many && !patch_filled && taps_open())
             name = launch_taps();
         if (!name && patch_ok)
             name = launch_conv2d_mfma(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,

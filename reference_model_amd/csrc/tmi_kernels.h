@@ -115,7 +115,8 @@ const char* launch_conv2d_stem(hipStream_t st, int32_t in_dtype, int32_t out_dty
 const char* launch_conv2d_taps(hipStream_t st, int32_t in_dtype, int32_t out_dtype, const ConvGeom& g, const void* in, const void* w,
                                const void* bias, int32_t in_zp, int32_t w_zp, const RescaleParams& rp, void* out, const void* pad_page,
                                uint32_t* flag_word);
-// what a layer takes in it, us (launch included; 1e9: too deep a reduction)
+// whether it takes a layer, and what the layer takes in it, us (launch included)
+bool conv2d_taps_takes(int32_t in_dtype, int32_t out_dtype, const ConvGeom& g, int32_t w_zp, const RescaleParams& rp, const void* out);
 double conv2d_taps_us(int32_t in_dtype, const ConvGeom& g);
 
 // conv_ksplit.hip: the form of launch_conv2d_pointwise's layers with both operands through LDS (IC = 512 ... 2048 in multiples

@@ -155,3 +155,35 @@ def test_values_out_of_range_are_latched(ctx):
             mult, sh = np.full(oc, 1 << 12, np.int32), np.full(oc, shift, np.int8)
             _, st = gpu_ops.conv2d(ctx, x, wt, bias, (1, 1, 1, 1), in_zp=0, w_zp=0, rescale=dict(mult=mult, shift=sh))
             assert "taps" in ctx.last_kernel and st == status
+
+
+@pytest.mark.parametrize("shape, form, kernel, copies", [
+    ((1, 40, 40, 5, 16), "16-bit scales", "conv2d_direct_i8_rescale", False),     # (this kernel would lead)
+    ((1, 40, 40, 3, 16), "off 16 bytes", "conv2d_direct_i8", False),
+    ((2, 35, 35, 45, 8), "16-bit scales", "conv2d_mfma_i8_rescale", True),        # rows of no whole words: padded first
+    ((2, 35, 35, 45, 8), "off 16 bytes", "conv2d_mfma_i8", True),
+    ((18, 21, 21, 48, 16), "16-bit scales", "conv2d_mfma_i8_rescale", False),     # whole words: the patch kernel, as they lie
+    ((18, 21, 21, 48, 16), "off 16 bytes", "conv2d_mfma_i8", False)])
+def test_what_it_declines_goes_where_it_leads(shape, form, kernel, copies):
+    """results off 16 bytes and 16-bit multipliers are not this kernel's: the rules that would hand it such a layer look for the next best"""
+    n, h, w, ic, oc = shape
+    rng = np.random.default_rng(ic)
+    x, wt = rng.integers(-128, 128, (n, h, w, ic)).astype(np.int8), rng.integers(-128, 128, (oc, 3, 3, ic)).astype(np.int8)
+    bias = rng.integers(-9999, 9999, oc).astype(np.int32)
+    want = oracle.conv2d("i8", x, wt, bias, (1, 1, 1, 1), (1, 1), (1, 1), in_zp=-11, w_zp=0)
+    c = Context(0)
+    try:
+        if form == "16-bit scales":
+            mult, shift = rng.integers(1 << 14, 1 << 15, oc).astype(np.int16), rng.integers(22, 25, oc).astype(np.int8)
+            r = dict(mult=mult, shift=shift, out_zp=3, scale32=False, rounding_mode=capi.ROUND_SINGLE)
+            want, wst = oracle.rescale(want, mult, shift, out_zp=3, scale32=False, rounding_mode=capi.ROUND_SINGLE)
+            got, st = gpu_ops.conv2d(c, x, wt, bias, (1, 1, 1, 1), in_zp=-11, w_zp=0, rescale=r)
+        else:
+            d = c.conv_desc(capi.INT8, capi.INT32, x.shape, oc, 3, 3, (h, w), (1, 1, 1, 1), (1, 1), (1, 1), oc)
+            out = c.empty((want.size + 1,), capi.INT32)
+            c.conv2d(d, *(c.upload(v) for v in (x, wt, bias)), -11, 0, out.ptr + 4)
+            st, wst, got = c.sync(), capi.VALID, out.numpy()[1:].reshape(want.shape)
+        assert st == wst and np.array_equal(got, want)
+        assert c.last_kernel == kernel and (c.workspace_bytes() != (0, 0)) == copies
+    finally:
+        c.close()
