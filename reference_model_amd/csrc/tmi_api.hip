@@ -671,8 +671,8 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // 9.2 / 4.0, [2,35,35,45]->8 6.3 / 4.7, [2,34,31,272]->480 stride 2 11.1 / 7.7, [7,24,24,112]->160 stride 2 10.6 / 4.7; fp16 1x1
         // [5,8,11,69]->440 8.1 / 3.6.  From 36 steps on, odd rows (loads that start between words, at a quarter of the rate) are
         // padded first: bf16 [1,45,9,219]->23 18.9 / 11, int8 [2,11,16,285]->42 5x5 34 / 18.
-        // (Up to 36 tiles the copies stay: they are a few microseconds either way, and the tests of the padded route lie there.)
-        if (padded && t_tiles > 36 && t_tiles * t_steps <= (t_row % 16 == 0 ? 24000 : 6000) && !(t_row % 4 != 0 && t_steps >= 36) && taps_open())
+        // A few tiles: [1,6,9,48]->16 int32 6.0 / 3.5, 1x1 [1,8,11,34]->32 int32 6.0 / 3.6, 5x5 [1,17,5,112]->24 stride 2 9.1 / 5.5, [2,12,12,73]->48 6.6 / 6.1.
+        if (padded && t_tiles * t_steps <= (t_row % 16 == 0 ? 24000 : 6000) && !(t_row % 4 != 0 && t_steps >= 36) && taps_open())
             padded = 0, name = launch_taps();
         if (name)
             return after_launch(ctx, name);
@@ -769,8 +769,14 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         if (!name && ctx->kernel_choice == 0 && (g.IC <= 112 || deep_first))
             name = launch_conv2d_pointwise(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                            ctx->flags_dev);
-        if (!name && ctx->kernel_choice == 0 && d->in_dtype == TMI_INT8 && direct_leads(g, total, rp.enabled) &&
-            (t_tiles <= 36 || !taps_open() || direct_us(g, total) < conv2d_taps_us(d->in_dtype, g)))
+        // The one-result-per-lane kernel or the one with resident weights, by what either takes.  us one result a lane / the other, eager calls of at
+        // most 36 tiles of 32 x 32: [1,18,8,6]->46 3x3 7.7 / 4.5, 1x1 [1,19,6,46]->204 6.5 / 3.9, [3,5,50,32]->22 6.3 / 3.8, [3,7,20,17]->16 4.1 / 3.9, even: int32
+        // [2,16,16,2]->41 3x3 4.6 / 4.5, 1x1 [2,17,7,14]->8 3.5 / 3.6 (34 layers: 0.77).  At once, before the stem kernel, whose pre-pass is a launch of its own:
+        // [2,26,7,4]->72 3x3 5.8 / 4.4, [6,11,15,4]->224 3x3 stride 2 6.0 / 4.6, [3,40,17,2]->16 5x5 stride 2 6.0 / 5.3.
+        const bool lane_leads = !name && ctx->kernel_choice == 0 && d->in_dtype == TMI_INT8 && direct_leads(g, total, rp.enabled);
+        if (lane_leads && taps_open() && conv2d_taps_us(d->in_dtype, g) <= direct_us(g, total))
+            name = launch_taps();
+        if (!name && lane_leads)
             name = launch_conv2d_direct(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                         ctx->flags_dev);
         // (left open, the slab kernel's layers with more than 128 input channels are the ones tried above)

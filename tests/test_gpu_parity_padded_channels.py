@@ -17,24 +17,33 @@ def ctx():
     c.close()
 
 
-CASES = {  # n, h, w, ic, oc, k, pad, stride: the kernel of the padded int8 layer (none of them takes it as it lies)
-    (1, 7, 9, 17, 24, 3, 1, 1): "conv2d_ksplit_i8",           # one byte past a piece
-    (2, 9, 7, 31, 8, 3, 1, 1): "conv2d_ksplit_i8",            # one short of a step
-    (1, 8, 8, 33, 13, 1, 0, 1): "conv2d_direct_i8",           # (tiny: stays as it lies)
-    (1, 8, 8, 65, 24, 1, 0, 1): "conv2d_pointwise_i8",
+CASES = {  # n, h, w, ic, oc, k, pad, stride: the kernel of the int8 layer
+    # copies padded first
+    (11, 45, 45, 17, 24, 3, 1, 1): "conv2d_taps_i8",     # one byte past a piece
+    (10, 47, 49, 31, 8, 3, 1, 1): "conv2d_mfma_i8",      # one short of a step
+    (20, 57, 57, 65, 24, 1, 0, 1): "conv2d_pointwise_i8",
     (3, 11, 5, 131, 40, 3, 1, 2): "conv2d_ksplit_i8",
-    (1, 6, 6, 207, 64, 2, 0, 1): "conv2d_ksplit_i8",
-    (2, 13, 13, 72, 72, 3, 1, 1): "conv2d_ksplit_i8",         # whole words
-    (2, 12, 12, 80, 80, 3, 1, 1): "conv2d_slab_i8",
-    (1, 10, 10, 245, 16, 3, 1, 1): "conv2d_ksplit_patch_i8",  # padded to 256: both operands in LDS
+    (6, 40, 41, 207, 64, 2, 0, 1): "conv2d_ksplit_i8",
+    (16, 16, 16, 72, 72, 3, 1, 1): "conv2d_ksplit_i8",    # whole words
+    (4, 53, 53, 80, 80, 3, 1, 1): "conv2d_slab_i8",
+    (1, 10, 10, 245, 16, 3, 1, 1): "conv2d_ksplit_patch_i8",    # padded to 256: both operands in LDS
+    # smaller ones: one launch, as they lie
+    (1, 7, 9, 17, 24, 3, 1, 1): "conv2d_taps_i8",
+    (2, 9, 7, 31, 8, 3, 1, 1): "conv2d_taps_i8",
+    (1, 8, 8, 33, 13, 1, 0, 1): "conv2d_taps_i8",
+    (1, 8, 8, 65, 24, 1, 0, 1): "conv2d_taps_i8",
+    (1, 6, 6, 207, 64, 2, 0, 1): "conv2d_taps_i8",
+    (2, 13, 13, 72, 72, 3, 1, 1): "conv2d_taps_i8",
+    (2, 12, 12, 80, 80, 3, 1, 1): "conv2d_taps_i8",
 }
 
 
 @pytest.mark.parametrize("ic, oc, fused, kernel", [
-    (17, 16, True, "conv2d_direct_i8_rescale"), (27, 32, True, "conv2d_direct_i8_rescale"), (45, 64, True, "conv2d_pointwise_i8_rescale"),
-    (21, 20, True, "conv2d_direct_i8_rescale"), (17, 16, False, "conv2d_direct_i8"), (37, 8, False, "conv2d_pointwise_i8")])
+    (17, 16, True, "conv2d_taps_i8_rescale"), (27, 32, True, "conv2d_taps_i8_rescale"), (45, 64, True, "conv2d_taps_i8_rescale"),
+    (21, 20, True, "conv2d_taps_i8_rescale"), (17, 16, False, "conv2d_taps_i8"), (37, 8, False, "conv2d_taps_i8"),
+    (7, 9, True, "conv2d_direct_i8_rescale"), (7, 9, False, "conv2d_direct_i8")])
 def test_tiny_layers_stay_one_launch(ic, oc, fused, kernel):
-    """below the border the one-result-per-lane kernel reads the operands as they lie, without a copy in scratch memory"""
+    """the one-result-per-lane kernel or the one with split reductions reads the operands as they lie, without a copy in scratch memory"""
     rng = np.random.default_rng(ic)
     x, wt = rng.integers(-128, 128, (1, 9, 8, ic)).astype(np.int8), rng.integers(-128, 128, (oc, 1, 1, ic)).astype(np.int8)
     bias = rng.integers(-999, 999, oc).astype(np.int32)
@@ -46,7 +55,20 @@ def test_tiny_layers_stay_one_launch(ic, oc, fused, kernel):
     try:
         got, st = gpu_ops.conv2d(c, x, wt, bias, in_zp=5, w_zp=0, rescale=dict(mult=mult, shift=shift, out_zp=3) if fused else None)
         assert st == capi.VALID and np.array_equal(got, want)
-        assert c.last_kernel == kernel and (c.workspace_bytes() == (0, 0)) == ("direct" in kernel)
+        assert c.last_kernel == kernel and c.workspace_bytes() == (0, 0)
+    finally:
+        c.close()
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_only_large_or_odd_layers_are_copied(case):
+    n, h, w, ic, oc, k, p, s = case
+    pad = (p, p - (h + 2 * p - k) % s, p, p - (w + 2 * p - k) % s)
+    c = Context(0)
+    try:
+        _, st = gpu_ops.conv2d(c, np.ones((n, h, w, ic), np.int8), np.ones((oc, k, k, ic), np.int8), np.zeros(oc, np.int32), pad, (s, s))
+        copied = list(CASES).index(case) < 8
+        assert st == capi.VALID and (c.workspace_bytes() != (0, 0)) == copied
     finally:
         c.close()
 
