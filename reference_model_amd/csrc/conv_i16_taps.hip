@@ -376,9 +376,11 @@ static bool launch_i16_taps(hipStream_t st, I16TapsArgs& a)
     constexpr auto kern = conv_i16_taps_kernel<CT, SPLIT, RAGGED>;
     if (lds > 65536 && !ensure_dynamic_lds<kern>((size_t)lds))
         return false;
-    // as many workgroups as the chip holds, for each channel block
+    // as many workgroups as the chip holds, for each channel block: the ragged forms' registers, 140 and more, leave three waves a SIMD, and a fourth
+    // workgroup of a CU would begin, and stage its weights, when another ends.  us four / three: 1x1 [14,127,114,11]->48 27.7 / 21.6, [30,86,86,40]->16
+    // 16.7 / 13.3, 3x3 [32,50,50,20]->164 38.4 / 30.6, [27,82,93,9]->16 22.9 / 18.8; the other way [21,72,72,104]->18 stride 2 12.7 / 13.9
     const int64_t blocks = (a.OC + 16 * CT - 1) / (16 * CT), rounds = SPLIT ? a.n_pt : (a.n_pt + 3) / 4;
-    const int64_t held = lds > 80 * 1024 ? 1 : (lds > 53 * 1024 ? 2 : (lds > 40 * 1024 ? 3 : 4)), most = (256 * held + blocks - 1) / blocks;
+    const int64_t held = lds > 80 * 1024 ? 1 : (lds > 53 * 1024 ? 2 : (RAGGED || lds > 40 * 1024 ? 3 : 4)), most = (256 * held + blocks - 1) / blocks;
     const int64_t each = (rounds + most - 1) / most;
     a.groups           = (int32_t)((rounds + each - 1) / each);
     if (!fastdiv_exact_up_to((uint64_t)a.groups * blocks, (uint32_t)a.groups))
