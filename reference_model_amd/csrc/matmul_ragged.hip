@@ -48,6 +48,8 @@ __device__ __forceinline__ v4i load16(const uint8_t* p)
 template <int EB>
 __device__ __forceinline__ v4i load_front(const uint8_t* p, int n)
 {
+    if (n >= 16)
+        return load16(p);
     uint32_t d[4] = { 0, 0, 0, 0 };
 #pragma unroll
     for (int i = 0; i < 16; i += EB)
@@ -90,7 +92,8 @@ constexpr int ragged_wave_lds()
     return SPLIT > 1 && block < 4096 * NC ? 4096 * NC : block;
 }
 
-// NC: column blocks of 32 in a tile.  TINY: an operand of less than 16 bytes, read element by element
+// NC: column blocks of 32 in a tile.  TINY: an operand of less than 16 bytes, or a tile beyond 32-bit offsets: 64-bit ones, and pieces of less than
+// 16 bytes element by element
 template <typename T, int SPLIT, int NC, bool TINY>
 __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_kernel(RaggedArgs p)
 {
@@ -411,7 +414,8 @@ template <typename T, int SPLIT, int NC = 2>
 static bool launch_split(hipStream_t st, RaggedArgs& p)
 {
     constexpr int EB = (int)sizeof(T);
-    // (and operands whose tile is beyond 32-bit offsets: element by element)
+    // (rows beyond 32-bit offsets, us with every piece element by element / now: int8 [1,66000001]x[66000001,1] 415800 / 72300, fp16
+    // [1,33000001]x[33000001,1] 265000 / 48600)
     const bool tiny = p.a_total < 16 || p.b_total < 16 || (int64_t)p.C * EB > INT32_MAX / 33 || (int64_t)p.W * EB > INT32_MAX / 65;
     return tiny ? launch_split_form<T, SPLIT, NC, true>(st, p) : launch_split_form<T, SPLIT, NC, false>(st, p);
 }

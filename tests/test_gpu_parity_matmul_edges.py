@@ -1,5 +1,7 @@
 """MATMUL by the kernel that splits K over waves: tiles of 32 columns, the last bytes of the operands wherever a load begins, operands of
 less than one load, and the eighths of the grid that share an L2."""
+import time
+
 import numpy as np
 import pytest
 
@@ -64,3 +66,23 @@ def test_nothing_around_the_operands_is_used(ctx, shape):
     assert ctx.sync() == capi.VALID
     af, bf = a.astype(np.float64), b.astype(np.float64)
     assert dp.check(out.numpy(), np.matmul(af, bf), np.matmul(np.abs(af), np.abs(bf)), "fp32", dp.kernel_size_bound(c, "fp32", has_bias=False))["ok"]
+
+
+def test_rows_beyond_32_bit_offsets(ctx):
+    """rows just below and just above what 32 rows' offsets reach in 32 bits: the same results, at the same rate (element by element the second
+    took five times as long)"""
+    rng = np.random.default_rng(1)
+    border = (2 ** 31 - 1) // 33
+    a, b = (rng.integers(-1, 2, border + 64).astype(np.int8) for _ in range(2))
+    da, db, out = ctx.upload(a), ctx.upload(b), ctx.empty((1,), capi.INT32)
+    took = []
+    for c in (border - 5, border + 5):
+        best = 1e9
+        for _ in range(3):
+            t0 = time.perf_counter()
+            ctx.matmul(capi.INT8, 1, 1, c, 1, da.ptr, db.ptr, 1, -1, out)
+            assert ctx.sync() == capi.VALID and ctx.last_kernel == "matmul_ragged_i8"
+            best = min(best, time.perf_counter() - t0)
+        took.append(best)
+        assert out.numpy()[0] == int(np.dot(a[:c].astype(np.int64) - 1, b[:c].astype(np.int64) + 1))
+    assert took[1] < 2 * took[0]
