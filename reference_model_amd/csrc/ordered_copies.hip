@@ -57,6 +57,7 @@ struct CopiedArgs
     int32_t zero_off;              // where the first operand's copy holds 64 bytes of zeros
     int32_t b_pitch;
     int32_t tiles, n_big;          // all; those not cut into quarters (a multiple of eight)
+    int32_t big_first;             // which of them come first
     int32_t IC, IH, IW, KH, pieces;
     int32_t pad_top, pad_left, stride_y, stride_x, dil_y, dil_x;
     int32_t padded;                // a tap can fall outside the image, and adds nothing there
@@ -460,16 +461,15 @@ __global__ __launch_bounds__(256, 2) void ordered_copied_kernel(CopiedArgs p)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const uint32_t n_big = (uint32_t)p.n_big, n_quarters = 4 * ((uint32_t)p.tiles - n_big);
-    if (blockIdx.x >= n_quarters)
+    if (p.big_first ? blockIdx.x < n_big : blockIdx.x >= n_quarters)
     {
         // neighbouring tiles share operand rows: a contiguous run of tiles for each of the eight L2s
-        const uint32_t at = blockIdx.x - n_quarters, tile = (at & 7) * (n_big >> 3) + (at >> 3);
+        const uint32_t at = blockIdx.x - (p.big_first ? 0 : n_quarters), tile = (at & 7) * (n_big >> 3) + (at >> 3);
         const uint32_t tm = fdiv(tile, p.tiles_n), tn = tile - tm * p.tiles_n.d;
         copied_tile<F64, 32, RING>(p, (int)tm * 64, (int)tn * 64, lds);
         return;
     }
-    // (the quarters first: their chain of dependent instructions is as long as a whole tile's and runs beside those)
-    const uint32_t quarter = blockIdx.x, tile = n_big + (quarter >> 2);
+    const uint32_t quarter = blockIdx.x - (p.big_first ? n_big : 0), tile = n_big + (quarter >> 2);
     const uint32_t tm = fdiv(tile, p.tiles_n), tn = tile - tm * p.tiles_n.d;
     const int m0 = (int)tm * 64 + 32 * (int)((quarter >> 1) & 1), n0 = (int)tn * 64 + 32 * (int)(quarter & 1);
     if (m0 >= p.M || n0 >= p.OC)
@@ -564,6 +564,10 @@ static bool launch_copied(hipStream_t st, CopiedArgs& p)
     p.tiles_n = make_fastdiv((uint32_t)tn);
     p.n_big   = tiles <= 192 || p.OC <= 32 ? 0 : (int32_t)(over <= 192 ? tiles - over : tiles / 8 * 8);
     const int64_t grid = p.n_big + 4 * (tiles - p.n_big);
+    // Quarters first, whose chain of dependent instructions is as long as a whole tile's and runs beside those - but where all do not fit at once (two
+    // workgroups a CU), for whole tiles would then wait for quarters to end.  us by ordered_gemm.hip / quarters first / whole tiles first: fp32 327 tiles,
+    // K 525 57 / 75 / 56, 390 tiles, K 2225 228 / 219 / 169, fp64 364 tiles, K 1107 111 / 103 / 71, IC % 4 = 0: 420 tiles, K 1656 127 / 154 / 121.
+    p.big_first = grid > 512;
     // few workgroups: a long ring, for the waves of one workgroup hide nothing of each other's loads
     const bool longer = grid <= 256 && ensure_dynamic_lds<ordered_copied_kernel<F64, 8>>(8 * 16384);
     if (longer)
