@@ -529,9 +529,14 @@ static bool copies_lead(const ConvGeom& g, bool f64)
     const int64_t K = (int64_t)g.KH * g.KW * g.IC;
     if (g.KH * g.KW < 4)    // (an image that is read once or twice)
         return false;
-    if (g.IC % 4 != 0)
-        return K >= (f64 ? 200 : 400);
     const int64_t tiles = (((int64_t)g.N * g.OH * g.OW + 63) / 64) * ((g.OC + 63) / 64);
+    // Rows of both operands for half a tile of results, over and over: fp32 610 tiles, K 425 59 / 102, 923 tiles, K 909 133 / 182, fp64 990 tiles,
+    // K 630 111 / 136, IC % 4 = 0: 632 tiles, K 1008 102 / 124, 875, K 1100 1.7 x; the other way fp32 571 tiles, K 1233 166 / 146, fp64 608, K 810 134 / 92.
+    if (g.OC <= 32 && tiles > 600)
+        return false;
+    // (129 ... 192 tiles, all quarters, fp32: K 425 27.5 / 37.7, 475 30.5 / 39.5, 567 37.0 / 33.7)
+    if (g.IC % 4 != 0)
+        return K >= (f64 ? 200 : (tiles > 128 && tiles <= 192 ? 500 : 400));
     return K > 900 && (f64 || (tiles <= 64 && g.IC % 32 != 0));
 }
 

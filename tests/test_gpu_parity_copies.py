@@ -99,3 +99,22 @@ def test_bounds_pass_multiplies_the_padding_out(ctx, shape, kernel, local):
             want = oracle.conv2d("f64", *(v.astype(np.float64) for v in (xs, wt, b)), (1, 1, 1, 1), (1, 1), (1, 1), abs_mode=bounds)
         assert np.array_equal(out.numpy(), want, equal_nan=True)
         assert np.isnan(want).any() and np.isinf(want).any()
+
+
+@pytest.mark.parametrize("case, f64, copied", [  # n, ih, iw, ic, oc, k
+    ((10, 61, 64, 17, 30, 5), False, False),     # 610 tiles of few channels: either operand read for half a tile of results
+    ((10, 57, 64, 17, 30, 5), False, True),      # 570
+    ((10, 64, 64, 112, 8, 3), True, False),      # 640
+    ((2, 52, 41, 17, 96, 5), False, False),      # 134 tiles in quarters, K 425
+    ((2, 52, 41, 21, 96, 5), False, True)])      # K 525
+def test_copies_where_they_lead(case, f64, copied):
+    n, h, w, ic, oc, k = case
+    c = Context(0)
+    try:
+        d = c.conv_desc(capi.FP32, capi.FP32, (n, h, w, ic), oc, k, k, (h, w), (k // 2,) * 4, (1, 1), (1, 1), oc)
+        dev = [c.upload(np.zeros(s, np.float32)) for s in ((n, h, w, ic), (oc, k, k, ic), (oc,))]
+        out = c.empty((n, h, w, oc), capi.F64 if f64 else capi.FP32)
+        c.conv2d_precise(d, *dev, False, out) if f64 else c.conv2d(d, *dev, 0, 0, out)
+        assert c.sync() == capi.VALID and ("copied" in c.last_kernel) == copied and not out.numpy().any()
+    finally:
+        c.close()
