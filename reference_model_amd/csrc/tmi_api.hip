@@ -672,7 +672,12 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // [5,8,11,69]->440 8.1 / 3.6.  From 36 steps on, odd rows (loads that start between words, at a quarter of the rate) are
         // padded first: bf16 [1,45,9,219]->23 18.9 / 11, int8 [2,11,16,285]->42 5x5 34 / 18.
         // A few tiles: [1,6,9,48]->16 int32 6.0 / 3.5, 1x1 [1,8,11,34]->32 int32 6.0 / 3.6, 5x5 [1,17,5,112]->24 stride 2 9.1 / 5.5, [2,12,12,73]->48 6.6 / 6.1.
-        if (padded && t_tiles * t_steps <= (t_row % 16 == 0 ? 24000 : 6000) && !(t_row % 4 != 0 && t_steps >= 36) && taps_open())
+        // More tiles than it has workgroups at once, 1x1 with the fused RESCALE: the pointwise kernel on copies.  us copies / this: [42,9,5,19]->416 (780
+        // tiles) 5.4 / 6.2, [15,13,8,26]->568 5.7 / 6.5, [2,39,45,95]->272 6.0 / 6.9; the other way [1,49,40,27]->360 (744) 5.6 / 4.9, [43,28,30,70]->16 7.5 /
+        // 6.1, even int32 results.
+        const bool pointwise_copies = rp.enabled && g.KH * g.KW == 1 && g.stride_y * g.stride_x == 1 && g.OC % 8 == 0 && g.OC > 32 && t_row % 4 != 0 &&
+                                      t_row <= 96 && t_tiles > 768;
+        if (padded && t_tiles * t_steps <= (t_row % 16 == 0 ? 24000 : 6000) && !(t_row % 4 != 0 && t_steps >= 36) && !pointwise_copies && taps_open())
             padded = 0, name = launch_taps();
         if (name)
             return after_launch(ctx, name);
@@ -842,7 +847,17 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // 5.5 / 6.8; the other way [14,92,75,48]->48 fp16 stride 2 11.3 / 7.8, [4,28,33,16]->264 8.1 / 5.4).
         const bool long_and_many = t_steps >= 90 && t_tiles > (t_steps >= 140 ? 380 : (t_steps >= 120 ? 480 : 700));
         const bool patch_filled  = g.KH * g.KW > 1 && t_tiles > 700 && t_tiles <= (t_steps >= 64 ? 3400 : 2400) && t_row % 8 == 0 && g.OC % 8 == 0;
-        if (!name && !long_and_many && !patch_filled && taps_open())
+        // 16-bit rows of a few words, filled up to 16 bytes a tap here and as they are there, from the same border on.  us patch kernel / this one: 3x3
+        // [6,91,61,4]->96 7.2 / 10.6, [9,30,14,10]->224 5.9 / 7.5, 5x5 [7,51,60,6]->56 6.6 / 9.0, [46,12,10,2]->224 6.6 / 9.3, 1x1 [3,87,100,12]->8 4.4 / 4.9; the
+        // other way 3x3 [7,36,38,2]->296 stride 2 (750 tiles) 5.8 / 5.2, [11,71,70,2]->88 (5127) 16.4 / 10.2, 1x1 [5,126,85,4]->40 (3348) 7.5 / 6.2.
+        // More than 5000 tiles: 3x3 [45,59,67,10]->32 (rows of 20 bytes) 10.9 / 14.6, 5x5 [11,134,113,6]->8 8.4 / 15.5; strided [51,124,107,14]->8 30.2 / 24.9.
+        const int32_t taps    = g.KH * g.KW;
+        const bool short_rows = fp16b && t_row % 4 == 0 && (t_row != 16 || taps > 9) && t_row <= (taps == 1 ? 24 : 28) && g.OC % 8 == 0 && t_tiles > 768 &&
+                                t_tiles <= (taps == 1 ? 2600 : ((taps > 9 || t_row > 16) && g.stride_y * g.stride_x == 1 ? 12000 : 5000));
+        // 5x5 on rows of 64 bytes (a block of the patch kernel) one round of it, whatever the output channels: int8 [14,55,51,39]->12 14.0 / 16.3 (padded),
+        // [4,35,26,55]->257 18.9 / 21.5, [30,40,16,43]->51 16.3 / 17.9; the other way [35,8,9,61]->474 25.1 / 20.8, even [20,32,22,49]->69 20.2 / 19.7.
+        const bool long_windows = taps > 9 && t_row == 64 && t_tiles > 960 && t_tiles <= 1400;
+        if (!name && !long_and_many && !patch_filled && !short_rows && !long_windows && taps_open())
             name = launch_taps();
         if (!name && patch_ok)
             name = launch_conv2d_mfma(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,

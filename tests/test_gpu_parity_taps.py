@@ -187,3 +187,34 @@ def test_what_it_declines_goes_where_it_leads(shape, form, kernel, copies):
         assert c.last_kernel == kernel and (c.workspace_bytes() != (0, 0)) == copies
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("dtype, shape, k, kernel", [
+    (capi.FP16, (6, 91, 61, 4, 96), 3, "conv2d_mfma_f16"),      # rows of two words, many tiles: not filled up to 16 bytes a tap
+    (capi.FP16, (1, 91, 61, 4, 96), 3, "conv2d_taps_f16"),      # fewer than it has workgroups
+    (capi.BF16, (7, 51, 60, 6, 56), 5, "conv2d_mfma_bf16"),
+    (capi.BF16, (7, 51, 60, 6, 60), 5, "conv2d_taps_bf16"),     # channels by fours
+    (capi.FP16, (3, 87, 100, 12, 8), 1, "conv2d_mfma_f16"),
+    (capi.FP16, (3, 87, 100, 16, 8), 1, "conv2d_taps_f16"),
+    (capi.INT8, (15, 13, 8, 26, 568), 1, "conv2d_pointwise_i8_rescale"),    # on copies
+    (capi.INT8, (1, 49, 40, 27, 360), 1, "conv2d_taps_i8_rescale"),
+    (capi.INT8, (30, 40, 16, 43, 51), 5, "conv2d_mfma_i8_rescale")])        # on copies of 64 bytes
+def test_many_tiles_of_short_rows_go_where_they_lead(ctx, dtype, shape, k, kernel):
+    n, h, w, ic, oc = shape
+    rng = np.random.default_rng(ic)
+    pad = (k // 2,) * 4
+    if dtype == capi.INT8:
+        x, wt = rng.integers(-128, 128, (n, h, w, ic)).astype(np.int8), rng.integers(-128, 128, (oc, k, k, ic)).astype(np.int8)
+        bias = rng.integers(-9999, 9999, oc).astype(np.int32)
+        mult, shift = rng.integers(1 << 30, 1 << 31, oc).astype(np.int32), rng.integers(40, 43, oc).astype(np.int8)
+        got, st = gpu_ops.conv2d(ctx, x, wt, bias, pad, in_zp=-11, w_zp=0, rescale=dict(mult=mult, shift=shift, out_zp=3))
+        want, wst = oracle.rescale(oracle.conv2d("i8", x[-1:], wt, bias, pad, in_zp=-11, w_zp=0), mult, shift, out_zp=3)
+        assert st == wst and np.array_equal(got[-1:], want)
+    else:
+        x, wt, bias = (rng.integers(-8, 9, s).astype(np.float32) / 4 for s in ((n, h, w, ic), (oc, k, k, ic), (oc,)))
+        args = [v.astype(np.float16) if dtype == capi.FP16 else (v.view(np.uint32) >> 16).astype(np.uint16) for v in (x, wt, bias)]
+        got, st = gpu_ops.conv2d(ctx, *args, pad, dtype=dtype)
+        got = got[-1:].astype(np.float64) if dtype == capi.FP16 else (got[-1:].astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+        want = oracle.conv2d("f64", *(v.astype(np.float64) for v in (x[-1:], wt, bias)), pad, (1, 1), (1, 1))
+        assert st == capi.VALID and np.all(np.abs(got - want) <= (2.0 ** -11 if dtype == capi.FP16 else 2.0 ** -8) * np.abs(want))
+    assert ctx.last_kernel == kernel
