@@ -88,7 +88,7 @@ def test_16_bit_floats(ctx, case, dtype):
     else:
         args = [(v.view(np.uint32) >> 16).astype(np.uint16) for v in (x, wt, bias)]
     got, st = gpu_ops.conv2d(ctx, *args, pad, stride, dil, dtype=dtype)
-    assert st == capi.VALID
+    assert st == capi.VALID and ctx.last_kernel == ("conv2d_taps_f16" if dtype == capi.FP16 else "conv2d_taps_bf16")
     if dtype == capi.BF16:
         got = (got.astype(np.uint32) << 16).view(np.float32)
     ulp = 2.0 ** -11 if dtype == capi.FP16 else 2.0 ** -8
