@@ -41,25 +41,6 @@ struct I16TapsArgs
 
 constexpr int kI16Dead = 1 << 26;    // table entry: no chunk at all
 
-__device__ __forceinline__ v4i load16_any(const uint8_t* p)    // of no alignment
-{
-    v4i v;
-    __builtin_memcpy(&v, p, 16);
-    return v;
-}
-// v without its first n bytes, zeros behind (n < 16)
-__device__ __forceinline__ v4i drop_front(v4i v, int n)
-{
-    if (n & 8)
-        v = v4i{ v[2], v[3], 0, 0 };
-    if (n & 4)
-        v = v4i{ v[1], v[2], v[3], 0 };
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-        v[k] = (int)__builtin_amdgcn_alignbyte(k < 3 ? v[k < 3 ? k + 1 : 3] : 0, v[k], n & 3);
-    return v;
-}
-
 __device__ __forceinline__ int64_t clip48(int64_t v)
 {
     const int64_t top = (int64_t(1) << 47) - 1;
@@ -115,16 +96,10 @@ __global__ __launch_bounds__(256, 2) void conv_i16_taps_kernel(I16TapsArgs a)
                 const int cc  = ok ? c : 0;
                 const int tap = (int)fdiv((uint32_t)cc, a.div_pieces), piece = cc - tap * a.pieces;
                 const int off = w_row + tap * a.IC + piece * 16, at = off <= a.w_last ? off : a.w_last;
-                wv[u]         = load16_any(a.w + (uint32_t)at);
+                wv[u]         = load16(a.w + (uint32_t)at);
                 if (__any(off > at))
                     wv[u] = drop_front(wv[u], off - at);
-                const int n = a.IC - piece * 16;    // channels of the chunk
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                {
-                    const int m = n - 4 * k;
-                    wv[u][k]    = m >= 4 ? wv[u][k] : (m <= 0 ? 0 : wv[u][k] & (int)((1u << (8 * m)) - 1u));
-                }
+                wv[u] = keep_bytes(wv[u], a.IC - piece * 16);    // channels of the chunk
             }
             if (!ok)
                 wv[u] = v4i{ 0, 0, 0, 0 };
@@ -172,14 +147,14 @@ __global__ __launch_bounds__(256, 2) void conv_i16_taps_kernel(I16TapsArgs a)
         if constexpr (!RAGGED)
             xv[d][0] = reinterpret_cast<const v4i*>(src)[0], xv[d][1] = reinterpret_cast<const v4i*>(src)[1];
         else if constexpr (!decltype(careful)::value)
-            xv[d][0] = load16_any(src), xv[d][1] = load16_any(src + 16);
+            xv[d][0] = load16(src), xv[d][1] = load16(src + 16);
         else
 #pragma unroll
             for (int j = 0; j < 2; j++)
             {
                 // (what lies 16 bytes or more past the last load is behind the channels: any value will do)
                 const int past = inside && off + 16 * j > a.in_last ? off + 16 * j - a.in_last : 0;
-                xv[d][j]       = drop_front(load16_any(src + 16 * j - past), past & 15);
+                xv[d][j]       = drop_front(load16(src + 16 * j - past), past & 15);
             }
     };
     auto enter_tile = [&](int pt) {

@@ -68,35 +68,6 @@ __host__ __device__ constexpr int taps_lds_bytes(int steps)
     return taps_fixed_lds<OCT>() + 2 * steps * (OCT * 512 + 16 + 8);
 }
 
-__device__ __forceinline__ v4i load16(const uint8_t* p)    // of no alignment
-{
-    v4i v;
-    __builtin_memcpy(&v, p, 16);
-    return v;
-}
-// v without its first n bytes, zeros behind
-__device__ __forceinline__ v4i drop_bytes(v4i v, int n)
-{
-    uint64_t lo = (uint32_t)v[0] | (uint64_t)(uint32_t)v[1] << 32, hi = (uint32_t)v[2] | (uint64_t)(uint32_t)v[3] << 32;
-    if (n & 8)
-        lo = hi, hi = 0;
-    const int bits = 8 * (n & 7);
-    if (bits)
-        lo = lo >> bits | hi << (64 - bits), hi >>= bits;
-    return v4i{ (int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32) };
-}
-// the first n bytes of v
-__device__ __forceinline__ v4i keep_bytes(v4i v, int n)
-{
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-    {
-        const int m = n - 4 * k;
-        v[k]        = m >= 4 ? v[k] : (m <= 0 ? 0 : v[k] & (int)((1u << (8 * m)) - 1u));
-    }
-    return v;
-}
-
 // What the epilogue reads of a tile of 32 channels.
 struct TapsTables
 {

@@ -35,15 +35,6 @@ struct RaggedArgs
     FastDiv per_batch, tiles_w;
 };
 
-struct __attribute__((packed)) Bytes16
-{
-    v4i v;
-};
-__device__ __forceinline__ v4i load16(const uint8_t* p)
-{
-    return reinterpret_cast<const Bytes16*>(p)->v;
-}
-
 // the first n bytes at p (n may be 0 or negative), then zeros
 template <int EB>
 __device__ __forceinline__ v4i load_front(const uint8_t* p, int n)
@@ -59,29 +50,6 @@ __device__ __forceinline__ v4i load_front(const uint8_t* p, int n)
             d[i >> 2] |= e << (8 * (i & 3));
         }
     return v4i{ (int)d[0], (int)d[1], (int)d[2], (int)d[3] };
-}
-
-// v without its first n bytes, zeros behind (n < 16)
-__device__ __forceinline__ v4i drop_bytes(v4i v, int n)
-{
-    uint64_t lo = (uint32_t)v[0] | (uint64_t)(uint32_t)v[1] << 32, hi = (uint32_t)v[2] | (uint64_t)(uint32_t)v[3] << 32;
-    if (n & 8)
-        lo = hi, hi = 0;
-    const int bits = 8 * (n & 7);
-    if (bits)
-        lo = lo >> bits | hi << (64 - bits), hi >>= bits;
-    return v4i{ (int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32) };
-}
-// the first n bytes of v, zeros behind (n may be negative)
-__device__ __forceinline__ v4i keep_bytes(v4i v, int n)
-{
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-    {
-        const int m = n - 4 * k;
-        v[k]        = m >= 4 ? v[k] : (m <= 0 ? 0 : v[k] & (int)((1u << (8 * m)) - 1u));
-    }
-    return v;
 }
 
 // bytes of LDS of a wave: a block of the second operand, then its partial tile

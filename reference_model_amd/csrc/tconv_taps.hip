@@ -49,25 +49,6 @@ struct TconvArgs    // (at most 256 bytes: a larger launch takes the host longer
 
 constexpr int kTconvDead = 1 << 26;    // table entry: no chunk at all
 
-__device__ __forceinline__ v4i load16_any(const uint8_t* p)    // of no alignment
-{
-    v4i v;
-    __builtin_memcpy(&v, p, 16);
-    return v;
-}
-// v without its first n bytes, zeros behind (n < 16)
-__device__ __forceinline__ v4i drop_front(v4i v, int n)
-{
-    if (n & 8)
-        v = v4i{ v[2], v[3], 0, 0 };
-    if (n & 4)
-        v = v4i{ v[1], v[2], v[3], 0 };
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-        v[k] = (int)__builtin_amdgcn_alignbyte(k < 3 ? v[k < 3 ? k + 1 : 3] : 0, v[k], n & 3);
-    return v;
-}
-
 template <int CT>
 constexpr int64_t tconv_lds(int64_t steps)
 {
@@ -119,16 +100,10 @@ __global__ __launch_bounds__(256, 2) void tconv_taps_kernel(TconvArgs a)
             else
             {
                 const int at = off <= a.w_last ? off : a.w_last;
-                wv[u]        = load16_any(a.w + (uint32_t)at);
+                wv[u]        = load16(a.w + (uint32_t)at);
                 if (__any(off > at))
                     wv[u] = drop_front(wv[u], off - at);
-                const int n = a.IC - piece * 16;    // channels of the chunk
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                {
-                    const int m = n - 4 * k;
-                    wv[u][k]    = m >= 4 ? wv[u][k] : (m <= 0 ? 0 : wv[u][k] & (int)((1u << (8 * m)) - 1u));
-                }
+                wv[u] = keep_bytes(wv[u], a.IC - piece * 16);    // channels of the chunk
             }
             if (!ok)
                 wv[u] = v4i{ 0, 0, 0, 0 };
@@ -175,11 +150,11 @@ __global__ __launch_bounds__(256, 2) void tconv_taps_kernel(TconvArgs a)
         if constexpr (!RAGGED)
             xv[d] = *reinterpret_cast<const v4i*>(src);
         else if constexpr (!decltype(careful)::value)
-            xv[d] = load16_any(src);
+            xv[d] = load16(src);
         else
         {
             const int past = inside && off > a.in_last ? off - a.in_last : 0;
-            xv[d]          = drop_front(load16_any(src - past), past);
+            xv[d]          = drop_front(load16(src - past), past);
         }
     };
     auto enter_tile = [&](int pt) {
