@@ -13,7 +13,7 @@
 // (28.7 ns alone, 30 with every CU at work), an fp32 step of four k 32 clocks and 64 of additions.  A layer of few tiles is that chain,
 // K / 4 instructions: [..,288]->24 3x3 (K 2592, 4 tiles), fp64 34.4 us of which the instructions are 18.6 and the first launch 3 (51.0 by
 // ordered_gemm.hip), and a wave must find its next operands in registers: without the fragments read a stage ahead it was 51.
-// [4,56,56,256]->256 3x3, fp64: 234 us, 212 of them matrix instructions (256 by ordered_gemm.hip).
+// [4,56,56,256]->256 3x3, fp64: 232 us, 212 of them matrix instructions (256 by ordered_gemm.hip).
 //
 // A tap outside the image multiplies a zero by a weight; where some weight of a tile's channels is infinite or NaN (the
 // first launch leaves a word per piece of a row that says so) the tile is summed again one result at a time without those taps.
@@ -518,7 +518,7 @@ static bool plan_copies(CopyPlan& c, const ConvGeom& g, bool f64)
 // element by element.  us by ordered_gemm.hip / here, 3x3 unless noted, K = taps x channels:
 //   fp64, IC % 4 != 0: K 225 17.4 / 12.2, 603 68 / 36, 1125 54 / 19, 1773 228 / 164, 3294 151 / 59; 135 11.0 / 9.4, 90 7.0 / 8.9, 81 10.1 /
 //     14.4; 1x1: 145 11.3 / 10.4, 113 18.8 / 22.1
-//   fp64, IC % 4 = 0: K 936 25.4 / 23.8, 1152 26 / 19, 2304 [4,56,56,256]->256 256 / 234, 2592 51 / 34 (few tiles) and 196.0 / 195.6 (495
+//   fp64, IC % 4 = 0: K 936 25.4 / 23.8, 1152 26 / 19, 2304 [4,56,56,256]->256 257 / 232, 2592 51 / 34 (few tiles) and 196.0 / 195.6 (495
 //     tiles), 4392 121 / 72; 648 56 / 66 (355 tiles) and 20.0 / 17.2 (23), 504 25 / 30; 1x1 424 19.4 / 24.4
 //   fp32, IC % 4 != 0: K 405 18.0 / 13.7, 846 50 / 41, 1125 44 / 23, 2178 (625 tiles) 276 / 223, 3114 282 / 187; 306 14.9 / 14.9
 //   fp32, IC % 4 = 0, up to 64 tiles: K 1008 28.2 / 24.5, 1296 37 / 30, 2232 61 / 41, 3312 89 / 61, 504 and shorter 0.9x; channels of whole

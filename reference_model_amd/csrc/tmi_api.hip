@@ -848,15 +848,15 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         const bool long_and_many = t_steps >= 90 && t_tiles > (t_steps >= 140 ? 380 : (t_steps >= 120 ? 480 : 700));
         const bool patch_filled  = g.KH * g.KW > 1 && t_tiles > 700 && t_tiles <= (t_steps >= 64 ? 3400 : 2400) && t_row % 8 == 0 && g.OC % 8 == 0;
         // 16-bit rows of a few words, filled up to 16 bytes a tap here and as they are there, from the same border on.  us patch kernel / this one: 3x3
-        // [6,91,61,4]->96 7.2 / 10.6, [9,30,14,10]->224 5.9 / 7.5, 5x5 [7,51,60,6]->56 6.6 / 9.0, [46,12,10,2]->224 6.6 / 9.3, 1x1 [3,87,100,12]->8 4.4 / 4.9; the
+        // [6,91,61,4]->96 7.2 / 10.6, [9,30,14,10]->224 5.9 / 7.5, 5x5 [7,51,60,6]->56 6.6 / 9.0, [46,12,10,2]->224 6.6 / 9.3, 7x7 [8,60,60,10]->64 11.9 / 21.2, 1x1 [3,87,100,12]->8 4.4 / 4.9; the
         // other way 3x3 [7,36,38,2]->296 stride 2 (750 tiles) 5.8 / 5.2, [11,71,70,2]->88 (5127) 16.4 / 10.2, 1x1 [5,126,85,4]->40 (3348) 7.5 / 6.2.
         // More than 5000 tiles: 3x3 [45,59,67,10]->32 (rows of 20 bytes) 10.9 / 14.6, 5x5 [11,134,113,6]->8 8.4 / 15.5; strided [51,124,107,14]->8 30.2 / 24.9.
         const int32_t taps    = g.KH * g.KW;
-        const bool short_rows = fp16b && t_row % 4 == 0 && (t_row != 16 || taps > 9) && t_row <= (taps == 1 ? 24 : 28) && g.OC % 8 == 0 && t_tiles > 768 &&
-                                t_tiles <= (taps == 1 ? 2600 : ((taps > 9 || t_row > 16) && g.stride_y * g.stride_x == 1 ? 12000 : 5000));
+        const bool short_rows = fp16b && t_row % 4 == 0 && (t_row != 16 || taps > 9) && t_row <= (taps == 1 ? 24 : 28) && g.OC % 8 == 0 &&
+                                t_tiles > 768 && t_tiles <= (taps == 1 ? 2600 : ((taps > 9 || t_row > 16) && g.stride_y * g.stride_x == 1 ? 12000 : 5000));
         // 5x5 on rows of 64 bytes (a block of the patch kernel) one round of it, whatever the output channels: int8 [14,55,51,39]->12 14.0 / 16.3 (padded),
         // [4,35,26,55]->257 18.9 / 21.5, [30,40,16,43]->51 16.3 / 17.9; the other way [35,8,9,61]->474 25.1 / 20.8, even [20,32,22,49]->69 20.2 / 19.7.
-        const bool long_windows = taps > 9 && t_row == 64 && t_tiles > 960 && t_tiles <= 1400;
+        const bool long_windows = taps > 9 && taps <= 25 && t_row == 64 && t_tiles > 960 && t_tiles <= 1400;
         if (!name && !long_and_many && !patch_filled && !short_rows && !long_windows && taps_open())
             name = launch_taps();
         if (!name && patch_ok)
@@ -865,6 +865,10 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         if (!name && gemm_ok && !gemm_1st)
             name = launch_gemm_mfma(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out, 0, 0,
                                     pad_page, ctx->flags_dev);
+        // Left to the patch kernel above, but its weights do not fit the LDS.  us one result a lane / this, 13x13: int8 [4,60,60,16]->64 4690 / 13.8, fp16
+        // [8,60,60,64]->64 57400 / 294
+        if (!name && taps_open())
+            name = launch_taps();
     }
     if (!name && ctx->kernel_choice >= 2)
         return fail(ctx, "%s: no MFMA / vector kernel is eligible for this shape", op);
