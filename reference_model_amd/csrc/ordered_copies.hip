@@ -534,6 +534,12 @@ static bool copies_lead(const ConvGeom& g, bool f64)
     // K 630 111 / 136, IC % 4 = 0: 632 tiles, K 1008 102 / 124, 875, K 1100 1.7 x; the other way fp32 571 tiles, K 1233 166 / 146, fp64 608, K 810 134 / 92.
     if (g.OC <= 32 && tiles > 600)
         return false;
+    // The chain grows by what fills the granules up (8 elements in fp64, 16 in fp32).  Times of ordered_gemm.hip's by channels, large windows: fp32 3
+    // channels 2.8, 6 1.3, 10 1.1 and from K 800 on 0.9, 11 0.9, 4 2.7, 8 1.4, 20 1.2, 12 and 24 1.0, 28 0.85; fp64 2 1.5, 3 1.1, 5 0.8, 4 1.4, 12 0.94, 20 0.85.
+    const int64_t kg  = f64 ? 8 : 16;
+    const double fill = (double)((g.IC + kg - 1) / kg * kg) / g.IC;
+    if (fill > (g.IC % 4 != 0 ? (f64 ? 1.8 : (K >= 800 ? 2.2 : 1.6)) : (f64 ? 1.34 : 1.3)))
+        return false;
     // (129 ... 192 tiles, all quarters, fp32: K 425 27.5 / 37.7, 475 30.5 / 39.5, 567 37.0 / 33.7)
     if (g.IC % 4 != 0)
         return K >= (f64 ? 200 : (tiles > 128 && tiles <= 192 ? 500 : 400));

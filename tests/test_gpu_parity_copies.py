@@ -102,11 +102,17 @@ def test_bounds_pass_multiplies_the_padding_out(ctx, shape, kernel, local):
 
 
 @pytest.mark.parametrize("case, f64, copied", [  # n, ih, iw, ic, oc, k
-    ((10, 61, 64, 17, 30, 5), False, False),     # 610 tiles of few channels: either operand read for half a tile of results
-    ((10, 57, 64, 17, 30, 5), False, True),      # 570
+    ((10, 61, 64, 21, 30, 5), False, False),     # 610 tiles of few channels: either operand read for half a tile of results
+    ((10, 57, 64, 21, 30, 5), False, True),      # 570
     ((10, 64, 64, 112, 8, 3), True, False),      # 640
-    ((2, 52, 41, 17, 96, 5), False, False),      # 134 tiles in quarters, K 425
-    ((2, 52, 41, 21, 96, 5), False, True)])      # K 525
+    ((2, 52, 41, 53, 96, 3), False, False),      # 134 tiles in quarters, K 477
+    ((2, 52, 41, 63, 96, 3), False, True),       # K 567
+    ((1, 20, 20, 6, 40, 11), False, False),      # few channels: the granules would be filled up with zeros
+    ((1, 20, 20, 4, 40, 17), False, False),
+    ((1, 20, 20, 28, 40, 7), False, True),
+    ((1, 20, 20, 2, 40, 13), True, False),
+    ((1, 20, 20, 4, 40, 17), True, False),
+    ((1, 20, 20, 5, 40, 13), True, True)])
 def test_copies_where_they_lead(case, f64, copied):
     n, h, w, ic, oc, k = case
     c = Context(0)
