@@ -852,8 +852,12 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // other way 3x3 [7,36,38,2]->296 stride 2 (750 tiles) 5.8 / 5.2, [11,71,70,2]->88 (5127) 16.4 / 10.2, 1x1 [5,126,85,4]->40 (3348) 7.5 / 6.2.
         // More than 5000 tiles: 3x3 [45,59,67,10]->32 (rows of 20 bytes) 10.9 / 14.6, 5x5 [11,134,113,6]->8 8.4 / 15.5; strided [51,124,107,14]->8 30.2 / 24.9.
         const int32_t taps    = g.KH * g.KW;
-        const bool short_rows = fp16b && t_row % 4 == 0 && (t_row != 16 || taps > 9) && t_row <= (taps == 1 ? 24 : 28) && g.OC % 8 == 0 &&
-                                t_tiles > 768 && t_tiles <= (taps == 1 ? 2600 : ((taps > 9 || t_row > 16) && g.stride_y * g.stride_x == 1 ? 12000 : 5000));
+        // Few channels or large windows, whatever the channels' number, the same: 7x7 [20,84,32,14]->4 8.9 / 20.5, 11x11 [45,29,27,4]->1 9.5 / 19.7; the other way 3x3
+        // [37,40,60,2]->28 11.7 / 8.5.
+        const bool few_oc     = g.OC < 24 || taps > 50;
+        const bool short_rows = fp16b && t_row % 4 == 0 && (t_row != 16 || taps > 9) && t_row <= (taps == 1 ? 24 : 28) && (g.OC % 8 == 0 || few_oc) &&
+                                t_tiles > 768 &&
+                                t_tiles <= (taps == 1 ? 2600 : ((taps > 9 || t_row > 16 || few_oc) && g.stride_y * g.stride_x == 1 ? 12000 : 5000));
         // 5x5 on rows of 64 bytes (a block of the patch kernel) one round of it, whatever the output channels: int8 [14,55,51,39]->12 14.0 / 16.3 (padded),
         // [4,35,26,55]->257 18.9 / 21.5, [30,40,16,43]->51 16.3 / 17.9; the other way [35,8,9,61]->474 25.1 / 20.8, even [20,32,22,49]->69 20.2 / 19.7.
         const bool long_windows = taps > 9 && taps <= 25 && t_row == 64 && t_tiles > 960 && t_tiles <= 1400;

@@ -200,6 +200,8 @@ def test_what_it_declines_goes_where_it_leads(shape, form, kernel, copies):
     (capi.INT8, (1, 49, 40, 27, 360), 1, "conv2d_taps_i8_rescale"),
     (capi.INT8, (30, 40, 16, 43, 51), 5, "conv2d_mfma_i8_rescale"),         # on copies of 64 bytes
     (capi.FP16, (8, 60, 60, 10, 64), 7, "conv2d_mfma_f16"),
+    (capi.FP16, (20, 84, 32, 14, 4), 7, "conv2d_mfma_f16"),                 # few channels
+    (capi.BF16, (45, 29, 27, 4, 1), 11, "conv2d_mfma_bf16"),
     (capi.FP16, (8, 60, 60, 10, 64), 9, "conv2d_taps_f16"),                 # windows whose weights do not fit the patch kernel's LDS
     (capi.FP16, (4, 60, 60, 8, 64), 13, "conv2d_taps_f16"),
     (capi.BF16, (2, 60, 60, 64, 256), 13, "conv2d_taps_bf16"),
