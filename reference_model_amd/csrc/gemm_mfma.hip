@@ -901,6 +901,10 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
 #pragma unroll
             for (int i = 0; i < PXT; i++)
                 psum[i] = tab_psum[wp * 32 * PXT + i * 32 + rho] + tab_psum[PROWS + wp * 32 * PXT + i * 32 + rho];
+            // (a thread per channel: every wave adding up the four parts of its channels was 24 more 16-byte reads each, half a microsecond)
+            if (tid < WROWS)
+                tab_wsum[tid] += tab_wsum[WROWS + tid] + tab_wsum[2 * WROWS + tid] + tab_wsum[3 * WROWS + tid];
+            __syncthreads();
         }
     }
     // Results leave through LDS: a lane holds 64 bytes of one pixel's row, so a store instruction straight from the accumulators is 64 separate
@@ -1032,11 +1036,7 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
 #pragma unroll
             for (int q = 0; q < 4; q++)
             {
-                const int* src = tab_wsum + tl + group_channel(q);
-                v4i sw         = *reinterpret_cast<const v4i*>(src);
-#pragma unroll
-                for (int r = 1; r < 4; r++)
-                    sw += *reinterpret_cast<const v4i*>(src + r * WROWS);
+                const v4i sw = *reinterpret_cast<const v4i*>(tab_wsum + tl + group_channel(q));
                 cb[4 * q] += kzz - a.za * sw.x, cb[4 * q + 1] += kzz - a.za * sw.y;
                 cb[4 * q + 2] += kzz - a.za * sw.z, cb[4 * q + 3] += kzz - a.za * sw.w;
             }
