@@ -59,6 +59,14 @@ template <int CT, bool RAGGED>
 __global__ __launch_bounds__(256, 2) void tconv_taps_kernel(TconvArgs a)
 {
     constexpr int DEPTH = 6;
+    // The arguments at once.  (Left to the compiler they come where they are used, and the classes' by vector loads: eight trips one after the other
+    // before the first operand; [1,7,5,42]->64 2x2 stride 2 4.3 us, so 3.8.)
+    asm volatile("" ::"s"(a.in), "s"(a.w), "s"(a.bias), "s"(a.out), "s"(a.page), "s"(a.OC), "s"(a.OH), "s"(a.OW), "s"(a.IH), "s"(a.IW), "s"(a.KH), "s"(a.KW),
+                 "s"(a.sy), "s"(a.sx), "s"(a.IC), "s"(a.pieces), "s"(a.groups), "s"(a.classes), "s"(a.w_last), "s"(a.bias_len), "s"(a.P), "s"(a.n_pt));
+    asm volatile("" ::"s"(a.div_groups.magic), "s"(a.div_groups.d), "s"(a.div_classes.magic), "s"(a.div_classes.d), "s"(a.div_sx.magic), "s"(a.div_sx.d),
+                 "s"(a.div_pieces.magic), "s"(a.div_pieces.d));
+    auto entry8  = [](const int8_t (&v)[kTconvStrides], int c) { uint32_t u; __builtin_memcpy(&u, v, 4); return (int)(int8_t)(u >> (8 * c)); };
+    auto entry16 = [](const auto& v, int c) { uint64_t u; __builtin_memcpy(&u, v, 8); return (uint32_t)(u >> (16 * c)) & 0xffffu; };
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     int* tab_base  = reinterpret_cast<int*>(lds);                   // bias - input_zp sum w of a channel
     int* tab_part  = reinterpret_cast<int*>(lds + 16 * CT * 4);     // a wave's part of sum w
@@ -71,8 +79,9 @@ __global__ __launch_bounds__(256, 2) void tconv_taps_kernel(TconvArgs a)
     const int ocb = (int)fdiv((uint32_t)unit, a.div_classes), cls = unit - ocb * a.classes;
     const int cy = (int)fdiv((uint32_t)cls, a.div_sx), cx = cls - cy * a.sx;
     const int oc0 = ocb * 16 * CT;
-    const int taps_y = a.y.taps[cy], taps_x = a.x.taps[cx], first_y = a.y.first[cy], first_x = a.x.first[cx];
-    const uint32_t magic_x = a.taps_x_magic[cx];    // (0: one tap)
+    const int taps_y = entry8(a.y.taps, cy), taps_x = entry8(a.x.taps, cx), first_y = entry8(a.y.first, cy), first_x = entry8(a.x.first, cx);
+    const int base_y = (int16_t)entry16(a.y.base, cy), base_x = (int16_t)entry16(a.x.base, cx);
+    const uint32_t magic_x = entry16(a.taps_x_magic, cx);    // (0: one tap)
     auto row_of = [&](int tap) { return magic_x ? (int)((uint32_t)tap * magic_x >> 16) : tap; };
     const int chunks = taps_y * taps_x * a.pieces, steps = (chunks + 3) >> 2;
 
@@ -83,13 +92,11 @@ __global__ __launch_bounds__(256, 2) void tconv_taps_kernel(TconvArgs a)
     const int w_oc     = oc0 + 16 * ct_w + l16;
     const int w_row    = (w_oc < a.OC ? w_oc : 0) * (a.KH * a.KW) * a.IC;
     v4i wv[WB];
+    int wfix[WB];    // RAGGED: what is left of a chunk after the load (bytes before it << 8 | its channels)
+    // (a load's result is not looked at here, so that all of a batch are in flight at once: [8,6,5,584]->176 4x4 14.4 us with the fix-ups behind each load, so 11.6)
     auto load_weights = [&](int s0) {
-#pragma unroll
-        for (int u = 0; u < WB; u++)
-        {
-            const int s = s0 + u * SKIP, c = 4 * s + q;
-            if (s >= steps)
-                continue;
+        auto load = [&](int u) {
+            const int c   = 4 * (s0 + u * SKIP) + q;
             const bool ok = w_oc < a.OC && c < chunks;
             const int cc  = ok ? c : 0;
             const int tap = (int)fdiv((uint32_t)cc, a.div_pieces), piece = cc - tap * a.pieces;
@@ -99,21 +106,34 @@ __global__ __launch_bounds__(256, 2) void tconv_taps_kernel(TconvArgs a)
                 wv[u] = *reinterpret_cast<const v4i*>(a.w + (uint32_t)off);
             else
             {
-                const int at = off <= a.w_last ? off : a.w_last;
+                const int at = off <= a.w_last ? off : a.w_last, n = a.IC - piece * 16;
                 wv[u]        = load16(a.w + (uint32_t)at);
-                if (__any(off > at))
-                    wv[u] = drop_front(wv[u], off - at);
-                wv[u] = keep_bytes(wv[u], a.IC - piece * 16);    // channels of the chunk
+                wfix[u]      = (off - at) << 8 | (ok ? (n < 16 ? n : 16) : 0);
             }
-            if (!ok)
-                wv[u] = v4i{ 0, 0, 0, 0 };
-        }
+        };
+        if (s0 + (WB - 1) * SKIP < steps)
+#pragma unroll
+            for (int u = 0; u < WB; u++)
+                load(u);
+        else
+#pragma unroll
+            for (int u = 0; u < WB; u++)
+                if (s0 + u * SKIP < steps)
+                    load(u);
     };
     auto store_weights = [&](int s0) {
 #pragma unroll
         for (int u = 0; u < WB; u++)
             if (s0 + u * SKIP < steps)
             {
+                if constexpr (RAGGED)
+                {
+                    if (__any(wfix[u] >> 8))
+                        wv[u] = drop_front(wv[u], wfix[u] >> 8);
+                    wv[u] = keep_bytes(wv[u], wfix[u] & 255);
+                }
+                else if (!(w_oc < a.OC && 4 * (s0 + u * SKIP) + q < chunks))
+                    wv[u] = v4i{ 0, 0, 0, 0 };
                 sum_w += dot4_ones(wv[u]);
                 *reinterpret_cast<v4i*>(wl + ((s0 + u * SKIP) * CT + ct_w) * 1024 + lane * 16) = wv[u];
             }
@@ -161,7 +181,7 @@ __global__ __launch_bounds__(256, 2) void tconv_taps_kernel(TconvArgs a)
         int p = pt * 16 + l16;
         p     = p < a.P ? p : a.P - 1;
         const int r = (int)fdiv((uint32_t)p, a.div_ow), x = p - r * (int)a.div_ow.d, n = (int)fdiv((uint32_t)r, a.div_oh), y = r - n * (int)a.div_oh.d;
-        const int y0 = y + a.y.base[cy], x0 = x + a.x.base[cx];
+        const int y0 = y + base_y, x0 = x + base_x;
         pix_off      = ((n * a.IH + y0) * a.IW + x0) * a.IC;
         // (classes are as large as the largest of them: a pixel may lie past the last row or column)
         out_pix      = pt * 16 + l16 < a.P && y * a.sy + cy < a.OH && x * a.sx + cx < a.OW ? (n * a.OH + y * a.sy + cy) * a.OW + x * a.sx + cx : -1;
