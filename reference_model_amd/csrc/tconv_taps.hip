@@ -11,7 +11,7 @@
 // What bounds it: the chain of a call (weights and the first pixels on their way together, a few steps, the stores).  us copies and CONV2D / here,
 // stride 2 (class pixels): 3x3 [1968,88]->21 7.3 / 4.7, [273,88]->48 2x2 6.4 / 4.5, [4465,48]->96 2x2 12.7 / 5.7, 4x4 [1368,88]->157 16.3 / 6.7,
 // [16632,184]->24 36.8 / 12.1, [4312,208]->48 2x2 15.0 / 5.5, [520,152]->56 3x3 7.4 / 6.6; the slab kernel's layers stay there ([6272,128]->64 3x3
-// 7.2 / 7.7: its patch serves all classes).
+// 7.2 / 7.7: its patch serves all classes).  (These before the arguments came in one trip and a batch of weights in flight: now 0.90 of it over 552 layers.)
 #include <algorithm>
 #include <type_traits>
 
