@@ -513,7 +513,8 @@ static bool plan_copies(CopyPlan& c, const ConvGeom& g, bool f64)
     return true;
 }
 
-// Whether the copies pay: their launch costs 3 us and the bytes written, and gains what ordered_gemm.hip spends on conversions, on masks and
+// Whether the copies pay, for what ordered_staged.hip leaves (channel vectors of no whole units of eight; times of such vectors below are from
+// before it): their launch costs 3 us and the bytes written, and gains what ordered_gemm.hip spends on conversions, on masks and
 // on waiting for stages it fetches through registers; most for channel vectors that end inside a group of four, which it reads
 // element by element.  us by ordered_gemm.hip / here, 3x3 unless noted, K = taps x channels:
 //   fp64, IC % 4 != 0: K 225 17.4 / 12.2, 603 68 / 36, 1125 54 / 19, 1773 228 / 164, 3294 151 / 59; 135 11.0 / 9.4, 90 7.0 / 8.9, 81 10.1 /

@@ -878,6 +878,9 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         return fail(ctx, "%s: no MFMA / vector kernel is eligible for this shape", op);
     // FP32 sums keep the reference's order: the tiles of ordered_gemm.hip, whose results are the one-result-per-lane kernel's bit
     // for bit
+    if (!name && !depthwise && ctx->kernel_choice == 0 && d->in_dtype == TMI_FP32 && ordered_staged_leads(TMI_FP32, false, g, in, w) &&
+        launch_ordered_conv_staged(ctx->stream, TMI_FP32, false, g, in, w, bias, false, out) != OrderedForm::none)
+        name = "conv2d_ordered_tail_f32";
     if (!name && !depthwise && ctx->kernel_choice == 0 && d->in_dtype == TMI_FP32 && own_scratch)
         if (void* copies = ordered_copies(ctx, ordered_conv_copies_bytes(false, g)))
             if (launch_ordered_conv_copied(ctx->stream, TMI_FP32, false, g, in, w, bias, false, nullptr, out, copies))
@@ -1739,8 +1742,8 @@ static int run_conv_precise(tmi_ctx* ctx, const char* op, bool depthwise, const 
     // one double of the context's 256-byte block (bytes 160..167) holds the input's largest magnitude
     double* abs_max_slot = (bounds_mode && !local_bound) ? reinterpret_cast<double*>(reinterpret_cast<uint8_t*>(ctx->flags_dev) + 160)
                                                          : nullptr;
-    const char* name = launch_conv_precise(ctx->stream, d->in_dtype, depthwise, g, in, w, bias, bounds_mode, abs_max_slot, out,
-                                           depthwise ? nullptr : ordered_copies(ctx, ordered_conv_copies_bytes(true, g)));
+    void* copies     = depthwise || (!abs_max_slot && ordered_staged_leads(d->in_dtype, true, g, in, w)) ? nullptr : ordered_copies(ctx, ordered_conv_copies_bytes(true, g));
+    const char* name = launch_conv_precise(ctx->stream, d->in_dtype, depthwise, g, in, w, bias, bounds_mode, abs_max_slot, out, copies);
     if (!name)
         return fail(ctx, "%s: operand type without a precise-mode kernel", op);
     return after_launch(ctx, name);

@@ -151,6 +151,10 @@ OrderedForm launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, cons
                          const void* bias, bool abs_mode, const double* input_abs_max, void* out);
 OrderedForm launch_ordered_matmul(hipStream_t st, int32_t in_dtype, bool f64, int32_t N, int32_t H, int32_t C, int32_t W, const void* a,
                            const void* b, bool abs_mode, void* out);
+// ordered_staged.hip: the same for CONV2D on whole units of eight channels; _leads: whether a layer runs there.
+bool ordered_staged_leads(int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w);
+OrderedForm launch_ordered_conv_staged(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w, const void* bias,
+                                       bool abs_mode, void* out);
 // ordered_copies.hip: the same on copies of the operands in `copies` (ordered_conv_copies_bytes() of 256-byte aligned memory; 0: not taken)
 size_t ordered_conv_copies_bytes(bool f64, const ConvGeom& g);
 bool launch_ordered_conv_copied(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w,
