@@ -12,9 +12,9 @@
 // the same 10.0 / 10.7).
 //
 // What bounds it: the first operand's fragments, a line per lane and load, for products of many tiles (fp16 at 130 TFLOP/s), the
-// chain of a wave's blocks otherwise.  us transposed copy + patch or GEMM kernel -> here: fp16 96 x [197,64]x[64,197] 33.6 -> 8.8
-// (34 MB with the next: 2.2 TB/s), 96 x [197,197]x[197,64] 45.3 -> 7.3, [1,4096]x[4096,4096] 49.7 -> 9.4, int8 4 x [700,701]x[701,703]
-// 13.4 (20.8 before its ends were read in one piece), [64,512]x[512,512] 11.5 -> 4.8.
+// chain of a wave's blocks otherwise.  us transposed copy + patch or GEMM kernel -> here: fp16 96 x [197,64]x[64,197] 33.6 -> 8.2
+// (34 MB with the next: 2.4 TB/s), 96 x [197,197]x[197,64] 45.3 -> 6.2, [1,4096]x[4096,4096] 49.7 -> 9.4, int8 4 x [700,701]x[701,703]
+// 13.4 (20.8 before its ends were read in one piece, 13.4 before its rows were read from words), [64,512]x[512,512] 11.5 -> 4.8.
 #include <type_traits>
 
 #include "tmi_mfma.h"
@@ -30,6 +30,7 @@ struct RaggedArgs
     int64_t a_total, b_total;    // bytes of the whole operands
     int32_t H, C, W;
     int32_t za, zb;
+    int32_t odd;      // bit 0 / 1: rows of the first / second operand begin between words
     int32_t tiles;    // of all batches
     uint32_t per_xcd;    // workgroups / 8, rounded down
     FastDiv per_batch, tiles_w;
@@ -62,7 +63,8 @@ constexpr int ragged_wave_lds()
 
 // NC: column blocks of 32 in a tile.  TINY: an operand of less than 16 bytes, or a tile beyond 32-bit offsets: 64-bit ones, and pieces of less than
 // 16 bytes element by element
-template <typename T, int SPLIT, int NC, bool TINY>
+// ODD: rows of an operand begin between words
+template <typename T, int SPLIT, int NC, bool TINY, bool ODD>
 __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_kernel(RaggedArgs p)
 {
     using M             = Mma<T>;
@@ -80,7 +82,7 @@ __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_ke
 
     // The arguments at once.  (Left to the compiler they come where they are used, seven trips one after the other before the first load: int8
     // [249,64]x[64,96] 4.11 us, so 3.71.)
-    asm volatile("" : "+s"(p.a_total), "+s"(p.b_total), "+s"(p.H), "+s"(p.C), "+s"(p.W), "+s"(p.za), "+s"(p.zb), "+s"(p.tiles), "+s"(p.per_xcd)
+    asm volatile("" : "+s"(p.a_total), "+s"(p.b_total), "+s"(p.H), "+s"(p.C), "+s"(p.W), "+s"(p.za), "+s"(p.zb), "+s"(p.odd), "+s"(p.tiles), "+s"(p.per_xcd)
                  : "s"(p.a), "s"(p.b), "s"(p.out));
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r32 = lane & 31, half = lane >> 5;
@@ -119,7 +121,25 @@ __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_ke
         const int64_t to = at < total - 16 ? at : total - 16, room = total - 16 - to;
         return Place{ t + to, (uint32_t)(at - to), room < INT32_MAX ? (uint32_t)room : (uint32_t)INT32_MAX };
     };
+    // A 16-byte load from between words occupies the memory pipeline for two and a half times as long (64 lanes, two to a row: 246 clocks,
+    // 92 from a word on).  Such rows are read from the word before; what a lane then lacks is the next piece's first word, which another
+    // lane has, and for the last piece is loaded (112 clocks).  Where a row's pieces begin in a word does not change along K.
+    // us before / now: bf16 2 x [64,2265]x[2265,796] 15.4 / 10.2, 2 x [14,2529]x[2529,160] 11.0 / 6.8, 2 x [758,191]x[191,1668] 13.5 / 9.6, fp16
+    // 96 x [197,197]x[197,64] 7.4 / 6.2, int8 8 x [300,701]x[701,701] 15.0 / 12.2.  The second operand's rows, whose pieces lie side by side, gain
+    // where a wave has a tile to itself, in 16 bits (fp16 96 x [197,64]x[64,197] 8.9 / 8.2, 8 x [1500,64]x[64,2001] 28.0 / 23.9); not where K is shared
+    // (bf16 2 x [64,2272]x[2272,797] 8.7 / 9.3) nor in int8 (64 x [200,64]x[64,301] 7.7 / 8.0).
+    constexpr bool kRealignB = SPLIT == 1 && EB == 2;
+    const bool odd_a = ODD && (p.odd & 1), odd_b = ODD && kRealignB && (p.odd & 2), last_piece = (lane & (CPR - 1)) == CPR - 1;
+    const int shift_a = odd_a ? (int)((uintptr_t)(p.a + a_tile + a_lane) & 3) : 0, shift_b = odd_b ? (int)((uintptr_t)(p.b + b_tile + b_lane) & 3) : 0;
+    auto k_ends = [&](int k0) { return k0 + KB > p.C; };
+    auto b_ends = [&](int k0) { return k_ends(k0) || b_tile + (k0 + KB - 1) * pitch + RB > p.b_total; };
     v4i av[2], bv[NL];
+    int a_next = 0, b_next[NL] = {};    // the word behind a lane's last piece
+    auto words  = [&](const uint8_t* at) {
+        v4i v;
+        __builtin_memcpy(&v, __builtin_assume_aligned(at, 4), 16);
+        return v;
+    };
     auto request = [&](int share) {
         const int k0 = (first + share * SPLIT) * KB;
         if constexpr (TINY)
@@ -137,23 +157,64 @@ __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_ke
             return;
         }
         const Place pa = place(p.a, p.a_total, a_tile + k0 * EB), pb = place(p.b, p.b_total, b_tile + k0 * pitch);
-#pragma unroll
-        for (int j = 0; j < 2; j++)
+        if (odd_a && !k_ends(k0))
         {
-            const uint32_t off = a_lane + pa.extra + 32 * j;
-            av[j]           = load16(pa.base + (off < pa.most ? off : pa.most));
+            const uint8_t* at = pa.base + a_lane - shift_a;
+            av[0] = words(at), av[1] = words(at + 32);
+            if (half)
+                a_next = *reinterpret_cast<const int*>(at + 32 + (shift_a ? 16 : 12));    // (a word of the row either way)
         }
+        else
 #pragma unroll
-        for (int j = 0; j < NL; j++)
+            for (int j = 0; j < 2; j++)
+            {
+                const uint32_t off = a_lane + pa.extra + 32 * j;
+                av[j]           = load16(pa.base + (off < pa.most ? off : pa.most));
+            }
+        if (odd_b && !b_ends(k0))
         {
-            const uint32_t off = b_lane + pb.extra + j * (64 / CPR) * (uint32_t)pitch;
-            bv[j]           = load16(pb.base + (off < pb.most ? off : pb.most));
+#pragma unroll
+            for (int j = 0; j < NL; j++)
+            {
+                const uint8_t* at = pb.base + b_lane - shift_b + j * (64 / CPR) * (uint32_t)pitch;
+                bv[j]             = words(at);
+                if (last_piece)
+                    b_next[j] = *reinterpret_cast<const int*>(at + (shift_b ? 16 : 12));
+            }
         }
+        else
+#pragma unroll
+            for (int j = 0; j < NL; j++)
+            {
+                const uint32_t off = b_lane + pb.extra + j * (64 / CPR) * (uint32_t)pitch;
+                bv[j]           = load16(pb.base + (off < pb.most ? off : pb.most));
+            }
+    };
+    auto shifted = [&](v4i v, int next, int by) {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            v[k] = (int)__builtin_amdgcn_alignbyte((uint32_t)(k < 3 ? v[k < 3 ? k + 1 : 3] : next), (uint32_t)v[k], by);
+        return v;
     };
     auto finish = [&](int share) {
         int k0 = (first + share * SPLIT) * KB;
         asm volatile("" : "+s"(k0));    // (worked out again rather than kept from request())
-        const bool k_tail = k0 + KB > p.C;
+        const bool k_tail = k_ends(k0);
+        if (odd_a && !k_tail)
+        {
+            // pieces in K order: lower half's first, upper half's first, lower half's second, upper half's second
+            const auto first_words = __builtin_amdgcn_permlane32_swap((uint32_t)av[0][0], (uint32_t)av[1][0], false, false);
+            const auto upper_words = __builtin_amdgcn_permlane32_swap((uint32_t)av[1][0], (uint32_t)av[1][0], false, false);
+            av[0] = shifted(av[0], (int)(half ? first_words[0] : first_words[1]), shift_a);
+            av[1] = shifted(av[1], half ? a_next : (int)upper_words[1], shift_a);
+        }
+        if (odd_b && !b_ends(k0))
+#pragma unroll
+            for (int j = 0; j < NL; j++)
+            {
+                const int right = __builtin_amdgcn_update_dpp(0, bv[j][0], 0x101, 0xf, 0xf, true);    // (the lane to the right; pieces of a row are 2, 4 or 8 lanes)
+                bv[j]           = shifted(bv[j], last_piece ? b_next[j] : right, shift_b);
+            }
         if (k_tail)
         {
             const Place pa = place(p.a, p.a_total, a_tile + k0 * EB);
@@ -166,7 +227,7 @@ __global__ __launch_bounds__(SPLIT > 4 ? 64 * SPLIT : 256) void matmul_ragged_ke
                 av[j] = keep_bytes(av[j], row_bytes - k0 * EB - 16 * half - 32 * j);
             }
         }
-        if (k_tail || b_tile + (k0 + KB - 1) * pitch + RB > p.b_total)
+        if (b_ends(k0))
         {
             const Place pb = place(p.b, p.b_total, b_tile + k0 * pitch);
 #pragma unroll
@@ -369,12 +430,12 @@ bool launch_matmul_pad(hipStream_t st, int32_t eb, int32_t N, int32_t H, int32_t
     return true;
 }
 
-template <typename T, int SPLIT, int NC, bool TINY>
+template <typename T, int SPLIT, int NC, bool TINY, bool ODD>
 static bool launch_split_form(hipStream_t st, RaggedArgs& p)
 {
     constexpr int kWaves       = SPLIT > 4 ? SPLIT : 4;
     constexpr size_t lds_bytes = (size_t)kWaves * ragged_wave_lds<T, SPLIT, NC>();
-    constexpr auto kern        = matmul_ragged_kernel<T, SPLIT, NC, TINY>;
+    constexpr auto kern        = matmul_ragged_kernel<T, SPLIT, NC, TINY, ODD>;
     if (lds_bytes > 65536 && !ensure_dynamic_lds<kern>(lds_bytes))
         return false;
     const int64_t grid = ((int64_t)p.tiles * SPLIT + kWaves - 1) / kWaves;
@@ -390,7 +451,9 @@ static bool launch_split(hipStream_t st, RaggedArgs& p)
     // (rows beyond 32-bit offsets, us with every piece element by element / now: int8 [1,66000001]x[66000001,1] 415800 / 72300, fp16
     // [1,33000001]x[33000001,1] 265000 / 48600)
     const bool tiny = p.a_total < 16 || p.b_total < 16 || (int64_t)p.C * EB > INT32_MAX / 33 || (int64_t)p.W * EB > INT32_MAX / 65;
-    return tiny ? launch_split_form<T, SPLIT, NC, true>(st, p) : launch_split_form<T, SPLIT, NC, false>(st, p);
+    if (tiny)
+        return launch_split_form<T, SPLIT, NC, true, false>(st, p);
+    return p.odd & (SPLIT == 1 && EB == 2 ? 3 : 1) ? launch_split_form<T, SPLIT, NC, false, true>(st, p) : launch_split_form<T, SPLIT, NC, false, false>(st, p);
 }
 
 template <typename T>
@@ -437,7 +500,7 @@ const char* launch_matmul_ragged(hipStream_t st, int32_t in_dtype, int32_t N, in
     RaggedArgs p{};
     p.a = (const uint8_t*)a, p.b = (const uint8_t*)b, p.out = (uint8_t*)out;
     p.a_total = (int64_t)N * H * C * eb, p.b_total = (int64_t)N * C * W * eb;
-    p.H = H, p.C = C, p.W = W, p.za = a_zp, p.zb = b_zp, p.tiles = (int32_t)tiles;
+    p.H = H, p.C = C, p.W = W, p.za = a_zp, p.zb = b_zp, p.odd = ((C * eb | (int)((uintptr_t)a & 3)) % 4 ? 1 : 0) | ((W * eb | (int)((uintptr_t)b & 3)) % 4 ? 2 : 0), p.tiles = (int32_t)tiles;
     p.per_batch = make_fastdiv((uint32_t)per), p.tiles_w = make_fastdiv((uint32_t)tw);
     switch (in_dtype)
     {
