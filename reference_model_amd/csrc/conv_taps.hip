@@ -17,6 +17,9 @@
 // [19,84,89,16]->108 3x3 63 / 22, [5,106,106,16]->232 3x3 stride 2 18.7 / 7.1, fp16 [15,54,65,68]->64 28.2 / 7.6.  Whole groups of
 // steps run without a test (a test and a branch a step: 4 ... 7 % slower over 257 layers).
 //
+// Channel vectors that begin between words (more than 32 bytes of them) are read from the word before and shifted where they are used: int8
+// [60,32,32,163]->16 1x1 8.0, with the copies such rows went through before 15.5; K split, [2,11,16,285]->44 5x5 34.4 -> 25.8, bf16 [1,45,9,219]->24 19.7 -> 13.2.
+//
 // The second kernel, for few tiles and a long reduction, splits K over the waves of a workgroup (see there).
 #include <type_traits>
 
@@ -300,9 +303,18 @@ __device__ __forceinline__ void sum_again(const TapsArgs& a, int p, int oc, int 
     }
 }
 
-template <typename T, int OCT, bool RAGGED>
+// How channel vectors lie: whole chunks from 16 bytes on; anywhere, beginning with words; anywhere.
+enum TapsRows
+{
+    kTapsWhole,
+    kTapsWords,
+    kTapsOdd
+};
+
+template <typename T, int OCT, int ROWS>
 __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs a)
 {
+    constexpr bool RAGGED = ROWS != kTapsWhole;
     using M             = Mma<T>;
     using acc_t         = typename M::acc_t;
     constexpr int NT    = kTapsWaves * 64;
@@ -437,29 +449,69 @@ __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs 
         if constexpr (RAGGED)
             edge = __any(pix_off > a.edge_off);
     };
+    // A 16-byte load from between words takes the memory pipeline more than twice as long as one from a word on: such chunks are read from the word
+    // before, with the word behind, and shifted where they are used.  So are they cut there to their channels: here a lane would wait for
+    // its load.
+    constexpr bool ODD = ROWS == kTapsOdd, CUT = RAGGED && !M::is_int;
     v4i fb[DEPTH];
+    int behind[ODD ? DEPTH : 1] = {};
+    uint32_t places = 0;    // where in a word each load's chunk begins, two bits each; from bit 16 on: whether it is a tap's last
+    auto note        = [&](int d, uint32_t place, int bits) {
+        if constexpr (ODD)
+            places = (places & ~(3u << (2 * d))) | place << (2 * d);
+        if constexpr (CUT)
+            places = (places & ~(65536u << d)) | (bits & kTapsPartial ? 65536u << d : 0u);
+    };
     auto load_pixels = [&](int d, v2i e, bool careful) {
         const bool inside  = (e.y & pix_miss) == 0;
         const int off      = pix_off + e.x;
         const uint8_t* src = inside ? a.in + (uint32_t)off : a.pad_page;
         if constexpr (!RAGGED)
             fb[d] = *reinterpret_cast<const v4i*>(src);
-        else
+        else if (careful)
         {
-            if (careful)
-            {
-                const int past = inside && off > a.last ? off - a.last : 0;
-                if (__any(past))
-                    fb[d] = drop_bytes(load16(src - past), past);
-                else
-                    fb[d] = load16(src);
-            }
+            const int past = inside && off > a.last ? off - a.last : 0;
+            if (__any(past))
+                fb[d] = drop_bytes(load16(src - past), past);
             else
                 fb[d] = load16(src);
-            if constexpr (!M::is_int)
-                if (e.y & kTapsPartial)
-                    fb[d] = keep_bytes(fb[d], partial);
+            note(d, 0, e.y);
         }
+        else if constexpr (ODD)
+        {
+            const uint8_t* word = reinterpret_cast<const uint8_t*>((uintptr_t)src & ~(uintptr_t)3);
+            __builtin_memcpy(&fb[d], __builtin_assume_aligned(word, 4), 16);
+            behind[d] = *reinterpret_cast<const int*>(word + 16);
+            note(d, (uint32_t)(uintptr_t)src & 3u, e.y);
+        }
+        else
+        {
+            fb[d] = load16(src);
+            note(d, 0, e.y);
+        }
+    };
+    auto pixels = [&](int d) {
+        v4i v = fb[d];
+        if constexpr (ODD)
+        {
+            const uint32_t by = places >> (2 * d) & 3u;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                v[k] = (int)__builtin_amdgcn_alignbyte((uint32_t)(k < 3 ? fb[d][k < 3 ? k + 1 : 3] : behind[d]), (uint32_t)fb[d][k], by);
+        }
+        if constexpr (CUT)
+            if (__any(places & (65536u << d)))
+            {
+                const int n = places & (65536u << d) ? partial : 16;
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                {
+                    // (channels are 16 bits: whole words, half of one, none)
+                    const int m = n - 4 * k;
+                    v[k]        = m >= 4 ? v[k] : (m == 2 ? v[k] & 0xffff : 0);
+                }
+            }
+        return v;
     };
     auto load_group = [&](bool careful) {
 #pragma unroll
@@ -541,9 +593,10 @@ __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs 
 #pragma unroll
                 for (int t = 0; t < OCT; t++)
                     fa[(d + 1) & 1][t] = *reinterpret_cast<const v4i*>(wf + (d + 1) * 2 * PITCH + t * 512);
+                const v4i px = pixels(d);
 #pragma unroll
                 for (int t = 0; t < OCT; t++)
-                    acc[t] = M::mma(fa[d & 1][t], fb[d], acc[t]);
+                    acc[t] = M::mma(fa[d & 1][t], px, acc[t]);
                 load_pixels(d, next[d], false);
             }
         }
@@ -560,9 +613,10 @@ __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs 
                 if (s0 + d >= a.steps)
                     break;
                 load_weight_fragments(s0 + d + 1, fa[(d + 1) & 1]);
+                const v4i px = pixels(d);
 #pragma unroll
                 for (int t = 0; t < OCT; t++)
-                    acc[t] = M::mma(fa[d & 1][t], fb[d], acc[t]);
+                    acc[t] = M::mma(fa[d & 1][t], px, acc[t]);
                 if (s0 + DEPTH + d < a.steps)
                     load_pixels(d, next[d], edge);
             }
@@ -620,13 +674,14 @@ __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs 
 // [9,31,41,240]->32 3x3 stride 2 28.9 / 8.2; with the weights staged in LDS first, as above, [2,79,7,88]->23 bf16 3x3 6.3 / 4.6.
 constexpr int kTapsShare = 8;
 
-template <typename T, int NW, bool RAGGED>
+template <typename T, int NW, int ROWS>
 __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_kernel(TapsArgs a)
 {
+    constexpr bool RAGGED = ROWS != kTapsWhole, ODD = ROWS == kTapsOdd;
     using M           = Mma<T>;
     using acc_t       = typename M::acc_t;
     using v4          = std::conditional_t<M::is_int, v4i, v4f>;
-    constexpr int KSW = kTapsShare;
+    constexpr int KSW = ODD ? 6 : kTapsShare;    // (what the registers of two workgroups hold)
     __shared__ __attribute__((aligned(16))) v4 red[NW][4][64];
     __shared__ __attribute__((aligned(16))) HighWordScale tab_hw[32];
     __shared__ __attribute__((aligned(16))) v2i tab_ms[32];
@@ -702,6 +757,22 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_ker
     const int wr  = 4 * (li & 4) + ((li >> 1) & 12) + (li & 3);    // the channel of operand row li
     const int w_row = (oc0 + wr < a.OC ? oc0 + wr : a.OC - 1) * (a.KH * a.KW) * a.row_bytes;    // (rows past the end are never stored)
     v4i fa[KSW], fb[KSW];
+    int fa_behind[ODD ? KSW : 1] = {}, fb_behind[ODD ? KSW : 1] = {};    // the words behind chunks that begin between words (see above)
+    uint32_t fa_places = 0, fb_places = 0;
+    auto load_words = [&](int d, const uint8_t* src, v4i& v, int& behind, uint32_t& places) {
+        const uint32_t place = (uint32_t)(uintptr_t)src & 3u;
+        const uint8_t* word  = reinterpret_cast<const uint8_t*>((uintptr_t)src & ~(uintptr_t)3);
+        __builtin_memcpy(&v, __builtin_assume_aligned(word, 4), 16);
+        behind = *reinterpret_cast<const int*>(word + (place ? 16 : 12));    // (never a word past the tensor)
+        places |= place << (2 * d);
+    };
+    auto shifted = [&](int d, v4i v, int behind, uint32_t places) {
+        const uint32_t by = places >> (2 * d) & 3u;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            v[k] = (int)__builtin_amdgcn_alignbyte((uint32_t)(k < 3 ? v[k < 3 ? k + 1 : 3] : behind), (uint32_t)v[k], by);
+        return v;
+    };
     auto load_pixels = [&](int d, const Chunk& q) {
         const bool inside  = q.index < a.chunks && (q.bits & pix_miss) == 0;
         const int off      = pix_off + q.off;
@@ -718,6 +789,8 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_ker
                 else
                     fb[d] = load16(src);
             }
+            else if constexpr (ODD)
+                load_words(d, src, fb[d], fb_behind[d], fb_places);
             else
                 fb[d] = load16(src);
         }
@@ -729,13 +802,24 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_ker
         else
         {
             const int at = off <= a.w_last ? off : a.w_last;
-            fa[d]        = load16(a.w + (uint32_t)at);
-            if (__any(off > a.w_last))
-                fa[d] = drop_bytes(fa[d], off - at);
+            if (ODD && !__any(off > a.w_last))
+                load_words(d, a.w + (uint32_t)at, fa[d], fa_behind[ODD ? d : 0], fa_places);
+            else
+            {
+                fa[d] = load16(a.w + (uint32_t)at);
+                if (__any(off > a.w_last))
+                    fa[d] = drop_bytes(fa[d], off - at);
+            }
         }
     };
     // what lies behind a channel vector counts for nothing, nor does the dead half of an odd count's last step
     auto trim = [&](int d, const Chunk& q, bool weights) {
+        if constexpr (ODD)
+        {
+            fb[d] = shifted(d, fb[d], fb_behind[d], fb_places);
+            if (weights)
+                fa[d] = shifted(d, fa[d], fa_behind[d], fa_places);
+        }
         if (RAGGED && partial && q.piece == a.pieces - 1)
         {
             if (weights)
@@ -795,7 +879,10 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_ker
         const bool weights = !keep || !have_start;
         for (int s0 = s_begin; s0 < s_end; s0 += KSW)
         {
-            Chunk qd = q;
+            Chunk qd  = q;
+            fb_places = 0;
+            if (weights)
+                fa_places = 0;
 #pragma unroll
             for (int d = 0; d < KSW; d++)
                 if (s0 + d < s_end)
@@ -891,13 +978,13 @@ static bool taps_grid(TapsArgs& a, int oct, int64_t wanted, int resident, unsign
     return all <= (1 << 24) && fastdiv_exact_up_to((uint64_t)all, (uint32_t)a.groups);
 }
 
-template <typename T, int OCT, bool RAGGED>
+template <typename T, int OCT, int ROWS>
 static bool launch_taps(hipStream_t st, TapsArgs& a)
 {
     // results whose rows are no whole words and all of one workgroup
     a.rows_bytes           = (a.OC & 3) && a.OC <= 32 * OCT && a.out_kind != 0 ? 32 * a.OC * (a.out_kind == 1 ? 1 : 2) : 0;
     const size_t lds_bytes = (size_t)taps_lds_bytes<OCT>(a.steps) + kTapsWaves * a.rows_bytes;
-    constexpr auto kern    = conv_taps_kernel<T, OCT, RAGGED>;
+    constexpr auto kern    = conv_taps_kernel<T, OCT, ROWS>;
     unsigned grid;
     if (!ensure_dynamic_lds<kern>(lds_bytes) ||
         !taps_grid(a, OCT, (a.n_pt + kTapsWaves - 1) / kTapsWaves, lds_bytes > 80 * 1024 ? 1 : (lds_bytes > 53 * 1024 ? 2 : 3), grid))
@@ -906,13 +993,13 @@ static bool launch_taps(hipStream_t st, TapsArgs& a)
     return true;
 }
 
-template <typename T, int NW, bool RAGGED>
+template <typename T, int NW, int ROWS>
 static bool launch_taps_split(hipStream_t st, TapsArgs& a)
 {
     unsigned grid;
     if (!taps_grid(a, 1, a.n_pt, NW == 4 ? 3 : (NW == 8 ? 2 : 1), grid))
         return false;
-    hipLaunchKernelGGL((conv_taps_split_kernel<T, NW, RAGGED>), dim3(grid), dim3(NW * 64), 0, st, a);
+    hipLaunchKernelGGL((conv_taps_split_kernel<T, NW, ROWS>), dim3(grid), dim3(NW * 64), 0, st, a);
     return true;
 }
 
@@ -973,9 +1060,14 @@ template <typename T>
 static bool launch_taps_t(hipStream_t st, TapsArgs& a, bool ragged)
 {
     const TapsForm form = taps_form(a.n_pt, a.OC, a.steps, !ragged ? 0 : (a.row_bytes % 4 == 0 ? 1 : 2));
+    // (up to 32 bytes a pixel, neighbouring pixels share lines and the other loads are no slower: [20,136,133,13]->488 3x3 stride 2 52.0 / 38.3,
+    // [5,14,14,30]->16 5x5 6.6 / 6.0)
+    const bool odd = a.row_bytes > 32 && (a.row_bytes % 4 != 0 || (((uintptr_t)a.in | (uintptr_t)a.w) & 3));
+    if (odd)
+        a.edge_off -= 4;    // (the word behind)
 #define TMI_TAPS(O)                                                                                                   \
     if (!form.split && form.oct == O)                                                                                 \
-        return ragged ? launch_taps<T, O, true>(st, a) : launch_taps<T, O, false>(st, a);
+        return !ragged ? launch_taps<T, O, kTapsWhole>(st, a) : (odd ? launch_taps<T, O, kTapsOdd>(st, a) : launch_taps<T, O, kTapsWords>(st, a));
     TMI_TAPS(1)
     TMI_TAPS(2)
     TMI_TAPS(3)
@@ -983,7 +1075,7 @@ static bool launch_taps_t(hipStream_t st, TapsArgs& a, bool ragged)
 #undef TMI_TAPS
 #define TMI_TAPS(NW)                                                                                                  \
     if (form.split == NW)                                                                                             \
-        return ragged ? launch_taps_split<T, NW, true>(st, a) : launch_taps_split<T, NW, false>(st, a);
+        return !ragged ? launch_taps_split<T, NW, kTapsWhole>(st, a) : (odd ? launch_taps_split<T, NW, kTapsOdd>(st, a) : launch_taps_split<T, NW, kTapsWords>(st, a));
     TMI_TAPS(4)
     TMI_TAPS(8)
     TMI_TAPS(16)

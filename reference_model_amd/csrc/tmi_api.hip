@@ -667,17 +667,39 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // 8.1, with 16-bit multipliers 17.1 / 14.6; the other way [2,35,35,45]->8 3x3 9.9 / 13.0).
         if (padded && t_row % 4 == 0 && ((((uintptr_t)out) & 15) || (rp.enabled && !rp.fast)))
             padded = 0;
-        // What would be padded and is small: one launch of the kernel that needs no whole steps.  us padded / this: int8 3x3 [18,21,21,48]->16
-        // 9.2 / 4.0, [2,35,35,45]->8 6.3 / 4.7, [2,34,31,272]->480 stride 2 11.1 / 7.7, [7,24,24,112]->160 stride 2 10.6 / 4.7; fp16 1x1
-        // [5,8,11,69]->440 8.1 / 3.6.  From 36 steps on, odd rows (loads that start between words, at a quarter of the rate) are
-        // padded first: bf16 [1,45,9,219]->23 18.9 / 11, int8 [2,11,16,285]->42 5x5 34 / 18.
-        // A few tiles: [1,6,9,48]->16 int32 6.0 / 3.5, 1x1 [1,8,11,34]->32 int32 6.0 / 3.6, 5x5 [1,17,5,112]->24 stride 2 9.1 / 5.5, [2,12,12,73]->48 6.6 / 6.1.
-        // More tiles than it has workgroups at once, 1x1 with the fused RESCALE: the pointwise kernel on copies.  us copies / this: [42,9,5,19]->416 (780
-        // tiles) 5.4 / 6.2, [15,13,8,26]->568 5.7 / 6.5, [2,39,45,95]->272 6.0 / 6.9; the other way [1,49,40,27]->360 (744) 5.6 / 4.9, [43,28,30,70]->16 7.5 /
-        // 6.1, even int32 results.
-        const bool pointwise_copies = rp.enabled && g.KH * g.KW == 1 && g.stride_y * g.stride_x == 1 && g.OC % 8 == 0 && g.OC > 32 && t_row % 4 != 0 &&
-                                      t_row <= 96 && t_tiles > 768;
-        if (padded && t_tiles * t_steps <= (t_row % 16 == 0 ? 24000 : 6000) && !(t_row % 4 != 0 && t_steps >= 36) && !pointwise_copies && taps_open())
+        // What would be padded and is small, or loses little to loads that begin anywhere: one launch of the kernel that needs no whole steps.  us
+        // padded / this: int8 3x3 [18,21,21,48]->16 9.2 / 4.0, [2,35,35,45]->8 6.3 / 4.7, [2,34,31,272]->480 stride 2 11.1 / 7.7, [7,24,24,112]->160 stride 2
+        // 10.6 / 4.7; fp16 1x1 [5,8,11,69]->440 8.1 / 3.6.  A few tiles: [1,6,9,48]->16 int32 6.0 / 3.5, 1x1 [1,8,11,34]->32 int32 6.0 / 3.6, 5x5 [1,17,5,112]->24
+        // stride 2 9.1 / 5.5, [2,12,12,73]->48 6.6 / 6.1.  Over 220 drawn layers of ragged rows:
+        //   1x1, an image that is read once: int8 [43,84,89,127]->96 47.1 / 24.7, [60,32,32,163]->16 15.5 / 8.0, [31,22,27,637]->24 15.1 / 8.7,
+        //     [5,89,86,495]->304 (11 960 tiles, 16 steps) 38.7 / 33.0, bf16 [12,100,73,39]->40 14.1 / 8.8, [15,23,39,75]->248 (3368, 5) 11.7 / 9.1; the other
+        //     way fp16 [8,27,53,277]->152 (1790, 18) 11.7 / 12.9.
+        //   rows of whole words: bf16 [10,88,14,242]->9 3x3 27.8 / 13.1, [6,25,67,122]->40 (630 tiles, 72 steps) 19.9 / 16.2, int8 [43,23,28,72]->16 14.9 / 8.5; the
+        //     other way [8,111,22,106]->36 (1222, 63) 20.1 / 21.6, [16,10,10,532]->160 (250, 153) 13.0 / 13.9.
+        //   rows between words, up to 3x3 and two chunks a tap: int8 [3,89,89,25]->96 13.6 / 9.7, [2,130,130,29]->240 stride 2 14.4 / 9.9; the other way [49,60,57,21]->384
+        //     (63 000 tiles) 51.9 / 70.8; up to 18 steps of few channels: [6,159,156,17]->16 16.3 / 12.7, [2,134,139,41]->26 11.5 / 9.0, [10,91,96,55]->40 stride 2 14.5 / 11.4, fp16 [14,83,23,17]->72 9.7 / 6.3; the other way int8
+        //     [30,21,26,66]->240 stride 2 9.3 / 12.3, [16,33,30,81]->96 10.0 / 15.3, [45,99,96,93]->16 (27 steps) 45.1 / 51.6, fp16 [2,55,89,41]->48 (27 steps) 6.4 / 8.7.  Longer ones, and larger
+        //     windows, are padded from 36 steps on: bf16 [1,45,9,219]->23 13.2 / 10.7 as they lie / padded, int8 [2,11,16,285]->42 5x5 25.8 / 19.1.
+        // More tiles than it has workgroups at once of many channels, 1x1 with the fused RESCALE: the pointwise kernel on copies.  us copies / this:
+        //   [42,9,5,19]->416 (780 tiles) 5.4 / 6.2, [26,40,40,54]->376 16.7 / 19.7, [16,50,47,29]->128 7.2 / 9.1, [63,21,21,62]->208 9.8 / 11.3; the other way
+        //   [1,49,40,27]->360 (744) 5.6 / 4.9, [10,53,50,79]->218 29.4 / 25.9, [17,122,122,75]->40 21.0 / 15.4, even int32 results.
+        const int64_t t_all         = t_tiles * t_steps;
+        const bool pointwise_copies = rp.enabled && g.KH * g.KW == 1 && g.stride_y * g.stride_x == 1 && g.OC % 8 == 0 && t_row % 4 != 0 && t_tiles > 768 &&
+                                      t_row <= 96 && g.OC > (t_row <= 64 ? 32 : 128);
+        auto as_they_lie = [&]() {
+            if (t_row % 16 == 0)
+                return t_all <= 24000;
+            if (t_all <= 6000)
+                return g.KH * g.KW == 1 ? !pointwise_copies : t_row % 4 == 0 || t_steps < 36;
+            if (g.OC % 4 != 0 && g.OC > 128)    // (results of no whole words that no workgroup has whole rows of: 1x1 [1,69,69,167]->607 13.6 / 17.6)
+                return false;
+            if (g.KH * g.KW == 1)
+                return t_all > 6500 && t_all <= (g.OC > 64 && d->in_dtype != TMI_INT8 ? 17000 : 200000) && !pointwise_copies;
+            if (t_row % 4 == 0)
+                return t_all <= (g.OC <= 64 ? 55000 : 8000);
+            return t_all > 6500 && g.KH * g.KW <= 9 && (g.OC <= 64 ? t_steps <= 18 : t_steps <= 9 && t_all <= 60000);
+        };    // (what lies between 6000 and 6500 keeps its copies, whose tests are there: 0.8 ... 1.05 of the time either way)
+        if (padded && as_they_lie() && taps_open())
             padded = 0, name = launch_taps();
         if (name)
             return after_launch(ctx, name);
