@@ -213,6 +213,111 @@ static const char* launch_rescale_fast(hipStream_t st, const RescaleParams& p, c
     return "rescale_fast";
 }
 
+// RESCALE of INT48 (16-bit multipliers, SINGLE rounding: what follows an INT16 convolution) in the manner of the kernel above: a lane owns four
+// channels, its constants in registers, and walks down the rows with four units of two 16-byte loads in flight.  Left to the general kernel,
+// which divides 64-bit indices by C and fetches every element's multiplier and shift, [8,56,56,64] -> INT16 (16 MB) took 5.5 us, [8,112,112,64] 15.8; here 4.4 (3.6 TB/s, the copy's rate and the
+// launch) and 12.9.  (First rows requested before the constants: 4.8.)
+template <typename OutT, bool NEG>
+__device__ __forceinline__ void rescale_i48_walk(const RescaleParams& p, const int32_t (&mul)[4], const int32_t (&sh)[4], const int64_t* __restrict__ in,
+                                                 OutT* __restrict__ out, int64_t rows, int32_t C, int32_t rpi, int slot, int c0, bool lane_on, uint32_t& flags,
+                                                 int32_t blocks)
+{
+    constexpr int U    = 4;
+    const int64_t step = (int64_t)blocks * rpi;    // rows between two units of a workgroup
+    int64_t r          = (int64_t)blockIdx.x * rpi + slot;
+    rs_v4i v[U][2];
+    auto load = [&](int u, int64_t row) {
+        const rs_v4i* from = reinterpret_cast<const rs_v4i*>(in + (lane_on && row < rows ? row * C + c0 : 0));
+        v[u][0] = from[0], v[u][1] = from[1];
+    };
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        load(u, r + u * step);
+    for (int64_t base = (int64_t)blockIdx.x * rpi; base < rows; base += U * step, r += U * step)
+    {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+        {
+            const int64_t ru = r + u * step;
+            int32_t res[4];
+            uint32_t met = 0;
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+            {
+                const uint32_t lo = (uint32_t)v[u][c >> 1][2 * (c & 1)];
+                uint32_t hi       = (uint32_t)v[u][c >> 1][2 * (c & 1) + 1];
+                hi |= (uint32_t)((int32_t)(hi << 16) >> 31) & 0xffff0000u;    // value_extend()
+                const uint64_t stored = (uint64_t)hi << 32 | lo, round = uint64_t(1) << (sh[c] - 1);
+                const int64_t scaled  = (int64_t)(stored * (NEG ? (uint64_t)(int64_t)mul[c] : (uint64_t)(uint32_t)mul[c]) + round) >> sh[c];
+                int32_t o             = (int32_t)scaled;
+                met |= o != scaled ? TMI_FLAG_SCALE_RESULT : 0;
+                met |= __builtin_sadd_overflow(o, p.out_zp, &o) ? TMI_FLAG_ZP_RESULT : 0;
+                o      = o < p.qmin ? p.qmin : o;
+                res[c] = o > p.qmax ? p.qmax : o;
+            }
+            load(u, ru + U * step);
+            if (lane_on && ru < rows)
+            {
+                flags |= met;
+                OutT* q = out + ru * C + c0;
+                if constexpr (sizeof(OutT) == 1)
+                    *reinterpret_cast<int*>(q) = (res[0] & 0xff) | ((res[1] & 0xff) << 8) | ((res[2] & 0xff) << 16) | ((res[3] & 0xff) << 24);
+                else if constexpr (sizeof(OutT) == 2)
+                    *reinterpret_cast<int2*>(q) = int2{ (res[0] & 0xffff) | (res[1] << 16), (res[2] & 0xffff) | (res[3] << 16) };
+                else
+                    *reinterpret_cast<rs_v4i*>(q) = rs_v4i{ res[0], res[1], res[2], res[3] };
+            }
+        }
+    }
+}
+
+template <typename OutT>
+__global__ __launch_bounds__(256) void rescale_i48_kernel(RescaleParams p, const int64_t* __restrict__ in, OutT* __restrict__ out, int64_t rows, int32_t C,
+                                                          int32_t cgs, int32_t rpi, FastDiv div_cgs, uint32_t* flag_word, int32_t blocks)
+{
+    const int tid      = threadIdx.x;
+    const int slot     = fdiv(tid, div_cgs);    // row slot of this lane inside a unit
+    const bool lane_on = slot < rpi;
+    const int c0       = lane_on ? (tid - slot * cgs) * 4 : 0;
+    uint32_t flags     = 0;
+    int32_t mul[4], sh[4];
+    bool negative = false;
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+    {
+        mul[c] = load_multiplier(p, c0 + c), sh[c] = load_shift(p, c0 + c);
+        if (lane_on && mul[c] < 0)
+            flags |= TMI_FLAG_SCALE_MULTIPLIER, negative = true;
+        if (lane_on && (sh[c] < 2 || sh[c] > 62))
+            flags |= TMI_FLAG_SCALE_SHIFT;
+    }
+    const bool illegal = flags & TMI_FLAG_SCALE_SHIFT;
+    if (__any(illegal))
+    {
+        // (apply_scale_16() returns 0 under such a shift)
+        for (int64_t r = (int64_t)blockIdx.x * rpi + slot; lane_on && r < rows; r += (int64_t)blocks * rpi)
+            for (int c = 0; c < 4; c++)
+                out[r * C + c0 + c] = (OutT)rescale_value<false>(p, in[r * C + c0 + c], load_multiplier(p, c0 + c), load_shift(p, c0 + c), flags);
+    }
+    else if (__any(negative))
+        rescale_i48_walk<OutT, true>(p, mul, sh, in, out, rows, C, rpi, slot, c0, lane_on, flags, blocks);
+    else
+        rescale_i48_walk<OutT, false>(p, mul, sh, in, out, rows, C, rpi, slot, c0, lane_on, flags, blocks);
+    raise_flags(flag_word, flags);
+}
+
+template <typename OutT>
+static const char* launch_rescale_i48(hipStream_t st, const RescaleParams& p, const void* in, void* out, int64_t n, int32_t C, uint32_t* flag_word)
+{
+    const int32_t cgs = C / 4, rpi = 256 / cgs;
+    const int64_t rows = n / C, units = (rows + rpi - 1) / rpi;
+    // as above: two workgroups per CU, equal shares
+    const int64_t visits = (units + 256 * 2 - 1) / (256 * 2), blocks = (units + visits - 1) / visits;
+    hipLaunchKernelGGL((rescale_i48_kernel<OutT>), dim3((unsigned)blocks), dim3(256), 0, st, p, (const int64_t*)in, (OutT*)out, rows, C, cgs, rpi,
+                       make_fastdiv(cgs), flag_word, (int32_t)blocks);
+    return "rescale_vec";
+}
+
 static int grid_for(int64_t work_items)
 {
     // 256 CUs x 8 blocks of 256 lanes keep every SIMD busy; beyond that the loop strides.
@@ -235,7 +340,9 @@ static const char* launch_rescale_t(hipStream_t st, const RescaleParams& p, cons
     if (n == 0)
         return "rescale_empty";
     const bool precise = p.inexact_round >= 2;
-    if (aligned && C % VEC == 0)
+    // (INT48 up to a few waves a SIMD: one element a lane has the shorter chain, us four a lane / one: 12 800 elements 3.2 / 2.4, 100 000 3.2 / 2.5,
+    // 226 000 3.3 / 2.8, 1 M 4.4 / 4.5)
+    if (aligned && C % VEC == 0 && !(sizeof(InT) == 8 && !precise && n <= 300000))
     {
         const int64_t n_vec = n / VEC;
         if (precise)
@@ -269,6 +376,16 @@ const char* launch_rescale(hipStream_t st, const RescaleParams& p, int32_t in_dt
             return launch_rescale_fast<int16_t>(st, p, in, out, n, C, flag_word);
         if (out_dtype == TMI_INT32)
             return launch_rescale_fast<int32_t>(st, p, in, out, n, C, flag_word);
+    }
+    if (in_dtype == TMI_INT48 && !p.scale32 && p.inexact_round == 0 && p.in_zp == 0 && p.in_bits == 48 && !p.has_clamp && n > 300000 && C >= 4 && (C & 3) == 0 &&
+        C <= 1024 && (((uintptr_t)in | (uintptr_t)out) & 15) == 0)
+    {
+        if (out_dtype == TMI_INT8)
+            return launch_rescale_i48<int8_t>(st, p, in, out, n, C, flag_word);
+        if (out_dtype == TMI_INT16)
+            return launch_rescale_i48<int16_t>(st, p, in, out, n, C, flag_word);
+        if (out_dtype == TMI_INT32)
+            return launch_rescale_i48<int32_t>(st, p, in, out, n, C, flag_word);
     }
 #define TMI_RESCALE_CASE(ID, IT, OD, OT)                                                                            \
     if (in_dtype == ID && out_dtype == OD)                                                                          \
