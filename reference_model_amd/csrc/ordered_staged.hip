@@ -88,7 +88,7 @@ __device__ __forceinline__ void staged_tile(const StagedArgs& p, int m0, int n0,
     uint32_t at = (uint32_t)((image + y * IW + x) * gp + chunk) * (uint32_t)UB, from = OUTSIDE;
     const uint32_t tap_skip = second ? 0u : p.tap_skip, row_skip = second ? 0u : p.row_skip;    // behind a tap's units
     auto enter = [&]() {
-        from = row_there & (ky < KH) & ((uint32_t)y < (uint32_t)IH) & ((uint32_t)x < (uint32_t)IW) ? at : OUTSIDE;
+        from = (row_there & (ky < KH) & ((uint32_t)y < (uint32_t)IH) & ((uint32_t)x < (uint32_t)IW)) ? at : OUTSIDE;
     };
     auto next_tap = [&]() {
         x += p.dil_x, at += tap_skip;
