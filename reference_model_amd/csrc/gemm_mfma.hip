@@ -119,6 +119,15 @@ enum
     PIPE_PIXEL_PAIRS = 2    // K-major weights: four stages of weight rows, three slots of two blocks of pixel rows
 };
 
+// Whether the two K-steps of a block go to two groups of waves with larger tiles each (KS below): the 128 x 128 shape, with zero points or
+// taps.  us without / with it: int8 MATMUL with zero points 8 x [512,K]x[K,512] K 2176 14.4 / 13.4, 4096 22.0 / 19.6, 8192 37.9 / 32.6; 3x3 stride 2
+// with RESCALE [32,28,28,384]->512 27.3 / 24.1, [32,28,28,1024]->512 58.7 / 49.4, without a stride [20,28,28,576]->144 36.6 / 32.6; fp16 3x3 stride 2
+// [16,56,56,128]->128 14.4 / 14.0, [32,28,28,512]->256 40.0 / 37.5, [64,7,7,512]->512 40.1 / 37.3.  The others wait for L2: without zero points
+// 1x1 bf16 [8,28,28,2048]->256 17.1 / 18.4, MATMUL 8 x [512,K]x[K,512] K 1536 12.6 / 12.1, 4096 27.6 / 28.5; the patch form 20.6 / 20.8 on
+// [16,28,28,256]->256; the 128 x 256 shape 0 to 8 % slower.
+template <int OCT, int PXT, bool ZP, int MODE, int PIPE>
+static constexpr bool kSplitWaves = PIPE == PIPE_PAIRS && OCT * PXT == 2 && (MODE == GEMM_TAPS || (ZP && MODE != GEMM_PATCH));
+
 template <typename T, int OCT, int PXT, bool ZP, int MODE, int kStages, int PIPE>
 __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
 {
@@ -134,6 +143,12 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     // block (tap, piece) are read from plane `piece` at the tap's offset.
     constexpr bool PATCH   = MODE == GEMM_PATCH;
     static_assert(!PATCH || (PIPE == PIPE_PAIRS && PXT == 1), "the patch form: pairs of weight blocks, 128 pixel rows");
+    // KS: two groups of four waves (2 x 2) take one of the two K-steps of every block each, and a wave owns OCT x 2 PXT accumulator
+    // tiles, half of which it hands to its partner in the other group after the loop.  A block of the 128 x 128 shape is 256 clocks
+    // of matrix instructions; with eight waves of 64 x 32 results over all of K it is also 384 clocks of fragment reads (the LDS serves
+    // 128 bytes a clock) beside 128 of the loads' writes, with waves of 64 x 64 results 256, and a third fewer instructions.
+    constexpr bool KS      = kSplitWaves<OCT, PXT, ZP, MODE, PIPE>;
+    constexpr int IT       = KS ? 2 * PXT : PXT;    // pixel tiles of a wave in the loop
     using M                = Mma<T>;
     constexpr int EB       = (int)sizeof(T);
     constexpr bool IDENT   = KM && EB == 1;    // accumulator row r of a channel tile is channel r
@@ -169,7 +184,10 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     const int rho  = lane & 31;
     const int h    = lane >> 5;
     const int wo   = wave & 1;
-    const int wp   = wave >> 1;
+    const int kg   = KS ? wave >> 2 : 0;    // K group
+    const int wp   = KS ? 2 * (wave >> 1 & 1) + kg : wave >> 1;    // which PXT pixel tiles the wave stores
+    // pixel tile i of the loop, of the workgroup's 4 PXT: those it stores first
+    auto pixel_tile = [&](int i) { return KS ? (wave >> 1 & 1) * IT + (i ^ (kg * PXT)) : wp * PXT + i; };
 
     // Workgroups are dealt round-robin to the 8 XCDs; each XCD takes a contiguous range of the tile list
     // (tiles with the same pixel rows are neighbours) so that its L2 sees every operand row few times.
@@ -395,12 +413,22 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     // ---- fragment addresses -----------------------------------------------------------------------------
     const int wrow = wo * 32 * OCT + row_channel(rho);
     const int prow = WROWS + wp * 32 * PXT + rho;
-    uint32_t aw[2], ap[2];
+    uint32_t aw[2], ap[KS ? IT : 2];    // of each K-step, or (KS) of the group's own, by pixel tile
 #pragma unroll
     for (int s = 0; s < 2; s++)
     {
-        aw[s] = wrow * 64 + (((2 * s + h) ^ swz(wrow)) * 16);
-        ap[s] = prow * 64 + (((2 * s + h) ^ swz(prow)) * 16);
+        aw[s] = wrow * 64 + (((2 * (KS ? kg : s) + h) ^ swz(wrow)) * 16);
+        if (!KS)
+            ap[s] = prow * 64 + (((2 * s + h) ^ swz(prow)) * 16);
+    }
+    if constexpr (KS)
+    {
+#pragma unroll
+        for (int i = 0; i < IT; i++)
+        {
+            const int row = WROWS + pixel_tile(i) * 32 + rho;
+            ap[i]         = row * 64 + (((2 * kg + h) ^ swz(row)) * 16);
+        }
     }
 
     // PATCH: the lane's pixel fragments of block (tap, piece) lie in plane `piece` at the patch pixel under that tap
@@ -458,23 +486,24 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                 const int m  = RB >= 256 ? m8 : (m8 >> 1);
                 akm[t]       = (16 * h + m8) * RB + ((((tile ^ m) << 1) + brho) << 4) + 8 * (sl & 1);
             }
+            akm[t] += (uint32_t)(KSTEP * kg * RB);
         }
     }
 
-    acc_t acc[PXT][OCT];
+    acc_t acc[IT][OCT];
 #pragma unroll
-    for (int i = 0; i < PXT; i++)
+    for (int i = 0; i < IT; i++)
 #pragma unroll
         for (int t = 0; t < OCT; t++)
 #pragma unroll
             for (int e = 0; e < 16; e++)
                 acc[i][t][e] = 0;
-    int wsum[OCT], psum[PXT];
+    int wsum[OCT], psum[IT];
 #pragma unroll
     for (int t = 0; t < OCT; t++)
         wsum[t] = 0;
 #pragma unroll
-    for (int i = 0; i < PXT; i++)
+    for (int i = 0; i < IT; i++)
         psum[i] = 0;
 
     // ---- main loop ----------------------------------------------------------------------------------------
@@ -486,28 +515,29 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     // Every LDS read and every direct load is placed behind a matrix instruction (and kept there with
     // scheduling barriers), so that the time those instructions spend waiting for a slot in the LDS and
     // address queues - all eight waves come out of the barrier together - passes while the matrix core works.
-    constexpr int NM = OCT * PXT;    // matrix instructions per step
+    // KS: a wave has one step of each block, and a pair of blocks takes the place of a block.
+    constexpr int NM = OCT * IT;    // matrix instructions per step
     constexpr int NW = KM ? 2 * OCT : OCT;    // weight fragment reads per step
-    constexpr int NR = NW + PXT;              // fragment reads per step
-    v4i fa[2][OCT], fb[2][PXT];
+    constexpr int NR = NW + IT;               // fragment reads per step
+    v4i fa[2][OCT], fb[2][IT];
     // reads in the order the matrix instructions want them: pixel tile 0, channel tile 0, the other pixel tiles, the other
     // channel tiles
     // wb: the stage's weight rows; pb: its pixel rows minus their offset in a whole stage (ap[] includes it)
     auto read_one = [&](const uint8_t* wb, const uint8_t* pb, int s, int j) {
         const uint8_t* sb = wb;
         constexpr int W1 = KM ? 2 : 1;    // weight reads per channel tile
-        if (j == 0 || (j > W1 && j < W1 + PXT))
+        if (j == 0 || (j > W1 && j < W1 + IT))
         {
             const int i = j == 0 ? 0 : j - W1;
-            fb[s][i]    = *reinterpret_cast<const v4i*>(pb + ap[s] + i * 2048);
+            fb[s][i]    = *reinterpret_cast<const v4i*>(KS ? pb + ap[KS ? i : 0] : pb + ap[s] + i * 2048);
         }
         else
         {
-            const int w = j <= W1 ? j - 1 : j - PXT;    // which of the NW weight reads
+            const int w = j <= W1 ? j - 1 : j - IT;    // which of the NW weight reads
             if constexpr (KM)
             {
                 const int t = w >> 1, r = w & 1;
-                const uint8_t* src = sb + akm[t] + (KSTEP * s + (KSTEP / 4) * r) * RB;
+                const uint8_t* src = sb + akm[t] + (KSTEP * (KS ? 0 : s) + (KSTEP / 4) * r) * RB;
                 v2i half;
                 if constexpr (EB == 2)
                     half = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -524,21 +554,22 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     // The four waves that read the same weight rows take a fourth of the K-steps each for the rows' sums, the two that read the
     // same pixel rows a half (every wave adding up every step: 16 vector instructions beside the 4 matrix instructions of a
     // step of the 128 x 256 shape; int8 [8,1024,1024]x[8,1024,1024] 18.4 us, so 18.05); the parts meet in LDS after the loop.
+    // KS: two waves of a group read the same rows of either operand.
     auto sums = [&](int s, int odd) {
         if constexpr (ZP)
         {
-            if (wp == 2 * odd + s)
+            if (KS ? (wave >> 1 & 1) == s : wp == 2 * odd + s)
 #pragma unroll
                 for (int t = 0; t < OCT; t++)
                     wsum[t] += dot4_ones(fa[s][t]);
             if (wo == s)
 #pragma unroll
-                for (int i = 0; i < PXT; i++)
+                for (int i = 0; i < IT; i++)
                     psum[i] += dot4_ones(fb[s][i]);
         }
     };
     auto mma_one = [&](int s, int k) {
-        const int t = k / PXT, i = t & 1 ? PXT - 1 - k % PXT : k % PXT;    // (one operand changes at a time)
+        const int t = k / IT, i = t & 1 ? IT - 1 - k % IT : k % IT;    // (one operand changes at a time)
         acc[i][t]   = M::mma(fa[s][t], fb[s][i], acc[i][t]);
     };
     // A bare s_barrier: __syncthreads() would also drain this wave's LDS reads (the fragments of the step
@@ -672,10 +703,15 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                     }
                 }
             };
-            first_step(0, cur0, PATCH ? lds : cur0, none, no_load);
-            next_patch(sc + 1);
-            second_step(0, cur0 + STAGE, PATCH ? lds : cur0 + STAGE, none, no_load);
-            first_step(1, cur0 + STAGE, PATCH ? lds : cur0 + STAGE, none, no_load);
+            if constexpr (KS)
+                first_step(0, cur0 + STAGE, cur0 + STAGE, none, no_load);
+            else
+            {
+                first_step(0, cur0, PATCH ? lds : cur0, none, no_load);
+                next_patch(sc + 1);
+                second_step(0, cur0 + STAGE, PATCH ? lds : cur0 + STAGE, none, no_load);
+                first_step(1, cur0 + STAGE, PATCH ? lds : cur0 + STAGE, none, no_load);
+            }
             publish_pair();    // the next pair is in LDS for every wave, and every wave is past the pair before
             next_patch(sc + 2);
             second_step(1, lds + sn * STAGE, PATCH ? lds : lds + sn * STAGE, std::integral_constant<int, 2 * LOADS>{},
@@ -746,7 +782,8 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
             // the last block of an odd count: the first half of a pair whose second half is a repeat
             const uint8_t* cur = lds + sc * STAGE;
             first_step(0, cur, PATCH ? lds : cur, none, no_load);
-            second_step(0, cur + STAGE, PATCH ? lds : cur + STAGE, none, no_load);
+            if constexpr (!KS)
+                second_step(0, cur + STAGE, PATCH ? lds : cur + STAGE, none, no_load);
         }
     }
     else if constexpr (APAIR)
@@ -870,9 +907,45 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     // The loads issued past the last block are still on their way into LDS: let them land before a stage is
     // given another use.  The stage buffers are then free: the channel sums go through the first one.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (KS)
+    {
+        // the other half of K: a wave's last PXT pixel tiles are its partner's first.  (Read before the next barrier, behind which the LDS
+        // has another use.)
+        static_assert(OCT * PXT * 8 * 4096 <= kStages * STAGE, "the tiles handed over lie in the ring");
+        __syncthreads();
+        uint8_t* give       = lds + wave * (OCT * PXT * 4096) + lane * 16;
+        const uint8_t* take = lds + (wave ^ 4) * (OCT * PXT * 4096) + lane * 16;
+#pragma unroll
+        for (int i = 0; i < PXT; i++)
+#pragma unroll
+            for (int t = 0; t < OCT; t++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                {
+                    const acc_t& v = acc[PXT + i][t];
+                    typedef decltype(acc[0][0][0] + acc[0][0][0]) word;
+                    typedef word word4 __attribute__((ext_vector_type(4)));
+                    *reinterpret_cast<word4*>(give + ((i * OCT + t) * 4 + q) * 1024) = word4{ v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3] };
+                }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PXT; i++)
+#pragma unroll
+            for (int t = 0; t < OCT; t++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                {
+                    typedef decltype(acc[0][0][0] + acc[0][0][0]) word;
+                    typedef word word4 __attribute__((ext_vector_type(4)));
+                    const word4 v = *reinterpret_cast<const word4*>(take + ((i * OCT + t) * 4 + q) * 1024);
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        acc[i][t][4 * q + e] += v[e];
+                }
+    }
     int* tab_wsum = reinterpret_cast<int*>(lds);           // a row of WROWS words per wp
-    int* tab_psum = reinterpret_cast<int*>(lds + 5120);    // a row of PROWS words per wo
-    static_assert(WROWS * 16 <= 4096 && 5120 + PROWS * 8 <= 8192, "below the transposition buffers, beside the late bias table");
+    int* tab_psum = reinterpret_cast<int*>(lds + 5120);    // a row of PROWS words per wo (and K group)
+    static_assert(WROWS * 16 <= 4096 && 5120 + PROWS * (KS ? 16 : 8) <= 8192, "below the transposition buffers, beside the late bias table");
     if constexpr (ZP || APAIR)
     {
         __syncthreads();    // every wave has read its last fragments and seen its last loads land
@@ -885,14 +958,14 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
             {
                 const int sum = wsum[t] + __shfl_xor(wsum[t], 32);
                 if (h == 0)
-                    tab_wsum[wp * WROWS + wo * 32 * OCT + t * 32 + row_channel(rho)] = sum;
+                    tab_wsum[(wave >> 1) * WROWS + wo * 32 * OCT + t * 32 + row_channel(rho)] = sum;
             }
 #pragma unroll
-            for (int i = 0; i < PXT; i++)
+            for (int i = 0; i < IT; i++)
             {
                 const int sum = psum[i] + __shfl_xor(psum[i], 32);
                 if (h == 0)
-                    tab_psum[wo * PROWS + wp * 32 * PXT + i * 32 + rho] = sum;
+                    tab_psum[(2 * kg + wo) * PROWS + pixel_tile(i) * 32 + rho] = sum;
             }
         }
         __syncthreads();
@@ -900,7 +973,12 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
         {
 #pragma unroll
             for (int i = 0; i < PXT; i++)
-                psum[i] = tab_psum[wp * 32 * PXT + i * 32 + rho] + tab_psum[PROWS + wp * 32 * PXT + i * 32 + rho];
+            {
+                const int* part = tab_psum + wp * 32 * PXT + i * 32 + rho;
+                psum[i]         = part[0] + part[PROWS];
+                if constexpr (KS)
+                    psum[i] += part[2 * PROWS] + part[3 * PROWS];
+            }
             // (a thread per channel: every wave adding up the four parts of its channels was 24 more 16-byte reads each, half a microsecond)
             if (tid < WROWS)
                 tab_wsum[tid] += tab_wsum[WROWS + tid] + tab_wsum[2 * WROWS + tid] + tab_wsum[3 * WROWS + tid];
