@@ -1,0 +1,444 @@
+// CONV2D with taps on 16-bit floats whose input patch streams through LDS, 128 bytes of channels at a time.
+//
+// A workgroup of 8 waves owns 64 output channels x IT * 128 pixels, whole output rows of one image.  K is walked in stages of one tap and 128 bytes of
+// channels, all taps of a slice of channels before the next slice: the slice's patch (with its halo) lies in one of two buffers, loaded
+// under the taps of the slice before, and a stage's 64 weight rows, whole lines, pass through a ring of eight.  Both go straight into LDS, one barrier a
+// stage.  Two groups of four waves take half of a stage's channels each, so that a wave owns 64 channels x IT * 32 pixels and reads four (IT 1: three)
+// fragments for four (two) matrix instructions; after the loop a wave hands half of its sums to its partner.
+//
+// What bounds it: on few tiles the chain of a stage (0.215 us, 0.11 of it matrix instructions; 0.416 of 0.21 with 256 pixels), on all CUs the clock under the
+// matrix instructions: [16,28,28,256]->256 3x3 14.9 us without any operand in the loop, 18.8 with its fragment reads.  A wave's loads straight into LDS go
+// one after the other, 0.3 us each, so the second group fetches the patch through registers (all loads straight into LDS: 26.2, so 21.5), in a loop of its own,
+// or the compiler has the first group wait for them too (28.9).
+// us before / here: [16,14,14,512]->512 40.1 / 24.2, [16,28,28,256]->64 20.7 / 13.4, 5x5 [2,20,20,480]->592 129 / 53, stride 2 [14,36,28,328]->240 46.9 / 22.7.
+#include <type_traits>
+
+#include "tmi_mfma.h"
+
+namespace tmi
+{
+
+struct PlanesArgs
+{
+    const uint8_t *x, *w, *pad_page;    // pad_page: 16 zero bytes
+    const void* bias;
+    void* out;
+    int32_t N;                   // output channels, a multiple of 8
+    int32_t kb, icb;             // bytes of a weight row, of a channel vector (multiples of 16)
+    int32_t slices, taps, KW;    // of 128 bytes
+    int32_t IH, IW, OH, OW;
+    int32_t sy, sx, dy, dx, pad_top, pad_left;
+    int32_t bias_len;
+    int32_t rows;                      // output rows of a tile
+    int32_t patch_w, patch_pixels;
+    int32_t buffer_bytes;              // of a slice's patch in LDS
+    int32_t tiles, per_xcd;
+    FastDiv tiles_n, tiles_image, div_pw, div_ow;
+};
+
+static constexpr int kPlanesRing = 8, kPlanesLoads = 12;    // stages of weights; KB of a slice's patch a wave fetches at most
+static constexpr int kPlanesPatches = 160 * 1024 - kPlanesRing * 8192 - 256;    // LDS for the two patches
+
+// 16-byte chunk c of a 128-byte row lies at c ^ key(row): the lanes the LDS serves in one cycle read one chunk of rows whose (row / 2) % 8 differ
+// or that lie in the two halves of the banks (no conflict for any 32 consecutive rows, nor for the weights' order).  A patch pixel's key is that of
+// its row * OW + column: consecutive outputs read consecutive ones, past the halo between two rows too.
+__device__ __forceinline__ int planes_key(int row)
+{
+    return (row >> 1) & 7;
+}
+
+template <typename T, int IT>
+__global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
+{
+    constexpr int D = kPlanesRing, STAGE = 64 * 128;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    const int lane = threadIdx.x & 63, rho = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int kg = wave >> 2, wq = wave & 3;    // half of a stage's channels, pixel tiles
+
+    // a contiguous range of tiles for each of the eight L2s; those of the same pixels are neighbours
+    const int L = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
+    if (L >= a.tiles)
+        return;
+    const uint32_t tm = fdiv((uint32_t)L, a.tiles_n), tn = (uint32_t)L - tm * a.tiles_n.d;
+    const uint32_t image = fdiv(tm, a.tiles_image);
+    const int oy0 = (int)(tm - image * a.tiles_image.d) * a.rows, oc0 = (int)tn * 64;
+    const int rows_here = a.OH - oy0 < a.rows ? a.OH - oy0 : a.rows, pixels = rows_here * a.OW;
+    const uint8_t* x = a.x + (size_t)image * a.IH * a.IW * a.icb;
+
+    // ---- loads: 64 lanes move eight rows of 128 bytes ---------------------------------------------------------
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    const uint8_t* zeros = a.pad_page;
+    // the first group of waves: weights, two of a stage's eight loads each
+    uint32_t w_off[2];
+    int w_at[2];    // of the lane's chunk
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+    {
+        const int row = (2 * wq + q) * 8 + (lane >> 3), oc = oc0 + row < a.N ? oc0 + row : a.N - 1;    // (rows past the last are not stored)
+        w_at[q]  = ((lane & 7) ^ planes_key(row)) * 16;
+        w_off[q] = (uint32_t)oc * (uint32_t)a.kb + (uint32_t)w_at[q];
+    }
+    const int whole = a.icb >> 7;    // slices of 128 bytes
+    int l_tap = 0, l_slice = 0;      // the next stage whose weights are requested; past the end the last slice again, which nobody reads
+    const uint8_t* l_base = a.w;
+    auto load_weights = [&](int slot) {
+        const uint32_t dst = lds0 + slot * STAGE + wq * 2048;
+        if (l_slice < whole)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %3\n\ts_add_u32 m0, %2, 1024\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3"
+                         :
+                         : "v"(w_off[0]), "v"(w_off[1]), "s"(dst), "s"(l_base)
+                         : "memory", "scc");
+        else    // (a slice of fewer than 128 bytes: zeros for the others)
+        {
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+            {
+                const uint8_t* src = l_slice * 128 + w_at[q] < a.icb ? l_base + w_off[q] : zeros;
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(dst + 1024 * q) : "memory");
+            }
+        }
+        l_base += a.icb;
+        if (++l_tap == a.taps)
+        {
+            l_tap   = 0;
+            l_slice = l_slice + 1 < a.slices ? l_slice + 1 : l_slice;
+            l_base  = a.w + l_slice * 128;
+        }
+    };
+    // the second group: the patch, through registers (a wave's loads straight into LDS go one after the other, these are in flight together)
+    const int iy0 = oy0 * a.sy - a.pad_top;
+    v4i held[kPlanesLoads];
+    auto fetch_patch = [&](int slice) {
+#pragma unroll
+        for (int j = 0; j < kPlanesLoads; j++)
+        {
+            const int u = (j * 4 + wq) * 8;    // the wave's first pixel
+            if (u >= a.patch_pixels)
+                break;
+            const int pix = u + (lane >> 3), r = (int)fdiv((uint32_t)pix, a.div_pw), c = pix - r * a.patch_w;
+            const int iy = iy0 + r, ix = c - a.pad_left, at = slice * 128 + (((lane & 7) ^ planes_key(r * a.OW + c)) * 16);
+            const bool there   = (uint32_t)iy < (uint32_t)a.IH && (uint32_t)ix < (uint32_t)a.IW && at < a.icb && pix < a.patch_pixels;
+            const uint8_t* src = there ? x + (uint32_t)((iy * a.IW + ix) * a.icb + at) : zeros;
+            held[j]            = *reinterpret_cast<const v4i*>(src);
+        }
+    };
+    auto store_patch = [&](int slice) {
+        uint8_t* to = lds + D * STAGE + (slice & 1) * a.buffer_bytes + wq * 1024 + lane * 16;
+#pragma unroll
+        for (int j = 0; j < kPlanesLoads; j++)
+        {
+            if ((j * 4 + wq) * 8 >= a.patch_pixels)
+                break;
+            *reinterpret_cast<v4i*>(to + j * 4096) = held[j];
+        }
+    };
+    float* tab_bias = reinterpret_cast<float*>(lds + D * STAGE + 2 * a.buffer_bytes);
+    if (threadIdx.x < 64)
+    {
+        const int oc          = oc0 + (int)threadIdx.x < a.N ? oc0 + (int)threadIdx.x : a.N - 1;
+        tab_bias[threadIdx.x] = load_as_float<T>(a.bias, a.bias_len == 1 ? 0 : oc);
+    }
+    if (kg)
+    {
+        fetch_patch(0);
+        store_patch(0);
+    }
+    else
+    {
+#pragma unroll
+        for (int s = 0; s < D - 1; s++)
+            load_weights(s);
+    }
+
+    // ---- fragments --------------------------------------------------------------------------------------------
+    // Tile i of the wave is the workgroup's pixel tile wq * IT + (i ^ kg): the one it stores (IT 2) first.
+    const int w_frag = channel_of_row(rho);
+    const uint32_t aw0 = (uint32_t)(w_frag * 128 + (((4 * kg + h) ^ planes_key(w_frag)) * 16));
+    int pbase[IT], pkey[IT];
+#pragma unroll
+    for (int i = 0; i < IT; i++)
+    {
+        int p = (wq * IT + (IT == 2 ? i ^ kg : 0)) * 32 + rho;
+        p     = p < pixels ? p : 0;    // (not stored)
+        const int py = (int)fdiv((uint32_t)p, a.div_ow);
+        pbase[i]     = py * a.sy * a.patch_w + (p - py * a.OW) * a.sx;
+        pkey[i]      = py * a.sy * a.OW + (p - py * a.OW) * a.sx;
+    }
+    // where the stage read next lies
+    uint32_t aw = aw0, ap[IT];
+    int tap = 0, kx = 0, slice = 0, tap_at = 0, tap_key = 0, slot = 0;
+    auto address = [&](int i) {    // of pixel tile i; of the weights
+        if (i == IT)
+            aw = aw0 + (uint32_t)slot * STAGE;
+        else
+        {
+            const int pp = pbase[i] + tap_at;
+            ap[i] = (uint32_t)(D * STAGE + (slice & 1) * a.buffer_bytes + pp * 128 + (((4 * kg + h) ^ planes_key(pkey[i] + tap_key)) * 16));
+        }
+    };
+    auto next_stage = [&]() {
+        slot = (slot + 1) & (D - 1);
+        kx++, tap++, tap_at += a.dx, tap_key += a.dx;
+        if (kx == a.KW)
+            kx = 0, tap_at += a.dy * a.patch_w - a.KW * a.dx, tap_key += a.dy * a.OW - a.KW * a.dx;
+        if (tap == a.taps)
+            tap = 0, tap_at = 0, tap_key = 0, slice++;
+    };
+    using acc_t = typename Mma<T>::acc_t;
+    acc_t acc[IT][2];
+#pragma unroll
+    for (int i = 0; i < IT; i++)
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int e = 0; e < 16; e++)
+                acc[i][t][e] = 0;
+    v4i fa[2][2], fb[2][IT];
+    auto read_one = [&](int s, int j) {    // j: pixel tile 0, channel tile 0, the others
+        if (j == 0 || (IT == 2 && j == 2))
+            fb[s][j >> 1] = *reinterpret_cast<const v4i*>(lds + (ap[j >> 1] ^ (32 * s)));
+        else
+            fa[s][j == 1 ? 0 : 1] = *reinterpret_cast<const v4i*>(lds + (aw ^ (32 * s)) + (j == 1 ? 0 : 4096));
+    };
+    constexpr int NM = 2 * IT, NR = 2 + IT;
+    // Step S; behind its instructions the requests for the next step's fragments and what `behind` does there.
+    auto multiply = [&](auto S_tag, auto&& behind) {
+        constexpr int S = decltype(S_tag)::value;
+#pragma unroll
+        for (int k = 0; k < NM; k++)
+        {
+            const int t = k / IT, i = t & 1 ? IT - 1 - k % IT : k % IT;
+            acc[i][t]   = Mma<T>::mma(fa[S][t], fb[S][i], acc[i][t]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+                if (j * (NM - 1) / NR == k)
+                    read_one(1 - S, j);
+            behind(k);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // the patch and the first stage
+    if (kg)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    else
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * (D - 2)) : "memory");
+    asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+    for (int i = 0; i <= IT; i++)
+        address(i);
+#pragma unroll
+    for (int j = 0; j < NR; j++)
+        read_one(0, j);
+
+    // One stage: its first step, the barrier behind which the next stage is there and every wave is past the one before this, its second.
+    auto stage = [&](auto&& wait, auto&& loads) {
+        multiply(std::integral_constant<int, 0>{}, [&](int k) {
+            if (k == NM - 1)
+            {
+                // (every request of this step's fragments is out)
+                next_stage();
+#pragma unroll
+                for (int i = 0; i <= IT; i++)
+                    address(i);
+            }
+        });
+        wait();
+        asm volatile("s_barrier" ::: "memory");
+        multiply(std::integral_constant<int, 1>{}, [&](int k) {
+            if (k == 0)
+                loads();
+        });
+    };
+    auto none = []() {};
+    // (a loop for each group: the compiler would have the one with loads to wait for also wait in the other's place)
+    if (!kg)
+    {
+        // the next stage's weights, with those of D - 3 later ones on their way
+        int free_slot = D - 1;
+#pragma unroll 1
+        for (int s = a.slices * a.taps; s > 0; s--)
+            stage([]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (D - 3)) : "memory"); },
+                  [&]() {
+                      load_weights(free_slot);
+                      free_slot = (free_slot + 1) & (D - 1);
+                  });
+    }
+    else
+    {
+        // the next slice's patch: fetched in the first stage of a slice, stored in the last but one
+#pragma unroll 1
+        for (int next = 1; next < a.slices; next++)
+        {
+            stage(none, [&]() { fetch_patch(next); });
+#pragma unroll 1
+            for (int t = a.taps - 3; t > 0; t--)
+                stage(none, none);
+            stage(none, [&]() { store_patch(next); });
+            stage([]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }, none);
+        }
+#pragma unroll 1
+        for (int t = a.taps; t > 0; t--)
+            stage(none, none);
+    }
+
+    // ---- the other half of the channels: a wave's second pixel tile (IT 1: its channel tile 1 - kg) is its partner's ---------
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    constexpr int HT = IT == 2 ? 2 : 1;    // channel tiles a wave stores
+    uint8_t* give       = lds + wave * (HT * 4096) + lane * 16;
+    const uint8_t* take = lds + (wave ^ 4) * (HT * 4096) + lane * 16;
+#pragma unroll
+    for (int t = 0; t < HT; t++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+            v4f v;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                v[e] = IT == 2 ? acc[IT - 1][t][4 * q + e] : (kg ? acc[0][0][4 * q + e] : acc[0][1][4 * q + e]);
+            *reinterpret_cast<v4f*>(give + (t * 4 + q) * 1024) = v;
+        }
+    __syncthreads();
+    float sum[HT][16];
+#pragma unroll
+    for (int t = 0; t < HT; t++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+            const v4f v = *reinterpret_cast<const v4f*>(take + (t * 4 + q) * 1024);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                sum[t][4 * q + e] = v[e] + (IT == 2 ? acc[0][t][4 * q + e] : (kg ? acc[0][1][4 * q + e] : acc[0][0][4 * q + e]));
+        }
+    __syncthreads();
+
+    // ---- results: gathered by pixel, so that whole lines leave ----------------------------------------------------
+    constexpr int ROW = HT * 64, PITCH = ROW + 16;
+    uint8_t* tbuf = lds + wave * (32 * PITCH);
+    const int oc_w = oc0 + (IT == 2 ? 0 : 32 * kg), p_w = (IT == 2 ? wq * 2 + kg : wq) * 32;
+#pragma unroll
+    for (int t = 0; t < HT; t++)
+    {
+        alignas(16) T packed[16];
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+            const v4f b = *reinterpret_cast<const v4f*>(tab_bias + oc_w - oc0 + 32 * t + 16 * h + 4 * q);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                store_from_float(packed + 4 * q + e, sum[t][4 * q + e] + b[e]);
+        }
+        uint8_t* d = tbuf + rho * PITCH + t * 64 + h * 32;
+        reinterpret_cast<v4i*>(d)[0] = reinterpret_cast<const v4i*>(packed)[0];
+        reinterpret_cast<v4i*>(d)[1] = reinterpret_cast<const v4i*>(packed)[1];
+    }
+    constexpr int PIECES = ROW / 16, RPI = 64 / PIECES;
+    uint8_t* to = reinterpret_cast<uint8_t*>(a.out) + (((size_t)(image * a.OH + oy0) * a.OW + p_w) * a.N + oc_w) * 2;
+#pragma unroll
+    for (int j = 0; j < 32 / RPI; j++)
+    {
+        const int row = lane / PIECES + RPI * j, piece = lane % PIECES;
+        const v4i d   = *reinterpret_cast<const v4i*>(tbuf + row * PITCH + piece * 16);
+        if (p_w + row < pixels && oc_w + piece * 8 < a.N)
+            *reinterpret_cast<v4i*>(to + (size_t)row * a.N * 2 + piece * 16) = d;
+    }
+}
+
+struct PlanesPlan
+{
+    int32_t rows = 0;    // of a tile; 0: none
+    int64_t patch_pixels, slices, tiles_image, tiles;
+    double us;           // a prediction: 230 layers of 0.3 to 30 GFLOP, half of them within 5 %, nine in ten within 13 %
+    bool wide;           // more than 128 pixels a tile
+};
+
+// The tile of whole output rows that takes the chip the shortest time
+static PlanesPlan plan_planes(const ConvGeom& g)
+{
+    PlanesPlan best;
+    const int64_t slices = ((int64_t)g.IC * 2 + 127) / 128, taps = (int64_t)g.KH * g.KW, tn = (g.OC + 63) / 64;
+    const int64_t patch_w = (int64_t)(g.OW - 1) * g.stride_x + (int64_t)(g.KW - 1) * g.dil_x + 1;
+    for (int rows = 1; rows <= g.OH && (int64_t)rows * g.OW <= 256; rows++)
+    {
+        PlanesPlan p;
+        p.rows         = rows;
+        p.patch_pixels = ((int64_t)(rows - 1) * g.stride_y + (int64_t)(g.KH - 1) * g.dil_y + 1) * patch_w;
+        if (p.patch_pixels > 8 * 4 * kPlanesLoads || 2 * ((p.patch_pixels + 7) / 8 * 1024) > kPlanesPatches)
+            break;
+        p.slices      = slices;
+        p.tiles_image = (g.OH + rows - 1) / rows;
+        p.tiles       = (int64_t)g.N * p.tiles_image * tn;
+        p.wide        = (int64_t)rows * g.OW > 128;
+        p.us          = 1.6 + (double)((p.tiles + 255) / 256) * (3.2 + (double)(slices * taps) * (p.wide ? 0.416 : 0.215) + 0.0029 * (double)(p.patch_pixels * slices));
+        if (best.rows == 0 || p.us < best.us * 0.999)
+            best = p;
+    }
+    return best;
+}
+
+static bool planes_take(int32_t in_dtype, const ConvGeom& g)
+{
+    const int64_t taps = (int64_t)g.KH * g.KW, icb = (int64_t)g.IC * 2;
+    return (in_dtype == TMI_FP16 || in_dtype == TMI_BF16) && taps >= 3 && taps <= 64 && g.IC % 8 == 0 && g.OC % 8 == 0 && g.OW <= 256 && icb * taps * g.OC < INT32_MAX &&
+           (int64_t)g.IH * g.IW * icb < INT32_MAX;
+}
+
+// Whether a layer runs here: one round of workgroups and 18 stages or more.  us the kernel it would go to / here, 3x3 unless noted:
+//   the patch kernel (conv2d_mfma.hip): [16,14,14,512]->512 40.1 / 24.2, [16,28,28,256]->64 20.7 / 13.4, [26,10,22,376]->160 32.8 / 20.8, 5x5 [2,20,20,480]->592 129 / 53,
+//     [11,58,21,96]->96 30.9 / 19.3, stride 2 [14,36,28,328]->240 46.9 / 22.7; over 34 of them 0.41 ... 0.96.  Two rounds: [4,29,109,136]->136 19.7 / 26.9,
+//     [22,75,13,288]->144 stride 2 27.6 / 34.6; 9 stages: [20,50,50,64]->72 stride 2 11.5 / 13.3, [11,28,28,32]->104 5.9 / 7.6.
+//   split reductions (conv_taps.hip), from 115 TFLOP/s predicted on: [2,18,18,384]->448 26.4 / 17.9, [7,14,21,200]->288 19.9 / 14.7; below [3,14,14,512]->160
+//     18.6 / 21.1 (39), [2,26,26,192]->88 1.24 times (35).
+//   the GEMM kernel, only with tiles of up to 128 pixels and whole slices: [14,22,22,384]->176 31.8 / 18.8, 5x5 [24,52,10,64]->128 15.2 / 10.6, [10,22,22,128]->296 20.7 / 17.7; else
+//     [16,28,28,256]->256 (196 pixels) 20.2 / 21.5, [16,40,15,160]->136 (two and a half slices) 12.6 / 13.0.
+bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, bool to_gemm)
+{
+    if (!planes_take(in_dtype, g))
+        return false;
+    const PlanesPlan p = plan_planes(g);
+    if (p.rows == 0 || p.tiles > 256 || p.slices * g.KH * g.KW < 18)
+        return false;
+    if (to_gemm)
+        return !p.wide && g.IC % 64 == 0;
+    if (p.slices == 1 && g.IC < 64)    // (a slice cut short and no other under which a patch is fetched: 5x5 [5,47,47,48]->48 10.2 / 11.9)
+        return false;
+    return 2e-6 * (double)g.N * g.OH * g.OW * g.OC * g.IC * g.KH * g.KW >= 115 * p.us;
+}
+
+bool launch_conv_planes(hipStream_t st, int32_t in_dtype, const ConvGeom& g, const void* in, const void* w, const void* bias, const void* pad_page, void* out)
+{
+    if (!planes_take(in_dtype, g) || (((uintptr_t)in | (uintptr_t)w | (uintptr_t)out | (uintptr_t)pad_page) & 15) != 0)
+        return false;
+    const PlanesPlan p = plan_planes(g);
+    if (p.rows == 0)
+        return false;
+    const int64_t icb = (int64_t)g.IC * 2, taps = (int64_t)g.KH * g.KW, kb = icb * taps, tn = (g.OC + 63) / 64, tiles_m = (int64_t)g.N * p.tiles_image;
+    PlanesArgs a{};
+    a.patch_w = (int32_t)((int64_t)(g.OW - 1) * g.stride_x + (int64_t)(g.KW - 1) * g.dil_x + 1);
+    if (p.tiles > (1 << 22) || !fastdiv_exact_up_to((uint64_t)p.tiles, (uint32_t)tn) || !fastdiv_exact_up_to((uint64_t)tiles_m, (uint32_t)p.tiles_image) ||
+        !fastdiv_exact_up_to((uint64_t)p.patch_pixels + 8, (uint32_t)a.patch_w) || !fastdiv_exact_up_to(256, (uint32_t)g.OW))
+        return false;
+    a.x = (const uint8_t*)in, a.w = (const uint8_t*)w, a.pad_page = (const uint8_t*)pad_page, a.bias = bias, a.out = out;
+    a.N = g.OC, a.kb = (int32_t)kb, a.icb = (int32_t)icb, a.slices = (int32_t)p.slices, a.taps = (int32_t)taps, a.KW = g.KW;
+    a.IH = g.IH, a.IW = g.IW, a.OH = g.OH, a.OW = g.OW;
+    a.sy = g.stride_y, a.sx = g.stride_x, a.dy = g.dil_y, a.dx = g.dil_x, a.pad_top = g.pad_top, a.pad_left = g.pad_left;
+    a.bias_len = g.bias_len, a.rows = p.rows, a.patch_pixels = (int32_t)p.patch_pixels;
+    a.buffer_bytes = (int32_t)((p.patch_pixels + 7) / 8 * 1024);
+    a.tiles = (int32_t)p.tiles, a.per_xcd = (int32_t)((p.tiles + 7) / 8);
+    a.tiles_n = make_fastdiv((uint32_t)tn), a.tiles_image = make_fastdiv((uint32_t)p.tiles_image);
+    a.div_pw = make_fastdiv((uint32_t)a.patch_w), a.div_ow = make_fastdiv((uint32_t)g.OW);
+    const size_t lds = (size_t)kPlanesRing * 8192 + 2 * (size_t)a.buffer_bytes + 256;    // and the bias
+    auto run = [&](auto kernel) {
+        if (!ensure_dynamic_lds<kernel.value>(lds))
+            return false;
+        hipLaunchKernelGGL(kernel.value, dim3((unsigned)(a.per_xcd * 8)), dim3(512), lds, st, a);
+        return true;
+    };
+    if (in_dtype == TMI_FP16)
+        return p.wide ? run(kernel_constant<conv_planes_kernel<_Float16, 2>>{}) : run(kernel_constant<conv_planes_kernel<_Float16, 1>>{});
+    return p.wide ? run(kernel_constant<conv_planes_kernel<bf16_t, 2>>{}) : run(kernel_constant<conv_planes_kernel<bf16_t, 1>>{});
+}
+
+}    // namespace tmi

@@ -77,12 +77,6 @@ __device__ __forceinline__ int swz(int r)
     return (r >> 3) & 3;
 }
 
-// accumulator row -> channel of its tile
-__device__ __forceinline__ int channel_of_row(int rho)
-{
-    return 16 * ((rho >> 2) & 1) + 4 * (rho >> 3) + (rho & 3);
-}
-
 // Stage buffers of a workgroup: four 64-byte blocks per row.  The 256x256 shape fills the LDS with them; two
 // workgroups of a smaller shape with three stages each were measured and are slower (the operand traffic per
 // matrix instruction, not the barrier, is what the smaller shapes wait for).
@@ -1330,6 +1324,14 @@ static bool patch_form_geometry(int OH, int OW, int KH, int KW, int sy, int sx, 
     patch_w              = (OW - 1) * sx + (KW - 1) * dx + 1;
     const int64_t bytes  = ((int64_t)patch_h * patch_w * icb + 1023) / 1024 * 1024;
     return kRing + bytes + kTables <= kLds;
+}
+
+bool gemm_patch_form(const ConvGeom& g, int32_t in_dtype)
+{
+    int rows = 0, patch_h = 0, patch_w = 0;
+    const int64_t icb = (int64_t)g.IC * (in_dtype == TMI_INT8 ? 1 : 2);
+    return patch_form_geometry(g.OH, g.OW, g.KH, g.KW, g.stride_y, g.stride_x, g.dil_y, g.dil_x, icb, g.OC, rows, patch_h, patch_w) &&
+           (int64_t)g.N * ((g.OH + rows - 1) / rows) * ((g.OC + 127) / 128) >= 48;
 }
 
 template <typename T>

@@ -53,6 +53,13 @@ struct Mma<bf16_t>
     }
 };
 
+// The row of a weight operand's tile that lane rho reads: accumulator row 8q + 4h' + j is then channel 16h' + 4q + j, and a lane owns 16
+// consecutive channels of one pixel
+__device__ __forceinline__ int channel_of_row(int rho)
+{
+    return 16 * ((rho >> 2) & 1) + 4 * (rho >> 3) + (rho & 3);
+}
+
 // min(max(v, lo), hi) as one instruction; lo <= hi
 __device__ __forceinline__ int32_t clamp_med3(int32_t v, int32_t lo, int32_t hi)
 {

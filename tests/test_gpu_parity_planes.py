@@ -1,0 +1,52 @@
+"""GPU parity of the streaming-patch CONV2D kernel (16-bit floats with taps): slices of channels whole and cut, windows of two taps and
+more, ragged rows, images and output channels.  Operands are small whole numbers, so that every sum is exact in fp32 and a
+result has one right value in every type."""
+import numpy as np
+import pytest
+
+import cases
+import gpu_ops
+from reference_model_amd import Context, capi
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # n, ih, iw, ic, oc, kh, kw, pad, stride, dilation
+    (16, 28, 28, 256, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
+    (10, 28, 30, 200, 56, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),     # channels of no whole slices, output channels cut
+    (12, 30, 28, 520, 128, 1, 3, (0, 0, 1, 1), (1, 1), (1, 1)),    # three taps: the next patch stored in a slice's second stage
+    (24, 21, 23, 448, 136, 3, 1, (1, 1, 0, 0), (1, 1), (1, 1)),
+    (9, 33, 41, 128, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1)),
+    (12, 14, 14, 384, 264, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
+    (14, 24, 28, 176, 56, 3, 3, (2, 2, 2, 2), (1, 1), (2, 2)),     # dilation
+    (16, 29, 29, 328, 240, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1)),    # stride
+    (27, 40, 40, 264, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),     # more than 128 pixels a tile, the last rows of an image fewer
+    (2, 60, 111, 256, 48, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),     # a row a tile
+    (16, 14, 14, 512, 512, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
+]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("kind", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_small_whole_numbers(ctx, kind, shape):
+    n, ih, iw, ic, oc, kh, kw, pad, stride, dil = shape
+    rng = np.random.default_rng(ic + oc)
+    x = rng.integers(-2, 3, (n, ih, iw, ic)).astype(np.int8)
+    w = rng.integers(-2, 3, (oc, kh, kw, ic)).astype(np.int8)
+    bias = rng.integers(-9, 10, oc).astype(np.int32)
+    want = cases.conv2d_exact_blas(x, w, bias, pad, stride, dil)
+    if kind == "fp16":
+        got, st = gpu_ops.conv2d(ctx, *(v.astype(np.float16) for v in (x, w, bias)), pad, stride, dil, dtype=capi.FP16)
+        want = want.astype(np.float16)
+    else:
+        got, st = gpu_ops.conv2d(ctx, *(cases.float_to_bf16_bits(v.astype(np.float32)) for v in (x, w, bias)), pad, stride, dil, dtype=capi.BF16)
+        want = cases.float_to_bf16_bits(want.astype(np.float32))
+    assert st == capi.VALID
+    print(shape, ctx.last_kernel)
+    assert np.array_equal(got, want)
