@@ -1,4 +1,4 @@
-// CONV2D with taps on 16-bit floats whose input patch streams through LDS, 128 bytes of channels at a time.
+// CONV2D with taps on 16-bit floats, or on int8 with the fused RESCALE, whose input patch streams through LDS, 128 bytes of channels at a time.
 //
 // A workgroup of 8 waves owns 64 output channels x IT * 128 pixels, whole output rows of one image.  K is walked in stages of one tap and 128 bytes of
 // channels, all taps of a slice of channels before the next slice: the slice's patch (with its halo) lies in one of two buffers, loaded
@@ -20,7 +20,7 @@ namespace tmi
 
 struct PlanesArgs
 {
-    const uint8_t *x, *w, *pad_page;    // pad_page: 16 zero bytes
+    const uint8_t *x, *w, *pad_page, *zeros;    // pad_page: 16 bytes of the input's zero point; 16 zero bytes
     const void* bias;
     void* out;
     int32_t N;                   // output channels, a multiple of 8
@@ -34,10 +34,13 @@ struct PlanesArgs
     int32_t buffer_bytes;              // of a slice's patch in LDS
     int32_t tiles, per_xcd;
     FastDiv tiles_n, tiles_image, div_pw, div_ow;
+    int32_t za;             // int8: the input's zero point; the weights' is 0
+    RescaleParams rp;
+    uint32_t* flag_word;    // where its REQUIRE conditions are latched
 };
 
 static constexpr int kPlanesRing = 8, kPlanesLoads = 12;    // stages of weights; KB of a slice's patch a wave fetches at most
-static constexpr int kPlanesPatches = 160 * 1024 - kPlanesRing * 8192 - 256;    // LDS for the two patches
+static constexpr int kPlanesPatches = 160 * 1024 - kPlanesRing * 8192 - 256 - 64 * 32;    // LDS for the two patches, beside the tables
 
 // 16-byte chunk c of a 128-byte row lies at c ^ key(row): the lanes the LDS serves in one cycle read one chunk of rows whose (row / 2) % 8 differ
 // or that lie in the two halves of the banks (no conflict for any 32 consecutive rows, nor for the weights' order).  A patch pixel's key is that of
@@ -51,6 +54,9 @@ template <typename T, int IT>
 __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
 {
     constexpr int D = kPlanesRing, STAGE = 64 * 128;
+    constexpr bool I8 = Mma<T>::is_int;
+    using word_t      = std::conditional_t<I8, int, float>;
+    using word4_t     = std::conditional_t<I8, v4i, v4f>;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const int lane = threadIdx.x & 63, rho = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -68,7 +74,6 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
 
     // ---- loads: 64 lanes move eight rows of 128 bytes ---------------------------------------------------------
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
-    const uint8_t* zeros = a.pad_page;
     // the first group of waves: weights, two of a stage's eight loads each
     uint32_t w_off[2];
     int w_at[2];    // of the lane's chunk
@@ -94,7 +99,7 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
 #pragma unroll
             for (int q = 0; q < 2; q++)
             {
-                const uint8_t* src = l_slice * 128 + w_at[q] < a.icb ? l_base + w_off[q] : zeros;
+                const uint8_t* src = l_slice * 128 + w_at[q] < a.icb ? l_base + w_off[q] : a.zeros;
                 asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(dst + 1024 * q) : "memory");
             }
         }
@@ -119,7 +124,7 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
             const int pix = u + (lane >> 3), r = (int)fdiv((uint32_t)pix, a.div_pw), c = pix - r * a.patch_w;
             const int iy = iy0 + r, ix = c - a.pad_left, at = slice * 128 + (((lane & 7) ^ planes_key(r * a.OW + c)) * 16);
             const bool there   = (uint32_t)iy < (uint32_t)a.IH && (uint32_t)ix < (uint32_t)a.IW && at < a.icb && pix < a.patch_pixels;
-            const uint8_t* src = there ? x + (uint32_t)((iy * a.IW + ix) * a.icb + at) : zeros;
+            const uint8_t* src = there ? x + (uint32_t)((iy * a.IW + ix) * a.icb + at) : a.pad_page;
             held[j]            = *reinterpret_cast<const v4i*>(src);
         }
     };
@@ -133,11 +138,21 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
             *reinterpret_cast<v4i*>(to + j * 4096) = held[j];
         }
     };
-    float* tab_bias = reinterpret_cast<float*>(lds + D * STAGE + 2 * a.buffer_bytes);
+    word_t* tab_bias     = reinterpret_cast<word_t*>(lds + D * STAGE + 2 * a.buffer_bytes);
+    ChannelScale* tab_cs = reinterpret_cast<ChannelScale*>(tab_bias + 64);
+    uint32_t flags       = 0;
     if (threadIdx.x < 64)
     {
-        const int oc          = oc0 + (int)threadIdx.x < a.N ? oc0 + (int)threadIdx.x : a.N - 1;
-        tab_bias[threadIdx.x] = load_as_float<T>(a.bias, a.bias_len == 1 ? 0 : oc);
+        const bool ok = oc0 + (int)threadIdx.x < a.N;
+        const int oc  = ok ? oc0 + (int)threadIdx.x : a.N - 1;
+        if constexpr (I8)
+        {
+            tab_bias[threadIdx.x] = reinterpret_cast<const int32_t*>(a.bias)[a.bias_len == 1 ? 0 : oc];
+            const int32_t m = load_multiplier(a.rp, oc), sh = load_shift(a.rp, oc);    // (channels past the end: neutral constants, nothing raised)
+            tab_cs[threadIdx.x] = make_channel_scale(ok ? m : 0, ok ? sh : 32, a.rp.double_round != 0, flags);
+        }
+        else
+            tab_bias[threadIdx.x] = load_as_float<T>(a.bias, a.bias_len == 1 ? 0 : oc);
     }
     if (kg)
     {
@@ -202,9 +217,20 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
             fa[s][j == 1 ? 0 : 1] = *reinterpret_cast<const v4i*>(lds + (aw ^ (32 * s)) + (j == 1 ? 0 : 4096));
     };
     constexpr int NM = 2 * IT, NR = 2 + IT;
+    // int8, sum((x - za) w) = sum(x w) - za sum(w): of the four waves that read the same weights each adds up one channel tile of one step
+    int wsum            = 0;
+    const int sums_step = I8 && a.za != 0 ? wq >> 1 : -1;
     // Step S; behind its instructions the requests for the next step's fragments and what `behind` does there.
     auto multiply = [&](auto S_tag, auto&& behind) {
         constexpr int S = decltype(S_tag)::value;
+        if constexpr (I8)
+            if (sums_step == S)
+            {
+                if (wq & 1)
+                    wsum += dot4_ones(fa[S][1]);
+                else
+                    wsum += dot4_ones(fa[S][0]);
+            }
 #pragma unroll
         for (int k = 0; k < NM; k++)
         {
@@ -287,6 +313,13 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     constexpr int HT = IT == 2 ? 2 : 1;    // channel tiles a wave stores
+    int* tab_wsum       = reinterpret_cast<int*>(lds + D * STAGE);    // a row of 64 words for each part
+    if constexpr (I8)
+    {
+        const int both = wsum + __shfl_xor(wsum, 32);
+        if (h == 0)
+            tab_wsum[(2 * kg + (wq >> 1)) * 64 + (wq & 1) * 32 + channel_of_row(rho)] = both;
+    }
     uint8_t* give       = lds + wave * (HT * 4096) + lane * 16;
     const uint8_t* take = lds + (wave ^ 4) * (HT * 4096) + lane * 16;
 #pragma unroll
@@ -294,20 +327,20 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
 #pragma unroll
         for (int q = 0; q < 4; q++)
         {
-            v4f v;
+            word4_t v;
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 v[e] = IT == 2 ? acc[IT - 1][t][4 * q + e] : (kg ? acc[0][0][4 * q + e] : acc[0][1][4 * q + e]);
-            *reinterpret_cast<v4f*>(give + (t * 4 + q) * 1024) = v;
+            *reinterpret_cast<word4_t*>(give + (t * 4 + q) * 1024) = v;
         }
     __syncthreads();
-    float sum[HT][16];
+    word_t sum[HT][16];
 #pragma unroll
     for (int t = 0; t < HT; t++)
 #pragma unroll
         for (int q = 0; q < 4; q++)
         {
-            const v4f v = *reinterpret_cast<const v4f*>(take + (t * 4 + q) * 1024);
+            const word4_t v = *reinterpret_cast<const word4_t*>(take + (t * 4 + q) * 1024);
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 sum[t][4 * q + e] = v[e] + (IT == 2 ? acc[0][t][4 * q + e] : (kg ? acc[0][1][4 * q + e] : acc[0][0][4 * q + e]));
@@ -315,35 +348,72 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
     __syncthreads();
 
     // ---- results: gathered by pixel, so that whole lines leave ----------------------------------------------------
-    constexpr int ROW = HT * 64, PITCH = ROW + 16;
+    constexpr int EB = (int)sizeof(T), ROW = HT * 32 * EB, PITCH = ROW + 16;
     uint8_t* tbuf = lds + wave * (32 * PITCH);
     const int oc_w = oc0 + (IT == 2 ? 0 : 32 * kg), p_w = (IT == 2 ? wq * 2 + kg : wq) * 32;
 #pragma unroll
     for (int t = 0; t < HT; t++)
     {
+        const int at = oc_w - oc0 + 32 * t + 16 * h;    // the lane's channels
         alignas(16) T packed[16];
-#pragma unroll
-        for (int q = 0; q < 4; q++)
+        if constexpr (I8)
         {
-            const v4f b = *reinterpret_cast<const v4f*>(tab_bias + oc_w - oc0 + 32 * t + 16 * h + 4 * q);
+            if (p_w + rho < pixels && oc0 + at < a.N)
+            {
+                v4i out;
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                store_from_float(packed + 4 * q + e, sum[t][4 * q + e] + b[e]);
+                for (int q = 0; q < 4; q++)
+                {
+                    v4i b = *reinterpret_cast<const v4i*>(tab_bias + at + 4 * q);
+                    if (a.za != 0)
+                    {
+                        v4i ws = *reinterpret_cast<const v4i*>(tab_wsum + at + 4 * q);
+#pragma unroll
+                        for (int part = 1; part < 4; part++)
+                            ws += *reinterpret_cast<const v4i*>(tab_wsum + part * 64 + at + 4 * q);
+                        b -= a.za * ws;
+                    }
+                    int word = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                    {
+                        const ChannelScale cs = tab_cs[at + 4 * q + e];
+                        word |= (fast_rescale(sum[t][4 * q + e] + b[e], cs, a.rp.out_zp, a.rp.lo, a.rp.hi, flags) & 0xff) << (8 * e);
+                    }
+                    out[q] = word;
+                }
+                *reinterpret_cast<v4i*>(tbuf + rho * PITCH + t * 32 + h * 16) = out;
+            }
         }
-        uint8_t* d = tbuf + rho * PITCH + t * 64 + h * 32;
-        reinterpret_cast<v4i*>(d)[0] = reinterpret_cast<const v4i*>(packed)[0];
-        reinterpret_cast<v4i*>(d)[1] = reinterpret_cast<const v4i*>(packed)[1];
+        else
+        {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+            {
+                const v4f b = *reinterpret_cast<const v4f*>(tab_bias + at + 4 * q);
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    store_from_float(packed + 4 * q + e, sum[t][4 * q + e] + b[e]);
+            }
+            uint8_t* d = tbuf + rho * PITCH + t * 64 + h * 32;
+            reinterpret_cast<v4i*>(d)[0] = reinterpret_cast<const v4i*>(packed)[0];
+            reinterpret_cast<v4i*>(d)[1] = reinterpret_cast<const v4i*>(packed)[1];
+        }
     }
-    constexpr int PIECES = ROW / 16, RPI = 64 / PIECES;
-    uint8_t* to = reinterpret_cast<uint8_t*>(a.out) + (((size_t)(image * a.OH + oy0) * a.OW + p_w) * a.N + oc_w) * 2;
+    // (pieces of eight channels)
+    using piece_t        = std::conditional_t<I8, v2i, v4i>;
+    constexpr int PIECES = ROW / (8 * EB), RPI = 64 / PIECES;
+    uint8_t* to = reinterpret_cast<uint8_t*>(a.out) + (((size_t)(image * a.OH + oy0) * a.OW + p_w) * a.N + oc_w) * EB;
 #pragma unroll
     for (int j = 0; j < 32 / RPI; j++)
     {
-        const int row = lane / PIECES + RPI * j, piece = lane % PIECES;
-        const v4i d   = *reinterpret_cast<const v4i*>(tbuf + row * PITCH + piece * 16);
+        const int row   = lane / PIECES + RPI * j, piece = lane % PIECES;
+        const piece_t d = *reinterpret_cast<const piece_t*>(tbuf + row * PITCH + piece * 8 * EB);
         if (p_w + row < pixels && oc_w + piece * 8 < a.N)
-            *reinterpret_cast<v4i*>(to + (size_t)row * a.N * 2 + piece * 16) = d;
+            *reinterpret_cast<piece_t*>(to + ((size_t)row * a.N + piece * 8) * EB) = d;
     }
+    if constexpr (I8)
+        raise_flags(a.flag_word, flags);
 }
 
 struct PlanesPlan
@@ -355,10 +425,10 @@ struct PlanesPlan
 };
 
 // The tile of whole output rows that takes the chip the shortest time
-static PlanesPlan plan_planes(const ConvGeom& g)
+static PlanesPlan plan_planes(const ConvGeom& g, int eb)
 {
     PlanesPlan best;
-    const int64_t slices = ((int64_t)g.IC * 2 + 127) / 128, taps = (int64_t)g.KH * g.KW, tn = (g.OC + 63) / 64;
+    const int64_t slices = ((int64_t)g.IC * eb + 127) / 128, taps = (int64_t)g.KH * g.KW, tn = (g.OC + 63) / 64;
     const int64_t patch_w = (int64_t)(g.OW - 1) * g.stride_x + (int64_t)(g.KW - 1) * g.dil_x + 1;
     for (int rows = 1; rows <= g.OH && (int64_t)rows * g.OW <= 256; rows++)
     {
@@ -380,8 +450,8 @@ static PlanesPlan plan_planes(const ConvGeom& g)
 
 static bool planes_take(int32_t in_dtype, const ConvGeom& g)
 {
-    const int64_t taps = (int64_t)g.KH * g.KW, icb = (int64_t)g.IC * 2;
-    return (in_dtype == TMI_FP16 || in_dtype == TMI_BF16) && taps >= 3 && taps <= 64 && g.IC % 8 == 0 && g.OC % 8 == 0 && g.OW <= 256 && icb * taps * g.OC < INT32_MAX &&
+    const int64_t taps = (int64_t)g.KH * g.KW, icb = (int64_t)g.IC * (in_dtype == TMI_INT8 ? 1 : 2);
+    return (in_dtype == TMI_FP16 || in_dtype == TMI_BF16 || in_dtype == TMI_INT8) && taps >= 3 && taps <= 64 && icb % 16 == 0 && g.OC % 8 == 0 && g.OW <= 256 && icb * taps * g.OC < INT32_MAX &&
            (int64_t)g.IH * g.IW * icb < INT32_MAX;
 }
 
@@ -393,34 +463,42 @@ static bool planes_take(int32_t in_dtype, const ConvGeom& g)
 //     18.6 / 21.1 (39), [2,26,26,192]->88 1.24 times (35).
 //   the GEMM kernel, only with tiles of up to 128 pixels and whole slices: [14,22,22,384]->176 31.8 / 18.8, 5x5 [24,52,10,64]->128 15.2 / 10.6, [10,22,22,128]->296 20.7 / 17.7; else
 //     [16,28,28,256]->256 (196 pixels) 20.2 / 21.5, [16,40,15,160]->136 (two and a half slices) 12.6 / 13.0.
+//   int8 with RESCALE, where the patch kernel has the layer, at most a third of the slices cut off: [8,29,29,208]->248 19.8 / 13.1, [14,30,30,592]->96 30.9 / 23.1, [4,31,36,480]->240 25.7 / 19.6, 5x5
+//     [18,20,20,624]->64 85 / 48; over 36 of them 0.56 ... 0.94; beyond a third [3,61,61,160]->176 19.0 / 17.8, [10,25,94,176]->64 12.7 / 13.4.  The kernels with resident weights
+//     or split reductions keep theirs: of 83 layers 9 gained, [11,7,8,416]->616 10.4 / 17.8, [8,30,86,160]->128 14.4 / 18.0.
 bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, bool to_gemm)
 {
     if (!planes_take(in_dtype, g))
         return false;
-    const PlanesPlan p = plan_planes(g);
+    const int eb       = in_dtype == TMI_INT8 ? 1 : 2;
+    const PlanesPlan p = plan_planes(g, eb);
     if (p.rows == 0 || p.tiles > 256 || p.slices * g.KH * g.KW < 18)
         return false;
+    if (in_dtype == TMI_INT8)
+        return p.slices * 128 * 3 <= (int64_t)g.IC * 4;
     if (to_gemm)
-        return !p.wide && g.IC % 64 == 0;
-    if (p.slices == 1 && g.IC < 64)    // (a slice cut short and no other under which a patch is fetched: 5x5 [5,47,47,48]->48 10.2 / 11.9)
+        return !p.wide && g.IC * eb % 128 == 0;
+    if (p.slices == 1 && g.IC * eb < 128)    // (a slice cut short and no other under which a patch is fetched: 5x5 [5,47,47,48]->48 10.2 / 11.9)
         return false;
     return 2e-6 * (double)g.N * g.OH * g.OW * g.OC * g.IC * g.KH * g.KW >= 115 * p.us;
 }
 
-bool launch_conv_planes(hipStream_t st, int32_t in_dtype, const ConvGeom& g, const void* in, const void* w, const void* bias, const void* pad_page, void* out)
+bool launch_conv_planes(hipStream_t st, int32_t in_dtype, const ConvGeom& g, const void* in, const void* w, const void* bias, const void* pad_page,
+                        const void* zeros, int32_t in_zp, const RescaleParams& rp, uint32_t* flag_word, void* out)
 {
-    if (!planes_take(in_dtype, g) || (((uintptr_t)in | (uintptr_t)w | (uintptr_t)out | (uintptr_t)pad_page) & 15) != 0)
+    if (!planes_take(in_dtype, g) || (in_dtype == TMI_INT8) != (rp.enabled != 0) || (rp.enabled && !rp.fast) || (((uintptr_t)in | (uintptr_t)w | (uintptr_t)out | (uintptr_t)pad_page) & 15) != 0)
         return false;
-    const PlanesPlan p = plan_planes(g);
+    const int eb       = in_dtype == TMI_INT8 ? 1 : 2;
+    const PlanesPlan p = plan_planes(g, eb);
     if (p.rows == 0)
         return false;
-    const int64_t icb = (int64_t)g.IC * 2, taps = (int64_t)g.KH * g.KW, kb = icb * taps, tn = (g.OC + 63) / 64, tiles_m = (int64_t)g.N * p.tiles_image;
+    const int64_t icb = (int64_t)g.IC * eb, taps = (int64_t)g.KH * g.KW, kb = icb * taps, tn = (g.OC + 63) / 64, tiles_m = (int64_t)g.N * p.tiles_image;
     PlanesArgs a{};
     a.patch_w = (int32_t)((int64_t)(g.OW - 1) * g.stride_x + (int64_t)(g.KW - 1) * g.dil_x + 1);
     if (p.tiles > (1 << 22) || !fastdiv_exact_up_to((uint64_t)p.tiles, (uint32_t)tn) || !fastdiv_exact_up_to((uint64_t)tiles_m, (uint32_t)p.tiles_image) ||
         !fastdiv_exact_up_to((uint64_t)p.patch_pixels + 8, (uint32_t)a.patch_w) || !fastdiv_exact_up_to(256, (uint32_t)g.OW))
         return false;
-    a.x = (const uint8_t*)in, a.w = (const uint8_t*)w, a.pad_page = (const uint8_t*)pad_page, a.bias = bias, a.out = out;
+    a.x = (const uint8_t*)in, a.w = (const uint8_t*)w, a.pad_page = (const uint8_t*)pad_page, a.zeros = (const uint8_t*)zeros, a.bias = bias, a.out = out;
     a.N = g.OC, a.kb = (int32_t)kb, a.icb = (int32_t)icb, a.slices = (int32_t)p.slices, a.taps = (int32_t)taps, a.KW = g.KW;
     a.IH = g.IH, a.IW = g.IW, a.OH = g.OH, a.OW = g.OW;
     a.sy = g.stride_y, a.sx = g.stride_x, a.dy = g.dil_y, a.dx = g.dil_x, a.pad_top = g.pad_top, a.pad_left = g.pad_left;
@@ -429,13 +507,16 @@ bool launch_conv_planes(hipStream_t st, int32_t in_dtype, const ConvGeom& g, con
     a.tiles = (int32_t)p.tiles, a.per_xcd = (int32_t)((p.tiles + 7) / 8);
     a.tiles_n = make_fastdiv((uint32_t)tn), a.tiles_image = make_fastdiv((uint32_t)p.tiles_image);
     a.div_pw = make_fastdiv((uint32_t)a.patch_w), a.div_ow = make_fastdiv((uint32_t)g.OW);
-    const size_t lds = (size_t)kPlanesRing * 8192 + 2 * (size_t)a.buffer_bytes + 256;    // and the bias
+    a.za = in_zp, a.rp = rp, a.flag_word = flag_word;
+    const size_t lds = (size_t)kPlanesRing * 8192 + 2 * (size_t)a.buffer_bytes + 256 + 64 * 32;    // and the tables
     auto run = [&](auto kernel) {
         if (!ensure_dynamic_lds<kernel.value>(lds))
             return false;
         hipLaunchKernelGGL(kernel.value, dim3((unsigned)(a.per_xcd * 8)), dim3(512), lds, st, a);
         return true;
     };
+    if (in_dtype == TMI_INT8)
+        return p.wide ? run(kernel_constant<conv_planes_kernel<int8_t, 2>>{}) : run(kernel_constant<conv_planes_kernel<int8_t, 1>>{});
     if (in_dtype == TMI_FP16)
         return p.wide ? run(kernel_constant<conv_planes_kernel<_Float16, 2>>{}) : run(kernel_constant<conv_planes_kernel<_Float16, 1>>{});
     return p.wide ? run(kernel_constant<conv_planes_kernel<bf16_t, 2>>{}) : run(kernel_constant<conv_planes_kernel<bf16_t, 1>>{});

@@ -658,36 +658,38 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         return launch_conv2d_taps(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                   ctx->pages_dev + (d->in_dtype == TMI_INT8 ? (in_zp & 255) * 64 : 0), ctx->flags_dev);
     };
-    // 16-bit layers with taps, one round of workgroups and a reduction of some length: the patch streams through LDS.  With the fp16 / bf16 name of the
-    // kernel that has the layer otherwise.  row_bytes: of the channel vectors that kernel would see.
-    auto launch_planes = [&](int32_t row_bytes) {
-        if (depthwise || ctx->kernel_choice != 0 || out_dtype != d->in_dtype || rp.enabled || (d->in_dtype != TMI_FP16 && d->in_dtype != TMI_BF16))
+    // Layers with taps, one round of workgroups and a reduction of some length: the patch streams through LDS.  With the name of the kernel that has
+    // the layer otherwise.  row_bytes: of the channel vectors that kernel would see; int8 layers (fused RESCALE) only where the patch kernel has them.
+    auto launch_planes = [&](int32_t row_bytes, bool at_patch_kernel) {
+        const bool i8 = d->in_dtype == TMI_INT8, f16 = d->in_dtype == TMI_FP16;
+        if (depthwise || ctx->kernel_choice != 0 || out_dtype != d->in_dtype || i8 != at_patch_kernel || (i8 ? !rp.enabled || !rp.fast || w_zp != 0 : rp.enabled) ||
+            (!i8 && !f16 && d->in_dtype != TMI_BF16))
             return;
         // (what is too short or too small for it in any case, before anything is planned: some 0.1 us of the host's time)
-        if ((row_bytes + 127) / 128 * g.KH * g.KW < 18 || total * row_bytes / 2 * g.KH * g.KW < 400000000)
+        if ((row_bytes + 127) / 128 * g.KH * g.KW < 18 || total * g.IC * g.KH * g.KW < 400000000)
             return;
         ConvGeom seen         = g;
-        seen.IC               = row_bytes / 2;
+        seen.IC               = i8 ? row_bytes : row_bytes / 2;
         const int64_t pixels  = (int64_t)g.N * g.OH * g.OW;
         const bool patch_form = gemm_patch_form(seen, d->in_dtype);
-        const bool to_gemm    = row_bytes % 64 == 0 && g.OC >= 64 && pixels >= 128 && gemm_mfma_preferred(d->in_dtype, seen) &&
+        const bool to_gemm    = !i8 && row_bytes % 64 == 0 && g.OC >= 64 && pixels >= 128 && gemm_mfma_preferred(d->in_dtype, seen) &&
                              (patch_form || (pixels + 127) / 128 * ((g.OC + 127) / 128) >= 96);
-        if (!conv_planes_leads(d->in_dtype, seen, to_gemm) || !launch_conv_planes(ctx->stream, d->in_dtype, g, in, w, bias, ctx->pages_dev, out))
+        if (!conv_planes_leads(d->in_dtype, seen, to_gemm) ||
+            !launch_conv_planes(ctx->stream, d->in_dtype, g, in, w, bias, ctx->pages_dev + (i8 ? (in_zp & 255) * 64 : 0), ctx->pages_dev, in_zp, rp, ctx->flags_dev, out))
             return;
-        const bool f16 = d->in_dtype == TMI_FP16;
         if (to_gemm && patch_form)
             name = f16 ? "gemm_mfma_f16_patch" : "gemm_mfma_bf16_patch";
         else if (to_gemm)
             name = f16 ? "gemm_mfma_f16" : "gemm_mfma_bf16";
         else
-            name = f16 ? "conv2d_mfma_f16" : "conv2d_mfma_bf16";
+            name = i8 ? "conv2d_mfma_i8_rescale" : f16 ? "conv2d_mfma_f16" : "conv2d_mfma_bf16";
     };
     // Channel vectors of no whole steps, where kernels that need whole ones lead by more than the copies cost
     if (!depthwise && ctx->kernel_choice == 0 && own_scratch && w_zp == 0)
     {
         int32_t padded = padded_channel_bytes(d->in_dtype, g, total, rp.enabled);
         if (padded)
-            launch_planes(padded);
+            launch_planes(padded, false);
         if (name)
             return after_launch(ctx, name);
         // Results off 16 bytes or 16-bit multipliers: the kernels that lead on whole steps decline, and the patch kernel has the layer either way;
@@ -750,7 +752,7 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         const bool gemm_ok   = ctx->kernel_choice == 0 || ctx->kernel_choice == 3;
         const bool patch_ok  = ctx->kernel_choice == 0 || ctx->kernel_choice == 2;
         const bool gemm_1st  = gemm_ok && (!patch_ok || gemm_mfma_preferred(d->in_dtype, g));
-        launch_planes(t_row);
+        launch_planes(t_row, false);
         if (name)
             return after_launch(ctx, name);
         // A pointwise layer with int32 results and more than 2 M of them: the GEMM kernel, whose results leave as
@@ -916,6 +918,8 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         const bool long_windows = taps > 9 && taps <= 25 && t_row == 64 && t_tiles > 960 && t_tiles <= 1400;
         if (!name && !long_and_many && !patch_filled && !short_rows && !long_windows && taps_open())
             name = launch_taps();
+        if (!name && patch_ok)
+            launch_planes(t_row, true);
         if (!name && patch_ok)
             name = launch_conv2d_mfma(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                       ctx->flags_dev);

@@ -151,10 +151,11 @@ OrderedForm launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, cons
                          const void* bias, bool abs_mode, const double* input_abs_max, void* out);
 OrderedForm launch_ordered_matmul(hipStream_t st, int32_t in_dtype, bool f64, int32_t N, int32_t H, int32_t C, int32_t W, const void* a,
                            const void* b, bool abs_mode, void* out);
-// conv_planes.hip: CONV2D with taps on 16-bit floats, results of the same type; pad_page: 16 zero bytes.  False: not taken.  _leads: whether it
-// should be; to_gemm: the layer is the GEMM kernel's otherwise.
+// conv_planes.hip: CONV2D with taps on 16-bit floats (results of the same type) or int8 (weights' zero point 0, fused RESCALE to int8 in its fast form);
+// pad_page: 16 bytes of in_zp, zeros: 16 zero bytes.  False: not taken.  _leads: whether it should be; to_gemm: the layer is the GEMM kernel's otherwise.
 bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, bool to_gemm);
-bool launch_conv_planes(hipStream_t st, int32_t in_dtype, const ConvGeom& g, const void* in, const void* w, const void* bias, const void* pad_page, void* out);
+bool launch_conv_planes(hipStream_t st, int32_t in_dtype, const ConvGeom& g, const void* in, const void* w, const void* bias, const void* pad_page,
+                        const void* zeros, int32_t in_zp, const RescaleParams& rp, uint32_t* flag_word, void* out);
 // ordered_staged.hip: the same for CONV2D on whole units of eight channels; _leads: whether a layer runs there.
 bool ordered_staged_leads(int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w);
 OrderedForm launch_ordered_conv_staged(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w, const void* bias,

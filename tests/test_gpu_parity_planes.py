@@ -6,6 +6,7 @@ import pytest
 
 import cases
 import gpu_ops
+import oracle
 from reference_model_amd import Context, capi
 
 pytestmark = pytest.mark.gpu
@@ -49,4 +50,33 @@ def test_small_whole_numbers(ctx, kind, shape):
         want = cases.float_to_bf16_bits(want.astype(np.float32))
     assert st == capi.VALID
     print(shape, ctx.last_kernel)
+    assert np.array_equal(got, want)
+
+
+I8_SHAPES = [  # the same for int8 with the fused RESCALE
+    (14, 30, 30, 592, 96, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
+    (32, 13, 10, 480, 136, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
+    (9, 33, 41, 256, 72, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1)),
+    (12, 30, 28, 768, 128, 1, 3, (0, 0, 1, 1), (1, 1), (1, 1)),
+    (27, 40, 40, 400, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
+    (16, 29, 29, 512, 264, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1)),
+]
+
+
+@pytest.mark.parametrize("in_zp, double_round, clamp", [(0, True, None), (-128, False, (-100, 90)), (17, True, (5, 127))])
+@pytest.mark.parametrize("shape", I8_SHAPES)
+def test_int8_rescale(ctx, shape, in_zp, double_round, clamp):
+    n, ih, iw, ic, oc, kh, kw, pad, stride, dil = shape
+    rng = np.random.default_rng(ic + oc + in_zp)
+    x = rng.integers(-128, 128, (n, ih, iw, ic)).astype(np.int8)
+    w = rng.integers(-128, 128, (oc, kh, kw, ic)).astype(np.int8)
+    bias = rng.integers(-(1 << 18), 1 << 18, oc).astype(np.int32)
+    mult = rng.integers(1 << 30, (1 << 31) - 1, oc).astype(np.int32)
+    shift = rng.integers(41, 45, oc).astype(np.int8)
+    mode = capi.ROUND_DOUBLE if double_round else capi.ROUND_SINGLE
+    want, wst = oracle.rescale(cases.conv2d_exact_blas(x, w, bias, pad, stride, dil, in_zp), mult, shift, out_zp=5, rounding_mode=mode)
+    if clamp:
+        want = oracle.clamp(want, *clamp)
+    got, st = gpu_ops.conv2d(ctx, x, w, bias, pad, stride, dil, in_zp=in_zp, rescale=dict(mult=mult, shift=shift, out_zp=5, rounding_mode=mode), clamp=clamp)
+    assert st == wst == capi.VALID
     assert np.array_equal(got, want)
