@@ -34,6 +34,7 @@ struct PlanesArgs
     int32_t buffer_bytes;              // of a slice's patch in LDS
     int32_t tiles, per_xcd;
     FastDiv tiles_n, tiles_image, div_pw, div_ow;
+    int32_t padded;         // a tap can fall outside the image
     int32_t za;             // int8: the input's zero point; the weights' is 0
     RescaleParams rp;
     uint32_t* flag_word;    // where its REQUIRE conditions are latched
@@ -400,6 +401,43 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
             reinterpret_cast<v4i*>(d)[1] = reinterpret_cast<const v4i*>(packed)[1];
         }
     }
+    // A tap outside the image adds nothing in the reference (tensor_ops.cpp:856-862); here it added 0 * weight, which is NaN where the weight is infinite
+    // or NaN.  A lane with such sums makes them again without those taps.
+    if constexpr (!I8)
+        if (a.padded)
+        {
+            uint32_t odd = 0;
+#pragma unroll
+            for (int t = 0; t < HT; t++)
+#pragma unroll
+                for (int e = 0; e < 16; e += 2)
+                    odd |= __builtin_isunordered(sum[t][e], sum[t][e + 1]) ? 3u << (16 * t + e) : 0u;
+            if (p_w + rho >= pixels)
+                odd = 0;
+            while (odd)
+            {
+                const int i = __builtin_ctz(odd), t = i >> 4, oc = oc_w + 32 * t + 16 * h + (i & 15);
+                odd &= odd - 1;
+                if (oc >= a.N)
+                    break;
+                const int py = (int)fdiv((uint32_t)(p_w + rho), a.div_ow), yb = (oy0 + py) * a.sy - a.pad_top, xb = (p_w + rho - py * a.OW) * a.sx - a.pad_left;
+                const int channels = a.icb / EB, KH = a.taps / a.KW;
+                const T* wt = reinterpret_cast<const T*>(a.w + (size_t)oc * a.kb);
+                float again = 0;
+                for (int ky = 0; ky < KH; ky++)
+                    for (int kx = 0; kx < a.KW; kx++, wt += channels)
+                    {
+                        const int iy = yb + ky * a.dy, ix = xb + kx * a.dx;
+                        if ((uint32_t)iy < (uint32_t)a.IH && (uint32_t)ix < (uint32_t)a.IW)
+                        {
+                            const T* px = reinterpret_cast<const T*>(x + (uint32_t)((iy * a.IW + ix) * a.icb));
+                            for (int c = 0; c < channels; c++)
+                                again += load_as_float<T>(px, c) * load_as_float<T>(wt, c);
+                        }
+                    }
+                store_from_float(reinterpret_cast<T*>(tbuf + rho * PITCH + t * 64 + h * 32) + (i & 15), again + tab_bias[oc - oc0]);
+            }
+        }
     // (pieces of eight channels)
     using piece_t        = std::conditional_t<I8, v2i, v4i>;
     constexpr int PIECES = ROW / (8 * EB), RPI = 64 / PIECES;
@@ -507,6 +545,8 @@ bool launch_conv_planes(hipStream_t st, int32_t in_dtype, const ConvGeom& g, con
     a.tiles = (int32_t)p.tiles, a.per_xcd = (int32_t)((p.tiles + 7) / 8);
     a.tiles_n = make_fastdiv((uint32_t)tn), a.tiles_image = make_fastdiv((uint32_t)p.tiles_image);
     a.div_pw = make_fastdiv((uint32_t)a.patch_w), a.div_ow = make_fastdiv((uint32_t)g.OW);
+    a.padded = g.pad_top > 0 || g.pad_left > 0 || (int64_t)(g.OH - 1) * g.stride_y - g.pad_top + (int64_t)(g.KH - 1) * g.dil_y >= g.IH ||
+               (int64_t)(g.OW - 1) * g.stride_x - g.pad_left + (int64_t)(g.KW - 1) * g.dil_x >= g.IW;
     a.za = in_zp, a.rp = rp, a.flag_word = flag_word;
     const size_t lds = (size_t)kPlanesRing * 8192 + 2 * (size_t)a.buffer_bytes + 256 + 64 * 32;    // and the tables
     auto run = [&](auto kernel) {

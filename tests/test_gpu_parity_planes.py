@@ -53,6 +53,29 @@ def test_small_whole_numbers(ctx, kind, shape):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("shape", [(7, 14, 21, 200, 288), (16, 28, 28, 256, 64)])
+def test_infinite_weights_outside_the_image(ctx, shape):
+    """a tap outside the image adds nothing, also where its weight is infinite or NaN"""
+    n, ih, iw, ic, oc = shape
+    rng = np.random.default_rng(3)
+    x = rng.integers(1, 4, (n, ih, iw, ic)).astype(np.float16)
+    w = rng.integers(-2, 3, (oc, 3, 3, ic)).astype(np.float16)
+    w[:, :, :, 0] = 1
+    plain = w.copy()
+    w[3, 0, 0, 5], w[oc - 1, 1, 2, ic - 1], w[8, 2, 2, 1] = np.inf, np.nan, -np.inf    # the top left tap, right, bottom right
+    b = np.zeros(oc, np.float16)
+    want, _ = gpu_ops.conv2d(ctx, x, plain, b, (1, 1, 1, 1), dtype=capi.FP16)
+    got, st = gpu_ops.conv2d(ctx, x, w, b, (1, 1, 1, 1), dtype=capi.FP16)
+    assert st == capi.VALID
+    # without a channel of the tap that lies outside: the results of finite weights there
+    one = [c for c in range(oc) if c not in (3, 8, oc - 1)]
+    assert np.array_equal(got[..., one], want[..., one])
+    assert np.array_equal(got[:, 0, :, 3], want[:, 0, :, 3]) and np.array_equal(got[:, :, 0, 3], want[:, :, 0, 3])
+    assert np.isposinf(got[:, 1:, 1:, 3]).all()
+    assert np.array_equal(got[:, -1, :, 8], want[:, -1, :, 8]) and np.isneginf(got[:, :-1, :-1, 8]).all()
+    assert np.array_equal(got[:, :, -1, oc - 1], want[:, :, -1, oc - 1]) and np.isnan(got[:, :, :-1, oc - 1]).all()
+
+
 I8_SHAPES = [  # the same for int8 with the fused RESCALE
     (14, 30, 30, 592, 96, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
     (32, 13, 10, 480, 136, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
