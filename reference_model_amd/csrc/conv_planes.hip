@@ -6,7 +6,7 @@
 // stage.  Two groups of four waves take half of a stage's channels each, so that a wave owns 64 channels x IT * 32 pixels and reads four (IT 1: three)
 // fragments for four (two) matrix instructions; after the loop a wave hands half of its sums to its partner.
 //
-// What bounds it: on few tiles the chain of a stage (0.215 us, 0.11 of it matrix instructions; 0.416 of 0.21 with 256 pixels), on all CUs the clock under the
+// What bounds it: on few tiles the instructions of a stage (0.21 us, 0.11 of it matrix instructions; 0.41 of 0.21 with 256 pixels), on all CUs the clock under the
 // matrix instructions: [16,28,28,256]->256 3x3 14.9 us without any operand in the loop, 18.8 with its fragment reads.  A wave's loads straight into LDS go
 // one after the other, 0.3 us each, so the second group fetches the patch through registers (all loads straight into LDS: 26.2, so 21.5), in a loop of its own,
 // or the compiler has the first group wait for them too (28.9).
@@ -88,8 +88,9 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
     const int whole = a.icb >> 7;    // slices of 128 bytes
     int l_tap = 0, l_slice = 0;      // the next stage whose weights are requested; past the end the last slice again, which nobody reads
     const uint8_t* l_base = a.w;
-    auto load_weights = [&](int slot) {
-        const uint32_t dst = lds0 + slot * STAGE + wq * 2048;
+    const uint32_t w_dst = lds0 + wq * 2048;
+    auto load_weights = [&](int slot_at) {
+        const uint32_t dst = w_dst + slot_at;
         if (l_slice < whole)
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %3\n\ts_add_u32 m0, %2, 1024\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3"
                          :
@@ -164,42 +165,45 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
     {
 #pragma unroll
         for (int s = 0; s < D - 1; s++)
-            load_weights(s);
+            load_weights(s * STAGE);
     }
 
     // ---- fragments --------------------------------------------------------------------------------------------
     // Tile i of the wave is the workgroup's pixel tile wq * IT + (i ^ kg): the one it stores (IT 2) first.
     const int w_frag = channel_of_row(rho);
     const uint32_t aw0 = (uint32_t)(w_frag * 128 + (((4 * kg + h) ^ planes_key(w_frag)) * 16));
-    int pbase[IT], pkey[IT];
+    uint32_t pbase[IT];    // byte of the patch under the first tap, and its position for the key
+    int pkey[IT];
 #pragma unroll
     for (int i = 0; i < IT; i++)
     {
         int p = (wq * IT + (IT == 2 ? i ^ kg : 0)) * 32 + rho;
         p     = p < pixels ? p : 0;    // (not stored)
         const int py = (int)fdiv((uint32_t)p, a.div_ow);
-        pbase[i]     = py * a.sy * a.patch_w + (p - py * a.OW) * a.sx;
+        pbase[i]     = (uint32_t)(py * a.sy * a.patch_w + (p - py * a.OW) * a.sx) * 128u;
         pkey[i]      = py * a.sy * a.OW + (p - py * a.OW) * a.sx;
     }
-    // where the stage read next lies
-    uint32_t aw = aw0, ap[IT];
-    int tap = 0, kx = 0, slice = 0, tap_at = 0, tap_key = 0, slot = 0;
+    // Where the stage read next lies: its weights, its tap in the slice's patch (byte and position).  Scalars that go on by additions: a stage of few tiles is
+    // as long as its instructions.
+    const int dx_at = a.dx * 128, row_at = (a.dy * a.patch_w - a.KW * a.dx) * 128, row_key = a.dy * a.OW - a.KW * a.dx;
+    uint32_t aw = aw0, ap[IT], w_at_stage = 0, patch_at = D * STAGE, tap_at = patch_at;
+    int taps_left = a.taps, kx_left = a.KW, tap_key = 0;
     auto address = [&](int i) {    // of pixel tile i; of the weights
         if (i == IT)
-            aw = aw0 + (uint32_t)slot * STAGE;
+            aw = aw0 + w_at_stage;
         else
-        {
-            const int pp = pbase[i] + tap_at;
-            ap[i] = (uint32_t)(D * STAGE + (slice & 1) * a.buffer_bytes + pp * 128 + (((4 * kg + h) ^ planes_key(pkey[i] + tap_key)) * 16));
-        }
+            ap[i] = pbase[i] + tap_at + (uint32_t)(((4 * kg + h) ^ planes_key(pkey[i] + tap_key)) << 4);
     };
     auto next_stage = [&]() {
-        slot = (slot + 1) & (D - 1);
-        kx++, tap++, tap_at += a.dx, tap_key += a.dx;
-        if (kx == a.KW)
-            kx = 0, tap_at += a.dy * a.patch_w - a.KW * a.dx, tap_key += a.dy * a.OW - a.KW * a.dx;
-        if (tap == a.taps)
-            tap = 0, tap_at = 0, tap_key = 0, slice++;
+        w_at_stage = (w_at_stage + STAGE) & (D * STAGE - 1);
+        tap_at += dx_at, tap_key += a.dx;
+        if (--kx_left == 0)
+            kx_left = a.KW, tap_at += row_at, tap_key += row_key;
+        if (--taps_left == 0)
+        {
+            patch_at  = 2 * D * STAGE + (uint32_t)a.buffer_bytes - patch_at;    // the other buffer
+            taps_left = a.taps, tap_at = patch_at, tap_key = 0;
+        }
     };
     using acc_t = typename Mma<T>::acc_t;
     acc_t acc[IT][2];
@@ -283,13 +287,13 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
     if (!kg)
     {
         // the next stage's weights, with those of D - 3 later ones on their way
-        int free_slot = D - 1;
+        int free_slot = (D - 1) * STAGE;
 #pragma unroll 1
         for (int s = a.slices * a.taps; s > 0; s--)
             stage([]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (D - 3)) : "memory"); },
                   [&]() {
                       load_weights(free_slot);
-                      free_slot = (free_slot + 1) & (D - 1);
+                      free_slot = (free_slot + STAGE) & (D * STAGE - 1);
                   });
     }
     else
@@ -497,8 +501,8 @@ static bool planes_take(int32_t in_dtype, const ConvGeom& g)
 //   the patch kernel (conv2d_mfma.hip): [16,14,14,512]->512 40.1 / 24.2, [16,28,28,256]->64 20.7 / 13.4, [26,10,22,376]->160 32.8 / 20.8, 5x5 [2,20,20,480]->592 129 / 53,
 //     [11,58,21,96]->96 30.9 / 19.3, stride 2 [14,36,28,328]->240 46.9 / 22.7; over 34 of them 0.41 ... 0.96.  Two rounds: [4,29,109,136]->136 19.7 / 26.9,
 //     [22,75,13,288]->144 stride 2 27.6 / 34.6; 9 stages: [20,50,50,64]->72 stride 2 11.5 / 13.3, [11,28,28,32]->104 5.9 / 7.6.
-//   split reductions (conv_taps.hip), from 115 TFLOP/s predicted on: [2,18,18,384]->448 26.4 / 17.9, [7,14,21,200]->288 19.9 / 14.7; below [3,14,14,512]->160
-//     18.6 / 21.1 (39), [2,26,26,192]->88 1.24 times (35).
+//   split reductions (conv_taps.hip), from 106 TFLOP/s predicted on: [2,18,18,384]->448 (115) 26.4 / 17.9, [2,54,54,512]->48 (107) 33.9 / 23.2, [7,14,21,200]->288 19.9 / 14.7, the least
+//     gain [1,85,85,88]->96 (108) 11.5 / 11.6; below [4,14,14,448]->320 (103) 17.1 / 19.8, [3,25,25,600]->128 (98) 23.2 / 28.1, [3,14,14,512]->160 (39) 18.6 / 21.1.
 //   the GEMM kernel, only with tiles of up to 128 pixels and whole slices: [14,22,22,384]->176 31.8 / 18.8, 5x5 [24,52,10,64]->128 15.2 / 10.6, [10,22,22,128]->296 20.7 / 17.7; else
 //     [16,28,28,256]->256 (196 pixels) 20.2 / 21.5, [16,40,15,160]->136 (two and a half slices) 12.6 / 13.0.
 //   int8 with RESCALE, where the patch kernel has the layer, at most a third of the slices cut off: [8,29,29,208]->248 19.8 / 13.1, [14,30,30,592]->96 30.9 / 23.1, [4,31,36,480]->240 25.7 / 19.6, 5x5
@@ -518,7 +522,7 @@ bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, bool to_gemm)
         return !p.wide && g.IC * eb % 128 == 0;
     if (p.slices == 1 && g.IC * eb < 128)    // (a slice cut short and no other under which a patch is fetched: 5x5 [5,47,47,48]->48 10.2 / 11.9)
         return false;
-    return 2e-6 * (double)g.N * g.OH * g.OW * g.OC * g.IC * g.KH * g.KW >= 115 * p.us;
+    return 2e-6 * (double)g.N * g.OH * g.OW * g.OC * g.IC * g.KH * g.KW >= 106 * p.us;
 }
 
 bool launch_conv_planes(hipStream_t st, int32_t in_dtype, const ConvGeom& g, const void* in, const void* w, const void* bias, const void* pad_page,
