@@ -10,7 +10,7 @@
 // matrix instructions: [16,28,28,256]->256 3x3 14.9 us without any operand in the loop, 18.8 with its fragment reads.  A wave's loads straight into LDS go
 // one after the other, 0.3 us each, so the second group fetches the patch through registers (all loads straight into LDS: 26.2, so 21.5), in a loop of its own,
 // or the compiler has the first group wait for them too (28.9).
-// us before / here: [16,14,14,512]->512 40.1 / 24.2, [16,28,28,256]->64 20.7 / 13.4, 5x5 [2,20,20,480]->592 129 / 53, stride 2 [14,36,28,328]->240 46.9 / 22.7.
+// us before / here: [16,14,14,512]->512 40.0 / 23.9, [16,28,28,256]->64 20.7 / 13.0, 5x5 [2,20,20,480]->592 129 / 51, stride 2 [14,36,28,328]->240 46.6 / 22.2.
 #include <type_traits>
 
 #include "tmi_mfma.h"
