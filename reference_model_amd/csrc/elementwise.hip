@@ -315,7 +315,7 @@ static const char* launch_rescale_i48(hipStream_t st, const RescaleParams& p, co
     const int64_t visits = (units + 256 * 2 - 1) / (256 * 2), blocks = (units + visits - 1) / visits;
     hipLaunchKernelGGL((rescale_i48_kernel<OutT>), dim3((unsigned)blocks), dim3(256), 0, st, p, (const int64_t*)in, (OutT*)out, rows, C, cgs, rpi,
                        make_fastdiv(cgs), flag_word, (int32_t)blocks);
-    return "rescale_vec";
+    return "rescale_i48";
 }
 
 static int grid_for(int64_t work_items)

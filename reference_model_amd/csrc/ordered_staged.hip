@@ -374,8 +374,8 @@ bool ordered_staged_leads(int32_t in_dtype, bool f64, const ConvGeom& g, const v
     return K >= (eb == 4 && g.IC % 32 == 0 ? 224 : 96);
 }
 
-OrderedForm launch_ordered_conv_staged(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w, const void* bias,
-                                       bool abs_mode, void* out)
+bool launch_ordered_conv_staged(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w, const void* bias, bool abs_mode,
+                                void* out)
 {
     const int64_t pixels = (int64_t)g.N * g.OH * g.OW, K = (int64_t)g.KH * g.KW * g.IC, eb = in_dtype == TMI_FP32 ? 4 : 2;
     const int64_t tn = (g.OC + 63) / 64, tiles = ((pixels + 63) / 64) * tn, over = tiles % 256;
@@ -396,18 +396,15 @@ OrderedForm launch_ordered_conv_staged(hipStream_t st, int32_t in_dtype, bool f6
     p.tiles            = (int32_t)tiles;
     p.n_big            = tiles <= 192 || g.OC <= 32 || !f64 ? 0 : (int32_t)(over <= 192 ? tiles - over : tiles / 8 * 8);
     p.quarters_per_xcd = (int32_t)((4 * (tiles - p.n_big) + 7) / 8);
-    bool launched = false;
     if (!f64)
-        launched = in_dtype == TMI_FP32 && launch_staged<float, false>(st, p, abs_mode);
-    else
-        switch (in_dtype)
-        {
-            case TMI_FP16: launched = launch_staged<_Float16, true>(st, p, abs_mode); break;
-            case TMI_BF16: launched = launch_staged<bf16_t, true>(st, p, abs_mode); break;
-            case TMI_FP32: launched = launch_staged<float, true>(st, p, abs_mode); break;
-            default: break;
-        }
-    return launched ? OrderedForm::quarters : OrderedForm::none;
+        return in_dtype == TMI_FP32 && launch_staged<float, false>(st, p, abs_mode);
+    switch (in_dtype)
+    {
+        case TMI_FP16: return launch_staged<_Float16, true>(st, p, abs_mode);
+        case TMI_BF16: return launch_staged<bf16_t, true>(st, p, abs_mode);
+        case TMI_FP32: return launch_staged<float, true>(st, p, abs_mode);
+        default: return false;
+    }
 }
 
 }    // namespace tmi

@@ -240,8 +240,8 @@ const char* launch_conv_precise(hipStream_t st, int32_t in_dtype, bool depthwise
         a.input_abs_max = abs_max_slot;
     }
     if (!depthwise && !copies && !a.input_abs_max && ordered_staged_leads(in_dtype, true, g, in, w) &&
-        launch_ordered_conv_staged(st, in_dtype, true, g, in, w, bias, abs_mode != 0, out) != OrderedForm::none)
-        return abs_mode ? "conv_bounds_ordered_tail_f64" : "conv_precise_ordered_tail_f64";
+        launch_ordered_conv_staged(st, in_dtype, true, g, in, w, bias, abs_mode != 0, out))
+        return abs_mode ? "conv_bounds_ordered_staged_f64" : "conv_precise_ordered_staged_f64";
     if (!depthwise && copies && launch_ordered_conv_copied(st, in_dtype, true, g, in, w, bias, abs_mode != 0, a.input_abs_max, out, copies))
         return abs_mode ? "conv_bounds_copied_f64" : "conv_precise_copied_f64";
     if (!depthwise)

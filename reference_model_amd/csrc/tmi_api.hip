@@ -658,8 +658,8 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         return launch_conv2d_taps(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                   ctx->pages_dev + (d->in_dtype == TMI_INT8 ? (in_zp & 255) * 64 : 0), ctx->flags_dev);
     };
-    // Layers with taps, one round of workgroups and a reduction of some length: the patch streams through LDS.  With the name of the kernel that has
-    // the layer otherwise.  row_bytes: of the channel vectors that kernel would see; int8 layers (fused RESCALE) only where the patch kernel has them.
+    // Layers with taps, one round of workgroups and a reduction of some length: the patch streams through LDS.  row_bytes: of the channel vectors that the
+    // kernel which has the layer otherwise would see; int8 layers (fused RESCALE) only where that is the patch kernel.
     auto launch_planes = [&](int32_t row_bytes, bool at_patch_kernel) {
         const bool i8 = d->in_dtype == TMI_INT8, f16 = d->in_dtype == TMI_FP16;
         if (depthwise || ctx->kernel_choice != 0 || out_dtype != d->in_dtype || i8 != at_patch_kernel || (i8 ? !rp.enabled || !rp.fast || w_zp != 0 : rp.enabled) ||
@@ -671,18 +671,12 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         ConvGeom seen         = g;
         seen.IC               = i8 ? row_bytes : row_bytes / 2;
         const int64_t pixels  = (int64_t)g.N * g.OH * g.OW;
-        const bool patch_form = gemm_patch_form(seen, d->in_dtype);
         const bool to_gemm    = !i8 && row_bytes % 64 == 0 && g.OC >= 64 && pixels >= 128 && gemm_mfma_preferred(d->in_dtype, seen) &&
-                             (patch_form || (pixels + 127) / 128 * ((g.OC + 127) / 128) >= 96);
+                             (gemm_patch_form(seen, d->in_dtype) || (pixels + 127) / 128 * ((g.OC + 127) / 128) >= 96);
         if (!conv_planes_leads(d->in_dtype, seen, to_gemm) ||
             !launch_conv_planes(ctx->stream, d->in_dtype, g, in, w, bias, ctx->pages_dev + (i8 ? (in_zp & 255) * 64 : 0), ctx->pages_dev, in_zp, rp, ctx->flags_dev, out))
             return;
-        if (to_gemm && patch_form)
-            name = f16 ? "gemm_mfma_f16_patch" : "gemm_mfma_bf16_patch";
-        else if (to_gemm)
-            name = f16 ? "gemm_mfma_f16" : "gemm_mfma_bf16";
-        else
-            name = i8 ? "conv2d_mfma_i8_rescale" : f16 ? "conv2d_mfma_f16" : "conv2d_mfma_bf16";
+        name = i8 ? "conv2d_planes_i8_rescale" : f16 ? "conv2d_planes_f16" : "conv2d_planes_bf16";
     };
     // Channel vectors of no whole steps, where kernels that need whole ones lead by more than the copies cost
     if (!depthwise && ctx->kernel_choice == 0 && own_scratch && w_zp == 0)
@@ -936,8 +930,8 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
     // FP32 sums keep the reference's order: the tiles of ordered_gemm.hip, whose results are the one-result-per-lane kernel's bit
     // for bit
     if (!name && !depthwise && ctx->kernel_choice == 0 && d->in_dtype == TMI_FP32 && ordered_staged_leads(TMI_FP32, false, g, in, w) &&
-        launch_ordered_conv_staged(ctx->stream, TMI_FP32, false, g, in, w, bias, false, out) != OrderedForm::none)
-        name = "conv2d_ordered_tail_f32";
+        launch_ordered_conv_staged(ctx->stream, TMI_FP32, false, g, in, w, bias, false, out))
+        name = "conv2d_ordered_staged_f32";
     if (!name && !depthwise && ctx->kernel_choice == 0 && d->in_dtype == TMI_FP32 && own_scratch)
         if (void* copies = ordered_copies(ctx, ordered_conv_copies_bytes(false, g)))
             if (launch_ordered_conv_copied(ctx->stream, TMI_FP32, false, g, in, w, bias, false, nullptr, out, copies))

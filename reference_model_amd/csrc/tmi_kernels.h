@@ -156,10 +156,10 @@ OrderedForm launch_ordered_matmul(hipStream_t st, int32_t in_dtype, bool f64, in
 bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, bool to_gemm);
 bool launch_conv_planes(hipStream_t st, int32_t in_dtype, const ConvGeom& g, const void* in, const void* w, const void* bias, const void* pad_page,
                         const void* zeros, int32_t in_zp, const RescaleParams& rp, uint32_t* flag_word, void* out);
-// ordered_staged.hip: the same for CONV2D on whole units of eight channels; _leads: whether a layer runs there.
+// ordered_staged.hip: the same for CONV2D on whole units of eight channels; false: not launched.  _leads: whether a layer runs there.
 bool ordered_staged_leads(int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w);
-OrderedForm launch_ordered_conv_staged(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w, const void* bias,
-                                       bool abs_mode, void* out);
+bool launch_ordered_conv_staged(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w, const void* bias, bool abs_mode,
+                                void* out);
 // ordered_copies.hip: the same on copies of the operands in `copies` (ordered_conv_copies_bytes() of 256-byte aligned memory; 0: not taken)
 size_t ordered_conv_copies_bytes(bool f64, const ConvGeom& g);
 bool launch_ordered_conv_copied(hipStream_t st, int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w,

@@ -233,7 +233,7 @@ def test_fp32_conv_and_matmul_compliance_on_the_device(ctx, data_set):
         tx, tw, tb = ctx.upload(xs, capi.FP32), ctx.upload(ws, capi.FP32), ctx.upload(bs, capi.FP32)
         imp, ref, bnd = ctx.empty(shape, capi.FP32), ctx.empty(shape, capi.F64), ctx.empty(shape, capi.F64)
         ctx.conv2d(d, tx, tw, tb, 0, 0, imp)
-        assert ctx.last_kernel == "conv2d_ordered_tail_f32"
+        assert ctx.last_kernel == "conv2d_ordered_staged_f32"
         ctx.conv2d_precise(d, tx, tw, tb, False, ref)
         ctx.conv2d_precise(d, tx, tw, tb, True, bnd)
         r = ctx.dot_product_check(capi.FP32, int(np.prod(shape)), imp, ref, bnd, dp.kernel_size_bound(ks, "fp32"), data_set)

@@ -427,7 +427,8 @@ def test_conv2d_fused_rescale_gemm_reports_require_conditions(ctx):
     (capi.INT8, (64, 7, 7, 640, 512, 3, 1), "gemm_mfma_i8"),           # on 640 channels: the GEMM kernel
     (capi.FP16, (16, 28, 28, 256, 256, 3, 1), "gemm_mfma_f16_patch"),  # 3x3 fp16, deep K, the patch fits the LDS
     (capi.FP16, (8, 28, 28, 512, 512, 3, 1), "gemm_mfma_f16"),         # the same with a patch that does not fit
-    (capi.FP16, (4, 28, 28, 256, 256, 3, 1), "gemm_mfma_f16_patch"),   # 56 tiles of four output rows: enough for the patch form
+    (capi.FP16, (4, 28, 28, 256, 256, 3, 1), "conv2d_planes_f16"),     # 56 tiles of four output rows, one round of at most 128 pixels: the streaming patch
+    (capi.FP16, (4, 28, 28, 224, 256, 3, 1), "gemm_mfma_f16_patch"),   # channels of three and a half of its slices: enough for the patch form
     (capi.INT8, (16, 14, 14, 256, 256, 3, 1), "conv2d_ksplit_patch_i8"),    # 50 tiles, 1.8 G multiply-adds: K split over the waves of small workgroups
     (capi.INT8, (32, 14, 14, 256, 256, 3, 1), "conv2d_ksplit_patch_i8"),       # 98 tiles, 3.7 G
     (capi.INT8, (32, 14, 14, 320, 256, 3, 1), "conv2d_mfma_i8"),       # 4.6 G on 320 channels: too much for that, too few tiles for the GEMM kernel
@@ -435,14 +436,17 @@ def test_conv2d_fused_rescale_gemm_reports_require_conditions(ctx):
     (capi.INT8, (8, 7, 7, 2048, 512, 1, 0), "conv2d_pointwise_split_i8"),    # 2048 channels, 411 M multiply-adds on 16 tiles: K split over waves
     (capi.INT8, (8, 28, 28, 512, 256, 1, 0), "conv2d_slab_i8"),        # pointwise on 512 channels, one round of workgroups: the slab kernel
     (capi.INT8, (16, 28, 28, 512, 256, 1, 0), "gemm_mfma_i8"),         # two rounds: the GEMM kernel
-    (capi.FP16, (2, 28, 28, 256, 256, 3, 1), "conv2d_mfma_f16"),       # 28 tiles: too few
+    (capi.FP16, (2, 28, 28, 256, 256, 3, 1), "conv2d_planes_f16"),     # 28 tiles: too few for the patch form
+    (capi.FP16, (2, 28, 28, 256, 250, 3, 1), "conv2d_mfma_f16"),       # the same with output channels of no whole pieces of eight: the patch kernel
     (capi.FP16, (1, 14, 14, 1024, 1024, 1, 0), "gemm_mfma_f16"),       # pointwise with 16 tiles: still the GEMM kernel
     (capi.FP16, (64, 7, 7, 512, 512, 3, 1), "gemm_mfma_f16"),          # 3x3, no patch form (49 pixels a tile), 100 tiles
-    (capi.FP16, (32, 7, 7, 512, 512, 3, 1), "conv2d_mfma_f16"),        # the same with 52 tiles: the patch kernel
+    (capi.FP16, (32, 7, 7, 512, 512, 3, 1), "conv2d_planes_f16"),      # the same with 52 tiles: the streaming patch
+    (capi.FP16, (32, 7, 7, 512, 508, 3, 1), "conv2d_mfma_f16"),        # and what that one does not take: the patch kernel
     (capi.FP16, (8, 56, 56, 64, 64, 3, 1), "conv2d_slab_f16"),         # 3x3 fp16 on 128-byte channel vectors: the slab kernel
     (capi.FP16, (8, 56, 56, 64, 128, 3, 1), "conv2d_slab_f16"),        # the same with 128 output channels
     (capi.FP16, (32, 56, 56, 64, 128, 3, 1, 2), "gemm_mfma_f16"),      # and with stride 2, 196 tiles: the GEMM kernel's taps form
-    (capi.FP16, (16, 56, 56, 128, 64, 3, 1), "conv2d_mfma_f16"),       # 128 channels in, 64 out: half of the GEMM kernel's tile empty
+    (capi.FP16, (16, 56, 56, 128, 64, 3, 1), "conv2d_planes_f16"),     # 128 channels in, 64 out: half of the GEMM kernel's tile empty
+    (capi.FP16, (4, 100, 130, 128, 64, 3, 1), "conv2d_mfma_f16"),      # the same with rows the streaming patch would need two rounds for
     (capi.FP16, (16, 56, 56, 128, 96, 3, 1), "gemm_mfma_f16"),         # 96 out
     (capi.FP16, (16, 56, 56, 64, 128, 3, 1, 2), "conv2d_slab_f16"),    # 98 tiles: the slab kernel
     (capi.FP16, (8, 56, 56, 64, 256, 1, 0), "gemm_mfma_f16"),          # pointwise with two blocks of K

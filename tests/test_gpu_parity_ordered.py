@@ -17,10 +17,16 @@ def ctx():
     c.close()
 
 
-CONVS = [  # n, ih, iw, ic, oc, k, pad, stride
-    (1, 8, 8, 32, 64, 3, 1, 1),      # one whole tile, stages inside a tap
-    (1, 5, 13, 64, 65, 3, 1, 1),     # one row and one column past a tile
-    (2, 9, 7, 96, 31, 3, 1, 2),      # narrow channels: 64 x 32 tiles
+# n, ih, iw, ic, oc, k, pad, stride; reductions of whole units of eight channels from 224 (the fp32 operator: 400) on run on operands staged through LDS
+STAGED = [
+    (1, 8, 8, 32, 64, 3, 1, 1),
+    (1, 5, 13, 64, 65, 3, 1, 1),
+    (2, 9, 7, 96, 31, 3, 1, 2),
+]
+CONVS = STAGED + [
+    (1, 9, 9, 32, 64, 2, 0, 1),      # one whole tile, stages inside a tap
+    (1, 6, 14, 32, 65, 2, 0, 1),     # one row and one column past a tile
+    (2, 9, 7, 32, 31, 2, 1, 2),      # narrow channels: 64 x 32 tiles
     (1, 5, 5, 32, 200, 2, 0, 1),     # few pixels: 32 x 64 tiles
     (1, 9, 9, 20, 70, 3, 1, 1),      # groups of four, stages across taps
     (2, 7, 9, 5, 66, 3, 1, 1),       # single elements
@@ -35,7 +41,8 @@ CONVS = [  # n, ih, iw, ic, oc, k, pad, stride
 @pytest.mark.parametrize("infinite", [False, True])
 def test_conv2d_in_the_references_order(ctx, case, infinite):
     n, ih, iw, ic, oc, k, p, s = case
-    tiles = "_ordered" if case == CONVS[-1] else "_ordered_tail"
+    tiles = "_ordered" if case == CONVS[-1] else "_ordered_staged" if case in STAGED else "_ordered_tail"
+    op_tiles = "_ordered_tail" if case == STAGED[0] else tiles
     rng = np.random.default_rng(ic * oc)
     x = rng.normal(0, 1, (n, ih, iw, ic)).astype(np.float32)
     w = rng.normal(0, 0.3, (oc, k, k, ic)).astype(np.float32)
@@ -49,7 +56,7 @@ def test_conv2d_in_the_references_order(ctx, case, infinite):
     with np.errstate(invalid="ignore"):
         want = oracle.conv2d("f32", x, w, b, pad, (s, s), (1, 1))
         got, st = gpu_ops.conv2d(ctx, x, w, b, pad, (s, s), (1, 1), dtype=capi.FP32)
-        assert st == capi.VALID and np.array_equal(got, want, equal_nan=True) and ctx.last_kernel == "conv2d" + tiles + "_f32"
+        assert st == capi.VALID and np.array_equal(got, want, equal_nan=True) and ctx.last_kernel == "conv2d" + op_tiles + "_f32"
         d = ctx.conv_desc(capi.FP32, capi.FP32, x.shape, oc, k, k, (oh, ow), pad, (s, s), (1, 1), oc)
         dev = [ctx.upload(v) for v in (x, w, b)]
         for bounds in (False,) if infinite else (False, True):    # (the oracle's bounds pass multiplies the padding out: NaN)

@@ -1,4 +1,4 @@
-"""GPU parity of the streaming-patch CONV2D kernel (16-bit floats with taps): slices of channels whole and cut, windows of two taps and
+"""GPU parity of the streaming-patch CONV2D kernel (16-bit floats with taps, int8 with the fused RESCALE): slices of channels whole and cut, windows of two taps and
 more, ragged rows, images and output channels.  Operands are small whole numbers, so that every sum is exact in fp32 and a
 result has one right value in every type."""
 import numpy as np
@@ -15,7 +15,7 @@ SHAPES = [  # n, ih, iw, ic, oc, kh, kw, pad, stride, dilation
     (16, 28, 28, 256, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
     (10, 28, 30, 200, 56, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),     # channels of no whole slices, output channels cut
     (12, 30, 28, 520, 128, 1, 3, (0, 0, 1, 1), (1, 1), (1, 1)),    # three taps: the next patch stored in a slice's second stage
-    (24, 21, 23, 448, 136, 3, 1, (1, 1, 0, 0), (1, 1), (1, 1)),
+    (24, 42, 23, 448, 56, 3, 1, (1, 1, 0, 0), (1, 1), (1, 1)),     # a window of one column
     (9, 33, 41, 128, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1)),
     (12, 14, 14, 384, 264, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
     (14, 24, 28, 176, 56, 3, 3, (2, 2, 2, 2), (1, 1), (2, 2)),     # dilation
@@ -48,8 +48,7 @@ def test_small_whole_numbers(ctx, kind, shape):
     else:
         got, st = gpu_ops.conv2d(ctx, *(cases.float_to_bf16_bits(v.astype(np.float32)) for v in (x, w, bias)), pad, stride, dil, dtype=capi.BF16)
         want = cases.float_to_bf16_bits(want.astype(np.float32))
-    assert st == capi.VALID
-    print(shape, ctx.last_kernel)
+    assert st == capi.VALID and ctx.last_kernel == ("conv2d_planes_f16" if kind == "fp16" else "conv2d_planes_bf16")
     assert np.array_equal(got, want)
 
 
@@ -66,7 +65,7 @@ def test_infinite_weights_outside_the_image(ctx, shape):
     b = np.zeros(oc, np.float16)
     want, _ = gpu_ops.conv2d(ctx, x, plain, b, (1, 1, 1, 1), dtype=capi.FP16)
     got, st = gpu_ops.conv2d(ctx, x, w, b, (1, 1, 1, 1), dtype=capi.FP16)
-    assert st == capi.VALID
+    assert st == capi.VALID and ctx.last_kernel == "conv2d_planes_f16"
     # without a channel of the tap that lies outside: the results of finite weights there
     one = [c for c in range(oc) if c not in (3, 8, oc - 1)]
     assert np.array_equal(got[..., one], want[..., one])
@@ -82,7 +81,7 @@ I8_SHAPES = [  # the same for int8 with the fused RESCALE
     (9, 33, 41, 256, 72, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1)),
     (12, 30, 28, 768, 128, 1, 3, (0, 0, 1, 1), (1, 1), (1, 1)),
     (27, 40, 40, 400, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
-    (16, 29, 29, 512, 264, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1)),
+    (16, 29, 29, 640, 264, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1)),
 ]
 
 
@@ -101,5 +100,5 @@ def test_int8_rescale(ctx, shape, in_zp, double_round, clamp):
     if clamp:
         want = oracle.clamp(want, *clamp)
     got, st = gpu_ops.conv2d(ctx, x, w, bias, pad, stride, dil, in_zp=in_zp, rescale=dict(mult=mult, shift=shift, out_zp=5, rounding_mode=mode), clamp=clamp)
-    assert st == wst == capi.VALID
+    assert st == wst == capi.VALID and ctx.last_kernel == "conv2d_planes_i8_rescale"
     assert np.array_equal(got, want)

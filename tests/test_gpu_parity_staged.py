@@ -46,15 +46,16 @@ def test_conv2d_staged(ctx, case, dtype, infinite):
     code = {"fp32": capi.FP32, "fp16": capi.FP16, "bf16": capi.BF16}[dtype]
     oh, ow = oracle.conv_out_hw(ih, iw, kh, kw, pad, stride, dil)
     bias = np.broadcast_to(b, oc)
+    staged_op = ic * kh * kw >= 400 and n * oh * ow * oc <= 192 * 64 * 64    # (the fp32 operator stages long reductions on few tiles)
     d = ctx.conv_desc(code, code, (n, ih, iw, ic), oc, kh, kw, (oh, ow), pad, stride, dil, len(b))
     with np.errstate(invalid="ignore"):
         if dtype == "fp32":
             got, st = gpu_ops.conv2d(ctx, x, w, b, pad, stride, dil, dtype=capi.FP32)
-            assert st == capi.VALID and np.array_equal(got, oracle.conv2d("f32", x, w, bias, pad, stride, dil), equal_nan=True)
+            assert st == capi.VALID and (ctx.last_kernel == "conv2d_ordered_staged_f32") == staged_op and np.array_equal(got, oracle.conv2d("f32", x, w, bias, pad, stride, dil), equal_nan=True)
         dev = [ctx.upload(np.ascontiguousarray(v), code) for v in bits]    # (behind gpu_ops, which frees the context's tensors)
         for bounds in (False, True):    # (the bounds pass multiplies the padding out: an infinite weight there makes NaN)
             out = ctx.empty((n, oh, ow, oc), capi.F64)
             ctx.conv2d_precise(d, *dev, bounds, out)
-            assert ctx.sync() == capi.VALID and ctx.last_kernel == ("conv_bounds" if bounds else "conv_precise") + "_ordered_tail_f64"
+            assert ctx.sync() == capi.VALID and ctx.last_kernel == ("conv_bounds" if bounds else "conv_precise") + "_ordered_staged_f64"
             want = oracle.conv2d("f64", *(v.astype(np.float64) for v in (x, w, bias)), pad, stride, dil, abs_mode=bounds)
             assert np.array_equal(out.numpy(), want, equal_nan=True)

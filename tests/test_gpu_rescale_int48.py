@@ -35,6 +35,7 @@ def test_int48(ctx, rows, c, out, kind):
     zp = 3 if out == np.int8 else 0
     args = dict(out_zp=3 if out == np.int8 else 0, out_dtype=out, scale32=False, rounding_mode=capi.ROUND_SINGLE, per_channel=n > 1)
     got, st = gpu_ops.rescale(ctx, x, mult, shift, **args)
+    assert ctx.last_kernel == "rescale_i48"
     want, wst = oracle.rescale(x, mult, shift, **args)
     assert st == wst and (st == capi.VALID) == (kind in ("plain", "uniform"))
     if st != capi.VALID:    # (the oracle has no values then: the general kernel's, on pieces that are left to it)
