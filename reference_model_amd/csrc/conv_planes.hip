@@ -13,7 +13,7 @@
 // us before / here: [16,14,14,512]->512 40.0 / 23.9, [16,28,28,256]->64 20.7 / 13.0, 5x5 [2,20,20,480]->592 129 / 51, stride 2 [14,36,28,328]->240 46.6 / 22.2.
 #include <type_traits>
 
-#include "tmi_mfma.h"
+#include "outside_taps.h"
 
 namespace tmi
 {
@@ -350,6 +350,12 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
             for (int e = 0; e < 4; e++)
                 sum[t][4 * q + e] = v[e] + (IT == 2 ? acc[0][t][4 * q + e] : (kg ? acc[0][1][4 * q + e] : acc[0][0][4 * q + e]));
         }
+    bool met_nan = false;    // (see outside_taps.h)
+    if constexpr (!I8)
+        if (a.padded)
+#pragma unroll
+            for (int t = 0; t < HT; t++)
+                met_nan |= any_nan<16>(sum[t]);
     __syncthreads();
 
     // ---- results: gathered by pixel, so that whole lines leave ----------------------------------------------------
@@ -405,43 +411,6 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
             reinterpret_cast<v4i*>(d)[1] = reinterpret_cast<const v4i*>(packed)[1];
         }
     }
-    // A tap outside the image adds nothing in the reference (tensor_ops.cpp:856-862); here it added 0 * weight, which is NaN where the weight is infinite
-    // or NaN.  A lane with such sums makes them again without those taps.
-    if constexpr (!I8)
-        if (a.padded)
-        {
-            uint32_t odd = 0;
-#pragma unroll
-            for (int t = 0; t < HT; t++)
-#pragma unroll
-                for (int e = 0; e < 16; e += 2)
-                    odd |= __builtin_isunordered(sum[t][e], sum[t][e + 1]) ? 3u << (16 * t + e) : 0u;
-            if (p_w + rho >= pixels)
-                odd = 0;
-            while (odd)
-            {
-                const int i = __builtin_ctz(odd), t = i >> 4, oc = oc_w + 32 * t + 16 * h + (i & 15);
-                odd &= odd - 1;
-                if (oc >= a.N)
-                    break;
-                const int py = (int)fdiv((uint32_t)(p_w + rho), a.div_ow), yb = (oy0 + py) * a.sy - a.pad_top, xb = (p_w + rho - py * a.OW) * a.sx - a.pad_left;
-                const int channels = a.icb / EB, KH = a.taps / a.KW;
-                const T* wt = reinterpret_cast<const T*>(a.w + (size_t)oc * a.kb);
-                float again = 0;
-                for (int ky = 0; ky < KH; ky++)
-                    for (int kx = 0; kx < a.KW; kx++, wt += channels)
-                    {
-                        const int iy = yb + ky * a.dy, ix = xb + kx * a.dx;
-                        if ((uint32_t)iy < (uint32_t)a.IH && (uint32_t)ix < (uint32_t)a.IW)
-                        {
-                            const T* px = reinterpret_cast<const T*>(x + (uint32_t)((iy * a.IW + ix) * a.icb));
-                            for (int c = 0; c < channels; c++)
-                                again += load_as_float<T>(px, c) * load_as_float<T>(wt, c);
-                        }
-                    }
-                store_from_float(reinterpret_cast<T*>(tbuf + rho * PITCH + t * 64 + h * 32) + (i & 15), again + tab_bias[oc - oc0]);
-            }
-        }
     // (pieces of eight channels)
     using piece_t        = std::conditional_t<I8, v2i, v4i>;
     constexpr int PIECES = ROW / (8 * EB), RPI = 64 / PIECES;
@@ -456,6 +425,18 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
     }
     if constexpr (I8)
         raise_flags(a.flag_word, flags);
+    else if (a.padded)
+    {
+        const int channels = a.N - oc0 < 64 ? a.N - oc0 : 64;
+        if (met_odd_weights<T, 8>(met_nan, tab_wsum, a.w + (size_t)oc0 * a.kb, (int64_t)channels * a.kb))
+        {
+            __threadfence();    // (results were stored by other lanes)
+            const PlanesArgs g = args_read_anew<PlanesArgs>();
+            const int p = p_w + rho, py = p / g.OW;
+            without_outside_taps<T>(OutsideTaps{ g.x, g.w, g.bias, g.out, g.icb, g.IH, g.IW, g.N, g.OH, g.OW, g.taps / g.KW, g.KW, g.sy, g.sx, g.dy, g.dx, g.pad_top, g.pad_left, g.bias_len },
+                                    p < pixels, (int)image, oy0 + py, p - py * g.OW, oc_w + 16 * h, HT, 16);
+        }
+    }
 }
 
 struct PlanesPlan
