@@ -15,7 +15,7 @@
 // (190 of matrix instructions); fp32 sums: [9,50,66,224]->16 stride 2 52.5 / 36.9.
 #include <type_traits>
 
-#include "tmi_mfma.h"
+#include "outside_taps.h"
 
 namespace tmi
 {
@@ -250,9 +250,20 @@ __device__ __forceinline__ void staged_tile(const StagedArgs& p, int m0, int n0,
             }
         }
     };
+    // A tap outside the image adds nothing in the reference (but in its bounds pass); here it adds 0 * weight, which is not nothing when the weight is
+    // infinite or NaN (see outside_taps.h): results that are NaN under a window that leaves the image, in channels with such a weight, are summed again.
+    // us a call on a NaN image, every NaN summed again / so (on finite values): [4,14,14,256]->64 3x3 fp64 1050 / 33 (29), fp32 1062 / 48 (43).
+    auto met_odd = [&](bool nan) {
+        if (ABS || !p.padded)
+            return false;
+        const int64_t row_bytes = (int64_t)p.KH * p.KW * p.IC * (int)sizeof(T);
+        const int channels      = p.OC - n0 < 2 * WT ? p.OC - n0 : 2 * WT;
+        return met_odd_weights<T, 4>(__any(nan) != 0, reinterpret_cast<int32_t*>(lds + RING * STAGE), reinterpret_cast<const uint8_t*>(p.b) + n0 * row_bytes, channels * row_bytes);
+    };
     if (m0 + wm >= p.M || n0 + wn >= p.OC)
     {
         walk(std::false_type{});    // a wave without results: only its part of the stages
+        met_odd(false);
         return;
     }
     walk(std::true_type{});
@@ -268,7 +279,7 @@ __device__ __forceinline__ void staged_tile(const StagedArgs& p, int m0, int n0,
         const float b = widened<T>(reinterpret_cast<const T*>(p.bias)[p.bias_len == 1 ? 0 : oc]);
         reinterpret_cast<acc_t*>(p.out)[(size_t)m * p.OC + oc] = v + (acc_t)(ABS ? __builtin_fabsf(b) : b);
     };
-    bool odd = false;
+    bool nan = false;
 #pragma unroll
     for (int i = 0; i < RESULTS; i++)
     {
@@ -278,33 +289,43 @@ __device__ __forceinline__ void staged_tile(const StagedArgs& p, int m0, int n0,
         else
             v = acc4[i];
         int m, oc;
-        odd |= v != v;
+        nan |= v != v;
         if (place(i, m, oc))
             store_result(m, oc, v);
     }
-    // A tap outside the image adds nothing in the reference (but in its bounds pass); here it added 0 * weight, which is not nothing when
-    // the weight is infinite or NaN.  Such sums are not numbers: a lane that has one makes its sums again without those taps.
-    if (!ABS && p.padded && odd)
-        for (int i = 0; i < RESULTS; i++)
-        {
-            int m, oc;
-            if (!place(i, m, oc))
-                continue;
-            const uint32_t t = fdiv((uint32_t)m, p.ow), n = fdiv(t, p.oh);
-            const int yb = (int32_t)(t - n * p.oh.d) * p.stride_y - p.pad_top, xb = (int32_t)((uint32_t)m - t * p.ow.d) * p.stride_x - p.pad_left;
-            const T* img = reinterpret_cast<const T*>(p.a) + (int64_t)n * p.IH * p.IW * p.IC;
-            const T* w   = reinterpret_cast<const T*>(p.b) + (int64_t)oc * p.KH * p.KW * p.IC;
-            acc_t sum    = 0;
-            for (int ky = 0; ky < p.KH; ky++)
-                for (int kx = 0; kx < p.KW; kx++, w += p.IC)
-                {
-                    const int iy = yb + ky * p.dil_y, ix = xb + kx * p.dil_x;
-                    if ((uint32_t)iy < (uint32_t)p.IH && (uint32_t)ix < (uint32_t)p.IW)
-                        for (int c = 0; c < p.IC; c++)
-                            sum = sum + (acc_t)widened<T>(img[(iy * p.IW + ix) * p.IC + c]) * (acc_t)widened<T>(w[c]);
-                }
-            store_result(m, oc, sum);
-        }
+    if (!met_odd(nan))
+        return;
+    const int64_t row_bytes = (int64_t)p.KH * p.KW * p.IC * (int)sizeof(T);
+    uint32_t odd = 0;    // a bit for each column of the lane
+    for (int t = 0; t < TW; t++)
+    {
+        const int oc        = n0 + wn + 16 * t + l16;
+        const uint64_t part = __ballot(weights_not_finite<T>(reinterpret_cast<const uint8_t*>(p.b) + (oc < p.OC ? oc : n0) * row_bytes, row_bytes, q, 4));
+        odd |= (part >> l16 & 0x0001000100010001u) != 0 ? 1u << t : 0u;
+    }
+    for (int i = 0; i < RESULTS; i++)
+    {
+        int m, oc;
+        if (!place(i, m, oc) || (odd >> ((i >> 2) % TW) & 1) == 0)
+            continue;
+        const uint32_t t = fdiv((uint32_t)m, p.ow), n = fdiv(t, p.oh);
+        const int yb = (int32_t)(t - n * p.oh.d) * p.stride_y - p.pad_top, xb = (int32_t)((uint32_t)m - t * p.ow.d) * p.stride_x - p.pad_left;
+        const acc_t stored = reinterpret_cast<const acc_t*>(p.out)[(size_t)m * p.OC + oc];
+        if (stored == stored || (yb >= 0 && xb >= 0 && yb + (p.KH - 1) * p.dil_y < p.IH && xb + (p.KW - 1) * p.dil_x < p.IW))
+            continue;
+        const T* img = reinterpret_cast<const T*>(p.a) + (int64_t)n * p.IH * p.IW * p.IC;
+        const T* w   = reinterpret_cast<const T*>(p.b) + (int64_t)oc * p.KH * p.KW * p.IC;
+        acc_t sum    = 0;
+        for (int ky = 0; ky < p.KH; ky++)
+            for (int kx = 0; kx < p.KW; kx++, w += p.IC)
+            {
+                const int iy = yb + ky * p.dil_y, ix = xb + kx * p.dil_x;
+                if ((uint32_t)iy < (uint32_t)p.IH && (uint32_t)ix < (uint32_t)p.IW)
+                    for (int c = 0; c < p.IC; c++)
+                        sum = sum + (acc_t)widened<T>(img[(iy * p.IW + ix) * p.IC + c]) * (acc_t)widened<T>(w[c]);
+            }
+        store_result(m, oc, sum);
+    }
 }
 
 // The first n_big tiles of 64 x 64 results whole, each of the others as four workgroups of 32 x 32.
@@ -334,7 +355,7 @@ __global__ __launch_bounds__(256, 2) void ordered_staged_kernel(StagedArgs p)
 template <typename T, bool F64>
 static bool launch_staged(hipStream_t st, const StagedArgs& p, bool abs_mode)
 {
-    constexpr int kLds  = 3 * 64 * 2 * 8 * (F64 ? 16 : 8);
+    constexpr int kLds  = 3 * 64 * 2 * 8 * (F64 ? 16 : 8) + 64;    // the ring, and the words of met_odd_weights()
     const unsigned grid = (unsigned)(p.n_big + 8 * p.quarters_per_xcd);
     auto run = [&](auto kernel) {
         if (!ensure_dynamic_lds<kernel.value>(kLds))

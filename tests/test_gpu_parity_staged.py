@@ -1,5 +1,7 @@
 """The ordered sums on units of eight channels staged through LDS (fp64 passes, fp32 operator on few tiles): bit for bit the oracle's loop
 nest at the edges of tiles, units, stages and taps, and where a weight is infinite under a tap outside the image."""
+import time
+
 import numpy as np
 import pytest
 
@@ -59,3 +61,28 @@ def test_conv2d_staged(ctx, case, dtype, infinite):
             assert ctx.sync() == capi.VALID and ctx.last_kernel == ("conv_bounds" if bounds else "conv_precise") + "_ordered_staged_f64"
             want = oracle.conv2d("f64", *(v.astype(np.float64) for v in (x, w, bias)), pad, stride, dil, abs_mode=bounds)
             assert np.array_equal(out.numpy(), want, equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype, precise", [("fp32", False), ("fp32", True), ("bf16", True)])
+def test_a_nan_image_costs_no_sums(ctx, dtype, precise):
+    """A result that is NaN through its window costs a look at the weights; summed again one product after the other it took 25 to 37 times as long."""
+    rng = np.random.default_rng(1)
+    n, h, w, ic, oc = 4, 14, 14, 256, 64
+    store = {"fp32": lambda v: v.astype(np.float32), "bf16": lambda v: (v.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)}[dtype]
+    code = {"fp32": capi.FP32, "bf16": capi.BF16}[dtype]
+    wt, b = ctx.upload(store(rng.normal(0, 0.1, (oc, 3, 3, ic))), code), ctx.upload(store(np.zeros(oc)), code)
+    d = ctx.conv_desc(code, code, (n, h, w, ic), oc, 3, 3, (h, w), (1, 1, 1, 1), (1, 1), (1, 1), oc)
+    out = ctx.empty((n, h, w, oc), capi.F64 if precise else code)
+
+    def seconds(x):
+        call = (lambda: ctx.conv2d_precise(d, x, wt, b, False, out)) if precise else (lambda: ctx.conv2d(d, x, wt, b, 0, 0, out))
+        call(), ctx.sync()
+        start = time.perf_counter()
+        for _ in range(10):
+            call()
+        assert ctx.sync() == capi.VALID and "ordered_staged" in ctx.last_kernel
+        return time.perf_counter() - start
+    finite = seconds(ctx.upload(store(rng.normal(0, 1, (n, h, w, ic))), code))
+    nan = seconds(ctx.upload(store(np.full((n, h, w, ic), np.nan)), code))
+    print("us a call, finite / NaN:", finite / 10e-6, nan / 10e-6)
+    assert np.isnan(out.numpy()).all() and nan < 4 * finite
