@@ -46,7 +46,7 @@
 // LDS table; every lane then spends about ten instructions per output element.
 #include <type_traits>
 
-#include "tmi_mfma.h"
+#include "outside_taps.h"
 
 namespace tmi
 {
@@ -795,6 +795,7 @@ __global__ __launch_bounds__(512) void conv2d_patch_kernel(PatchArgs a)
     {
         // floating point: out = bias + acc, rounded to the output type (16 channels = 32 bytes per pixel), or
         // kept in fp32 (MATMUL: 64 bytes per pixel)
+        float largest = 0.0f;    // (see outside_taps.h)
 #pragma unroll
         for (int t = 0; t < OCT; t++)
         {
@@ -827,6 +828,7 @@ __global__ __launch_bounds__(512) void conv2d_patch_kernel(PatchArgs a)
                     }
                     continue;
                 }
+                largest = largest_or_nan<16>(largest, acc[i][t]);
                 union
                 {
                     v4i v[2];
@@ -854,6 +856,25 @@ __global__ __launch_bounds__(512) void conv2d_patch_kernel(PatchArgs a)
                     for (int j = 0; j < 16; j++)
                         if (oc0 + oclt + j < g.OC)
                             o[j] = u.e[j];
+                }
+            }
+        }
+        // (each wave by itself: with a barrier for all of them layers of several short rounds lose 2 to 4 %)
+        if (__builtin_expect(__any(largest != largest), 0))
+        {
+            const PatchArgs b       = args_read_anew<PatchArgs>();
+            const int64_t row_bytes = (int64_t)b.g.KH * b.g.KW * b.g.IC * EB;
+            const int c_w = oc0 + woc * OCT * 32, channels = b.g.OC - c_w < OCT * 32 ? b.g.OC - c_w : OCT * 32;
+            if (b.out_dtype != TMI_FP32 && channels > 0 && __any(weights_not_finite<T>(b.w + c_w * row_bytes, channels * row_bytes, lane_counted(), 64)))
+            {
+                __threadfence();
+#pragma unroll 1
+                for (int i = 0; i < PXT; i++)
+                {
+                    const int lane = lane_counted(), p = (wpx * PXT + i) * 32 + (lane & 31), ty = (int)fdiv((uint32_t)p, b.div_tw), oy = oy0 + ty, ox = ox0 + p - ty * b.TW;
+                    without_outside_taps<T>(OutsideTaps{ b.in, b.w, b.bias, b.out, b.g.IC * EB, b.g.IH, b.g.IW, b.g.OC, b.g.OH, b.g.OW, b.g.KH, b.g.KW, b.g.stride_y, b.g.stride_x, b.g.dil_y, b.g.dil_x, b.g.pad_top,
+                                                         b.g.pad_left, b.g.bias_len },
+                                            p < b.TH * b.TW && oy < b.g.OH && ox < b.g.OW, n, oy, ox, oc0 + woc * OCT * 32 + 16 * (lane >> 5), OCT, 16);
                 }
             }
         }

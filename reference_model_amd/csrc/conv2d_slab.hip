@@ -27,7 +27,7 @@
 #include <cstring>
 #include <type_traits>
 
-#include "tmi_mfma.h"
+#include "outside_taps.h"
 
 namespace tmi
 {
@@ -397,6 +397,7 @@ __global__ __launch_bounds__(512) void conv2d_slab_kernel(std::conditional_t<(TC
         }
     }
     const bool chan_ok = oc0 + ocl < a.OC;    // OC is a multiple of 16: a lane's 16 channels are in or out together
+    float largest      = 0.0f;                // (see outside_taps.h)
 #pragma unroll
     for (int k = 0; k < NPT; k++)
     {
@@ -409,6 +410,7 @@ __global__ __launch_bounds__(512) void conv2d_slab_kernel(std::conditional_t<(TC
     const size_t obase = (uint32_t)(((n * a.OH + oy) * a.OW + ox) * a.OC + oc0 + ocl);
     if constexpr (!Mma<T>::is_int)
     {
+        largest = largest_or_nan<16>(largest, acck);
         // 16 consecutive channels of one pixel, rounded to the tensor's type: 32 bytes
         if (pix_ok && chan_ok)
         {
@@ -532,6 +534,27 @@ __global__ __launch_bounds__(512) void conv2d_slab_kernel(std::conditional_t<(TC
         }
     }
     }
+    // (each wave by itself: a barrier for all of them is a fiftieth of the smallest layers)
+    if constexpr (!Mma<T>::is_int)
+        if (__builtin_expect(__any(largest != largest) && oc0 + oct * 32 < a.OC, 0))
+        {
+            constexpr int WB   = TAPS * KB;
+            const SlabArgs g   = args_read_anew<SlabArgs>();
+            const int c_w      = oc0 + oct * 32;
+            const int channels = g.OC - c_w < 32 ? g.OC - c_w : 32;
+            if (__any(weights_not_finite<T>(g.w + (size_t)c_w * WB, (int64_t)channels * WB, lane_counted(), 64)))
+            {
+                __threadfence();
+#pragma unroll 1
+                for (int k = 0; k < NPT; k++)
+                {
+                    const int oy = oy0 + (k ? ty[NPT - 1] : ty[0]), ox = ox0 + (k ? tx[NPT - 1] : tx[0]);
+                    const bool there = (k ? second_active && p_in_tile[NPT - 1] : p_in_tile[0]) && wave_active && oy < g.OH && ox < g.OW;
+                    without_outside_taps<T>(OutsideTaps{ g.in, g.w, g.bias, g.out, KB, g.IH, g.IW, g.OC, g.OH, g.OW, KH, KW, g.sy, g.sx, g.dy, g.dx, g.pad_top, g.pad_left, g.bias_len },
+                                            there, n, oy, ox, oc0 + ocl, 1, 16);
+                }
+            }
+        }
     raise_flags(a.flag_word, flags);
 }
 

@@ -350,12 +350,12 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
             for (int e = 0; e < 4; e++)
                 sum[t][4 * q + e] = v[e] + (IT == 2 ? acc[0][t][4 * q + e] : (kg ? acc[0][1][4 * q + e] : acc[0][0][4 * q + e]));
         }
-    bool met_nan = false;    // (see outside_taps.h)
+    float largest = 0.0f;    // (see outside_taps.h)
     if constexpr (!I8)
         if (a.padded)
 #pragma unroll
             for (int t = 0; t < HT; t++)
-                met_nan |= any_nan<16>(sum[t]);
+                largest = largest_or_nan<16>(largest, sum[t]);
     __syncthreads();
 
     // ---- results: gathered by pixel, so that whole lines leave ----------------------------------------------------
@@ -427,8 +427,11 @@ __global__ __launch_bounds__(512) void conv_planes_kernel(PlanesArgs a)
         raise_flags(a.flag_word, flags);
     else if (a.padded)
     {
-        const int channels = a.N - oc0 < 64 ? a.N - oc0 : 64;
-        if (met_odd_weights<T, 8>(met_nan, tab_wsum, a.w + (size_t)oc0 * a.kb, (int64_t)channels * a.kb))
+        auto weights = [&](auto&& look) {
+            const PlanesArgs g = args_read_anew<PlanesArgs>();
+            look(g.w + (size_t)oc0 * g.kb, (int64_t)(g.N - oc0 < 64 ? g.N - oc0 : 64) * g.kb);
+        };
+        if (__builtin_expect(met_odd_weights<T, 8>(largest, wave, tab_wsum, weights), 0))
         {
             __threadfence();    // (results were stored by other lanes)
             const PlanesArgs g = args_read_anew<PlanesArgs>();

@@ -26,7 +26,7 @@
 //
 // Zero points (int8): sum(a*w) - zw*sum(a) - za*sum(w) + K*za*zw.  The sums are taken with v_dot4 from the
 // fragments as they pass through registers on their way to the matrix core (only in the ZP instantiation).
-#include "tmi_mfma.h"
+#include "outside_taps.h"
 #include <type_traits>
 
 namespace tmi
@@ -1034,6 +1034,13 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
     {
         if (half_lines)
         {
+            float largest = 0.0f;    // (see outside_taps.h)
+            if constexpr (TAPS || PATCH)
+#pragma unroll
+                for (int i = 0; i < PXT; i++)
+#pragma unroll
+                    for (int t = 0; t < OCT; t++)
+                        largest = largest_or_nan<16>(largest, acc[i][t]);
 #pragma unroll
             for (int i = 0; i < PXT; i++)
             {
@@ -1085,6 +1092,25 @@ __global__ __launch_bounds__(512) void gemm_lds_kernel(GemmArgs a)
                             if (64 * u + lane < left)
                                 *reinterpret_cast<uint16_t*>(to + 128 * u + 2 * lane) = *reinterpret_cast<const uint16_t*>(tbuf + row * HPITCH + 128 * u + 2 * lane);
                         to += (size_t)a.N * 2;
+                    }
+                }
+            }
+            if constexpr (TAPS || PATCH)
+            {
+                auto weights = [&](auto&& look) {
+                    const GemmArgs g = args_read_anew<GemmArgs>();
+                    look(g.w + (size_t)oc0 * g.kb, (int64_t)(g.N - oc0 < WROWS ? g.N - oc0 : WROWS) * g.kb);
+                };
+                if (__builtin_expect(met_odd_weights<T, 8>(largest, wave, reinterpret_cast<int32_t*>(lds), weights), 0))
+                {
+                    __threadfence();    // (results were stored by other lanes)
+                    const GemmArgs g = args_read_anew<GemmArgs>();
+#pragma unroll 1
+                    for (int i = 0; i < PXT; i++)
+                    {
+                        const int lane = lane_counted(), p = p0 + (wp * PXT + i) * 32 + (lane & 31), y = (int)((uint32_t)p / (uint32_t)g.OW), n = (int)((uint32_t)y / (uint32_t)g.OH);
+                        without_outside_taps<T>(OutsideTaps{ g.a, g.w, g.bias, g.out, g.icb, g.IH, g.IW, g.N, g.OH, g.OW, g.taps / g.KW, g.KW, g.sy, g.sx, g.dy, g.dx, g.pad_top, g.pad_left, g.bias_len },
+                                                p < m_end, n, y - n * g.OH, p - y * g.OW, oc0 + wo * 32 * OCT + 16 * (lane >> 5), OCT, 16);
                     }
                 }
             }

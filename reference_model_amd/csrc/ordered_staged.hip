@@ -258,7 +258,8 @@ __device__ __forceinline__ void staged_tile(const StagedArgs& p, int m0, int n0,
             return false;
         const int64_t row_bytes = (int64_t)p.KH * p.KW * p.IC * (int)sizeof(T);
         const int channels      = p.OC - n0 < 2 * WT ? p.OC - n0 : 2 * WT;
-        return met_odd_weights<T, 4>(__any(nan) != 0, reinterpret_cast<int32_t*>(lds + RING * STAGE), reinterpret_cast<const uint8_t*>(p.b) + n0 * row_bytes, channels * row_bytes);
+        return met_odd_weights<T, 4>(nan ? __builtin_nanf("") : 0.0f, wave, reinterpret_cast<int32_t*>(lds + RING * STAGE),
+                                     [&](auto&& look) { look(reinterpret_cast<const uint8_t*>(p.b) + n0 * row_bytes, channels * row_bytes); });
     };
     if (m0 + wm >= p.M || n0 + wn >= p.OC)
     {

@@ -1,12 +1,15 @@
 // CONV2D results whose window leaves the image, on kernels that multiply what lies outside as zeros.
 //
 // A tap outside the image adds nothing in the reference (tensor_ops.cpp:845-852); zero times the weight is nothing too, unless the weight is infinite or
-// NaN.  A workgroup that met a sum that is NaN looks at its channels' weights behind its stores, once and with all lanes side by side; where one is no
-// number, its waves go over their tiles once more and sum one at a time, without those taps, the results that are NaN, whose window leaves the image and
-// whose channel has such a weight.  Every other result keeps the sum it has, and a NaN that came from the image costs the look.  us a call on a NaN
-// image, every NaN summed again / so (on finite values): streaming patch fp16 3x3 [7,14,21,200]->288 2600 / 24 (17), bf16 [16,28,28,256]->64 3679 / 24 (16).
-// (Behind the loop and from arguments read anew it costs the loop a test of the results and no register: summed again in the loop, two channel tiles
-// a wave of conv_taps.hip fall from four waves a SIMD to two.)
+// NaN.  A workgroup (the patch and the slab kernel: a wave) that met a sum that is NaN looks at its channels' weights behind its stores, once and with all
+// lanes side by side; where one is no number, its waves go over their tiles once more and sum one at a time, without those taps, the results that are NaN,
+// whose window leaves the image and whose channel has such a weight.  Every other result keeps the sum it has, and a NaN that came from the image costs
+// the look.  us a call on a NaN image, every NaN summed again / so (on finite values): streaming patch fp16 3x3 [7,14,21,200]->288 2600 / 23 (17), bf16
+// [16,28,28,256]->64 3679 / 24 (16); GEMM kernel [4,28,28,224]->256 31 (18), bf16 [64,7,7,512]->512 90 (44); patch kernel [2,28,28,256]->250 53 (25); slab
+// kernel [8,56,56,64]->64 13.8 (5.9).
+// (Behind the loop and from arguments read anew it costs the loop a test of the results and no vector register: summed again in the loop, two channel
+// tiles a wave of conv_taps.hip fall from four waves a SIMD to two.  On finite values, over 36 layers of the patch and the GEMM kernel, 1.001 of the time
+// without any of this; the most, [4,100,130,128]->64 on the patch kernel, 29.0 / 29.8.  A workgroup's barrier in the patch kernel: layers of short rounds 2 to 4 % more.)
 #pragma once
 #include <type_traits>
 
@@ -26,15 +29,20 @@ struct OutsideTaps
     int32_t bias_len;
 };
 
-// Whether one of N sums of any lane is NaN
+// The largest of so_far and N sums, or NaN if one of them is: an instruction for two of them, and one test behind the last
 template <int N, typename R>
-__device__ __forceinline__ bool any_nan(const R& v)
+__device__ __forceinline__ float largest_or_nan(float so_far, const R& v)
 {
-    bool nan = false;
 #pragma unroll
     for (int e = 0; e < N; e += 2)
-        nan |= __builtin_isunordered(v[e], v[e + 1]);
-    return __any(nan);
+        so_far = __builtin_elementwise_maximum(__builtin_elementwise_maximum(v[e], v[e + 1]), so_far);
+    return so_far;
+}
+
+// The lane's number, counted and not kept from the kernel's start
+__device__ __forceinline__ int lane_counted()
+{
+    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
 }
 
 // The kernel's arguments from memory: not the values it began with, which would have to be kept
@@ -56,7 +64,7 @@ __device__ __forceinline__ bool weights_not_finite(const uint8_t* w, int64_t byt
     auto odd = [](uint32_t word) { return (word & EXPONENT) == EXPONENT || (sizeof(T) < 4 && (word >> 16 & EXPONENT) == EXPONENT); };
     bool found          = false;
     const int64_t whole = bytes & ~(int64_t)15;
-#pragma unroll 4
+#pragma unroll 8
     for (int64_t at = 16 * part; at < whole; at += 16 * parts)
     {
         const v4i v = load16(w + at);
@@ -67,19 +75,23 @@ __device__ __forceinline__ bool weights_not_finite(const uint8_t* w, int64_t byt
     return found;
 }
 
-// Whether a wave of the workgroup met a NaN and the weights of the workgroup's channels are not all finite.  For all waves alike, behind their loops;
-// words: 2 WAVES words of LDS that no wave uses any more.
-template <typename T, int WAVES>
-__device__ __forceinline__ bool met_odd_weights(bool met_nan, int32_t* words, const uint8_t* w, int64_t bytes)
+// Whether a wave of the workgroup met a NaN (largest_or_nan() of its sums) and the weights of the workgroup's channels are not all finite.  For all waves alike, behind their loops;
+// words: 2 WAVES words of LDS that no wave uses any more; weights(look): calls look(w, bytes), from arguments read anew where registers are short.
+template <typename T, int WAVES, typename Weights>
+__device__ __forceinline__ bool met_odd_weights(float largest, int wave, int32_t* words, Weights&& weights)
 {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int lane   = lane_counted();
     auto in_any_wave = [&](bool flag, int32_t* word) {
         if (lane == 0)
             word[wave] = flag;
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");    // (stores need not have arrived)
         return __any(lane < WAVES && word[lane < WAVES ? lane : 0]) != 0;
     };
-    return in_any_wave(met_nan, words) && in_any_wave(__any(weights_not_finite<T>(w, bytes, threadIdx.x, WAVES * 64)), words + WAVES);
+    if (__builtin_expect(!in_any_wave(__any(largest != largest), words), 1))
+        return false;
+    bool odd = false;
+    weights([&](const uint8_t* w, int64_t bytes) { odd = weights_not_finite<T>(w, bytes, wave * 64 + lane, WAVES * 64); });
+    return in_any_wave(__any(odd), words + WAVES);
 }
 
 // The lane's pixel (n, oy, ox), if it is there; of `tiles` tiles of 32 channels the lane holds `each` from channel c0 on, the same for all lanes of a
@@ -87,7 +99,7 @@ __device__ __forceinline__ bool met_odd_weights(bool met_nan, int32_t* words, co
 template <typename T>
 __device__ __forceinline__ void without_outside_taps(const OutsideTaps& g, bool there, int n, int oy, int ox, int c0, int tiles, int each)
 {
-    const int lane = threadIdx.x & 63;
+    const int lane = lane_counted();
     const int y0 = oy * g.sy - g.pad_top, x0 = ox * g.sx - g.pad_left;
     const bool leaves = there && (y0 < 0 || x0 < 0 || y0 + (g.KH - 1) * g.dy >= g.IH || x0 + (g.KW - 1) * g.dx >= g.IW);
     if (!__any(leaves))
