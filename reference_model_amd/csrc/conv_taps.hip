@@ -672,7 +672,8 @@ __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs 
 // memory pipeline, two loads a step with a line per lane: 23 ns a step of the workgroup, whatever NW is.  us patch kernel / this
 // kernel: int8 [1,49,49,616]->59 3x3 stride 2 77 / 11.8, [2,13,18,200]->40 5x5 stride 2 47 / 11.2, [5,24,29,8]->48 3x3 stride 2 7.4 / 4.2, fp16
 // [9,31,41,240]->32 3x3 stride 2 28.9 / 8.2; with the weights staged in LDS first, as above, [2,79,7,88]->23 bf16 3x3 6.3 / 4.6.
-constexpr int kTapsShare = 8;
+// (Rows between words, with the words behind them: six.)
+constexpr int kTapsShare = 8, kTapsOddShare = 6;
 
 template <typename T, int NW, int ROWS>
 __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_kernel(TapsArgs a)
@@ -681,7 +682,7 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_ker
     using M           = Mma<T>;
     using acc_t       = typename M::acc_t;
     using v4          = std::conditional_t<M::is_int, v4i, v4f>;
-    constexpr int KSW = ODD ? 6 : kTapsShare;    // (what the registers of two workgroups hold)
+    constexpr int KSW = ODD ? kTapsOddShare : kTapsShare;    // (what the registers of two workgroups hold)
     __shared__ __attribute__((aligned(16))) v4 red[NW][4][64];
     __shared__ __attribute__((aligned(16))) HighWordScale tab_hw[32];
     __shared__ __attribute__((aligned(16))) v2i tab_ms[32];
@@ -1013,8 +1014,14 @@ struct TapsForm
     int32_t oct, split;    // split 0: the form with resident weights
     double us;
 };
-static TapsForm taps_form(int64_t n_pt, int64_t oc, int64_t steps, int odd)
+// rows: 0 whole chunks, 1 whole words, 2 any, 3 any and read from the word before, of which a wave holds kTapsOddShare steps
+static int taps_rows(int64_t row)
 {
+    return row % 16 == 0 ? 0 : (row % 4 == 0 ? 1 : (row <= 32 ? 2 : 3));
+}
+static TapsForm taps_form(int64_t n_pt, int64_t oc, int64_t steps, int rows)
+{
+    const int odd = rows < 3 ? rows : 2;
     static const double split_base[3] = { 3.3, 3.8, 3.5 }, split_step[3] = { 0.0235, 0.038, 0.1 }, split_all[3] = { 0.035, 0.037, 0.053 };
     static const double base[3] = { 4.5, 4.6, 4.9 }, weights[3] = { 0.018, 0.078, 0.08 }, chain[3] = { 0.0, 0.06, 0.05 }, step[3] = { 0.047, 0.045, 0.085 },
                         tile[3] = { 0.028, 0.008, 0.008 };
@@ -1024,8 +1031,14 @@ static TapsForm taps_form(int64_t n_pt, int64_t oc, int64_t steps, int odd)
     {
         const int64_t most = 256 * (nw == 4 ? 3 : (nw == 8 ? 2 : 1));
         const int64_t each = (tiles + most - 1) / most;
-        const double us    = split_base[odd] + (nw == 4 ? (steps > 32 ? 0.4 : 0.0) : (nw == 8 ? 0.1 : 0.3)) + split_step[odd] * (double)steps +
+        double us          = split_base[odd] + (nw == 4 ? (steps > 32 ? 0.4 : 0.0) : (nw == 8 ? 0.1 : 0.3)) + split_step[odd] * (double)steps +
                           split_all[odd] * (double)(tiles * steps) / 256 * (nw == 16 ? 0.9 : 1.0) + 1.4 * (double)(each - 1);
+        // A share of seven or eight steps of rows read from the word before is fetched and shifted again for every tile.  us so / with weights in LDS: 1x1
+        // int8 [5,32,33,939]->200 19.8 / 16.5, [9,31,32,823]->99 18.7 / 17.5, [9,31,30,945]->128 17.9 / 16.3; up to two tiles of channels, where many workgroups
+        // would lay the same weights out, it stays: [35,32,32,930]->24 18.3 / 23.7, fp16 [35,32,32,491]->9 16.0 / 22.5, bf16 [35,32,32,455]->14 16.1 / 20.9.
+        const int64_t share = (steps + nw - 1) / nw;
+        if (rows == 3 && each > 1 && tiles_oc > 2 && share > kTapsOddShare && share <= kTapsShare)
+            us += 2.0;
         if (us < best.us)
             best = TapsForm{ 1, nw, us };
     }
@@ -1053,13 +1066,13 @@ static int64_t taps_steps(int64_t taps, int64_t row)
 double conv2d_taps_us(int32_t in_dtype, const ConvGeom& g)
 {
     const int64_t row = (int64_t)g.IC * (in_dtype == TMI_INT8 ? 1 : 2), steps = taps_steps((int64_t)g.KH * g.KW, row);
-    return taps_form(((int64_t)g.N * g.OH * g.OW + 31) / 32, g.OC, steps, row % 16 == 0 ? 0 : (row % 4 == 0 ? 1 : 2)).us;
+    return taps_form(((int64_t)g.N * g.OH * g.OW + 31) / 32, g.OC, steps, taps_rows(row)).us;
 }
 
 template <typename T>
 static bool launch_taps_t(hipStream_t st, TapsArgs& a, bool ragged)
 {
-    const TapsForm form = taps_form(a.n_pt, a.OC, a.steps, !ragged ? 0 : (a.row_bytes % 4 == 0 ? 1 : 2));
+    const TapsForm form = taps_form(a.n_pt, a.OC, a.steps, !ragged ? 0 : (a.row_bytes % 4 == 0 ? 1 : taps_rows(a.row_bytes)));
     // (up to 32 bytes a pixel, neighbouring pixels share lines and the other loads are no slower: [20,136,133,13]->488 3x3 stride 2 52.0 / 38.3,
     // [5,14,14,30]->16 5x5 6.6 / 6.0)
     const bool odd = a.row_bytes > 32 && (a.row_bytes % 4 != 0 || (((uintptr_t)a.in | (uintptr_t)a.w) & 3));

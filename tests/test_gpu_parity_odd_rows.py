@@ -39,13 +39,15 @@ def test_rows_between_words(ctx, shape, dtype, offset):
 
 
 EVERY, FLOATS = ("int8", "fp16", "bf16"), ("fp16", "bf16")
-ON_COPIES = {    # 36 steps and more with taps; more than 18 on many tiles
-    (1, 10, 11, 163, 24, 3, 1): EVERY, (2, 4, 4, 331, 9, 5, 1): EVERY, (9, 40, 40, 57, 12, 3, 1): FLOATS, (30, 21, 20, 37, 40, 3, 1): FLOATS}
+ON_COPIES = {    # 36 steps and more with taps; more than 18 on many tiles; many tiles and channels
+    (1, 10, 11, 163, 24, 3, 1): EVERY, (2, 4, 4, 331, 9, 5, 1): EVERY, (9, 40, 40, 57, 12, 3, 1): FLOATS, (30, 21, 20, 37, 40, 3, 1): FLOATS,
+    (5, 32, 33, 939, 200, 1, 1): FLOATS}    # (of many channels: to the GEMM kernel)
 
 
 @pytest.mark.parametrize("shape", [  # n, h, w, ic, oc, k, stride
     (1, 5, 7, 33, 17, 1, 1), (2, 9, 8, 35, 40, 3, 1), (1, 8, 9, 49, 8, 3, 2), (1, 6, 5, 101, 33, 2, 1), (1, 10, 11, 163, 24, 3, 1), (2, 4, 4, 331, 9, 5, 1), (1, 10, 11, 467, 24, 1, 1), (2, 4, 4, 1331, 9, 1, 1),
-    (9, 40, 40, 57, 12, 3, 1), (40, 20, 20, 163, 20, 1, 1), (30, 21, 20, 37, 40, 3, 1), (12, 40, 40, 29, 12, 3, 1), (24, 30, 30, 41, 100, 1, 1)])    # weights resident: several tiles a wave
+    (9, 40, 40, 57, 12, 3, 1), (40, 20, 20, 163, 20, 1, 1), (30, 21, 20, 37, 40, 3, 1), (12, 40, 40, 29, 12, 3, 1), (24, 30, 30, 41, 100, 1, 1),    # weights resident: several tiles a wave
+    (33, 32, 32, 761, 24, 1, 1), (33, 32, 32, 829, 18, 1, 1), (33, 32, 32, 930, 9, 1, 1), (5, 32, 33, 939, 200, 1, 1)])    # int8: K split, two tiles a workgroup on shares of six (kept in registers), seven and eight steps; too many channels for that
 @pytest.mark.parametrize("dtype, offset", [("int8", 0), ("int8", 1), ("int8", 2), ("fp16", 0), ("fp16", 1), ("bf16", 1)])
 def test_channel_vectors_between_words(shape, dtype, offset):
     n, h, w, ic, oc, k, s = shape
