@@ -697,7 +697,8 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // stride 2 9.1 / 5.5, [2,12,12,73]->48 6.6 / 6.1.  Over 220 drawn layers of ragged rows:
         //   1x1, an image that is read once: int8 [43,84,89,127]->96 47.1 / 24.7, [60,32,32,163]->16 15.5 / 8.0, [31,22,27,637]->24 15.1 / 8.7,
         //     [5,89,86,495]->304 (11 960 tiles, 16 steps) 38.7 / 33.0, bf16 [12,100,73,39]->40 14.1 / 8.8, [15,23,39,75]->248 (3368, 5) 11.7 / 9.1; the other
-        //     way fp16 [8,27,53,277]->152 (1790, 18) 11.7 / 12.9.
+        //     way fp16 [8,27,53,277]->152 (1790, 18) 11.7 / 12.9.  From 6000 tile-steps on at once, 72 layers of 6000 to 6500 0.79 of the time on copies, none above 1.02:
+        //     fp16 1x1 [24,13,77,114]->8 9.6 / 4.5, int8 3x3 [10,51,44,23]->24 8.8 / 6.3.
         //   rows of whole words: bf16 [10,88,14,242]->9 3x3 27.8 / 13.1, [6,25,67,122]->40 (630 tiles, 72 steps) 19.9 / 16.2, int8 [43,23,28,72]->16 14.9 / 8.5; the
         //     other way [8,111,22,106]->36 (1222, 63) 20.1 / 21.6, [16,10,10,532]->160 (250, 153) 13.0 / 13.9.
         //   rows between words, up to 3x3 and two chunks a tap: int8 [3,89,89,25]->96 13.6 / 9.7, [2,130,130,29]->240 stride 2 14.4 / 9.9; the other way [49,60,57,21]->384
@@ -718,11 +719,11 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
             if (g.OC % 4 != 0 && g.OC > 128)    // (results of no whole words that no workgroup has whole rows of: 1x1 [1,69,69,167]->607 13.6 / 17.6)
                 return false;
             if (g.KH * g.KW == 1)
-                return t_all > 6500 && t_all <= (g.OC > 64 && d->in_dtype != TMI_INT8 ? 17000 : 200000) && !pointwise_copies;
+                return t_all <= (g.OC > 64 && d->in_dtype != TMI_INT8 ? 17000 : 200000) && !pointwise_copies;
             if (t_row % 4 == 0)
                 return t_all <= (g.OC <= 64 ? 55000 : 8000);
-            return t_all > 6500 && g.KH * g.KW <= 9 && (g.OC <= 64 ? t_steps <= 18 : t_steps <= 9 && t_all <= 60000);
-        };    // (what lies between 6000 and 6500 keeps its copies, whose tests are there: 0.8 ... 1.05 of the time either way)
+            return g.KH * g.KW <= 9 && (g.OC <= 64 ? t_steps <= 18 : t_steps <= 9 && t_all <= 60000);
+        };
         if (padded && as_they_lie() && taps_open())
             padded = 0, name = launch_taps();
         if (name)

@@ -19,15 +19,18 @@ def ctx():
 
 CASES = {  # n, h, w, ic, oc, k, pad, stride: the kernel of the int8 layer
     # copies padded first
-    (11, 45, 45, 17, 24, 3, 1, 1): "conv2d_taps_i8",     # one byte past a piece
-    (10, 47, 49, 31, 8, 3, 1, 1): "conv2d_mfma_i8",      # one short of a step
-    (20, 57, 57, 65, 24, 1, 0, 1): "conv2d_pointwise_i8",
+    (6, 45, 45, 65, 24, 3, 1, 1): "conv2d_taps_i8",      # one byte past a piece
+    (10, 47, 49, 31, 8, 5, 2, 1): "conv2d_mfma_i8",      # one short of a step
+    (40, 57, 57, 33, 131, 1, 0, 1): "gemm_mfma_i8",
     (3, 11, 5, 131, 40, 3, 1, 2): "conv2d_ksplit_i8",
     (6, 40, 41, 207, 64, 2, 0, 1): "conv2d_ksplit_i8",
     (16, 16, 16, 72, 72, 3, 1, 1): "conv2d_ksplit_i8",    # whole words
     (4, 53, 53, 80, 80, 3, 1, 1): "conv2d_slab_i8",
     (1, 10, 10, 245, 16, 3, 1, 1): "conv2d_ksplit_patch_i8",    # padded to 256: both operands in LDS
-    # smaller ones: one launch, as they lie
+    # smaller ones, and few channels in short reductions: one launch, as they lie
+    (11, 45, 45, 17, 24, 3, 1, 1): "conv2d_taps_i8",
+    (10, 47, 49, 31, 8, 3, 1, 1): "conv2d_taps_i8",
+    (20, 57, 57, 65, 24, 1, 0, 1): "conv2d_taps_i8",
     (1, 7, 9, 17, 24, 3, 1, 1): "conv2d_taps_i8",
     (2, 9, 7, 31, 8, 3, 1, 1): "conv2d_taps_i8",
     (1, 8, 8, 33, 13, 1, 0, 1): "conv2d_taps_i8",
@@ -91,6 +94,23 @@ def test_int8(ctx, case, fused):
     want, wst = oracle.rescale(want, mult, shift, out_zp=3)
     got, st = gpu_ops.conv2d(ctx, x, wt, bias, pad, (s, s), in_zp=-11, w_zp=0, rescale=dict(mult=mult, shift=shift, out_zp=3))
     assert st == wst and np.array_equal(got, want) and len(np.unique(got)) > 20 and ctx.last_kernel == CASES[case] + "_rescale"
+
+
+def test_pointwise_layer_on_copies():
+    """many channels on more tiles than the kernel that reads as they lie has workgroups: copies, and the kernel that keeps its weights in registers"""
+    n, h, w, ic, oc = 40, 20, 20, 65, 136
+    rng = np.random.default_rng(3)
+    x, wt = rng.integers(-128, 128, (n, h, w, ic)).astype(np.int8), rng.integers(-128, 128, (oc, 1, 1, ic)).astype(np.int8)
+    bias = rng.integers(-9999, 9999, oc).astype(np.int32)
+    mult, shift = rng.integers(1 << 30, 1 << 31, oc).astype(np.int32), rng.integers(38, 43, oc).astype(np.int8)
+    want, wst = oracle.rescale(oracle.conv2d("i8", x, wt, bias, in_zp=-11, w_zp=0), mult, shift, out_zp=3)
+    c = Context(0)
+    try:
+        got, st = gpu_ops.conv2d(c, x, wt, bias, in_zp=-11, w_zp=0, rescale=dict(mult=mult, shift=shift, out_zp=3))
+        assert st == wst and np.array_equal(got, want) and len(np.unique(got)) > 20
+        assert c.last_kernel == "conv2d_pointwise_i8_rescale" and c.workspace_bytes() != (0, 0)
+    finally:
+        c.close()
 
 
 def test_padded_layer_with_its_sums_in_the_scratch_buffer():
