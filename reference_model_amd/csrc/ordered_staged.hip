@@ -376,7 +376,8 @@ static bool launch_staged(hipStream_t st, const StagedArgs& p, bool abs_mode)
 //     90.5 / 90.0.
 //   Few channels on many tiles, where half the waves have no results: 938 tiles of 16 channels K 144 19.3 / 32.4, 1152 94 / 112; 407 tiles none slower.
 //   fp32 sums, up to 192 tiles: K 504 15.5 / 13.0, 1152 25.0 / 21.8, 2376 49.4 / 44.4; 288 8.8 / 8.2 and 13.3 / 14.1; 160 8.6 / 10.0.
-//   Images of fewer than 16 pixels stay on the copies, whose tests are about them ([1,4,3,128]->65 3x3 18.0 / 14.1).
+//   The same on images of a few pixels: 1 to 15 of them, [1,4,3,128]->65 3x3 17.9 / 14.3, [1,1,1,1024]->256 1x1 20.6 / 12.4, fp32 sums [1,2,2,512]->512 3x3 87.4 / 74.8;
+//     over 15 layers of seven shapes 0.55 ... 0.89 of the time.
 bool ordered_staged_leads(int32_t in_dtype, bool f64, const ConvGeom& g, const void* in, const void* w)
 {
     const int64_t pixels = (int64_t)g.N * g.OH * g.OW, K = (int64_t)g.KH * g.KW * g.IC, eb = in_dtype == TMI_FP32 ? 4 : 2;
@@ -384,8 +385,6 @@ bool ordered_staged_leads(int32_t in_dtype, bool f64, const ConvGeom& g, const v
     if (g.IC % 8 != 0 || (((uintptr_t)in | (uintptr_t)w) & 15) != 0 || K < 1 || K > INT32_MAX / 8 || (int64_t)g.N * g.IH * g.IW * g.IC * eb >= INT32_MAX ||
         (int64_t)g.OC * K * eb >= INT32_MAX || pixels > INT32_MAX - 64 || tiles > INT32_MAX / 8 || !fastdiv_exact_up_to((uint64_t)tiles, (uint32_t)tn) ||
         !fastdiv_exact_up_to((uint64_t)pixels, (uint32_t)g.OW) || !fastdiv_exact_up_to((uint64_t)pixels / g.OW, (uint32_t)g.OH))
-        return false;
-    if (pixels < 16)
         return false;
     if (!f64)
         return tiles <= 192 && K >= 400;

@@ -23,7 +23,8 @@ CASES = [  # n, ih, iw, ic, oc, kh, kw, pads, strides, dilations, fp32 sums on c
     (1, 9, 9, 26, 66, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1), False),      # 234
     (1, 7, 8, 65, 64, 2, 4, (2, 2, 1, 3), (1, 2), (2, 1), True),       # dilated, strided, uneven padding
     (1, 6, 4, 116, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), True),      # 1044, whole groups of four
-    (1, 6, 5, 128, 65, 3, 3, (0, 0, 0, 0), (1, 1), (1, 1), False),     # 1152, whole stages, no padding
+    (1, 6, 5, 128, 65, 3, 3, (0, 0, 0, 0), (1, 1), (1, 1), False),     # 1152, whole stages, no padding: copies for the bounds pass of the largest magnitude
+    (1, 7, 6, 60, 65, 4, 4, (0, 0, 0, 0), (1, 1), (1, 1), False),      # 960, whole stages
     (1, 2, 3, 51, 5, 2, 2, (0, 0, 0, 0), (1, 1), (1, 1), False),       # two results in a row of 204
     (1, 114, 113, 59, 65, 2, 2, (1, 0, 0, 1), (1, 1), (1, 1), False),  # a whole round of tiles and quarters
 ]
@@ -52,7 +53,8 @@ def test_conv2d_on_copies(ctx, case, infinite):
             for local in (True, False) if bounds else (True,):
                 out = ctx.empty((n, oh, ow, oc), capi.F64)
                 ctx.conv2d_precise(d, *dev, bounds, out, local_bound=local)
-                assert ctx.sync() == capi.VALID and ctx.last_kernel == ("conv_bounds" if bounds else "conv_precise") + "_copied_f64"
+                kind = "_ordered_staged_f64" if ic % 8 == 0 and local else "_copied_f64"    # (units of eight channels are staged as they lie)
+                assert ctx.sync() == capi.VALID and ctx.last_kernel == ("conv_bounds" if bounds else "conv_precise") + kind
                 xs = x.astype(np.float64) if local else np.full(x.shape, np.abs(x).max(), np.float64)
                 want = oracle.conv2d("f64", xs, w.astype(np.float64), bias.astype(np.float64), pad, stride, dil, abs_mode=bounds)
                 assert np.array_equal(out.numpy(), want, equal_nan=True)

@@ -28,6 +28,8 @@ CASES = [  # n, ih, iw, ic, oc, kh, kw, pads, strides, dilations
     (1, 9, 8, 64, 65, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),         # whole stages, one column past a tile
     (1, 66, 65, 32, 250, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),      # a whole round of tiles and quarters, whole stages
     (1, 66, 65, 24, 250, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),      # the same across taps
+    (1, 2, 3, 128, 33, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),        # six pixels
+    (1, 1, 1, 512, 5, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1)),         # one
 ]
 
 
