@@ -152,6 +152,39 @@ struct alignas(16) ChanEntry
     int64_t rnd_pos, rnd_neg;
 };
 
+// Which tile a workgroup has
+struct PatchTile
+{
+    int32_t n, oy0, ox0, oc0;
+    uint32_t tile, ocb;
+};
+template <int OCB>
+__device__ __forceinline__ PatchTile patch_tile(const PatchArgs& a, uint32_t bid)
+{
+    if (a.xcd_remap)
+    {
+        // consecutive workgroups are dealt to the 8 XCDs in turn; give each XCD a contiguous run of tiles
+        // so that neighbouring tiles (which share halo rows) share an L2
+        const uint32_t per = (uint32_t)a.xcd_remap;
+        bid                = (bid & 7) * per + (bid >> 3);
+    }
+    // Grouped order: a run of kGroup pixel tiles times all channel blocks, the pixel tile running fastest.
+    // The workgroups that are resident on an XCD together then share a few patches and a few weight blocks
+    // instead of one weight block and many patches, which is what keeps GEMM-sized operands in L2.
+    constexpr uint32_t kGroup = 4;
+    const uint32_t grp        = fdiv(bid, a.div_group);
+    const uint32_t first      = grp * kGroup;
+    const uint32_t in_grp     = bid - grp * kGroup * a.n_ocb;
+    const uint32_t rows       = a.n_tiles - first < kGroup ? a.n_tiles - first : kGroup;
+    const uint32_t ocb        = rows == kGroup ? in_grp / kGroup : in_grp / rows;
+    const uint32_t tile       = first + in_grp - ocb * rows;
+    const uint32_t trow       = fdiv(tile, a.div_tiles_x);
+    const int txi             = tile - trow * a.tiles_x;
+    const int n               = fdiv(trow, a.div_tiles_y);
+    const int tyi             = trow - n * a.tiles_y;
+    return PatchTile{ n, tyi * a.TH, txi * a.TW, (int)ocb * OCB, tile, ocb };
+}
+
 // Per-lane chunk budget of one staging round (weights, patch) and K-loop group size of an instantiation.
 template <int OCT, int PXT, bool MULTI>
 struct TileTraits
@@ -226,31 +259,11 @@ __global__ __launch_bounds__(512) void conv2d_patch_kernel(PatchArgs a)
     const int w_bytes      = OCB * a.wstride;
 
     // ---- which tile ------------------------------------------------------------------------------------
-    uint32_t bid = blockIdx.x;
-    if (a.xcd_remap)
-    {
-        // consecutive workgroups are dealt to the 8 XCDs in turn; give each XCD a contiguous run of tiles
-        // so that neighbouring tiles (which share halo rows) share an L2
-        const uint32_t per = (uint32_t)a.xcd_remap;
-        bid                = (bid & 7) * per + (bid >> 3);
-    }
-    // Grouped order: a run of kGroup pixel tiles times all channel blocks, the pixel tile running fastest.
-    // The workgroups that are resident on an XCD together then share a few patches and a few weight blocks
-    // instead of one weight block and many patches, which is what keeps GEMM-sized operands in L2.
-    constexpr uint32_t kGroup = 4;
-    const uint32_t grp        = fdiv(bid, a.div_group);
-    const uint32_t first      = grp * kGroup;
-    const uint32_t in_grp     = bid - grp * kGroup * a.n_ocb;
-    const uint32_t rows       = a.n_tiles - first < kGroup ? a.n_tiles - first : kGroup;
-    const uint32_t ocb        = rows == kGroup ? in_grp / kGroup : in_grp / rows;
-    const uint32_t tile       = first + in_grp - ocb * rows;
-    const uint32_t trow = fdiv(tile, a.div_tiles_x);
-    const int txi       = tile - trow * a.tiles_x;
-    const int n         = fdiv(trow, a.div_tiles_y);
-    const int tyi       = trow - n * a.tiles_y;
-    const int oy0       = tyi * a.TH;
-    const int ox0       = txi * a.TW;
-    const int oc0       = ocb * OCB;
+    if constexpr (!M::is_int)
+        keep_place(reinterpret_cast<v4i*>(mbtab));    // (the table is the integers')
+    const PatchTile at = patch_tile<OCB>(a, blockIdx.x);
+    const int n = at.n, oy0 = at.oy0, ox0 = at.ox0, oc0 = at.oc0;
+    const uint32_t tile = at.tile, ocb = at.ocb;
     const int y0        = oy0 * g.stride_y - g.pad_top;
     const int x0        = ox0 * g.stride_x - g.pad_left;
     const int P         = a.TH * a.TW;
@@ -862,19 +875,23 @@ __global__ __launch_bounds__(512) void conv2d_patch_kernel(PatchArgs a)
         // (each wave by itself: with a barrier for all of them layers of several short rounds lose 2 to 4 %)
         if (__builtin_expect(__any(largest != largest), 0))
         {
-            const PatchArgs b       = args_read_anew<PatchArgs>();
+            uint32_t block;
+            const PatchArgs b       = args_kept<PatchArgs>(reinterpret_cast<const v4i*>(mbtab), block);
             const int64_t row_bytes = (int64_t)b.g.KH * b.g.KW * b.g.IC * EB;
-            const int c_w = oc0 + woc * OCT * 32, channels = b.g.OC - c_w < OCT * 32 ? b.g.OC - c_w : OCT * 32;
+            // (the tile worked out again: three scalars kept across the stores, whose masks fill the registers, and each of them reloads some: up to 8 % of a layer)
+            const PatchTile at = patch_tile<OCB>(b, block);
+            const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), wpx = wave % WPX;
+            const int c_w = at.oc0 + wave / WPX * OCT * 32, channels = b.g.OC - c_w < OCT * 32 ? b.g.OC - c_w : OCT * 32;
             if (b.out_dtype != TMI_FP32 && channels > 0 && __any(weights_not_finite<T>(b.w + c_w * row_bytes, channels * row_bytes, lane_counted(), 64)))
             {
                 __threadfence();
 #pragma unroll 1
                 for (int i = 0; i < PXT; i++)
                 {
-                    const int lane = lane_counted(), p = (wpx * PXT + i) * 32 + (lane & 31), ty = (int)fdiv((uint32_t)p, b.div_tw), oy = oy0 + ty, ox = ox0 + p - ty * b.TW;
+                    const int lane = lane_counted(), p = (wpx * PXT + i) * 32 + (lane & 31), ty = (int)fdiv((uint32_t)p, b.div_tw), oy = at.oy0 + ty, ox = at.ox0 + p - ty * b.TW;
                     without_outside_taps<T>(OutsideTaps{ b.in, b.w, b.bias, b.out, b.g.IC * EB, b.g.IH, b.g.IW, b.g.OC, b.g.OH, b.g.OW, b.g.KH, b.g.KW, b.g.stride_y, b.g.stride_x, b.g.dil_y, b.g.dil_x, b.g.pad_top,
                                                          b.g.pad_left, b.g.bias_len },
-                                            p < b.TH * b.TW && oy < b.g.OH && ox < b.g.OW, n, oy, ox, oc0 + woc * OCT * 32 + 16 * (lane >> 5), OCT, 16);
+                                            p < b.TH * b.TW && oy < b.g.OH && ox < b.g.OW, at.n, oy, ox, c_w + 16 * (lane >> 5), OCT, 16);
                 }
             }
         }

@@ -8,8 +8,9 @@
 // [16,28,28,256]->64 3679 / 24 (16); GEMM kernel [4,28,28,224]->256 31 (18), bf16 [64,7,7,512]->512 90 (44); patch kernel [2,28,28,256]->250 53 (25); slab
 // kernel [8,56,56,64]->64 13.8 (5.9).
 // (Behind the loop and from arguments read anew it costs the loop a test of the results and no vector register: summed again in the loop, two channel
-// tiles a wave of conv_taps.hip fall from four waves a SIMD to two.  On finite values, over 36 layers of the patch and the GEMM kernel, 1.001 of the time
-// without any of this; the most, [4,100,130,128]->64 on the patch kernel, 29.0 / 29.8.  A workgroup's barrier in the patch kernel: layers of short rounds 2 to 4 % more.)
+// tiles a wave of conv_taps.hip fall from four waves a SIMD to two.  On finite values, over 15 layers of the GEMM kernel 1.002 of the time
+// without any of this, over 77 of the patch kernel 0.994, where arguments kept by way of LDS spare the loop's scalars; with its scalars kept across the stores bf16
+// [4,71,71,280]->136 58.2 / 63.4, so 56.3.  A workgroup's barrier in the patch kernel: layers of short rounds 2 to 4 % more.)
 #pragma once
 #include <type_traits>
 
@@ -53,6 +54,32 @@ __device__ __forceinline__ Args args_read_anew()
     asm volatile("" : "+s"(args));
     Args a;
     __builtin_memcpy(&a, (const void*)args, sizeof(a));
+    return a;
+}
+
+// The same, and the workgroup's number, by way of 16 bytes of LDS (written before the first barrier) where scalar registers are short up to the end
+__device__ __forceinline__ void keep_place(v4i* place)
+{
+    if (threadIdx.x == 0)
+    {
+        const uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+        *place              = v4i{ (int)(uint32_t)args, (int)(uint32_t)(args >> 32), (int)blockIdx.x, 0 };
+    }
+}
+template <typename Args>
+__device__ __forceinline__ Args args_kept(const v4i* place, uint32_t& block)
+{
+    const v4i p      = *place;
+    const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane(p[0]), h = (uint32_t)__builtin_amdgcn_readfirstlane(p[1]);
+    block            = (uint32_t)__builtin_amdgcn_readfirstlane(p[2]);
+    static_assert(sizeof(Args) % 4 == 0, "by words");
+    const auto* from = (const __attribute__((address_space(4))) uint32_t*)((uint64_t)h << 32 | l);
+    uint32_t words[sizeof(Args) / 4];
+#pragma unroll
+    for (int i = 0; i < (int)sizeof(Args) / 4; i++)
+        words[i] = from[i];
+    Args a;
+    __builtin_memcpy(&a, words, sizeof(a));
     return a;
 }
 
