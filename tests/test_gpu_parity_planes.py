@@ -15,7 +15,7 @@ SHAPES = [  # n, ih, iw, ic, oc, kh, kw, pad, stride, dilation
     (16, 28, 28, 256, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
     (10, 28, 30, 200, 56, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),     # channels of no whole slices, output channels cut
     (12, 30, 28, 520, 128, 1, 3, (0, 0, 1, 1), (1, 1), (1, 1)),    # three taps: the next patch stored in a slice's second stage
-    (24, 42, 23, 448, 56, 3, 1, (1, 1, 0, 0), (1, 1), (1, 1)),     # a window of one column
+    (24, 21, 23, 448, 136, 3, 1, (1, 1, 0, 0), (1, 1), (1, 1)),
     (9, 33, 41, 128, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1)),
     (12, 14, 14, 384, 264, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
     (14, 24, 28, 176, 56, 3, 3, (2, 2, 2, 2), (1, 1), (2, 2)),     # dilation
@@ -48,7 +48,8 @@ def test_small_whole_numbers(ctx, kind, shape):
     else:
         got, st = gpu_ops.conv2d(ctx, *(cases.float_to_bf16_bits(v.astype(np.float32)) for v in (x, w, bias)), pad, stride, dil, dtype=capi.BF16)
         want = cases.float_to_bf16_bits(want.astype(np.float32))
-    assert st == capi.VALID and ctx.last_kernel == ("conv2d_planes_f16" if kind == "fp16" else "conv2d_planes_bf16")
+    assert st == capi.VALID
+    print(shape, ctx.last_kernel)
     assert np.array_equal(got, want)
 
 
@@ -65,7 +66,7 @@ def test_infinite_weights_outside_the_image(ctx, shape):
     b = np.zeros(oc, np.float16)
     want, _ = gpu_ops.conv2d(ctx, x, plain, b, (1, 1, 1, 1), dtype=capi.FP16)
     got, st = gpu_ops.conv2d(ctx, x, w, b, (1, 1, 1, 1), dtype=capi.FP16)
-    assert st == capi.VALID and ctx.last_kernel == "conv2d_planes_f16"
+    assert st == capi.VALID
     # without a channel of the tap that lies outside: the results of finite weights there
     one = [c for c in range(oc) if c not in (3, 8, oc - 1)]
     assert np.array_equal(got[..., one], want[..., one])
@@ -81,7 +82,7 @@ I8_SHAPES = [  # the same for int8 with the fused RESCALE
     (9, 33, 41, 256, 72, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1)),
     (12, 30, 28, 768, 128, 1, 3, (0, 0, 1, 1), (1, 1), (1, 1)),
     (27, 40, 40, 400, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
-    (16, 29, 29, 640, 264, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1)),
+    (16, 29, 29, 512, 264, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1)),
 ]
 
 
@@ -100,5 +101,24 @@ def test_int8_rescale(ctx, shape, in_zp, double_round, clamp):
     if clamp:
         want = oracle.clamp(want, *clamp)
     got, st = gpu_ops.conv2d(ctx, x, w, bias, pad, stride, dil, in_zp=in_zp, rescale=dict(mult=mult, shift=shift, out_zp=5, rounding_mode=mode), clamp=clamp)
-    assert st == wst == capi.VALID and ctx.last_kernel == "conv2d_planes_i8_rescale"
+    assert st == wst == capi.VALID
     assert np.array_equal(got, want)
+
+
+# Which of them the kernel has, so that a change of its rule does not leave the tests above to others.  The window of one column on 448 channels
+# (161 pixels a tile) is the GEMM kernel's and the strided int8 layer on 512 channels a split reduction's; shapes that stay stand in for them.
+ELSEWHERE = [(24, 21, 23, 448, 136, 3, 1, (1, 1, 0, 0), (1, 1), (1, 1)), (16, 29, 29, 512, 264, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1))]
+
+
+@pytest.mark.parametrize("kind", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape", [s for s in SHAPES if s not in ELSEWHERE] + [(24, 42, 23, 448, 56, 3, 1, (1, 1, 0, 0), (1, 1), (1, 1))])
+def test_which_kernel(ctx, kind, shape):
+    test_small_whole_numbers(ctx, kind, shape)
+    assert ctx.last_kernel == ("conv2d_planes_f16" if kind == "fp16" else "conv2d_planes_bf16")
+
+
+@pytest.mark.parametrize("in_zp", [0, 17])
+@pytest.mark.parametrize("shape", [s for s in I8_SHAPES if s not in ELSEWHERE] + [(16, 29, 29, 640, 264, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1))])
+def test_which_kernel_int8(ctx, shape, in_zp):
+    test_int8_rescale(ctx, shape, in_zp, True, None)
+    assert ctx.last_kernel == "conv2d_planes_i8_rescale"
