@@ -23,7 +23,7 @@
 // The second kernel, for few tiles and a long reduction, splits K over the waves of a workgroup (see there).
 #include <type_traits>
 
-#include "tmi_mfma.h"
+#include "outside_taps.h"
 
 namespace tmi
 {
@@ -243,15 +243,8 @@ __device__ __forceinline__ void finish_taps(const TapsArgs& a, const TapsTables&
     }
 }
 
-// A tap outside the image adds nothing in the reference (tensor_ops.cpp:845-852); in the matrix instruction it adds zero times the
-// weight, which is NaN where the weight is infinite or NaN.  A wave that met a NaN in a layer with padding goes over its tiles once more
-// at the end, and sums results that are NaN and whose window leaves the image one at a time without those taps.  (Here, behind the
-// loop and from arguments read anew, it costs the loop a test of the results and no register: summed again in the loop, two channel
-// tiles a wave fall from four waves a SIMD to two.)
-__device__ __forceinline__ bool leaves_image(const TapsArgs& a, int y0, int x0)
-{
-    return y0 < 0 || x0 < 0 || y0 + (a.KH - 1) * a.dy >= a.IH || x0 + (a.KW - 1) * a.dx >= a.IW;
-}
+// Results that are NaN because of a tap outside the image (see outside_taps.h): a wave that met a NaN looks at its channels' weights behind its loop, and goes
+// over its tiles once more where one is infinite or NaN.
 template <int N, typename R>
 __device__ __forceinline__ bool any_nan(const R& v)
 {
@@ -261,46 +254,21 @@ __device__ __forceinline__ bool any_nan(const R& v)
         nan |= __builtin_isunordered(v[e], v[e + 1]);
     return __any(nan);
 }
-__device__ __forceinline__ TapsArgs args_read_anew()
+// `channels` of the weights from channel oc on, by all lanes of the wave
+template <typename T>
+__device__ __forceinline__ bool odd_weights(const TapsArgs& a, int oc, int channels)
 {
-    auto* args = __builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(args));    // (not the values the kernel began with, which would have to be kept)
-    TapsArgs a;
-    __builtin_memcpy(&a, (const void*)args, sizeof(a));
-    return a;
+    const int64_t row = (int64_t)a.KH * a.KW * a.row_bytes;
+    channels          = a.OC - oc < channels ? a.OC - oc : channels;
+    return channels > 0 && __any(weights_not_finite<T>(a.w + oc * row, channels * row, lane_counted(), 64));
 }
 // the lane's pixel p, `tiles` tiles of 32 channels of which it holds `each` from channel oc on
 template <typename T>
 __device__ __forceinline__ void sum_again(const TapsArgs& a, int p, int oc, int tiles, int each)
 {
-    if (p >= a.P)
-        return;
-    const int r = (int)fdiv((uint32_t)p, a.div_ow), n = (int)fdiv((uint32_t)r, a.div_oh), IC = a.row_bytes / 2;
-    const int y0 = (r - n * a.OH) * a.sy - a.pad_top, x0 = (p - r * a.OW) * a.sx - a.pad_left;
-    if (!leaves_image(a, y0, x0))
-        return;
-    T* out = reinterpret_cast<T*>(a.out) + (size_t)p * a.OC;
-#pragma unroll 1
-    for (int k = 0; k < tiles * each; k++)
-    {
-        const int c = oc + k / each * 32 + k % each;
-        if (c >= a.OC || load_as_float<T>(out, c) == load_as_float<T>(out, c))
-            continue;
-        float sum = 0.0f;
-#pragma unroll 1
-        for (int tap = 0; tap < a.KH * a.KW; tap++)
-        {
-            const int ky = (int)fdiv((uint32_t)tap, a.div_kw), y = y0 + ky * a.dy, x = x0 + (tap - ky * a.KW) * a.dx;
-            if ((unsigned)y >= (unsigned)a.IH || (unsigned)x >= (unsigned)a.IW)
-                continue;
-            const uint8_t* u = a.in + (uint32_t)(((n * a.IH + y) * a.IW + x) * a.row_bytes);
-            const uint8_t* w = a.w + (uint32_t)((c * a.KH * a.KW + tap) * a.row_bytes);
-#pragma unroll 1
-            for (int i = 0; i < IC; i++)
-                sum += load_as_float<T>(u, i) * load_as_float<T>(w, i);
-        }
-        store_from_float(out + c, sum + load_as_float<T>(a.bias, a.bias_len == 1 ? 0 : c));
-    }
+    const int r = (int)fdiv((uint32_t)p, a.div_ow), n = (int)fdiv((uint32_t)r, a.div_oh);
+    without_outside_taps<T>(OutsideTaps{ a.in, a.w, a.bias, a.out, a.row_bytes, a.IH, a.IW, a.OC, a.OH, a.OW, a.KH, a.KW, a.sy, a.sx, a.dy, a.dx, a.pad_top, a.pad_left, a.bias_len },
+                            p < a.P, n, r - n * a.OH, p - r * a.OW, oc, tiles, each);
 }
 
 // How channel vectors lie: whole chunks from 16 bytes on; anywhere, beginning with words; anywhere.
@@ -658,10 +626,18 @@ __global__ __launch_bounds__(kTapsWaves * 64, 2) void conv_taps_kernel(TapsArgs 
         raise_flags(a.flag_word, flags);
     else if (met_nan)
     {
-        __threadfence();    // (gathered rows were stored by other lanes)
-        const TapsArgs b = args_read_anew();
-        while ((pt -= pt_step) >= 0)
-            sum_again<T>(b, pt * 32 + li, oc0 + 16 * lh, OCT, 16);
+        const TapsArgs b = args_read_anew<TapsArgs>();
+        // (its channels' weights as they lie in LDS)
+        const uint8_t* w_lds = lds + taps_fixed_lds<OCT>() + 2 * b.steps * 8;
+        bool odd             = false;
+        for (int i = lane_counted(); i < OCB * b.chunks; i += 64)
+            odd |= not_finite<T>(*reinterpret_cast<const v4i*>(w_lds + i / OCB * PITCH + i % OCB * 16));
+        if (__any(odd))
+        {
+            __threadfence();    // (gathered rows were stored by other lanes)
+            while ((pt -= pt_step) >= 0)
+                sum_again<T>(b, pt * 32 + li, oc0 + 16 * lh, OCT, 16);
+        }
     }
 }
 
@@ -960,9 +936,10 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 4 : 2) void conv_taps_split_ker
         raise_flags(a.flag_word, flags);
     else if (met_nan)
     {
-        const TapsArgs b = args_read_anew();
-        while ((pt -= b.groups) >= 0)
-            sum_again<T>(b, pt * 32 + li, oc0 + 16 * lh + 4 * wave, 1, 4);
+        const TapsArgs b = args_read_anew<TapsArgs>();
+        if (odd_weights<T>(b, oc0 + 4 * wave, 4) || odd_weights<T>(b, oc0 + 16 + 4 * wave, 4))
+            while ((pt -= b.groups) >= 0)
+                sum_again<T>(b, pt * 32 + li, oc0 + 16 * lh + 4 * wave, 1, 4);
     }
 }
 

@@ -1,12 +1,13 @@
 // CONV2D results whose window leaves the image, on kernels that multiply what lies outside as zeros.
 //
 // A tap outside the image adds nothing in the reference (tensor_ops.cpp:845-852); zero times the weight is nothing too, unless the weight is infinite or
-// NaN.  A workgroup (the patch and the slab kernel: a wave) that met a sum that is NaN looks at its channels' weights behind its stores, once and with all
+// NaN.  A workgroup (the patch kernel, the slab kernel and those with resident weights: a wave) that met a sum that is NaN looks at its channels' weights behind its stores, once and with all
 // lanes side by side; where one is no number, its waves go over their tiles once more and sum one at a time, without those taps, the results that are NaN,
 // whose window leaves the image and whose channel has such a weight.  Every other result keeps the sum it has, and a NaN that came from the image costs
 // the look.  us a call on a NaN image, every NaN summed again / so (on finite values): streaming patch fp16 3x3 [7,14,21,200]->288 2600 / 23 (17), bf16
 // [16,28,28,256]->64 3679 / 24 (16); GEMM kernel [4,28,28,224]->256 31 (18), bf16 [64,7,7,512]->512 90 (44); patch kernel [2,28,28,256]->250 53 (25); slab
-// kernel [8,56,56,64]->64 13.8 (5.9).
+// kernel [8,56,56,64]->64 13.8 (5.9); resident weights fp16 [15,54,65,68]->64 1860 / 32 (24), bf16 [2,79,7,88]->23 276 / 9.4 (5.5); K split bf16 5x5 [2,14,13,200]->40
+// 1701 / 35 (15), fp16 stride 2 [9,31,41,240]->32 764 / 16 (8.7).  (A __threadfence() of every wave that met a NaN, before it knew of such a weight: 113 in the place of the 32.)
 // (Behind the loop and from arguments read anew it costs the loop a test of the results and no vector register: summed again in the loop, two channel
 // tiles a wave of conv_taps.hip fall from four waves a SIMD to two.  On finite values, over 15 layers of the GEMM kernel 1.002 of the time
 // without any of this, over 77 of the patch kernel 0.994, where arguments kept by way of LDS spare the loop's scalars; with its scalars kept across the stores bf16
@@ -83,22 +84,30 @@ __device__ __forceinline__ Args args_kept(const v4i* place, uint32_t& block)
     return a;
 }
 
+// Whether a word, 16 bytes of weights hold one that is infinite or NaN
+template <typename T>
+__device__ __forceinline__ bool not_finite(uint32_t word)
+{
+    constexpr uint32_t EXPONENT = sizeof(T) == 4 ? 0x7f800000u : (std::is_same_v<T, bf16_t> ? 0x7f80u : 0x7c00u);
+    return (word & EXPONENT) == EXPONENT || (sizeof(T) < 4 && (word >> 16 & EXPONENT) == EXPONENT);
+}
+template <typename T>
+__device__ __forceinline__ bool not_finite(const v4i& v)
+{
+    return not_finite<T>((uint32_t)v[0]) || not_finite<T>((uint32_t)v[1]) || not_finite<T>((uint32_t)v[2]) || not_finite<T>((uint32_t)v[3]);
+}
+
 // Whether the lane's part of the weights from w on, every parts-th 16 bytes from the part-th on, holds one that is infinite or NaN
 template <typename T>
 __device__ __forceinline__ bool weights_not_finite(const uint8_t* w, int64_t bytes, int part, int parts)
 {
-    constexpr uint32_t EXPONENT = sizeof(T) == 4 ? 0x7f800000u : (std::is_same_v<T, bf16_t> ? 0x7f80u : 0x7c00u);
-    auto odd = [](uint32_t word) { return (word & EXPONENT) == EXPONENT || (sizeof(T) < 4 && (word >> 16 & EXPONENT) == EXPONENT); };
     bool found          = false;
     const int64_t whole = bytes & ~(int64_t)15;
 #pragma unroll 8
     for (int64_t at = 16 * part; at < whole; at += 16 * parts)
-    {
-        const v4i v = load16(w + at);
-        found |= odd(v[0]) || odd(v[1]) || odd(v[2]) || odd(v[3]);
-    }
+        found |= not_finite<T>(load16(w + at));
     for (int64_t at = whole + part * (int)sizeof(T); at < bytes; at += parts * (int)sizeof(T))
-        found |= odd(sizeof(T) == 4 ? *reinterpret_cast<const uint32_t*>(w + at) : *reinterpret_cast<const uint16_t*>(w + at));
+        found |= not_finite<T>(sizeof(T) == 4 ? *reinterpret_cast<const uint32_t*>(w + at) : (uint32_t)*reinterpret_cast<const uint16_t*>(w + at));
     return found;
 }
 

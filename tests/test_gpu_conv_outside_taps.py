@@ -28,6 +28,11 @@ CASES = [  # kernel, kernel choice, n, ih, iw, ic, oc, k, stride, dilation
     ("conv2d_slab_bf16", 0, 4, 29, 29, 48, 96, 3, 2, 1),
     ("conv2d_slab_f16", 4, 1, 9, 9, 32, 48, 3, 1, 1),              # half a block of channels
     ("conv2d_slab_bf16", 0, 8, 28, 28, 256, 128, 1, 1, 1),
+    ("conv2d_taps_f16", 0, 15, 54, 65, 68, 64, 3, 1, 1),           # weights resident, two tiles of channels
+    ("conv2d_taps_bf16", 0, 2, 79, 7, 88, 23, 3, 1, 1),
+    ("conv2d_taps_f16", 0, 9, 31, 41, 240, 32, 3, 2, 1),           # K split
+    ("conv2d_taps_bf16", 0, 2, 14, 13, 200, 40, 5, 1, 1),
+    ("conv2d_taps_f16", 0, 2, 12, 11, 45, 48, 3, 1, 2),            # rows between words
 ]
 
 
