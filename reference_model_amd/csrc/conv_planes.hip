@@ -492,6 +492,9 @@ static bool planes_take(int32_t in_dtype, const ConvGeom& g)
 //   int8 with RESCALE, where the patch kernel has the layer, at most a third of the slices cut off: [8,29,29,208]->248 19.8 / 13.1, [14,30,30,592]->96 30.9 / 23.1, [4,31,36,480]->240 25.7 / 19.6, 5x5
 //     [18,20,20,624]->64 85 / 48; over 36 of them 0.56 ... 0.94; beyond a third [3,61,61,160]->176 19.0 / 17.8, [10,25,94,176]->64 12.7 / 13.4.  The kernels with resident weights
 //     or split reductions keep theirs: of 83 layers 9 gained, [11,7,8,416]->616 10.4 / 17.8, [8,30,86,160]->128 14.4 / 18.0.
+//   Up to 32 channels on tiles of more than 128 pixels, half of whose matrix instructions have no channel: the patch kernel keeps int8 and rows of less than 600 bytes.  Over 69
+//     and 40 drawn layers of these here 1.07 and 1.10 of its time: int8 [21,48,48,192]->32 11.6 / 16.2, [13,34,89,192]->8 12.4 / 16.4, bf16 [16,55,55,96]->32 10.9 / 15.1, fp16
+//     [9,71,71,80]->32 10.4 / 13.7; the most given up bf16 5x5 [23,35,35,128]->32 25.1 / 22.9, int8 [14,46,46,624]->16 30.3 / 28.1.  Longer rows 0.92 over 30: [31,52,22,512]->16 39.9 / 32.8.
 bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, bool to_gemm)
 {
     if (!planes_take(in_dtype, g))
@@ -499,6 +502,8 @@ bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, bool to_gemm)
     const int eb       = in_dtype == TMI_INT8 ? 1 : 2;
     const PlanesPlan p = plan_planes(g, eb);
     if (p.rows == 0 || p.tiles > 256 || p.slices * g.KH * g.KW < 18)
+        return false;
+    if (p.wide && g.OC <= 32 && (in_dtype == TMI_INT8 || g.IC * eb < 600))
         return false;
     if (in_dtype == TMI_INT8)
         return p.slices * 128 * 3 <= (int64_t)g.IC * 4;

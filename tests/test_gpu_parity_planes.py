@@ -122,3 +122,25 @@ def test_which_kernel(ctx, kind, shape):
 def test_which_kernel_int8(ctx, shape, in_zp):
     test_int8_rescale(ctx, shape, in_zp, True, None)
     assert ctx.last_kernel == "conv2d_planes_i8_rescale"
+
+
+@pytest.mark.parametrize("kind, shape, kernel", [  # n, h, w, ic, oc, k, stride
+    # up to 32 output channels on tiles of more than 128 pixels: the patch kernel's, but for long rows of 16-bit floats
+    ("int8", (21, 48, 48, 192, 32, 3, 1), "conv2d_mfma_i8_rescale"),
+    ("int8", (13, 34, 89, 192, 8, 3, 1), "conv2d_mfma_i8_rescale"),
+    ("bf16", (16, 55, 55, 96, 32, 3, 1), "conv2d_mfma_bf16"),
+    ("fp16", (9, 71, 71, 80, 32, 3, 1), "conv2d_mfma_f16"),
+    ("fp16", (5, 52, 22, 512, 16, 3, 1), "conv2d_taps_f16"),
+    ("fp16", (31, 52, 22, 512, 16, 3, 1), "conv2d_planes_f16"),
+    ("bf16", (16, 55, 55, 96, 40, 3, 1), "conv2d_planes_bf16"),
+])
+def test_layers_it_leaves(ctx, kind, shape, kernel):
+    n, h, w, ic, oc, k, s = shape
+    p = k // 2
+    pad = (p, p - (h + 2 * p - k) % s, p, p - (w + 2 * p - k) % s)
+    case = (n, h, w, ic, oc, k, k, pad, (s, s), (1, 1))
+    if kind == "int8":
+        test_int8_rescale(ctx, case, 17, True, None)
+    else:
+        test_small_whole_numbers(ctx, kind, case)
+    assert ctx.last_kernel == kernel
