@@ -487,6 +487,9 @@ static bool planes_take(int32_t in_dtype, const ConvGeom& g)
 //     [22,75,13,288]->144 stride 2 27.6 / 34.6; 9 stages: [20,50,50,64]->72 stride 2 11.5 / 13.3, [11,28,28,32]->104 5.9 / 7.6.
 //   split reductions (conv_taps.hip), from 106 TFLOP/s predicted on: [2,18,18,384]->448 (115) 26.4 / 17.9, [2,54,54,512]->48 (107) 33.9 / 23.2, [7,14,21,200]->288 19.9 / 14.7, the least
 //     gain [1,85,85,88]->96 (108) 11.5 / 11.6; below [4,14,14,448]->320 (103) 17.1 / 19.8, [3,25,25,600]->128 (98) 23.2 / 28.1, [3,14,14,512]->160 (39) 18.6 / 21.1.
+//     Where the last slice is cut off (its stages choose every source) and four fifths of their last round of tiles are filled, they keep theirs: over 49 drawn layers here 1.07 of their time,
+//     [9,14,61,136]->328 stride 2 (682 tiles) 11.1 / 14.5, 5x5 [11,23,8,88]->216 (448) 14.2 / 18.4, [4,47,8,144]->320 (470) 9.9 / 12.1; the most given up [6,26,42,120]->384 stride 2 (624) 14.3 / 11.7.
+//     Less filled 0.88 over 55, [12,96,21,176]->96 stride 2 (594) 21.0 / 13.5; the most lost [7,16,16,208]->216 (392) 12.1 / 15.1.
 //   the GEMM kernel, only with tiles of up to 128 pixels and whole slices: [14,22,22,384]->176 31.8 / 18.8, 5x5 [24,52,10,64]->128 15.2 / 10.6, [10,22,22,128]->296 20.7 / 17.7; else
 //     [16,28,28,256]->256 (196 pixels) 20.2 / 21.5, [16,40,15,160]->136 (two and a half slices) 12.6 / 13.0.
 //   int8 with RESCALE, where the patch kernel has the layer, at most a third of the slices cut off: [8,29,29,208]->248 19.8 / 13.1, [14,30,30,592]->96 30.9 / 23.1, [4,31,36,480]->240 25.7 / 19.6, 5x5
@@ -495,7 +498,7 @@ static bool planes_take(int32_t in_dtype, const ConvGeom& g)
 //   Up to 32 channels on tiles of more than 128 pixels, half of whose matrix instructions have no channel: the patch kernel keeps int8 and rows of less than 600 bytes.  Over 69
 //     and 40 drawn layers of these here 1.07 and 1.10 of its time: int8 [21,48,48,192]->32 11.6 / 16.2, [13,34,89,192]->8 12.4 / 16.4, bf16 [16,55,55,96]->32 10.9 / 15.1, fp16
 //     [9,71,71,80]->32 10.4 / 13.7; the most given up bf16 5x5 [23,35,35,128]->32 25.1 / 22.9, int8 [14,46,46,624]->16 30.3 / 28.1.  Longer rows 0.92 over 30: [31,52,22,512]->16 39.9 / 32.8.
-bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, bool to_gemm)
+bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, PlanesRival rival)
 {
     if (!planes_take(in_dtype, g))
         return false;
@@ -507,10 +510,16 @@ bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, bool to_gemm)
         return false;
     if (in_dtype == TMI_INT8)
         return p.slices * 128 * 3 <= (int64_t)g.IC * 4;
-    if (to_gemm)
+    if (rival == PLANES_GEMM)
         return !p.wide && g.IC * eb % 128 == 0;
     if (p.slices == 1 && g.IC * eb < 128)    // (a slice cut short and no other under which a patch is fetched: 5x5 [5,47,47,48]->48 10.2 / 11.9)
         return false;
+    if (rival == PLANES_SPLIT && !p.wide && g.IC * eb % 128 != 0)
+    {
+        const int64_t tiles = (((int64_t)g.N * g.OH * g.OW + 31) / 32) * ((g.OC + 31) / 32);    // of 32 x 32 results, a workgroup each
+        if (tiles * 5 >= (tiles + 255) / 256 * 256 * 4)
+            return false;
+    }
     return 2e-6 * (double)g.N * g.OH * g.OW * g.OC * g.IC * g.KH * g.KW >= 106 * p.us;
 }
 

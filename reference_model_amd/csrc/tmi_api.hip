@@ -654,6 +654,8 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
     const int32_t t_row   = g.IC * (d->in_dtype == TMI_INT8 ? 1 : 2);
     const int64_t t_steps = ((int64_t)g.KH * g.KW * ((t_row + 15) / 16) + 1) / 2;
     const int64_t t_tiles = ((total / g.OC + 31) / 32) * ((g.OC + 31) / 32);
+    // long reductions over many tiles, which it leaves to the patch kernel (measured below)
+    auto long_reduction = [&](int64_t steps) { return steps >= 90 && t_tiles > (steps >= 140 ? 380 : (steps >= 120 ? 480 : 700)); };
     auto launch_taps = [&]() {
         return launch_conv2d_taps(ctx->stream, d->in_dtype, out_dtype, g, in, w, bias, in_zp, w_zp, rp, out,
                                   ctx->pages_dev + (d->in_dtype == TMI_INT8 ? (in_zp & 255) * 64 : 0), ctx->flags_dev);
@@ -673,7 +675,8 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         const int64_t pixels  = (int64_t)g.N * g.OH * g.OW;
         const bool to_gemm    = !i8 && row_bytes % 64 == 0 && g.OC >= 64 && pixels >= 128 && gemm_mfma_preferred(d->in_dtype, seen) &&
                              (gemm_patch_form(seen, d->in_dtype) || (pixels + 127) / 128 * ((g.OC + 127) / 128) >= 96);
-        if (!conv_planes_leads(d->in_dtype, seen, to_gemm) ||
+        const bool to_split   = !to_gemm && t_tiles <= 700 && !long_reduction(((int64_t)g.KH * g.KW * ((row_bytes + 15) / 16) + 1) / 2);
+        if (!conv_planes_leads(d->in_dtype, seen, to_gemm ? PLANES_GEMM : (to_split ? PLANES_SPLIT : PLANES_PATCH)) ||
             !launch_conv_planes(ctx->stream, d->in_dtype, g, in, w, bias, ctx->pages_dev + (i8 ? (in_zp & 255) * 64 : 0), ctx->pages_dev, in_zp, rp, ctx->flags_dev, out))
             return;
         name = i8 ? "conv2d_planes_i8_rescale" : f16 ? "conv2d_planes_f16" : "conv2d_planes_bf16";
@@ -895,7 +898,7 @@ int run_conv(tmi_ctx* ctx, const char* op, bool depthwise, const tmi_conv_desc_t
         // (1364, 99) 23.4 / 34, [4,72,32,288]->48 bf16 (576, 162) 23.4 / 24.5) and layers with taps of 700 ... 2400 tiles whose rows are whole words, where its one round of large tiles
         // is well filled ([5,93,77,64]->56 fp16 12.5 / 16.8, [10,50,50,56]->56 5x5 14.4 / 17.8, [59,15,15,24]->96 5x5 9.9 / 11.8, [4,106,106,16]->32
         // 5.5 / 6.8; the other way [14,92,75,48]->48 fp16 stride 2 11.3 / 7.8, [4,28,33,16]->264 8.1 / 5.4).
-        const bool long_and_many = t_steps >= 90 && t_tiles > (t_steps >= 140 ? 380 : (t_steps >= 120 ? 480 : 700));
+        const bool long_and_many = long_reduction(t_steps);
         const bool patch_filled  = g.KH * g.KW > 1 && t_tiles > 700 && t_tiles <= (t_steps >= 64 ? 3400 : 2400) && t_row % 8 == 0 && g.OC % 8 == 0;
         // 16-bit rows of a few words, filled up to 16 bytes a tap here and as they are there, from the same border on.  us patch kernel / this one: 3x3
         // [6,91,61,4]->96 7.2 / 10.6, [9,30,14,10]->224 5.9 / 7.5, 5x5 [7,51,60,6]->56 6.6 / 9.0, [46,12,10,2]->224 6.6 / 9.3, 7x7 [8,60,60,10]->64 11.9 / 21.2, 1x1 [3,87,100,12]->8 4.4 / 4.9; the

@@ -152,8 +152,14 @@ OrderedForm launch_ordered_conv(hipStream_t st, int32_t in_dtype, bool f64, cons
 OrderedForm launch_ordered_matmul(hipStream_t st, int32_t in_dtype, bool f64, int32_t N, int32_t H, int32_t C, int32_t W, const void* a,
                            const void* b, bool abs_mode, void* out);
 // conv_planes.hip: CONV2D with taps on 16-bit floats (results of the same type) or int8 (weights' zero point 0, fused RESCALE to int8 in its fast form);
-// pad_page: 16 bytes of in_zp, zeros: 16 zero bytes.  False: not taken.  _leads: whether it should be; to_gemm: the layer is the GEMM kernel's otherwise.
-bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, bool to_gemm);
+// pad_page: 16 bytes of in_zp, zeros: 16 zero bytes.  False: not taken.  _leads: whether it should be; rival: the kernel that has the layer otherwise.
+enum PlanesRival
+{
+    PLANES_PATCH,    // conv2d_mfma.hip
+    PLANES_GEMM,     // gemm_mfma.hip
+    PLANES_SPLIT     // conv_taps.hip
+};
+bool conv_planes_leads(int32_t in_dtype, const ConvGeom& g, PlanesRival rival);
 bool launch_conv_planes(hipStream_t st, int32_t in_dtype, const ConvGeom& g, const void* in, const void* w, const void* bias, const void* pad_page,
                         const void* zeros, int32_t in_zp, const RescaleParams& rp, uint32_t* flag_word, void* out);
 // ordered_staged.hip: the same for CONV2D on whole units of eight channels; false: not launched.  _leads: whether a layer runs there.

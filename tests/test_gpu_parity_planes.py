@@ -133,6 +133,12 @@ def test_which_kernel_int8(ctx, shape, in_zp):
     ("fp16", (5, 52, 22, 512, 16, 3, 1), "conv2d_taps_f16"),
     ("fp16", (31, 52, 22, 512, 16, 3, 1), "conv2d_planes_f16"),
     ("bf16", (16, 55, 55, 96, 40, 3, 1), "conv2d_planes_bf16"),
+    # a slice cut off, and the split reductions' last round of tiles four fifths full; less full, or whole slices
+    ("bf16", (9, 14, 61, 136, 328, 3, 2), "conv2d_taps_bf16"),
+    ("fp16", (11, 23, 8, 88, 216, 5, 1), "conv2d_taps_f16"),
+    ("fp16", (4, 47, 8, 144, 320, 3, 1), "conv2d_taps_f16"),
+    ("fp16", (12, 96, 21, 176, 96, 3, 2), "conv2d_planes_f16"),
+    ("fp16", (3, 76, 20, 128, 104, 3, 1), "conv2d_planes_f16"),
 ])
 def test_layers_it_leaves(ctx, kind, shape, kernel):
     n, h, w, ic, oc, k, s = shape
