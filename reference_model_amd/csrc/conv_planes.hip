@@ -6,7 +6,7 @@
 // stage.  Two groups of four waves take half of a stage's channels each, so that a wave owns 64 channels x IT * 32 pixels and reads four (IT 1: three)
 // fragments for four (two) matrix instructions; after the loop a wave hands half of its sums to its partner.
 //
-// What bounds it: on few tiles the instructions of a stage (0.21 us, 0.11 of it matrix instructions; 0.41 of 0.21 with 256 pixels), on all CUs the clock under the
+// What bounds it: on few tiles the instructions of a stage (0.21 us, of which its matrix instructions are 0.11; with 256 pixels 0.41 and 0.21), on all CUs the clock under the
 // matrix instructions: [16,28,28,256]->256 3x3 14.9 us without any operand in the loop, 18.8 with its fragment reads.  A wave's loads straight into LDS go
 // one after the other, 0.3 us each, so the second group fetches the patch through registers (all loads straight into LDS: 26.2, so 21.5), in a loop of its own,
 // or the compiler has the first group wait for them too (28.9).
@@ -482,7 +482,7 @@ static bool planes_take(int32_t in_dtype, const ConvGeom& g)
 }
 
 // Whether a layer runs here: one round of workgroups and 18 stages or more.  us the kernel it would go to / here, 3x3 unless noted:
-//   the patch kernel (conv2d_mfma.hip): [16,14,14,512]->512 40.1 / 24.2, [16,28,28,256]->64 20.7 / 13.4, [26,10,22,376]->160 32.8 / 20.8, 5x5 [2,20,20,480]->592 129 / 53,
+//   the patch kernel (conv2d_mfma.hip): [16,28,28,256]->64 20.7 / 13.4, [26,10,22,376]->160 32.8 / 20.8, 5x5 [2,20,20,480]->592 129 / 53,
 //     [11,58,21,96]->96 30.9 / 19.3, stride 2 [14,36,28,328]->240 46.9 / 22.7; over 34 of them 0.41 ... 0.96.  Two rounds: [4,29,109,136]->136 19.7 / 26.9,
 //     [22,75,13,288]->144 stride 2 27.6 / 34.6; 9 stages: [20,50,50,64]->72 stride 2 11.5 / 13.3, [11,28,28,32]->104 5.9 / 7.6.
 //   split reductions (conv_taps.hip), from 106 TFLOP/s predicted on: [2,18,18,384]->448 (115) 26.4 / 17.9, [2,54,54,512]->48 (107) 33.9 / 23.2, [7,14,21,200]->288 19.9 / 14.7, the least
@@ -490,7 +490,7 @@ static bool planes_take(int32_t in_dtype, const ConvGeom& g)
 //     Where the last slice is cut off (its stages choose every source) and four fifths of their last round of tiles are filled, they keep theirs: over 49 drawn layers here 1.07 of their time,
 //     [9,14,61,136]->328 stride 2 (682 tiles) 11.1 / 14.5, 5x5 [11,23,8,88]->216 (448) 14.2 / 18.4, [4,47,8,144]->320 (470) 9.9 / 12.1; the most given up [6,26,42,120]->384 stride 2 (624) 14.3 / 11.7.
 //     Less filled 0.88 over 55, [12,96,21,176]->96 stride 2 (594) 21.0 / 13.5; the most lost [7,16,16,208]->216 (392) 12.1 / 15.1.
-//   the GEMM kernel, only with tiles of up to 128 pixels and whole slices: [14,22,22,384]->176 31.8 / 18.8, 5x5 [24,52,10,64]->128 15.2 / 10.6, [10,22,22,128]->296 20.7 / 17.7; else
+//   the GEMM kernel, only with tiles of up to 128 pixels and whole slices: [14,22,22,384]->176 31.8 / 18.8, [16,14,14,512]->512 40.1 / 24.2, 5x5 [24,52,10,64]->128 15.2 / 10.6, [10,22,22,128]->296 20.7 / 17.7; else
 //     [16,28,28,256]->256 (196 pixels) 20.2 / 21.5, [16,40,15,160]->136 (two and a half slices) 12.6 / 13.0.
 //   int8 with RESCALE, where the patch kernel has the layer, at most a third of the slices cut off: [8,29,29,208]->248 19.8 / 13.1, [14,30,30,592]->96 30.9 / 23.1, [4,31,36,480]->240 25.7 / 19.6, 5x5
 //     [18,20,20,624]->64 85 / 48; over 36 of them 0.56 ... 0.94; beyond a third [3,61,61,160]->176 19.0 / 17.8, [10,25,94,176]->64 12.7 / 13.4.  The kernels with resident weights
